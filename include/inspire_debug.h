@@ -91,8 +91,8 @@ int ipir_dbg_set_group_chunk(ipir_server* srv, size_t groups);
  * overrides it). 1 for values outside 0..3. */
 int ipir_dbg_set_tail_split(ipir_server* srv, int on);
 /* Select the Horner kernel a server's answers use: mode as variant above,
- * or -1 (the default) to use the pair only for serial answers with at most
- * two chains. Whatever the mode, the asynchronous device entry points
+ * or -1 (the default): one workgroup per chain, the faster one. Whatever
+ * the mode, the asynchronous device entry points
  * (ipir_answer_batch_device, ipir_answer_batch_packed_device) never use the
  * pair: its bounded wait reports through a status word that only the
  * blocking entry points and the serving loop read. */

@@ -10,6 +10,7 @@
 // acc = ext_prod(rgsw, acc) + packed[i] (src/gpu_online.cu:474-540). All
 // arithmetic is exact, so results equal the reference's bit for bit.
 #include "kernels.h"
+#include "ntt_regs.h"
 
 namespace ipx {
 
@@ -171,43 +172,64 @@ __global__ __launch_bounds__(1024) void k_pack_finalize_wg(const uint32_t* __res
 }
 
 // ------------------------------------------------------------ Horner chain
-// One workgroup per (response ciphertext, query); 4 teams of 256 lanes.
-// acc (a0, a1, b0, b1 polys, NTT form) lives in registers between steps;
-// per step: 4 INTTs, gadget split, 2 rounds of 4 NTTs, multiply-accumulate
-// against the query's RGSW rows, + packed[i]. L == 1 copies packed[start].
-// The RGSW rows are loaded once and kept in registers across steps; the
-// step's packed parts are loaded during round 0, a phase ahead of their
-// use, so HBM latency (long while a database pass streams through L2) hides
-// behind the round-1 transforms. STREAMED: beside a streamed pack, each
-// step first waits for its group's packed b-part (StreamWait).
+// One workgroup per (response ciphertext, query), two teams of 256 lanes,
+// one per limb. Per step (acc <- ext_prod(rgsw, acc) + packed[i]) a team
+// takes its limb's a and b parts from NTT form to coefficients, the teams
+// swap halves of the CRT lift through LDS so that each coefficient is
+// lifted and cut into digits once, and a team transforms the four digit
+// polynomials mod its prime together and multiplies them with the query's
+// RGSW rows. A lane holds the same 8 slots of every polynomial at both ends
+// of the transforms (ntt_regs.h), so the accumulators, the products and the
+// rows stay in registers and a step has 8 barriers. L == 1 copies
+// packed[start].
+// Bound: VALU issue of one CU (a serial chain; its workgroup has two waves
+// per SIMD with the four polynomials as independent work). One team of 256
+// lanes per polynomial (16 waves, every transform through LDS with folded
+// butterflies, products and digits exchanged through LDS: 20 barriers)
+// took 16.6 us per step alone, this form takes 8.7 (two chains of 256 groups
+// for 3 queries: 4245 and 2214 us).
+// The rows are kept times 2^32 so the four products of a slot are brought
+// back with one Montgomery step (2 instructions); the accumulators stay
+// below 5q and are made canonical where they leave the kernel.
+// The step's packed parts load while the digits are transformed. STREAMED:
+// beside a streamed pack the chain needs a group only where it adds the
+// group's b-part, so it waits for it (StreamWait) before the step's last
+// phase.
+struct HornerChain {
+    const uint32_t* pa_base;
+    size_t pa_stride;
+    uint32_t G, Da, T;
+    uint32_t* packed_b;
+    size_t pstride;
+    const uint32_t* rgsw;
+    size_t rstride;
+    uint64_t* out;
+    uint32_t* hstate;
+    uint32_t g_lo, g_hi;
+};
+
 template <bool STREAMED>
-__global__ __launch_bounds__(1024) void k_horner(const uint32_t* __restrict__ pa_base, size_t pa_stride, uint32_t G, uint32_t Da,
-                                                 uint32_t T, uint32_t* packed_b,
-                                                 size_t pstride, const uint32_t* __restrict__ rgsw,
-                                                 size_t rstride, uint64_t* __restrict__ out,
-                                                 uint32_t* __restrict__ hstate, uint32_t g_lo, uint32_t g_hi,
-                                                 NttConst nc, CrtConst cc, FusedPack fp, StreamWait sw) {
-    __shared__ uint32_t buf[4][POLY_LDS];
-    __shared__ uint32_t twl[8 * N];
+__global__ __launch_bounds__(512, 2) void k_horner(HornerChain h, NttConst nc, NrGadget gc, FusedPack fp,
+                                                   StreamWait sw) {
+    __shared__ __align__(16) uint32_t buf[2][4][POLY4_LDS];  // [limb][a, b or the four digit polynomials]
+    __shared__ __align__(16) nr_u32x2 tw2[2][N];
+    __shared__ uint32_t dx[2][8][2][256];  // digits by the team that made them: [4a + .., 4b + ..][d1, d2][lane]
     __shared__ uint32_t sw_abort;
-    const uint32_t ct = blockIdx.x, qi = blockIdx.y, tid = threadIdx.x;
-    const uint32_t team = tid >> 8, t = tid & 255;
-    const uint32_t start = ct * Da;
-    const uint32_t L = (G - start) < Da ? (G - start) : Da;
+    const uint32_t ct = blockIdx.x, qi = blockIdx.y, tid = threadIdx.x, t = tid & 255;
+    const int c = __builtin_amdgcn_readfirstlane((int)(tid >> 8));  // this team's limb
+    const uint32_t start = ct * h.Da;
+    const uint32_t L = (h.G - start) < h.Da ? (h.G - start) : h.Da;
     const uint32_t top = start + L - 1;
     // this launch covers the chain's groups in [lo, hi), highest first
-    const uint32_t lo = start > g_lo ? start : g_lo, hi = start + L < g_hi ? start + L : g_hi;
+    const uint32_t lo = start > h.g_lo ? start : h.g_lo, hi = start + L < h.g_hi ? start + L : h.g_hi;
     if (lo >= hi) return;
-    stage_twiddles(twl, nc, tid, 1024);
-    const int tlimb = (int)(team & 1);
-    const Tw tw = tw_lds(twl, tlimb);
-    const uint32_t inv_n = nc.inv_n[tlimb], inv_n_p = nc.inv_n_p[tlimb];
-    // Beside a streamed pack: wait until this chain's packed b-part of
-    // group g is published (lane 0 spins and acquires, then the block
-    // meets at a barrier; the hand-over rules in dev_common.h).
-    // False: the wait exceeded its bound (every lane returns the same).
+    const NrLimb m = nr_limb(c);
+    // Beside a streamed pack: lane 0 waits until this chain's packed b-part
+    // of group g is published and acquires (the hand-over rules in
+    // dev_common.h); the caller's next barrier publishes sw_abort, set where
+    // the wait exceeded its bound.
     const uint32_t* sw_done = sw.done + (size_t)(qi / sw.queries) * sw.stride;
-    auto wait_packed = [&](uint32_t g) -> bool {
+    auto wait_packed = [&](uint32_t g) {
         if (tid == 0) {
             uint32_t spins = 0, ab = 0;
             while (sw.spin_limit == 0 ||
@@ -222,179 +244,179 @@ __global__ __launch_bounds__(1024) void k_horner(const uint32_t* __restrict__ pa
             fence_acquire_agent_done();
             sw_abort = ab;
         }
-        __syncthreads();
-        return !sw_abort;
     };
-    constexpr bool streamed = STREAMED;
-    uint64_t* o = out + ((size_t)qi * T + ct) * 4 * N;
+    uint64_t* o = h.out + ((size_t)qi * h.T + ct) * 4 * N;
     auto poison = [&]() {  // an invalid response: no residue is all-ones
-#pragma unroll
-        for (int p = 0; p < 4; p++)
-#pragma unroll
-            for (int e = 0; e < 2; e++) o[(size_t)p * N + tid + 1024 * e] = ~0ull;
+        for (uint32_t x = tid; x < 4 * N; x += 512) o[x] = ~0ull;
     };
+    uint32_t* pbw = h.packed_b + qi * h.pstride;
     if (fp.interm) {
-        // this chain's packed b-parts of groups [lo, hi): team k%4 takes
-        // (group lo + k/2, limb k%2), the limb of its own twiddles (as
-        // k_pack_finalize_wg); written to packed_b and read back below
+        // this chain's packed b-parts of groups [lo, hi), team c the limb c
+        // (as k_pack_finalize): written to packed_b and read back below
         // after the block's barrier
-        const uint32_t npoly = 2 * (hi - lo), rounds = (npoly + 3) / 4;
-        uint32_t* b = buf[team];
-        for (uint32_t r = 0; r < rounds; r++) {  // every lane runs every round (barriers inside)
-            const uint32_t k = 4 * r + team;
-            const bool active = k < npoly;
-            const uint32_t g = lo + (active ? k >> 1 : 0), c = k & 1;
-            __syncthreads();  // twiddles staged, the previous round's reads done
-            if (active) {
-                const uint32_t* src = fp.interm + (size_t)qi * 2 * fp.C + (size_t)c * fp.C + (size_t)g * N;
+        const Tw gtw = tw_global(nc, c);
+        uint32_t* b = buf[c][0];
+        for (uint32_t g = lo; g < hi; g++) {  // every lane runs every round (barriers inside)
+            const uint32_t* src = fp.interm + (size_t)qi * 2 * fp.C + (size_t)c * fp.C + (size_t)g * N;
 #pragma unroll
-                for (int e = 0; e < 8; e++) b[ls(t + 256 * e)] = src[t + 256 * e];
+            for (int e = 0; e < 8; e++) b[ls(t + 256 * e)] = src[t + 256 * e];
+            __syncthreads();
+            ntt_fwd_lds(b, t, gtw, c);
+            const uint32_t* Df = fp.precomp + (size_t)g * PC_GROUP + PC_DF + (size_t)c * D_EFF * N;
+            const uint32_t* Kn = fp.keys + qi * fp.keys_stride + BLK + (size_t)c * N;
+            const uint32_t* p2 = fp.part2 + qi * fp.part2_stride + (size_t)g * 2 * N + (size_t)c * N;
+#pragma unroll 2
+            for (int e = 0; e < 8; e++) {
+                const uint32_t i = t + 256 * e;
+                const uint64_t sub = (uint64_t)Df[i] * Kn[i] + (uint64_t)Df[N + i] * Kn[2 * N + i] + p2[i];
+                pbw[(size_t)g * 2 * N + (size_t)c * N + i] = sub_mod(b[ls(i)], red64(sub, c), m.q);
             }
             __syncthreads();
-            ntt_fwd_lds(b, t, tw, (int)c, active);
-            if (active) {
-                const uint32_t q = qof((int)c);
-                const uint32_t* Df = fp.precomp + (size_t)g * PC_GROUP + PC_DF + (size_t)c * D_EFF * N;
-                const uint32_t* Kn = fp.keys + qi * fp.keys_stride + BLK + (size_t)c * N;
-                const uint32_t* p2 = fp.part2 + qi * fp.part2_stride + (size_t)g * 2 * N + (size_t)c * N;
-#pragma unroll 2
-                for (int e = 0; e < 8; e++) {
-                    const uint32_t i = t + 256 * e;
-                    const uint64_t sub = (uint64_t)Df[i] * Kn[i] + (uint64_t)Df[N + i] * Kn[2 * N + i] + p2[i];
-                    packed_b[qi * pstride + (size_t)g * 2 * N + (size_t)c * N + i] =
-                        sub_mod(b[ls(i)], red64(sub, (int)c), q);
-                }
-            }
         }
-        __syncthreads();  // the block's packed parts are in place
     }
-    const uint32_t* pb = packed_b + qi * pstride;
-    const uint32_t* rg = rgsw + qi * rstride;
-    uint32_t* hs = hstate + ((size_t)qi * T + ct) * 4 * N;  // chain state between launches
-    uint32_t acc[4][2];
+    const uint32_t* pb = pbw;
+    const uint32_t* rg = h.rgsw + qi * h.rstride;
+    uint32_t* hs = h.hstate + ((size_t)qi * h.T + ct) * 4 * N;  // chain state between launches
+    // 8 consecutive slots of this lane's limb
+    auto load8 = [&](uint32_t (&x)[8], const uint32_t* p) {
+        const u32x4* s = reinterpret_cast<const u32x4*>(p + (size_t)c * N + 8 * t);
+        const u32x4 l = s[0], u = s[1];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            x[k] = l[k];
+            x[k + 4] = u[k];
+        }
+    };
+    uint32_t acc[2][8];  // a and b part, slots 8t + k
     int first;
-    if (top < g_hi) {  // the chain starts here: acc = packed[top]
-        if constexpr (streamed)
-            if (!wait_packed(top)) {
+    if (top < h.g_hi) {  // the chain starts here: acc = packed[top]
+        if constexpr (STREAMED) {
+            wait_packed(top);
+            __syncthreads();
+            if (sw_abort) {
                 poison();
                 return;
             }
-        const uint32_t* pa = pa_base + (size_t)top * pa_stride;
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const uint32_t i = tid + 1024 * e;
-            acc[0][e] = pa[i]; acc[1][e] = pa[N + i];
-            acc[2][e] = pb[(size_t)top * 2 * N + i]; acc[3][e] = pb[(size_t)top * 2 * N + N + i];
         }
+        load8(acc[0], h.pa_base + (size_t)top * h.pa_stride);
+        load8(acc[1], pb + (size_t)top * 2 * N);
         first = (int)top - 1;
     } else {
-#pragma unroll
-        for (int p = 0; p < 4; p++)
-#pragma unroll
-            for (int e = 0; e < 2; e++) acc[p][e] = hs[(size_t)p * N + tid + 1024 * e];
+        load8(acc[0], hs);
+        load8(acc[1], hs + 2 * N);
         first = (int)hi - 1;
     }
-    // the query's RGSW rows [round][c][e][j] (round 0: top_a / top_b, round
-    // 1: bot_a / bot_b), the same for every step: loaded once, kept in
-    // registers across the steps
-    uint32_t rA[2][2][2][2], rB[2][2][2][2];
-#pragma unroll
-    for (int rd = 0; rd < 2; rd++)
-#pragma unroll
-        for (int c = 0; c < 2; c++)
-#pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const uint32_t i = tid + 1024 * e;
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    rA[rd][c][e][j] = rg[(size_t)(2 * rd) * BLK + (size_t)(j * 2 + c) * N + i];
-                    rB[rd][c][e][j] = rg[(size_t)(2 * rd + 1) * BLK + (size_t)(j * 2 + c) * N + i];
-                }
-            }
-    for (int gs = first; gs >= (int)lo; gs--) {
-        if constexpr (streamed)
-            if (!wait_packed((uint32_t)gs)) {
-                poison();
-                return;
-            }
-        const int st = gs - (int)start;
-        const uint32_t gi0 = start + (uint32_t)st;
-        uint32_t pav[2][2], pbv[2][2];  // packed a / b parts [c][e], loaded a phase ahead
+    if (first >= (int)lo) {
+        nr_stage_twiddles(tw2, nc, tid, 512);  // published by the barrier below
+        // the query's rows of this limb, [top_a | top_b | bot_a | bot_b][digit][slot], times 2^32 mod q
+        const uint32_t r32 = c ? (uint32_t)(4294967296ull % Q1) : (uint32_t)(4294967296ull % Q0);
+        const uint32_t qneg = c ? nr_neg_inverse(Q1) : nr_neg_inverse(Q0);
+        uint32_t rows[4][2][8];
 #pragma unroll
         for (int p = 0; p < 4; p++)
 #pragma unroll
-            for (int e = 0; e < 2; e++) buf[p][ls(tid + 1024 * e)] = acc[p][e];
-        __syncthreads();
-        ntt_inv_lds(buf[team], t, tw, tlimb, inv_n, inv_n_p);
-        uint32_t da0[2][2], da1[2][2], db0[2][2], db1[2][2];  // [e][digit], residue mod Q0 / Q1
+            for (int j = 0; j < 2; j++) {
+                load8(rows[p][j], rg + (size_t)p * BLK + (size_t)j * 2 * N);
 #pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const uint32_t i = tid + 1024 * e;
-            gadget2(buf[0][ls(i)], buf[1][ls(i)], cc, da0[e], da1[e]);
-            gadget2(buf[2][ls(i)], buf[3][ls(i)], cc, db0[e], db1[e]);
-        }
-        uint64_t ra[2][2], rb[2][2];  // [limb][e]
-#pragma unroll
-        for (int round = 0; round < 2; round++) {
-            __syncthreads();
-#pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const uint32_t i = tid + 1024 * e;
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    buf[j * 2 + 0][ls(i)] = round ? db0[e][j] : da0[e][j];
-                    buf[j * 2 + 1][ls(i)] = round ? db1[e][j] : da1[e][j];
-                }
+                for (int k = 0; k < 8; k++) rows[p][j][k] = mul_mod(rows[p][j][k], r32, c);
             }
+        const nr_u32x2* tw = tw2[c];
+        uint32_t(*xs)[256] = reinterpret_cast<uint32_t(*)[256]>(buf[c][2]);            // lift shares sent
+        const uint32_t(*xr)[256] = reinterpret_cast<const uint32_t(*)[256]>(buf[1 - c][2]);  // and received
+        __syncthreads();
+        for (int gs = first; gs >= (int)lo; gs--) {
+            uint32_t cf[2][8];  // a and b part, coefficients t + 256k
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+#pragma unroll
+                for (int k = 0; k < 8; k++) cf[p][k] = acc[p][k];
+            nr_inverse<2>(cf, buf[c], tw, t, m);
+            // this limb's shares of the CRT lift; team c lifts the
+            // coefficients k in [4c, 4c + 4) and sends the others
+            uint32_t keep[2][4];
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+#pragma unroll
+                for (int k = 0; k < 8; k++) cf[p][k] = nr_crt_part(cf[p][k], gc, c, m);
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    keep[p][k] = c ? cf[p][k + 4] : cf[p][k];
+                    xs[4 * p + k][t] = c ? cf[p][k] : cf[p][k + 4];
+                }
             __syncthreads();
-            ntt_fwd_lds(buf[team], t, tw, tlimb);
-            // RGSW parts: 0 top_a, 1 top_b, 2 bot_a, 3 bot_b; [part][digit][limb][N]
+            uint32_t x[4][8];  // digit polynomials a1, a2, b1, b2: residues + q mod this limb's prime
 #pragma unroll
-            for (int c = 0; c < 2; c++)
+            for (int p = 0; p < 2; p++)
 #pragma unroll
-                for (int e = 0; e < 2; e++) {
-                    const uint32_t i = tid + 1024 * e;
-                    uint64_t sa = round ? ra[c][e] : 0, sb = round ? rb[c][e] : 0;
+                for (int k = 0; k < 4; k++) {
+                    const uint32_t other = xr[4 * p + k][t];
+                    const nr_u32x2 d = nr_digits(c ? other : keep[p][k], c ? keep[p][k] : other);
+                    dx[c][4 * p + k][0][t] = d.x;
+                    dx[c][4 * p + k][1][t] = d.y;
+                }
+            __syncthreads();
+            uint32_t pav[8], pbv[8];  // the step's packed parts, in flight during the transforms
+            load8(pav, h.pa_base + (size_t)gs * h.pa_stride);
+            if constexpr (!STREAMED) load8(pbv, pb + (size_t)gs * 2 * N);
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+#pragma unroll
+                for (int s = 0; s < 2; s++)
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        x[2 * p][4 * s + k] = dx[s][4 * p + k][0][t] + (m.q - (1u << 17));
+                        x[2 * p + 1][4 * s + k] = dx[s][4 * p + k][1][t] + m.q;
+                    }
+            nr_forward<4>(x, buf[c], tw, t, m, [&]() {
+                if constexpr (STREAMED) wait_packed((uint32_t)gs);
+            });
+            if constexpr (STREAMED) {
+                if (sw_abort) {
+                    poison();
+                    return;
+                }
+                load8(pbv, pb + (size_t)gs * 2 * N);
+            }
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                // digits below 23.1q, rows below q: the sums stay below 93 q^2 < 2^59.6
+                uint64_t sa = 0, sb = 0;
+#pragma unroll
+                for (int s = 0; s < 2; s++)
 #pragma unroll
                     for (int j = 0; j < 2; j++) {
-                        const uint64_t d = buf[j * 2 + c][ls(i)];
-                        sa += d * rA[round][c][e][j];
-                        sb += d * rB[round][c][e][j];
+                        sa += (uint64_t)x[2 * s + j][k] * rows[2 * s][j][k];
+                        sb += (uint64_t)x[2 * s + j][k] * rows[2 * s + 1][j][k];
                     }
-                    ra[c][e] = sa; rb[c][e] = sb;
-                }
-            if (round == 0) {  // the step's packed parts, issued before round 1's transforms
-#pragma unroll
-                for (int c = 0; c < 2; c++)
-#pragma unroll
-                    for (int e = 0; e < 2; e++) {
-                        const uint32_t i = tid + 1024 * e;
-                        pav[c][e] = pa_base[(size_t)gi0 * pa_stride + (size_t)c * N + i];
-                        pbv[c][e] = pb[(size_t)gi0 * 2 * N + (size_t)c * N + i];
-                    }
+                acc[0][k] = nr_montgomery(sa, qneg, m.q) + pav[k];  // below 2.1q + q + q
+                acc[1][k] = nr_montgomery(sb, qneg, m.q) + pbv[k];
             }
         }
 #pragma unroll
-        for (int c = 0; c < 2; c++)
+        for (int p = 0; p < 2; p++)
 #pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const uint32_t q = qof(c);
-                acc[c][e] = add_mod(red64(ra[c][e], c), pav[c][e], q);
-                acc[2 + c][e] = add_mod(red64(rb[c][e], c), pbv[c][e], q);
-            }
-        __syncthreads();
+            for (int k = 0; k < 8; k++) acc[p][k] = fold(fold(fold(acc[p][k], 4 * m.q), 2 * m.q), m.q);
     }
     if (lo > start) {  // the chain continues in a later launch
 #pragma unroll
-        for (int p = 0; p < 4; p++)
-#pragma unroll
-            for (int e = 0; e < 2; e++) hs[(size_t)p * N + tid + 1024 * e] = acc[p][e];
+        for (int p = 0; p < 2; p++) {
+            u32x4* d = reinterpret_cast<u32x4*>(hs + (size_t)(2 * p + c) * N + 8 * t);
+            d[0] = u32x4{acc[p][0], acc[p][1], acc[p][2], acc[p][3]};
+            d[1] = u32x4{acc[p][4], acc[p][5], acc[p][6], acc[p][7]};
+        }
         return;
     }
+    // the response, through LDS for whole lines of 8-byte words (a lane's own
+    // words of the last exchange)
+    nr_store<3, 2>(buf[c], acc, t);
+    __syncthreads();
 #pragma unroll
-    for (int p = 0; p < 4; p++)
+    for (int p = 0; p < 2; p++)
 #pragma unroll
-        for (int e = 0; e < 2; e++) o[(size_t)p * N + tid + 1024 * e] = acc[p][e];
+        for (int k = 0; k < 8; k++)
+            o[(size_t)(2 * p + c) * N + t + 256 * k] = buf[c][p][nr_base(0, t) + nr_stride<0>() * k];
 }
 
 // ------------------------------------------------------------ streamed pack
@@ -574,14 +596,14 @@ hipError_t launch_horner(const uint32_t* pa_base, size_t pa_stride, size_t G, si
                          const CrtConst& cc, hipStream_t s, const FusedPack& pack, const StreamWait& wait) {
     if (nq == 0 || g_lo >= g_hi) return hipSuccess;
     if (wait.done && (!wait.status || wait.queries == 0)) return hipErrorInvalidValue;
+    const HornerChain h{pa_base, pa_stride, (uint32_t)G, (uint32_t)Da, (uint32_t)T, packed_b, packed_stride,
+                        rgsw, rgsw_stride, out, hstate, (uint32_t)g_lo, (uint32_t)g_hi};
+    const NrGadget gc = nr_gadget_const(nc, cc);
+    const dim3 grid((unsigned)T, (unsigned)nq);
     if (wait.done)
-        hipLaunchKernelGGL(k_horner<true>, dim3((unsigned)T, (unsigned)nq), dim3(1024), 0, s, pa_base, pa_stride,
-                           (uint32_t)G, (uint32_t)Da, (uint32_t)T, packed_b, packed_stride, rgsw, rgsw_stride, out,
-                           hstate, (uint32_t)g_lo, (uint32_t)g_hi, nc, cc, pack, wait);
+        hipLaunchKernelGGL(k_horner<true>, grid, dim3(512), 0, s, h, nc, gc, pack, wait);
     else
-        hipLaunchKernelGGL(k_horner<false>, dim3((unsigned)T, (unsigned)nq), dim3(1024), 0, s, pa_base, pa_stride,
-                           (uint32_t)G, (uint32_t)Da, (uint32_t)T, packed_b, packed_stride, rgsw, rgsw_stride, out,
-                           hstate, (uint32_t)g_lo, (uint32_t)g_hi, nc, cc, pack, wait);
+        hipLaunchKernelGGL(k_horner<false>, grid, dim3(512), 0, s, h, nc, gc, pack, wait);
     return hipGetLastError();
 }
 

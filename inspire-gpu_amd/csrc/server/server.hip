@@ -918,18 +918,17 @@ void GpuServerCtx::stage_finalize(size_t count, hipStream_t s, size_t slot0) {
                               d_packed_b + slot0 * packed_stride, packed_stride, count, nc, s));
 }
 
-bool GpuServerCtx::use_pair(size_t chains, bool beside_passes, bool status_read) const {
-    // never where nobody reads the status its bounded wait reports through;
-    // auto: the pair kernel shortens a lone chain run by itself (its per-step
-    // exchange costs more than it saves once many chains share the L2s, or
-    // while database passes stream through them)
-    if (!status_read) return false;
-    return horner_mode == 1 || (horner_mode < 0 && chains <= kPairMaxChains && !beside_passes);
+bool GpuServerCtx::use_pair(bool status_read) const {
+    // only where set by hand, and never where nobody reads the status its
+    // bounded wait reports through: the Horner stage of a serial one-query
+    // answer at 1 GB (7 steps) takes 87 us with the pair, 72 us with one
+    // workgroup
+    return status_read && horner_mode == 1;
 }
 
 void GpuServerCtx::horner_range(size_t count, uint64_t* d_out, size_t g_lo, size_t g_hi, hipStream_t s,
-                                size_t slot0, int lane, bool status_read, bool beside_passes, const FusedPack* fp) {
-    if (use_pair(count * T, beside_passes, status_read))
+                                size_t slot0, int lane, bool status_read, const FusedPack* fp) {
+    if (use_pair(status_read))
         HIPX(launch_horner_pair(d_precomp + PC_A, PC_GROUP, G, Da, T, d_packed_b + slot0 * packed_stride,
                                 packed_stride, d_rgsw + slot0 * rgsw_stride, rgsw_stride, d_out,
                                 d_hstate + slot0 * T * 4 * N, g_lo, g_hi, count,
@@ -1155,7 +1154,7 @@ void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, 
             if (cs != s) HIPX(hipStreamWaitEvent(hs, dbe, 0));
             HIPX(hipStreamWaitEvent(hs, ce, 0));
             // the pack: fused into the one-workgroup Horner chains, or a kernel of its own
-            const bool fuse = pack_wg == 2 && !use_pair(nq * T, true, status_read);
+            const bool fuse = pack_wg == 2 && !use_pair(status_read);
             const FusedPack fp{d_interm + q0 * 2 * C, C, p2, part2_stride, d_precomp, keys, keys_stride};
             if (fuse)
                 ;
@@ -1165,7 +1164,7 @@ void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, 
             else
                 HIPX(launch_pack_finalize(d_interm + q0 * 2 * C, C, p2, part2_stride, d_precomp, g_lo, ng, keys,
                                           keys_stride, packed, packed_stride, nq, nc, hs));
-            horner_range(nq, out, g_lo, g_hi, hs, q0, lane, status_read, true, fuse ? &fp : nullptr);
+            horner_range(nq, out, g_lo, g_hi, hs, q0, lane, status_read, fuse ? &fp : nullptr);
         }
         if (cs != s) {  // the next batch's key digits overwrite the lane's scratch
             HIPX(hipEventRecord(prep_ev[lane], cs));

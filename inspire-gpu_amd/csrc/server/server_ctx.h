@@ -146,11 +146,9 @@ struct GpuServerCtx {
     hipEvent_t pass_ev[kLanes] = {};                 // a split streamed pass's first launch done
     hipEvent_t horner_done[kLanes] = {};
     uint32_t* d_packed_b = nullptr;
-    // Horner: 0 = one workgroup per chain, 1 = a workgroup pair (one per
-    // limb), -1 = pair when a call has at most kPairMaxChains chains and its
-    // answer is serial (beside the passes the pair's exchange is slower)
+    // Horner: 1 = a workgroup pair per chain (one per limb) where its status
+    // is read, 0 and -1 = one workgroup per chain (faster everywhere)
     int horner_mode = -1;
-    static constexpr size_t kPairMaxChains = 2;
     // pack kernel of pipelined chunks: 1 one workgroup per query, 0 a grid
     // over (group, limb), -1 one workgroup for one-query calls, 2 fused into
     // the Horner chains' own workgroups (where the one-workgroup Horner runs)
@@ -226,11 +224,11 @@ struct GpuServerCtx {
     void stage_dbpass(size_t count, hipStream_t s, size_t slot0, int lane = 0, int force = -1);
     // The pair kernel only where the caller reads the lane's status after
     // the call (status_read): its bounded wait reports through it.
-    bool use_pair(size_t chains, bool beside_passes, bool status_read) const;
+    bool use_pair(bool status_read) const;
     // Horner chains of `count` queries over groups [g_lo, g_hi).
     // fp: the chains compute their groups' packed b-parts themselves first
     void horner_range(size_t count, uint64_t* d_out, size_t g_lo, size_t g_hi, hipStream_t s, size_t slot0,
-                      int lane, bool status_read, bool beside_passes = false, const ipx::FusedPack* fp = nullptr);
+                      int lane, bool status_read, const ipx::FusedPack* fp = nullptr);
     void stage_collapse(size_t count, hipStream_t s, size_t slot0, int lane = 0);
     void stage_finalize(size_t count, hipStream_t s, size_t slot0);
     void stage_horner(size_t count, uint64_t* d_out, hipStream_t s, size_t slot0, bool status_read);
