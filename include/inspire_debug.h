@@ -34,8 +34,9 @@ int ipir_dbg_db_pass(ipir_server* srv, const uint64_t* b, size_t nq, int path, u
 /* Device time of the full-width database pass alone (the pass kernel of
  * the plan answer_batch uses for nq <= 32 queries, and its slice reduction
  * if the plan has row slices, on the server stream) over the first nq
- * query slots as last staged, averaged over iters passes; the query digits
- * are prepared once, outside the timed launches. */
+ * query slots as last staged (by a host-staged answer or
+ * ipir_dbg_profile_batch), averaged over iters passes; the query digits are
+ * prepared once, outside the timed launches. */
 int ipir_dbg_time_dbpass(ipir_server* srv, size_t nq, int iters, double* ms_per_pass);
 /* The database-pass kernel (profiler name) and row-slice count the server
  * uses for a batch of nq queries, NUL-terminated into out[cap]. */

@@ -284,10 +284,18 @@ int ipir_dbg_db_pass(ipir_server* srv, const uint64_t* b, size_t nq, int path, u
         std::lock_guard<std::mutex> lk(c->mu);
         if (c->loop_active) return 5;
         c->order_before(c->stream);
-        std::vector<double> bd(nq * 2 * R);
-        for (size_t i = 0; i < bd.size(); i++) bd[i] = (double)b[i];
-        hip_check(hipMemcpy(c->d_bq, bd.data(), bd.size() * 8, hipMemcpyHostToDevice), "dbg db pass upload");
-        c->stage_dbpass(nq, c->stream, 0, 0, path);
+        // the LWE parts, 2R words apart, in the flat query staging
+        hip_check(hipMemcpy(c->d_q, b, nq * 2 * R * 8, hipMemcpyHostToDevice), "dbg db pass upload");
+        const size_t step = path == 0 ? 1 : ipx::kMfmaMaxQueries;
+        for (size_t q0 = 0; q0 < nq; q0 += step) {
+            const size_t n = nq - q0 < step ? nq - q0 : step;
+            ipx::DbPlan p = c->plan_for(n, C);
+            if (path == 0 && p.kind != ipx::DbPlan::F64) p = ipx::dbplan_f64(R, C, 4, 2048);
+            if (path == 1 && p.kind == ipx::DbPlan::F64)
+                p = ipx::dbplan_form(R, C, n, c->mfma_target, c->mfma_depth, c->mfma_form);
+            c->prep_lwe(c->d_q + q0 * 2 * R, 2 * R, q0, n, p, c->stream, 0);
+            c->dbpass_range(q0, n, 0, c->G, p, c->stream, 0);
+        }
         c->order_after(c->stream);
         hip_check(hipStreamSynchronize(c->stream), "dbg db pass");
         hip_check(hipMemcpy(interm, c->d_interm, nq * 2 * C * 4, hipMemcpyDeviceToHost), "dbg db pass download");
@@ -315,7 +323,7 @@ int ipir_dbg_time_dbpass(ipir_server* srv, size_t nq, int iters, double* ms_per_
         // the query digits once; then the pass's own launches (the kernel and,
         // for a plan with row slices, the slice reduction)
         const ipx::DbPlan p = c->plan_for(nq, c->pp.db_cols);
-        c->dbpass_prep(0, nq, p, c->stream, 0);
+        c->prep_lwe(c->d_q, c->qlen, 0, nq, p, c->stream, 0);
         c->dbpass_range(0, nq, 0, c->G, p, c->stream, 0);  // warm-up
         hip_check(hipEventRecord(e0, c->stream), "record");
         for (int i = 0; i < iters; i++) c->dbpass_range(0, nq, 0, c->G, p, c->stream, 0);
@@ -362,6 +370,9 @@ int ipir_dbg_tuning(const ipir_server* srv, char* out, size_t cap) {
         s += c->tail_split ? " (lowest split in 1/2, 1/4, 1/4" : " (";
         s += c->head_split ? std::string(c->tail_split ? "; " : "") + "highest split in 1/4, 1/4, 1/2)" : ")";
     }
+    if (c->pipe_single == 0 || c->pipe_batched == 0)
+        s += "; serial: batch1 " + plan(c->serial_plan(1)) + ", batch" + std::to_string(nq) + " " +
+             plan(c->serial_plan(nq));
     s += "; collapse variant " + std::to_string(c->collapse_variant) + "; pipeline shapes " +
          std::to_string(c->pipe_single) + "/" + std::to_string(c->pipe_batched);
     if (c->pipe_single >= 6 || c->pipe_batched >= 6) {  // streamed shapes
@@ -647,8 +658,8 @@ int ipir_dbg_stream_parts(ipir_server* srv, size_t nq, uint32_t slices, double* 
         uint32_t* part = direct ? c->d_interm : c->d_part;
         const size_t part_qstride = direct ? 2 * C : c->part_stride;
         c->order_before(s);
-        hip_check(hipMemsetAsync(c->d_bq, 0, nq * 2 * c->pp.db_rows * sizeof(double), s), "zero");
-        c->dbpass_prep(0, nq, p, s, 0);
+        hip_check(hipMemsetAsync(c->d_q, 0, nq * c->qlen * 8, s), "zero");
+        c->prep_lwe(c->d_q, c->qlen, 0, nq, p, s, 0);
         auto timed = [&](const std::function<void()>& fn) {
             fn();  // warm
             hip_check(hipEventRecord(e0, s), "event");
@@ -864,36 +875,53 @@ int ipir_dbg_profile_batch(ipir_server* srv, const uint64_t* d_queries, size_t c
     GpuServerCtx* c = srv->ctx;
     std::lock_guard<std::mutex> lk(c->mu);
     if (c->loop_active) return 5;
-    hipEvent_t ev[6];
-    for (auto& e : ev) (void)hipEventCreate(&e);
     hipStream_t s = c->stream;
+    // the serial answer stage by stage, sub-batch by sub-batch (their int8
+    // operands share one scratch set); events around every stage
+    const size_t step = ipx::kMfmaMaxQueries, nsub = (count + step - 1) / step;
+    std::vector<hipEvent_t> ev(5 * nsub + 2, nullptr);
     int rc = 0;
     try {
+        for (auto& e : ev) hip_check(hipEventCreate(&e), "event");
         c->order_before(s);
         c->clear_status(s, 0);
-        (void)hipEventRecord(ev[0], s);
-        c->stage_prep(d_queries, count, s, 0);
-        (void)hipEventRecord(ev[1], s);
-        c->stage_dbpass(count, s, 0);
-        (void)hipEventRecord(ev[2], s);
-        c->stage_collapse(count, s, 0);
-        (void)hipEventRecord(ev[3], s);
-        c->stage_finalize(count, s, 0);
-        (void)hipEventRecord(ev[4], s);
-        c->stage_horner(count, d_out, s, 0, true);
-        (void)hipEventRecord(ev[5], s);
-        c->order_after(s);
-        hip_check(hipEventSynchronize(ev[5]), "sync");
-        c->check_status(s, 0);
-        for (int i = 0; i < 5; i++) {
-            float ms = 0;
-            (void)hipEventElapsedTime(&ms, ev[i], ev[i + 1]);
-            stage_ms[i] = ms;
+        // kept as staged queries for ipir_dbg_time_dbpass
+        hip_check(hipMemcpyAsync(c->d_q, d_queries, count * c->qlen * 8, hipMemcpyDeviceToDevice, s), "stage queries");
+        size_t k = 0;
+        auto mark = [&] { hip_check(hipEventRecord(ev[k++], s), "event"); };
+        for (size_t q0 = 0; q0 < count; q0 += step) {
+            const size_t nq = count - q0 < step ? count - q0 : step;
+            const ipx::DbPlan p = c->serial_plan(nq);
+            mark();
+            c->prep_query(c->d_q + q0 * c->qlen, q0, nq, p, s, 0);
+            mark();
+            c->dbpass_whole(q0, nq, p, s, 0);
+            mark();
+            c->collapse_whole(q0, nq, s, 0);
+            mark();
+            c->pack_whole(q0, nq, p, s);
+            mark();
         }
+        mark();
+        c->horner_range(count, d_out, 0, c->G, s, 0, 0, true);
+        mark();
+        c->order_after(s);
+        hip_check(hipEventSynchronize(ev[k - 1]), "sync");
+        c->check_status(s, 0);
+        for (int i = 0; i < 5; i++) stage_ms[i] = 0;
+        float ms = 0;
+        for (size_t b = 0; b < nsub; b++)
+            for (int i = 0; i < 4; i++) {
+                hip_check(hipEventElapsedTime(&ms, ev[5 * b + i], ev[5 * b + i + 1]), "elapsed");
+                stage_ms[i] += ms;
+            }
+        hip_check(hipEventElapsedTime(&ms, ev[5 * nsub], ev[5 * nsub + 1]), "elapsed");
+        stage_ms[4] = ms;
     } catch (...) {
         rc = 4;
     }
-    for (auto& e : ev) (void)hipEventDestroy(e);
+    for (auto& e : ev)
+        if (e) (void)hipEventDestroy(e);
     return rc;
 }
 

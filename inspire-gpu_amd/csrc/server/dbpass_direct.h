@@ -10,6 +10,15 @@ namespace {
 
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 
+// sum_r b_pr[r] of pair pr = 2 q + limb, the database-offset correction, as
+// k_prep leaves it: one residue per row range, below 2^30 together.
+__device__ __forceinline__ uint32_t offset_sum(const uint32_t* __restrict__ S, uint32_t pr) {
+    static_assert(kOffsetSumParts == 8, "two 16-byte loads");
+    const i32x4* p = reinterpret_cast<const i32x4*>(S + (size_t)pr * kOffsetSumParts);
+    const i32x4 a = p[0], b = p[1];
+    return (uint32_t)(a[0] + a[1] + a[2] + a[3] + b[0] + b[1] + b[2] + b[3]);
+}
+
 // Recombine one lane's accumulators of pair pr and store the canonical residue.
 __device__ __forceinline__ void store_pair(const i32x4& al, const i32x4& ah, uint32_t pr, uint32_t nq, bool corr,
                                            const uint32_t* __restrict__ S, uint32_t* __restrict__ out,
@@ -17,7 +26,7 @@ __device__ __forceinline__ void store_pair(const i32x4& al, const i32x4& ah, uin
     const uint32_t q = pr >> 1;
     const int c = (int)(pr & 1);
     if (q >= nq) return;
-    int64_t s = corr ? (int64_t)32896 * S[pr] : 0;
+    int64_t s = corr ? (int64_t)32896 * offset_sum(S, pr) : 0;
 #pragma unroll
     for (int i = 0; i < 4; i++) s += ((int64_t)ah[i] * 256 + (int64_t)al[i]) * ((int64_t)1 << (8 * i));
     // |s| < 2^58.1 (|d_3| <= 8 bounds the top digit's term); add a multiple

@@ -24,8 +24,6 @@ struct SlotLayout {
     size_t query_u64s() const { return 2 * R + 6 * (size_t)D_EFF * 2 * N; }
 };
 
-hipError_t launch_unmarshal(const uint64_t* d_q, size_t count, size_t R, double* bq, uint32_t* keys,
-                            uint32_t* rgsw, hipStream_t s);
 // In-place forward NTT of `npoly` RNS polynomials laid out [npoly][2][N].
 hipError_t launch_ntt_rns(uint32_t* polys, size_t npoly, const NttConst& nc, bool inverse, hipStream_t s);
 // dst <- src, bytes a multiple of 16 (grid-stride, 16 bytes per lane).
@@ -84,6 +82,36 @@ size_t dbplan_max_queries(const DbPlan& p);
 size_t dbplan_mp(const DbPlan& p);
 // Column granularity of a plan (one block's columns): col0 and ncols are multiples of it.
 size_t dbplan_cols(const DbPlan& p);
+// One launch preparing nq (1..32) flat wire queries for their passes: keys
+// in NTT form with their int8 digits (kdig) and sums (KS), RGSW rows, and
+// the operand of plan p's database pass: digits (dig, R*Mp bytes) and sums
+// (S), or doubles (bq) for an fp64 plan. keys = nullptr prepares the LWE part
+// alone.
+constexpr uint32_t kOffsetSumParts = 8;  // row ranges of S: [query][limb][part], unused parts zero
+constexpr uint32_t kKeySumParts = 2;     // KS: [query][limb][digit]
+enum PrepForm : uint32_t { kPrepDoubles, kPrepDigits4, kPrepDigits7, kPrepPower };
+struct PrepArgs {
+    const uint64_t* q = nullptr;  // query 0's words (LWE part first), queries q_stride apart
+    size_t q_stride = 0, R = 0;
+    double* bq = nullptr;         // [query][limb][R]
+    int8_t* dig = nullptr;
+    uint32_t* S = nullptr;
+    uint32_t* keys = nullptr;     // [query][key][digit][limb][N]
+    size_t keys_stride = 0;
+    uint32_t* rgsw = nullptr;     // [query][part][digit][limb][N]
+    size_t rgsw_stride = 0;
+    int8_t* kdig = nullptr;
+    uint32_t* KS = nullptr;
+    uint32_t* zero = nullptr;     // zero_words words set to zero (hand-over flags)
+    uint32_t zero_words = 0;
+    uint32_t* status = nullptr;   // a word set to zero
+    uint32_t* part2 = nullptr;    // part2_words (a multiple of 4096) words per query set to zero
+    size_t part2_stride = 0, part2_words = 0;
+    bool skip_lwe = false;        // keys and RGSW rows only
+    // set by launch_prep
+    uint32_t form = 0, parts = 0, Mp = 0, kMp = 0, key_blocks = 0, lwe_blocks = 0, rgsw_blocks = 0;
+};
+hipError_t launch_prep(PrepArgs a, size_t nq, const DbPlan& p, const NttConst& nc, hipStream_t s);
 // Name of the kernel a plan launches (as profilers report it, without arguments).
 std::string dbplan_kernel(const DbPlan& p);
 // Output of the database passes: out points at the first column's residue
@@ -93,12 +121,8 @@ std::string dbplan_kernel(const DbPlan& p);
 // One query, fp64 FMA on the vector ALUs, over columns [col0, col0 + ncols).
 hipError_t launch_dbpass_f64(const uint8_t* db, const double* bq, uint32_t* out, size_t ostride, size_t R, size_t C,
                              size_t col0, size_t ncols, const DbPlan& p, hipStream_t s);
-// Query digits and offset sums of nq queries (bq [q][limb][R] doubles) for
-// an MFMA plan: dig (R*Mp bytes) and S (2*nq words).
-hipError_t launch_mfma_digits(const double* bq, size_t nq, size_t R, const DbPlan& p, int8_t* dig, uint32_t* S,
-                              hipStream_t s);
 // The int8-MFMA pass of nq queries over columns [col0, col0 + ncols), from
-// launch_mfma_digits' output for a plan with the same digit tile count.
+// launch_prep's dig and S for a plan with the same digit tile count.
 //
 // A streamed pass (ps set; full width, direct kernels and shared-digit
 // forms only) hands its groups over while it runs: its 1-D grid takes the
@@ -133,10 +157,8 @@ hipError_t launch_reduce_slices(const uint32_t* part, size_t part_stride, uint32
 
 // Queries one collapse pass serves.
 constexpr size_t kCollapseMaxQueries = 32;
-// Key digits and key sums of nq queries whose NTT-form keys sit at
-// keys + q*kstride, for launch_collapse: kdig (1 MiB) and KS (2*nq words).
-hipError_t launch_collapse_keys(const uint32_t* keys, size_t kstride, size_t nq, int8_t* kdig, uint32_t* KS,
-                                hipStream_t s);
+// Key-digit rows a collapse pass of nq queries stages per 16-row block.
+size_t collapse_mp(size_t nq);
 // Precomp-tensor pass in dot-product form (int8 MFMA, Dd read once) of ng
 // groups whose precomp blocks start at precomp_g0, for nq queries:
 // part2_g0 + q*p2_stride + g*2N holds [limb][N] of group g (relative).
@@ -148,25 +170,36 @@ hipError_t launch_collapse_keys(const uint32_t* keys, size_t kstride, size_t nq,
 // 5 in 8-wave blocks); fewer queries ignore the variant.
 constexpr int kCollapseVariants = 6;
 hipError_t launch_collapse(const uint32_t* precomp_g0, size_t ng, const int8_t* kdig, const uint32_t* KS, size_t nq,
-                           uint32_t* part2_g0, size_t p2_stride, hipStream_t s, int variant = 0);
-// A streamed pass of up to 8 queries with the collapse in the same launch:
-// per group from the top, the collapse (all groups' precomp, part2 as in
+                           uint32_t* part2_g0, size_t p2_stride, hipStream_t s, int variant = 0, bool zeroed = false);
+// Row slices that launch adds up (1: it stores, nothing needs zeroing).
+uint32_t collapse_row_slices(size_t nq, size_t ng, int variant);
+// The database pass of up to 8 queries and the collapse in one launch: per
+// group from the top, the collapse (all groups' precomp, part2 as in
 // launch_collapse) and the database pass of plan p (a direct-kernel plan,
-// 256-column tiles; out as a streamed pass's) as 256-lane work items;
-// group_done[g] counts them (zero before the launch) and reaches
-// pass_collapse_target(p, nq, G) when both halves of group g are in place.
-// The key digits (launch_collapse_keys) and query digits must be ready.
+// 256-column tiles; out as that pass's) as 256-lane work items. The key and
+// query digits (launch_prep) must be ready.
+// Streamed (group_done set): group_done[g] counts the items (zero before the
+// launch) and reaches pass_collapse_target(p, nq, G) when both halves of
+// group g are in place. Otherwise the collapse may be cut into
+// pass_collapse_ksplit(nq, G) row slices; above 1, part2 must be zero.
+inline bool pass_collapse_ok(const DbPlan& p, size_t nq) {
+    return p.kind == DbPlan::MFMA && p.param <= 4 && nq >= 1 && nq <= 8 && dbplan_cols(p) == 256;
+}
 uint32_t pass_collapse_target(const DbPlan& p, size_t nq, size_t G);
-hipError_t launch_pass_collapse_stream(const uint8_t* db, const int8_t* dig, const uint32_t* S, size_t nq,
-                                       uint32_t* out, size_t out_qstride, size_t R, size_t C, const DbPlan& p,
-                                       const uint32_t* precomp, const int8_t* kdig, const uint32_t* KS,
-                                       uint32_t* part2, size_t p2_stride, uint32_t* group_done, hipStream_t s);
-// packed_b[q][g] = NTT(interm[q] group slice) - collapse sums - Df*Kn, for
-// groups [g0, g0 + ng) (absolute indexes into every buffer).
-hipError_t launch_pack_finalize(const uint32_t* interm, size_t C, const uint32_t* part2, size_t part2_stride,
-                                const uint32_t* precomp, size_t g0, size_t ng, const uint32_t* keys,
-                                size_t keys_stride, uint32_t* packed_b, size_t packed_stride, size_t nq,
-                                const NttConst& nc, hipStream_t s);
+uint32_t pass_collapse_ksplit(size_t nq, size_t G);
+hipError_t launch_pass_collapse(const uint8_t* db, const int8_t* dig, const uint32_t* S, size_t nq, uint32_t* out,
+                                size_t out_qstride, size_t R, size_t C, const DbPlan& p, const uint32_t* precomp,
+                                const int8_t* kdig, const uint32_t* KS, uint32_t* part2, size_t p2_stride,
+                                uint32_t* group_done, hipStream_t s);
+// packed_b[q][g] = NTT(sum of the pass's row slices, group g) - collapse sums
+// - Df*Kn, for groups [g0, g0 + ng) (absolute indexes into every buffer).
+// part: [q][slice][limb][C] partials (one slice: interm). out (one group,
+// so every chain is one ciphertext): also write the flat u64 responses.
+hipError_t launch_pack_finalize(const uint32_t* part, size_t part_qstride, uint32_t slices, size_t C,
+                                const uint32_t* part2, size_t part2_stride, const uint32_t* precomp, size_t g0,
+                                size_t ng, const uint32_t* keys, size_t keys_stride, uint32_t* packed_b,
+                                size_t packed_stride, size_t nq, const NttConst& nc, hipStream_t s,
+                                uint64_t* out = nullptr);
 // The same output from one 1024-lane workgroup per query (for one-query
 // chunks beside database passes, where it starts without waiting for slots).
 hipError_t launch_pack_finalize_wg(const uint32_t* interm, size_t C, const uint32_t* part2, size_t part2_stride,

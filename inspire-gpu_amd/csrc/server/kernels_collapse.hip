@@ -121,54 +121,6 @@ __global__ __launch_bounds__(1024) void k_dd_relayout(const uint32_t* __restrict
 }
 
 // ------------------------------------------------------------ online
-// Key digits: kdig[c][kb][Mp][16 bytes], row m = q*4 + b holding digit b
-// (balanced base 256, as for the database pass) of K5_q[j][c][p] at
-// k = j*N + p = 16*kb + byte. Padding rows (q >= nq) are zero.
-__global__ __launch_bounds__(256) void k_kdigits(const uint32_t* __restrict__ keys, size_t kstride, uint32_t nq,
-                                                 uint32_t Mp, int8_t* __restrict__ kdig) {
-    const uint32_t nkb = DD_K / 16, nqp = Mp / 4;
-    const uint32_t x = blockIdx.x * 256 + threadIdx.x;
-    if (x >= 2 * nkb * nqp) return;
-    const uint32_t kb = x % nkb, q = (x / nkb) % nqp, c = x / (nkb * nqp);
-    u32x4 o[4];
-#pragma unroll
-    for (int b = 0; b < 4; b++) o[b] = u32x4{0, 0, 0, 0};
-    if (q < nq) {
-        const uint32_t k0 = kb * 16, j = k0 / N, p0 = k0 % N;
-        const uint32_t* K = keys + (size_t)q * kstride + ((size_t)j * 2 + c) * N + p0;
-#pragma unroll
-        for (int e = 0; e < 16; e++) {
-            int32_t v = (int32_t)K[e];
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                int32_t d = v;
-                if (b < 3) {
-                    d = ((v & 255) ^ 128) - 128;
-                    v = (v - d) >> 8;
-                }
-                o[b][e >> 2] |= ((uint32_t)d & 255u) << (8 * (e & 3));
-            }
-        }
-    }
-    u32x4* dst = reinterpret_cast<u32x4*>(kdig + (((size_t)c * nkb + kb) * Mp + (size_t)q * 4) * 16);
-#pragma unroll
-    for (int b = 0; b < 4; b++) dst[b] = o[b];
-}
-
-// KS[q*2 + c] = sum_{j,p} K5_q[j][c][p] mod q_c (the plane-offset correction).
-__global__ __launch_bounds__(1024) void k_ksum(const uint32_t* __restrict__ keys, size_t kstride,
-                                               uint32_t* __restrict__ KS) {
-    __shared__ uint64_t red[16];
-    const uint32_t q = blockIdx.x >> 1, c = blockIdx.x & 1;
-    // DD_K = 2N entries: digit d's limb-c polynomial at keys + (2d + c) N
-    const uint32_t* k = keys + (size_t)q * kstride + (size_t)c * N + threadIdx.x;
-    uint64_t a = 0;
-#pragma unroll
-    for (int e = 0; e < 4; e++) a += k[(size_t)(e >> 1) * 2 * N + (size_t)(e & 1) * 1024];
-    const uint64_t sum = block_sum_u64<1024>(a, red);
-    if (threadIdx.x == 0) KS[blockIdx.x] = red64(sum, (int)c);
-}
-
 // Recombine one lane's 16 accumulators (4 Dd planes x 4 key digits) of
 // query q for one slot and store the canonical residue. With Dd entry =
 // sum_a 256^a x_a + 128*65793 (x_a the signed planes, x_3 the top byte) and
@@ -186,16 +138,16 @@ struct KSlice {
     bool first = true;     // adds the 128*65793 sum(K) term
     bool add = false;      // atomic add (split) or store (whole)
 };
-// The slice of a split launch's grid, z = group * ksplit + slice.
-__device__ __forceinline__ KSlice slice_of(uint32_t ksplit) {
+__device__ __forceinline__ KSlice kslice(uint32_t sl, uint32_t ksplit) {
     KSlice k;
-    const uint32_t sl = blockIdx.z % ksplit;
     k.nks = (uint32_t)(DD_K / 64) / ksplit;
     k.k0 = sl * k.nks;
     k.first = sl == 0;
     k.add = ksplit > 1;
     return k;
 }
+// The slice of a split launch's grid, z = group * ksplit + slice.
+__device__ __forceinline__ KSlice slice_of(uint32_t ksplit) { return kslice(blockIdx.z % ksplit, ksplit); }
 __device__ __forceinline__ void collapse_store(const i32x4 (&acc)[4], uint32_t q, int c, uint32_t g, uint32_t i,
                                                const uint32_t* __restrict__ KS, uint32_t* __restrict__ part2,
                                                size_t p2_stride, const KSlice& ks = KSlice{}) {
@@ -205,7 +157,9 @@ __device__ __forceinline__ void collapse_store(const i32x4 (&acc)[4], uint32_t q
     for (int pl = 0; pl < 4; pl++)
 #pragma unroll
         for (int b = 0; b < 4; b++) lv[pl + b] += acc[pl][b];
-    int64_t s = ks.first ? (int64_t)8421504 * KS[q * 2 + c] : 0;  // 128*65793 * sum(K)
+    static_assert(kKeySumParts == 2, "one residue per digit");
+    const uint32_t* kp = KS + (size_t)(q * 2 + c) * kKeySumParts;
+    int64_t s = ks.first ? (int64_t)8421504 * (kp[0] + kp[1]) : 0;  // 128*65793 * sum(K)
     uint64_t wk = 1;                                // 256^k mod q_c
 #pragma unroll
     for (int k = 0; k < 7; k++) {
@@ -349,24 +303,31 @@ __global__ __launch_bounds__(256, 2) void k_collapse_mfma(const uint32_t* __rest
 // are complete (one agent-scope release per workgroup), adds 1 to its
 // group's counter; a group is in place at 2 N/(64 CNT) + (N/(64 PNT)) x
 // slices.
+// Without counters (group_done null) it is the serial answer's pass and
+// collapse in one launch, a table too small to fill the chip with either
+// alone cutting the collapse into ksplit row slices (KSlice).
 template <int PMT, int PNT, int CMT, int CNT>
 __global__ __launch_bounds__(256, 2) void k_pass_collapse_stream(
     const uint8_t* __restrict__ db, const int8_t* __restrict__ dig, const uint32_t* __restrict__ S,
     uint32_t* __restrict__ out, size_t out_qstride, uint32_t C, uint32_t kbps, const uint32_t* __restrict__ precomp,
     const int8_t* __restrict__ kdig, const uint32_t* __restrict__ KS, uint32_t* __restrict__ part2,
-    size_t p2_stride, uint32_t nq, uint32_t G, uint32_t slice_shift, uint32_t* __restrict__ group_done) {
+    size_t p2_stride, uint32_t nq, uint32_t G, uint32_t slice_shift, uint32_t ksplit,
+    uint32_t* __restrict__ group_done) {
     constexpr uint32_t CIT = N / (64 * CNT);  // collapse slot tiles per limb
-    constexpr uint32_t CB = 2 * CIT;          // collapse work items per group
     constexpr uint32_t TPG = N / (64 * PNT);  // pass column tiles per group
+    const uint32_t CB = 2 * CIT * ksplit;     // collapse work items per group
     const uint32_t per = CB + (TPG << slice_shift);
     const uint32_t b = blockIdx.x, gi = b / per, r = b - gi * per, g = G - 1 - gi;
     if (r < CB) {
-        collapse_mfma_body<CMT, CNT, false>(precomp, kdig, KS, part2, p2_stride, nq, r % CIT, (int)(r / CIT), g);
+        const uint32_t sl = r / (2 * CIT), it = r % (2 * CIT);
+        collapse_mfma_body<CMT, CNT, false>(precomp, kdig, KS, part2, p2_stride, nq, it % CIT, (int)(it / CIT), g,
+                                            kslice(sl, ksplit));
     } else {
         const uint32_t pr = r - CB;
         dbpass_direct_body<PMT, PNT>(db, dig, S, out, out_qstride, C, C, nq, kbps, g * TPG + (pr >> slice_shift),
                                      pr & ((1u << slice_shift) - 1));
     }
+    if (!group_done) return;
     __builtin_amdgcn_s_waitcnt(0);  // this wave's stores are complete
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -487,16 +448,15 @@ hipError_t launch_dd_relayout(const uint32_t* Dp, const uint32_t* Dm, size_t gst
 }
 
 static uint32_t collapse_mt(size_t nq) { return nq <= 4 ? 1 : nq <= 8 ? 2 : nq <= 16 ? 4 : 8; }  // 4 queries per tile
+size_t collapse_mp(size_t nq) { return 16 * collapse_mt(nq); }
 
-hipError_t launch_collapse_keys(const uint32_t* keys, size_t kstride, size_t nq, int8_t* kdig, uint32_t* KS,
-                                hipStream_t s) {
-    if (nq == 0 || nq > kCollapseMaxQueries) return hipErrorInvalidValue;
-    const uint32_t Mp = 16 * collapse_mt(nq);
-    const size_t nthr = 2 * (DD_K / 16) * (Mp / 4);
-    hipLaunchKernelGGL(k_kdigits, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, s, keys, kstride, (uint32_t)nq,
-                       Mp, kdig);
-    hipLaunchKernelGGL(k_ksum, dim3((unsigned)(2 * nq)), dim3(1024), 0, s, keys, kstride, KS);
-    return hipGetLastError();
+// Row slices of a collapse launch of `blocks` workgroups (2 limbs x tiles x
+// groups): a grid too small to fill the chip (one group, 16-column tiles:
+// 64 workgroups) splits its 4096-row contraction in up to 8 slices.
+static uint32_t collapse_ksplit(size_t blocks) {
+    uint32_t k = 1;
+    while (blocks * k < 512 && k < 8) k *= 2;
+    return k;
 }
 
 uint32_t pass_collapse_target(const DbPlan& p, size_t nq, size_t G) {
@@ -504,26 +464,33 @@ uint32_t pass_collapse_target(const DbPlan& p, size_t nq, size_t G) {
     return (uint32_t)(2 * (N / (64 * cnt)) + (N / dbplan_cols(p)) * p.slices);
 }
 
-hipError_t launch_pass_collapse_stream(const uint8_t* db, const int8_t* dig, const uint32_t* S, size_t nq,
-                                       uint32_t* out, size_t out_qstride, size_t R, size_t C, const DbPlan& p,
-                                       const uint32_t* precomp, const int8_t* kdig, const uint32_t* KS,
-                                       uint32_t* part2, size_t p2_stride, uint32_t* group_done, hipStream_t s) {
+// Row slices of the collapse in a counter-less pass_collapse launch.
+uint32_t pass_collapse_ksplit(size_t nq, size_t G) {
+    const uint32_t cnt = collapse_mt(nq) == 1 && G < 16 ? 1 : 2;
+    return collapse_ksplit(2 * (N / (64 * cnt)) * G);
+}
+
+hipError_t launch_pass_collapse(const uint8_t* db, const int8_t* dig, const uint32_t* S, size_t nq, uint32_t* out,
+                                size_t out_qstride, size_t R, size_t C, const DbPlan& p, const uint32_t* precomp,
+                                const int8_t* kdig, const uint32_t* KS, uint32_t* part2, size_t p2_stride,
+                                uint32_t* group_done, hipStream_t s) {
     const size_t G = C / N;
-    if (p.kind != DbPlan::MFMA || p.param > 4 || nq == 0 || nq > 8 || nq > dbplan_max_queries(p) || C % N ||
-        !group_done || p.slices == 0 || (p.slices & (p.slices - 1)) || dbplan_cols(p) != 256)
+    if (!pass_collapse_ok(p, nq) || nq > dbplan_max_queries(p) || C % N || p.slices == 0 ||
+        (p.slices & (p.slices - 1)))
         return hipErrorInvalidValue;
     const uint32_t kbps = (uint32_t)(R / 16 / p.slices);
     if (kbps % 8 || kbps == 0) return hipErrorInvalidValue;
     uint32_t sh = 0;
     while ((1u << sh) < p.slices) sh++;
     const uint32_t cmt = collapse_mt(nq), cnt = cmt == 1 && G < 16 ? 1 : 2;
-    const size_t blocks = G * pass_collapse_target(p, nq, G);
+    const uint32_t ks = group_done ? 1 : pass_collapse_ksplit(nq, G);
+    const size_t blocks = G * (2 * (N / (64 * cnt)) * ks + (N / dbplan_cols(p)) * p.slices);
     if (blocks > 0x7fffffffu) return hipErrorInvalidValue;
     const dim3 grid((unsigned)blocks);
     const uint32_t Cc = (uint32_t)C, Q = (uint32_t)nq, Gg = (uint32_t)G;
 #define PCS(PMT, CMT, CNT)                                                                                    \
     hipLaunchKernelGGL((k_pass_collapse_stream<PMT, 4, CMT, CNT>), grid, dim3(256), 0, s, db, dig, S, out, \
-                       out_qstride, Cc, kbps, precomp, kdig, KS, part2, p2_stride, Q, Gg, sh, group_done)
+                       out_qstride, Cc, kbps, precomp, kdig, KS, part2, p2_stride, Q, Gg, sh, ks, group_done)
     switch (p.param * 10 + cmt) {
         case 11: if (cnt == 1) PCS(1, 1, 1); else PCS(1, 1, 2); break;
         case 21: if (cnt == 1) PCS(2, 1, 1); else PCS(2, 1, 2); break;
@@ -543,24 +510,26 @@ __global__ __launch_bounds__(256) void k_zero_rows(uint32_t* __restrict__ p, siz
 }
 }  // namespace
 
-// Row slices of a collapse launch of `blocks` workgroups (2 limbs x tiles x
-// groups): a grid too small to fill the chip (one group, 16-column tiles:
-// 64 workgroups) splits its 4096-row contraction in up to 8 slices.
-static uint32_t collapse_ksplit(size_t blocks) {
-    uint32_t k = 1;
-    while (blocks * k < 512 && k < 8) k *= 2;
-    return k;
+uint32_t collapse_row_slices(size_t nq, size_t ng, int variant) {
+    // 16-column tiles per workgroup, as launched below
+    uint32_t cols;
+    switch (collapse_mt(nq)) {
+        case 1: cols = ng < 16 ? 64 : ng < 32 ? 128 : 256; break;
+        case 2: case 4: cols = 128; break;
+        default: cols = variant >= 3 ? 128 : 64; break;
+    }
+    return collapse_ksplit((size_t)(N / cols) * 2 * ng);
 }
 
 hipError_t launch_collapse(const uint32_t* precomp_g0, size_t ng, const int8_t* kdig, const uint32_t* KS, size_t nq,
-                           uint32_t* part2_g0, size_t p2_stride, hipStream_t s, int variant) {
+                           uint32_t* part2_g0, size_t p2_stride, hipStream_t s, int variant, bool zeroed) {
     if (nq == 0 || nq > kCollapseMaxQueries || variant < 0 || variant >= kCollapseVariants) return hipErrorInvalidValue;
     if (ng == 0) return hipSuccess;
     const uint32_t Q = (uint32_t)nq;
     // a split launch adds its slices' residues into part2, zeroed first
     auto split = [&](unsigned gx) {
         const uint32_t ks = collapse_ksplit((size_t)gx * 2 * ng);
-        if (ks > 1) {
+        if (ks > 1 && !zeroed) {
             const size_t row = ng * 2 * N, total = nq * row;
             hipLaunchKernelGGL(k_zero_rows, dim3((unsigned)((total + 255) / 256 < 1024 ? (total + 255) / 256 : 1024)),
                                dim3(256), 0, s, part2_g0, p2_stride, row, total);

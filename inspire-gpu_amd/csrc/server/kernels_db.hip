@@ -123,37 +123,6 @@ __global__ __launch_bounds__(256) void k_dbpass_f64(const uint8_t* __restrict__ 
 // rows 4*(l/16)+i, col l%16 in element i. A lane thus owns all four digits
 // of one pair for one column and recombines them locally.
 
-// dig for query pairs [0, 2*nq) and zero digits for padding pairs < Mp/4.
-__global__ __launch_bounds__(256) void k_digits(const double* __restrict__ bq, uint32_t R, uint32_t nq,
-                                                uint32_t Mp, int8_t* __restrict__ dig) {
-    const uint32_t nkb = R / 16;
-    const uint32_t x = blockIdx.x * 256 + threadIdx.x;
-    if (x >= nkb * (Mp / 4)) return;
-    const uint32_t pr = x / nkb, kb = x % nkb;
-    u32x4 o[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) o[k] = u32x4{0, 0, 0, 0};
-    if (pr < 2 * nq) {
-        const double* b = bq + (size_t)pr * R + (size_t)kb * 16;  // bq [q][c][R] = [pr][R]
-#pragma unroll
-        for (int e = 0; e < 16; e++) {
-            int32_t v = (int32_t)(uint32_t)b[e];
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                int32_t d = v;
-                if (k < 3) {
-                    d = ((v & 255) ^ 128) - 128;  // balanced digit in [-128, 127]
-                    v = (v - d) >> 8;
-                }
-                o[k][e >> 2] |= ((uint32_t)d & 255u) << (8 * (e & 3));
-            }
-        }
-    }
-    u32x4* dst = reinterpret_cast<u32x4*>(dig + ((size_t)kb * Mp + (size_t)pr * 4) * 16);
-#pragma unroll
-    for (int k = 0; k < 4; k++) dst[k] = o[k];
-}
-
 // 7-digit rows (17..32 queries): both limbs of a query share one digit
 // expansion, that of the CRT value B_r in [0, Q0*Q1) with B_r = b_{q,c}[r]
 // mod q_c. sum_r v_r B_r is congruent to either limb's sum mod q_c, and
@@ -166,43 +135,6 @@ constexpr uint32_t pow_mod_c(uint64_t b, uint64_t e, uint64_t m) {
         if (e & 1) r = r * b % m;
     return (uint32_t)r;
 }
-constexpr uint32_t kQ1InvQ0 = pow_mod_c(Q1, Q0 - 2, Q0);  // Q0 is prime
-
-// pmajor: rows (Mp/7) k + q (the power-row form) instead of 7q + k.
-__global__ __launch_bounds__(256) void k_digits7(const double* __restrict__ bq, uint32_t R, uint32_t nq,
-                                                 uint32_t Mp, int8_t* __restrict__ dig, uint32_t pmajor) {
-    const uint32_t nkb = R / 16;
-    const uint32_t x = blockIdx.x * 256 + threadIdx.x;
-    if (x >= nkb * (Mp / 7)) return;
-    const uint32_t q = x / nkb, kb = x % nkb;
-    u32x4 o[7];
-#pragma unroll
-    for (int k = 0; k < 7; k++) o[k] = u32x4{0, 0, 0, 0};
-    if (q < nq) {
-        const double* b0 = bq + (size_t)q * 2 * R + (size_t)kb * 16;  // bq [q][c][R]
-        const double* b1 = b0 + R;
-#pragma unroll
-        for (int e = 0; e < 16; e++) {
-            const uint32_t r0 = (uint32_t)b0[e], r1 = (uint32_t)b1[e];
-            // Garner: B = r1 + Q1 * ((r0 - r1) * Q1^-1 mod Q0)
-            const uint32_t t = mul_mod(sub_mod(r0, r1 % Q0, Q0), kQ1InvQ0, 0);
-            int64_t v = (int64_t)r1 + (int64_t)Q1 * t;
-#pragma unroll
-            for (int k = 0; k < 7; k++) {
-                int64_t d = v;
-                if (k < 6) {
-                    d = ((v & 255) ^ 128) - 128;
-                    v = (v - d) >> 8;
-                }
-                o[k][e >> 2] |= ((uint32_t)d & 255u) << (8 * (e & 3));
-            }
-        }
-    }
-    u32x4* dst = reinterpret_cast<u32x4*>(dig + (size_t)kb * Mp * 16);
-#pragma unroll
-    for (int k = 0; k < 7; k++) dst[pmajor ? (Mp / 7) * k + q : 7 * q + k] = o[k];
-}
-
 // Residue mod q_c of one output of the 7-digit form from the dot products
 // t_k = 256*H_k + L_k (|t_k| < 2^38.01, at most 2^16 rows per slice):
 //   sum_k 256^k t_k + 32896*S_c.
@@ -243,24 +175,6 @@ __device__ __forceinline__ uint32_t pow_residue(const int32_t (&p)[8], uint32_t 
         s += (uint64_t)red64((uint64_t)(p[k] + off32), c) * (c ? w1[k - 4] : w0[k - 4]);
     return red64(s, c);
 }
-
-// S[pr] = sum_r b_pr[r] mod q_c, the DB-offset correction. One block of
-// 1024 lanes per pair, R a multiple of 2048: R/2048 16-byte loads per lane,
-// all in flight together (a one-query answer waits for this kernel).
-__global__ __launch_bounds__(1024) void k_bsum(const double* __restrict__ bq, uint32_t R, uint32_t* __restrict__ S) {
-    __shared__ uint64_t red[16];
-    const uint32_t pr = blockIdx.x;
-    const double2* b = reinterpret_cast<const double2*>(bq + (size_t)pr * R) + threadIdx.x;
-    uint64_t a = 0;
-#pragma unroll 16
-    for (uint32_t i = 0; i < R / 2048; i++) {
-        const double2 v = b[(size_t)i * 1024];
-        a += (uint64_t)v.x + (uint64_t)v.y;
-    }
-    const uint64_t sum = block_sum_u64<1024>(a, red);
-    if (threadIdx.x == 0) S[pr] = red64(sum, (int)(pr & 1));
-}
-
 
 // Column tile and row slice of this workgroup: the 2-D grid's, or in a
 // streamed pass the 1-D index read as (tile counted from the top, slice).
@@ -494,8 +408,8 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void k_dbpass_mfma_sa(const uint8_
                     for (int k = 0; k < 8; k++) pk[k] = acc[QT * k + h][n][0][i];
                     uint32_t* o = out + (size_t)q * out_qstride + (size_t)slice * 2 * OC + col0 + n * 16 + cl;
                     if (q < nq) {
-                        const uint32_t r0 = pow_residue(pk, slice == 0 ? S[2 * q] : 0, 0);
-                        const uint32_t r1 = pow_residue(pk, slice == 0 ? S[2 * q + 1] : 0, 1);
+                        const uint32_t r0 = pow_residue(pk, slice == 0 ? offset_sum(S, 2 * q) : 0, 0);
+                        const uint32_t r1 = pow_residue(pk, slice == 0 ? offset_sum(S, 2 * q + 1) : 0, 1);
                         o[0] = r0;
                         o[OC] = r1;
                     }
@@ -525,7 +439,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void k_dbpass_mfma_sa(const uint8_
                 if (q < nq) {
                     uint32_t* o = out + (size_t)q * out_qstride + (size_t)slice * 2 * OC + col0 + cl;
 #pragma unroll
-                    for (int c = 0; c < 2; c++) o[(size_t)c * OC] = crt7_residue(t, slice == 0 ? S[2 * q + c] : 0, c);
+                    for (int c = 0; c < 2; c++) o[(size_t)c * OC] = crt7_residue(t, slice == 0 ? offset_sum(S, 2 * q + c) : 0, c);
                 }
             }
             __syncthreads();  // the second half reuses the region
@@ -740,22 +654,6 @@ hipError_t launch_dbpass_f64(const uint8_t* db, const double* bq, uint32_t* out,
         default: F64(4); break;
     }
 #undef F64
-    return hipGetLastError();
-}
-
-hipError_t launch_mfma_digits(const double* bq, size_t nq, size_t R, const DbPlan& p, int8_t* dig, uint32_t* S,
-                              hipStream_t s) {
-    if (p.kind != DbPlan::MFMA || nq == 0 || nq > kMfmaMaxQueries || R % 2048) return hipErrorInvalidValue;
-    const uint32_t Mp = (uint32_t)dbplan_mp(p);
-    if (nq > dbplan_max_queries(p)) return hipErrorInvalidValue;
-    const size_t nthr = (R / 16) * (p.crt ? Mp / 7 : Mp / 4);
-    const dim3 grid((unsigned)((nthr + 255) / 256));
-    if (p.crt)
-        hipLaunchKernelGGL(k_digits7, grid, dim3(256), 0, s, bq, (uint32_t)R, (uint32_t)nq, Mp, dig,
-                           (uint32_t)p.pow);
-    else
-        hipLaunchKernelGGL(k_digits, grid, dim3(256), 0, s, bq, (uint32_t)R, (uint32_t)nq, Mp, dig);
-    hipLaunchKernelGGL(k_bsum, dim3((unsigned)(2 * nq)), dim3(1024), 0, s, bq, (uint32_t)R, S);
     return hipGetLastError();
 }
 

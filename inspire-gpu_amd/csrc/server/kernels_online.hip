@@ -21,30 +21,6 @@ constexpr size_t BLK = (size_t)D_EFF * 2 * N;  // one key / RGSW part, u32 words
 // clocks); 4, 8, 16 and 32 measured no different from 2 at the 16 GB tier
 constexpr int kSpinSleep = 2;
 
-// ------------------------------------------------------------ unmarshal
-// Flat u64 wire query -> per-slot device layout, reducing every residue
-// mod its limb's prime (the reference narrows ksk/RGSW words without
-// reduction, src/gpu_protocol.cu:1066 and :50; canonical inputs agree).
-__global__ __launch_bounds__(256) void k_unmarshal(const uint64_t* __restrict__ q, size_t total, size_t R,
-                                                   double* __restrict__ bq, uint32_t* __restrict__ keys,
-                                                   uint32_t* __restrict__ rgsw) {
-    const size_t qlen = 2 * R + 6 * BLK;
-    for (size_t x = (size_t)blockIdx.x * blockDim.x + threadIdx.x; x < total; x += (size_t)gridDim.x * blockDim.x) {
-        const size_t qi = x / qlen, off = x - qi * qlen;
-        const uint64_t v = q[x];
-        if (off < 2 * R) {
-            const int limb = off >= R;
-            bq[qi * 2 * R + off] = (double)red64(v, limb);
-        } else if (off < 2 * R + 2 * BLK) {
-            const size_t o = off - 2 * R;
-            keys[qi * 2 * BLK + o] = red64(v, (int)((o / N) & 1));
-        } else {
-            const size_t o = off - 2 * R - 2 * BLK;
-            rgsw[qi * 4 * BLK + o] = red64(v, (int)((o / N) & 1));
-        }
-    }
-}
-
 // ------------------------------------------------------------ batched NTT
 __global__ __launch_bounds__(256) void k_ntt_rns(uint32_t* __restrict__ polys, NttConst nc, int inverse) {
     __shared__ uint32_t buf[POLY_LDS];
@@ -62,6 +38,7 @@ __global__ __launch_bounds__(256) void k_ntt_rns(uint32_t* __restrict__ polys, N
 
 // ------------------------------------------------------------ slice reduction
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // interm[q][limb][col] = sum over row slices of part mod q_limb, for columns
 // col0 + [0, gridDim.x*256); blockIdx.y = limb, blockIdx.z = query. A
@@ -99,30 +76,106 @@ __global__ __launch_bounds__(256) void k_reduce_slices(const uint32_t* __restric
 // ------------------------------------------------------------ pack finalize
 // packed_b[q][g][c] = NTT(interm[q][c][gN..gN+N-1]) - part2[q][g][c]
 //                     - sum_j Df[g][c][j] * Kn[j][c]  (reference
-// src/gpu_protocol.cu:1225-1283, src/gpu_online.cu:547-592).
-__global__ __launch_bounds__(256) void k_pack_finalize(const uint32_t* __restrict__ interm, uint32_t C,
-                                                       const uint32_t* __restrict__ part2,
-                                                       size_t p2_stride,
-                                                       const uint32_t* __restrict__ precomp,
-                                                       const uint32_t* __restrict__ keys, size_t kstride,
-                                                       uint32_t* __restrict__ packed_b, size_t pstride,
-                                                       uint32_t g0, NttConst nc) {
-    __shared__ uint32_t buf[POLY_LDS];
-    const uint32_t g = g0 + blockIdx.x, c = blockIdx.y, qi = blockIdx.z, t = threadIdx.x;
-    const uint32_t q = qof((int)c);
-    const uint32_t* pp = interm + (size_t)qi * 2 * C + (size_t)c * C + (size_t)g * N;
+// src/gpu_protocol.cu:1225-1283, src/gpu_online.cu:547-592), where interm is
+// the sum of the database pass's row-slice partials (one slice: itself). A
+// workgroup per (group, limb, query) of TH lanes: they all sum slices, then
+// 256 of them transform in registers (ntt_regs.h). A chain of dependent
+// latencies, so every load that depends on nothing (twiddles, Df, Kn, the
+// collapse sums) is issued first. Summing here saves a pass over the
+// partials and a launch: at 0.13 GB the reduction and the pack took 4.6 +
+// 5.6 us and two launches. Where every chain is one ciphertext long (out set)
+// the response is written here as well, without a Horner launch (another 5
+// us).
+template <int TH>
+__global__ __launch_bounds__(TH) void k_pack_finalize(const uint32_t* __restrict__ part, size_t part_qstride,
+                                                      uint32_t slices, uint32_t C,
+                                                      const uint32_t* __restrict__ part2, size_t p2_stride,
+                                                      const uint32_t* __restrict__ precomp,
+                                                      const uint32_t* __restrict__ keys, size_t kstride,
+                                                      uint32_t* __restrict__ packed_b, size_t pstride, uint32_t g0,
+                                                      uint64_t* __restrict__ out, NttConst nc) {
+    __shared__ __align__(16) uint32_t buf[1][POLY4_LDS];
+    const uint32_t g = g0 + blockIdx.x, c = blockIdx.y, qi = blockIdx.z, tid = threadIdx.x, t = tid & 255;
+    const bool lead = __builtin_amdgcn_readfirstlane((int)(tid >> 8)) == 0;
+    const NrLimb m = nr_limb((int)c);
+    const uint32_t* pp = part + (size_t)qi * part_qstride + (size_t)c * C + (size_t)g * N;
+    const size_t sstride = 2 * (size_t)C;
+    const uint32_t* pc = precomp + (size_t)g * PC_GROUP;
+    uint32_t x[1][8];
+    NrTw tw[4];
+    u32x4 d0[2], d1[2], k0[2], k1[2], s2[2];
+    if (lead) {
+        nr_tw_global(tw, nc, (int)c, t);
+        const u32x4* Df = reinterpret_cast<const u32x4*>(pc + PC_DF + (size_t)c * D_EFF * N + 8 * t);
+        const u32x4* Kn =  // key 1 = ksk_neg1, [digit][limb][N]
+            reinterpret_cast<const u32x4*>(keys + (size_t)qi * kstride + BLK + (size_t)c * N + 8 * t);
+        const u32x4* p2 = reinterpret_cast<const u32x4*>(part2 + (size_t)qi * p2_stride + (size_t)g * 2 * N +
+                                                         (size_t)c * N + 8 * t);
 #pragma unroll
-    for (int k = 0; k < 8; k++) buf[ls(t + 256 * k)] = pp[t + 256 * k];
+        for (int h = 0; h < 2; h++) {
+            d0[h] = Df[h];
+            d1[h] = Df[N / 4 + h];
+            k0[h] = Kn[h];
+            k1[h] = Kn[2 * N / 4 + h];
+            s2[h] = p2[h];
+        }
+    }
+    if (TH == 256) {
+        if (slices == 1) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) x[0][k] = pp[t + 256 * k];
+        } else {  // 2..4 slices: up to 32 loads in flight
+            uint32_t a[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // residues below 2^27
+#pragma unroll
+            for (uint32_t s = 0; s < 4; s++)
+                if (s < slices)
+#pragma unroll
+                    for (int k = 0; k < 8; k++) a[k] += pp[s * sstride + t + 256 * k];
+#pragma unroll
+            for (int k = 0; k < 8; k++) x[0][k] = a[k];  // up to 4q
+        }
+    } else {
+        // lane: 2 columns of every slice, 16 loads in flight
+        const u32x2* p = reinterpret_cast<const u32x2*>(pp) + tid;
+        uint64_t a0 = 0, a1 = 0;
+#pragma unroll 16
+        for (uint32_t s = 0; s < slices; s++) {
+            const u32x2 v = p[s * (sstride / 2)];
+            a0 += v.x;
+            a1 += v.y;
+        }
+        const uint32_t e = 2 * tid, w = e + 4 * (e >> 5);
+        *reinterpret_cast<u32x2*>(&buf[0][w]) = u32x2{red64(a0, (int)c), red64(a1, (int)c)};
+        __syncthreads();
+        if (lead) nr_load<0, 1>(buf, x, t);
+    }
+    nr_forward1(x, buf, tw, t, m, lead);
+    if (lead) {
+        u32x4* dst = reinterpret_cast<u32x4*>(packed_b + (size_t)qi * pstride + (size_t)g * 2 * N + (size_t)c * N + 8 * t);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            u32x4 r;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint64_t sub = (uint64_t)d0[h][e] * k0[h][e] + (uint64_t)d1[h][e] * k1[h][e] + s2[h][e];
+                const uint32_t v = fold(nr_reduce(x[0][4 * h + e], m), m.q);  // from at most 26q
+                r[e] = sub_mod(v, red64(sub, (int)c), m.q);
+                x[0][4 * h + e] = r[e];
+            }
+            dst[h] = r;
+        }
+    }
+    if (!out) return;
+    // a chain of one ciphertext: [a|b][limb][N] u64, whole lines through LDS
+    if (lead) nr_store<3, 1>(buf, x, t);
     __syncthreads();
-    ntt_fwd_lds(buf, t, tw_global(nc, (int)c), (int)c);
-    const uint32_t* Df = precomp + (size_t)g * PC_GROUP + PC_DF + (size_t)c * D_EFF * N;
-    const uint32_t* Kn = keys + qi * kstride + BLK + (size_t)c * N;  // key 1 = ksk_neg1, [digit][limb][N]
-    const uint32_t* p2 = part2 + qi * p2_stride + (size_t)g * 2 * N + (size_t)c * N;
+    if (!lead) return;
+    uint64_t* o = out + (size_t)qi * 4 * N + (size_t)c * N + t;
+    const uint32_t* pa = pc + PC_A + (size_t)c * N + t;
 #pragma unroll
     for (int k = 0; k < 8; k++) {
-        const uint32_t i = t + 256 * k;
-        const uint64_t sub = (uint64_t)Df[i] * Kn[i] + (uint64_t)Df[N + i] * Kn[2 * N + i] + p2[i];
-        packed_b[qi * pstride + (size_t)g * 2 * N + (size_t)c * N + i] = sub_mod(buf[ls(i)], red64(sub, (int)c), q);
+        o[256 * k] = pa[256 * k];
+        o[2 * N + 256 * k] = buf[0][nr_base(0, t) + nr_stride<0>() * k];
     }
 }
 
@@ -515,15 +568,6 @@ __global__ __launch_bounds__(1024) void k_pack_stream(PackStream ps, const uint3
 
 }  // namespace
 
-hipError_t launch_unmarshal(const uint64_t* d_q, size_t count, size_t R, double* bq, uint32_t* keys,
-                            uint32_t* rgsw, hipStream_t s) {
-    const size_t total = count * (2 * R + 6 * BLK);
-    size_t blocks = (total + 255) / 256;
-    if (blocks > 8192) blocks = 8192;
-    hipLaunchKernelGGL(k_unmarshal, dim3((unsigned)blocks), dim3(256), 0, s, d_q, total, R, bq, keys, rgsw);
-    return hipGetLastError();
-}
-
 namespace {
 // Plain grid-stride copy, 16 bytes per lane: the reference point that
 // scales the memory-traffic counters of the other kernels.
@@ -556,13 +600,20 @@ hipError_t launch_reduce_slices(const uint32_t* part, size_t part_stride, uint32
     return hipGetLastError();
 }
 
-hipError_t launch_pack_finalize(const uint32_t* interm, size_t C, const uint32_t* part2, size_t part2_stride,
-                                const uint32_t* precomp, size_t g0, size_t ng, const uint32_t* keys,
-                                size_t keys_stride, uint32_t* packed_b, size_t packed_stride, size_t nq,
-                                const NttConst& nc, hipStream_t s) {
+hipError_t launch_pack_finalize(const uint32_t* part, size_t part_qstride, uint32_t slices, size_t C,
+                                const uint32_t* part2, size_t part2_stride, const uint32_t* precomp, size_t g0,
+                                size_t ng, const uint32_t* keys, size_t keys_stride, uint32_t* packed_b,
+                                size_t packed_stride, size_t nq, const NttConst& nc, hipStream_t s, uint64_t* out) {
     if (ng == 0 || nq == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_pack_finalize, dim3((unsigned)ng, 2, (unsigned)nq), dim3(256), 0, s, interm, (uint32_t)C,
-                       part2, part2_stride, precomp, keys, keys_stride, packed_b, packed_stride, (uint32_t)g0, nc);
+    if (slices == 0 || (out && (g0 != 0 || ng != 1 || C != N))) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)ng, 2, (unsigned)nq);
+    // from 5 slices on the sums take 1024 lanes
+    if (slices > 4)
+        hipLaunchKernelGGL(k_pack_finalize<1024>, grid, dim3(1024), 0, s, part, part_qstride, slices, (uint32_t)C, part2,
+                           part2_stride, precomp, keys, keys_stride, packed_b, packed_stride, (uint32_t)g0, out, nc);
+    else
+        hipLaunchKernelGGL(k_pack_finalize<256>, grid, dim3(256), 0, s, part, part_qstride, slices, (uint32_t)C, part2,
+                           part2_stride, precomp, keys, keys_stride, packed_b, packed_stride, (uint32_t)g0, out, nc);
     return hipGetLastError();
 }
 

@@ -226,6 +226,53 @@ __device__ __forceinline__ void nr_forward(uint32_t (&x)[P][8], uint32_t (*buf)[
     nr_fwd_phase<P, false>(x, w, m);
 }
 
+// The four phases' twiddles of lane t from the device tables, all loads in
+// flight together: for kernels that transform one polynomial and leave.
+__device__ __forceinline__ void nr_tw_global(NrTw (&w)[4], const NttConst& nc, int c, uint32_t t) {
+    const uint32_t* f = nc.tw + (size_t)c * 4 * N;
+    const uint32_t* fp = f + N;
+#pragma unroll
+    for (int ph = 0; ph < 4; ph++) {
+        const uint32_t A = nr_node(ph, t);
+        const nr_u32x2 b = *reinterpret_cast<const nr_u32x2*>(f + 2 * A);
+        const nr_u32x2 bp = *reinterpret_cast<const nr_u32x2*>(fp + 2 * A);
+        const nr_u32x4 q = *reinterpret_cast<const nr_u32x4*>(f + 4 * A);
+        const nr_u32x4 qp = *reinterpret_cast<const nr_u32x4*>(fp + 4 * A);
+        if (ph < 3) w[ph].a = nr_u32x2{f[A], fp[A]};
+#pragma unroll
+        for (int h = 0; h < 2; h++) w[ph].b[h] = nr_u32x2{b[h], bp[h]};
+#pragma unroll
+        for (int h = 0; h < 4; h++) w[ph].c[h] = nr_u32x2{q[h], qp[h]};
+    }
+}
+// Forward transform of one polynomial with those twiddles (bounds and
+// layout as nr_forward; every lane of the workgroup calls it, lanes of other
+// teams with active = false).
+__device__ __forceinline__ void nr_forward1(uint32_t (&x)[1][8], uint32_t (*buf)[POLY4_LDS], const NrTw (&w)[4],
+                                            uint32_t t, const NrLimb& m, bool active = true) {
+    if (active) {
+        nr_fwd_phase<1, true>(x, w[0], m);
+        nr_store<0, 1>(buf, x, t);
+    }
+    __syncthreads();
+    if (active) {
+        nr_load<1, 1>(buf, x, t);
+        nr_fwd_phase<1, true>(x, w[1], m);
+        nr_store<1, 1>(buf, x, t);
+    }
+    __syncthreads();
+    if (active) {
+        nr_load<2, 1>(buf, x, t);
+        nr_fwd_phase<1, true>(x, w[2], m);
+        nr_store<2, 1>(buf, x, t);
+    }
+    __syncthreads();
+    if (active) {
+        nr_load<3, 1>(buf, x, t);
+        nr_fwd_phase<1, false>(x, w[3], m);
+    }
+}
+
 // Inverse transform without its N^-1 scale: in, NTT slots 8t + k up to
 // 5q; out, coefficients t + 256k up to 32q. buf as above, with the words
 // 8t + k (own) free.

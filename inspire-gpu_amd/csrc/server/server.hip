@@ -8,6 +8,7 @@
 // groups lives in one arena (one allocation, fixed group stride), the
 // answer pipeline is a fixed sequence of batched kernels on one stream (no
 // per-group launches), and errors surface as exceptions instead of exit().
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -299,6 +300,10 @@ DbPlan narrow_plan(const DbPlan& full, size_t target, size_t R, size_t C, size_t
 }
 }  // namespace
 
+// Tables (with their tensors) up to this size run the pass and the collapse
+// of up to 8 queries in one launch.
+constexpr size_t kMergeBytes = (size_t)1 << 30;
+
 size_t default_group_chunk(size_t G) {
     // group chunks of the pipelined answer: about 8, of at least 8 groups
     return G / 8 >= 8 ? G / 8 : (G < 8 ? G : 8);
@@ -337,7 +342,8 @@ ServerFootprint server_footprint(const PublicParams& pp, size_t gchunk) {
                  (horner_pair_xbuf_words(T) + 2 * T + T * 4 * N) * 4 +
                  query_packed_bytes(R) + T * 4 * N * 4 + T * GpuServerCtx::kCompressedCtBytes;
     f.fixed = R * C * 2 + G * PC_GROUP * 4 + 8 * N * 4 +
-              GpuServerCtx::kLanes * (R * 256 + GpuServerCtx::kKdigBytes + 2 * 64 * 4 + 4);
+              GpuServerCtx::kLanes *
+                  (R * 256 + GpuServerCtx::kKdigBytes + (GpuServerCtx::kSumWords + GpuServerCtx::kKeySumWords) * 4 + 4);
     // streamed answers' flags: one set per lane and 32 slots (rounded up)
     const size_t set_bytes = GpuServerCtx::kStreamSetWords * G * 4;
     f.fixed += GpuServerCtx::kLanes * set_bytes;
@@ -393,9 +399,9 @@ void GpuServerCtx::alloc_slots() {
     d_packed_b = dalloc<uint32_t>(B * packed_stride);
     for (int l = 0; l < kLanes; l++) {
         d_dig[l] = dalloc<int8_t>(R * 256);
-        d_S[l] = dalloc<uint32_t>(64);
+        d_S[l] = dalloc<uint32_t>(kSumWords);
         d_kdig[l] = dalloc<int8_t>(kKdigBytes);
-        d_KS[l] = dalloc<uint32_t>(64);
+        d_KS[l] = dalloc<uint32_t>(kKeySumWords);
     }
     d_hstate = dalloc<uint32_t>(B * T * 4 * N);
     trace_name_stream(stream, "server");
@@ -460,7 +466,6 @@ void GpuServerCtx::alloc_slots() {
     d_qpack = dalloc<uint8_t>(B * qpack_bytes);
     d_cmp = dalloc<uint32_t>(B * T * 4 * N);
     d_rcmp = dalloc<uint8_t>(B * T * kCompressedCtBytes);
-    HIPX(hipMemset(d_bq, 0, B * 2 * R * sizeof(double)));
     HIPX(hipHostMalloc((void**)&h_q, B * qlen * 8, hipHostMallocDefault));
     HIPX(hipHostMalloc((void**)&h_resp, B * resp_u64s * 8, hipHostMallocDefault));
     resident_bytes = fp.fixed + B * fp.per_slot;
@@ -512,7 +517,7 @@ void GpuServerCtx::autotune_dbpass() {
     // within tens of milliseconds, so timing the candidates one after
     // another would favour whichever ran first.
     auto fastest = [&](size_t n, auto&& prep, auto&& run, int rounds = 4) {
-        std::vector<float> tot(n, 0.f);
+        std::vector<std::vector<float>> got(n);
         for (int round = 0; round < rounds; round++)
             for (size_t i = 0; i < n; i++) {
                 prep(i);
@@ -522,17 +527,20 @@ void GpuServerCtx::autotune_dbpass() {
                 HIPX(hipEventSynchronize(e1));
                 float ms = 0;
                 HIPX(hipEventElapsedTime(&ms, e0, e1));
-                if (round) tot[i] += ms;
+                if (round) got[i].push_back(ms);
             }
+        // the lower median: one disturbed round does not decide
         size_t b = 0;
-        for (size_t i = 1; i < n; i++)
-            if (tot[i] < tot[b]) b = i;
+        for (size_t i = 0; i < n; i++) {
+            std::sort(got[i].begin(), got[i].end());
+            if (got[i][(got[i].size() - 1) / 2] < got[b][(got[b].size() - 1) / 2]) b = i;
+        }
         return b;
     };
     // one full-width database pass of plan x over nq staged queries (zeroed)
-    auto prep_plan = [&](const DbPlan& x, size_t nq) {
-        if (x.kind == DbPlan::MFMA) HIPX(launch_mfma_digits(d_bq, nq, R, x, d_dig[0], d_S[0], stream));
-    };
+    const size_t nq = cfg.max_batch < kMfmaMaxQueries ? cfg.max_batch : kMfmaMaxQueries;
+    HIPX(hipMemset(d_q, 0, nq * qlen * 8));
+    auto prep_plan = [&](const DbPlan& x, size_t n) { prep_lwe(d_q, qlen, 0, n, x, stream, 0); };
     auto run_plan = [&](const DbPlan& x, size_t nq) {
         if (x.kind == DbPlan::F64)
             HIPX(launch_dbpass_f64(db_planes(), d_bq, d_part, C, R, C, 0, C, x, stream));
@@ -560,7 +568,6 @@ void GpuServerCtx::autotune_dbpass() {
     // batched pass: target, depth and form at the largest batch this context
     // serves, and apart for 9..16 queries when that batch is larger (their
     // best form differs)
-    const size_t nq = cfg.max_batch < kMfmaMaxQueries ? cfg.max_batch : kMfmaMaxQueries;
     auto tune_batched = [&](size_t nqc, size_t& target_out, uint32_t& depth_out, int& form_out) {
         const uint32_t param = dbplan_mfma(R, C, nqc, target_out).param;
         // forms (dbplan_form): the shared DB tile and the 7-digit forms
@@ -613,8 +620,7 @@ void GpuServerCtx::autotune_dbpass() {
         }
         // the 17..32-query collapse pass form, over all groups (zeroed keys)
         if (nq > 16) {
-            HIPX(hipMemset(d_keys, 0, nq * keys_stride * 4));
-            HIPX(launch_collapse_keys(d_keys, keys_stride, nq, d_kdig[0], d_KS[0], stream));
+            prep_query(d_q, 0, nq, plan_for(nq, C), stream, 0);
             collapse_variant = (int)fastest(
                 (size_t)kCollapseVariants, [](size_t) {},
                 [&](size_t v) {
@@ -638,7 +644,6 @@ void GpuServerCtx::autotune_dbpass() {
     const bool chunked_ok = G / gchunk > 1;
     if (chunked_ok || can_stream(stream)) {
         const size_t ccols = gchunk * N;
-        HIPX(hipMemset(d_q, 0, nq * qlen * 8));
         for (const size_t count : {(size_t)1, nq}) {
             const DbPlan full = plan_for(count, C);
             const size_t blocks = ccols / dbplan_cols(full);
@@ -651,7 +656,21 @@ void GpuServerCtx::autotune_dbpass() {
             // the serial answer: with many chunks it can still win where a
             // sub-batch's Horner chains hold many of the CUs the chunked
             // passes would run beside them
-            if (!pipe_forced || forced == 0 || (!chunked_ok && forced < 6 && forced != 3)) cands.push_back({0, 0});
+            // of a table too small to chunk, also at other row slices than its
+            // plan's, which was timed without what reads its partials: the
+            // collapse beside the pass keeps the CUs busy, and each slice is
+            // more for the pack to sum
+            if (!pipe_forced || forced == 0 || (!chunked_ok && forced < 6 && forced != 3)) {
+                cands.push_back({0, 0});
+                const uint32_t most = count == 1 ? 64 : full.kind == DbPlan::MFMA ? full.slices / 2 : 0;
+                for (uint32_t sl = most; !chunked_ok && sl && sl * 16 > most; sl /= 2) {
+                    (count == 1 ? serial_slices1 : serial_slices) = sl;
+                    serial_param = full.param;
+                    if (serial_plan(count).slices == sl) cands.push_back({sl, 0});
+                }
+                serial_slices1 = count == 1 ? 0 : serial_slices1;
+                serial_slices = count == 1 ? serial_slices : 0;
+            }
             // one chunk: the collapse beside the whole pass (the two branches'
             // small kernels and launch gaps overlap)
             if (!chunked_ok && (!pipe_forced || forced == 3)) cands.push_back({0, 3});
@@ -690,11 +709,14 @@ void GpuServerCtx::autotune_dbpass() {
             auto use = [&](const Pick& p) {
                 const bool st = p.shape >= 6;
                 if (count == 1) {
-                    if (st) stream_slices1 = p.slices; else chunk_slices1 = p.slices;
+                    (st ? stream_slices1 : p.shape == 0 ? serial_slices1 : chunk_slices1) = p.slices;
                     if (!pipe_forced) pipe_single = p.shape;
                 } else {
                     if (st) {
                         stream_slices = p.slices;
+                    } else if (p.shape == 0) {
+                        serial_slices = p.slices;
+                        serial_param = full.param;
                     } else {
                         chunk_slices = p.slices;
                         chunk_param = p.slices ? full.param : 0;
@@ -727,10 +749,38 @@ void GpuServerCtx::autotune_dbpass() {
     (void)hipEventDestroy(e1);
 }
 
-void GpuServerCtx::stage_prep(const uint64_t* d_in, size_t count, hipStream_t s, size_t slot0) {
-    HIPX(launch_unmarshal(d_in, count, pp.db_rows, d_bq + slot0 * 2 * pp.db_rows, d_keys + slot0 * keys_stride,
-                          d_rgsw + slot0 * rgsw_stride, s));
-    HIPX(launch_ntt_rns(d_keys + slot0 * keys_stride, count * 2 * D_EFF, nc, false, s));
+PrepArgs GpuServerCtx::prep_args(const uint64_t* d_in, size_t stride, size_t q0, int lane) const {
+    PrepArgs a;
+    a.q = d_in;
+    a.q_stride = stride;
+    a.R = pp.db_rows;
+    a.bq = d_bq + q0 * 2 * pp.db_rows;
+    a.dig = d_dig[lane];
+    a.S = d_S[lane];
+    return a;
+}
+
+void GpuServerCtx::prep_lwe(const uint64_t* d_in, size_t stride, size_t q0, size_t nq, const DbPlan& p, hipStream_t s,
+                            int lane) {
+    HIPX(launch_prep(prep_args(d_in, stride, q0, lane), nq, p, nc, s));
+}
+
+void GpuServerCtx::prep_query(const uint64_t* d_in, size_t q0, size_t nq, const DbPlan& p, hipStream_t s, int lane,
+                              const PrepZero& z) {
+    PrepArgs a = prep_args(d_in, qlen, q0, lane);
+    a.keys = d_keys + q0 * keys_stride;
+    a.keys_stride = keys_stride;
+    a.rgsw = d_rgsw + q0 * rgsw_stride;
+    a.rgsw_stride = rgsw_stride;
+    a.kdig = d_kdig[lane];
+    a.KS = d_KS[lane];
+    a.skip_lwe = z.skip_lwe;
+    a.zero = z.flags;
+    a.zero_words = z.flag_words;
+    a.part2 = d_part2 + q0 * part2_stride;
+    a.part2_stride = part2_stride;
+    a.part2_words = z.part2 ? G * 2 * N : 0;
+    HIPX(launch_prep(a, nq, p, nc, s));
 }
 
 DbPlan GpuServerCtx::plan_for(size_t nq, size_t ncols) const {
@@ -861,9 +911,24 @@ bool GpuServerCtx::can_stream(hipStream_t s) const {
     return cap == hipStreamCaptureStatusNone;
 }
 
-void GpuServerCtx::dbpass_prep(size_t q0, size_t nq, const DbPlan& p, hipStream_t s, int lane) {
-    if (p.kind == DbPlan::MFMA)
-        HIPX(launch_mfma_digits(d_bq + q0 * 2 * pp.db_rows, nq, pp.db_rows, p, d_dig[lane], d_S[lane], s));
+uint32_t* GpuServerCtx::pass_out(size_t q0, const DbPlan& p, size_t& qstride) {
+    // one slice: straight into interm; else row-slice partials
+    const size_t C = pp.db_cols;
+    if (p.slices > 1 && (size_t)p.slices * 2 * C > part_stride)
+        throw std::logic_error("database pass: row-slice partials exceed their buffer");
+    qstride = p.slices == 1 ? 2 * C : part_stride;
+    return p.slices == 1 ? d_interm + q0 * 2 * C : d_part + q0 * part_stride;
+}
+
+void GpuServerCtx::dbpass_whole(size_t q0, size_t nq, const DbPlan& p, hipStream_t s, int lane) {
+    const size_t R = pp.db_rows, C = pp.db_cols;
+    size_t qstride;
+    uint32_t* out = pass_out(q0, p, qstride);
+    if (p.kind == DbPlan::F64)
+        for (size_t q = 0; q < nq; q++)
+            HIPX(launch_dbpass_f64(db_planes(), d_bq + (q0 + q) * 2 * R, out + q * qstride, C, R, C, 0, C, p, s));
+    else
+        HIPX(launch_dbpass_mfma(db_planes(), d_dig[lane], d_S[lane], nq, out, qstride, C, R, C, 0, C, p, s));
 }
 
 void GpuServerCtx::dbpass_range(size_t q0, size_t nq, size_t g_lo, size_t g_hi, const DbPlan& p, hipStream_t s,
@@ -889,33 +954,29 @@ void GpuServerCtx::dbpass_range(size_t q0, size_t nq, size_t g_lo, size_t g_hi, 
                                   ncols, s));
 }
 
-void GpuServerCtx::stage_dbpass(size_t count, hipStream_t s, size_t slot0, int lane, int force) {
-    const size_t R = pp.db_rows, C = pp.db_cols;
-    const size_t step = force == 0 ? 1 : kMfmaMaxQueries;
-    for (size_t q0 = slot0; q0 < slot0 + count; q0 += step) {
-        const size_t nq = slot0 + count - q0 < step ? slot0 + count - q0 : step;
-        DbPlan p = plan_for(nq, C);
-        if (force == 0 && p.kind != DbPlan::F64) p = dbplan_f64(R, C, 4, 2048);
-        if (force == 1 && p.kind == DbPlan::F64)
-            p = dbplan_form(R, C, nq, mfma_target, mfma_depth, mfma_form);
-        dbpass_prep(q0, nq, p, s, lane);
-        dbpass_range(q0, nq, 0, G, p, s, lane);
-    }
+DbPlan GpuServerCtx::serial_plan(size_t nq) const {
+    DbPlan p = plan_for(nq, pp.db_cols);
+    const uint32_t sl = nq == 1 ? serial_slices1 : serial_slices;
+    if (!sl) return p;
+    DbPlan x = nq == 1 ? dbplan_mfma(pp.db_rows, pp.db_cols, 1, 1) : p;
+    x.slices = sl;  // timed for plans of this kernel
+    const bool ok = x.kind == DbPlan::MFMA && (nq == 1 || (x.param == serial_param && sl < p.slices)) &&
+                    pp.db_rows / sl <= (x.pow ? 32768u : 65536u) && pp.db_rows / 16 / sl % 8 == 0 &&
+                    (sl == 1 || (size_t)sl * 2 * pp.db_cols <= part_stride);
+    return ok ? x : p;
 }
 
-void GpuServerCtx::stage_collapse(size_t count, hipStream_t s, size_t slot0, int lane) {
-    for (size_t q0 = slot0; q0 < slot0 + count; q0 += kCollapseMaxQueries) {
-        const size_t nq = slot0 + count - q0 < kCollapseMaxQueries ? slot0 + count - q0 : kCollapseMaxQueries;
-        HIPX(launch_collapse_keys(d_keys + q0 * keys_stride, keys_stride, nq, d_kdig[lane], d_KS[lane], s));
-        HIPX(launch_collapse(d_precomp, G, d_kdig[lane], d_KS[lane], nq, d_part2 + q0 * part2_stride, part2_stride,
-                             s, collapse_variant));
-    }
+void GpuServerCtx::collapse_whole(size_t q0, size_t nq, hipStream_t s, int lane, bool zeroed) {
+    HIPX(launch_collapse(d_precomp, G, d_kdig[lane], d_KS[lane], nq, d_part2 + q0 * part2_stride, part2_stride, s,
+                         collapse_variant, zeroed));
 }
 
-void GpuServerCtx::stage_finalize(size_t count, hipStream_t s, size_t slot0) {
-    HIPX(launch_pack_finalize(d_interm + slot0 * 2 * pp.db_cols, pp.db_cols, d_part2 + slot0 * part2_stride,
-                              part2_stride, d_precomp, 0, G, d_keys + slot0 * keys_stride, keys_stride,
-                              d_packed_b + slot0 * packed_stride, packed_stride, count, nc, s));
+void GpuServerCtx::pack_whole(size_t q0, size_t nq, const DbPlan& p, hipStream_t s, uint64_t* d_out) {
+    size_t qstride;
+    const uint32_t* part = pass_out(q0, p, qstride);
+    HIPX(launch_pack_finalize(part, qstride, p.slices, pp.db_cols, d_part2 + q0 * part2_stride, part2_stride,
+                              d_precomp, 0, G, d_keys + q0 * keys_stride, keys_stride, d_packed_b + q0 * packed_stride,
+                              packed_stride, nq, nc, s, d_out));
 }
 
 bool GpuServerCtx::use_pair(bool status_read) const {
@@ -940,15 +1001,10 @@ void GpuServerCtx::horner_range(size_t count, uint64_t* d_out, size_t g_lo, size
                            count, nc, cc, s, fp ? *fp : FusedPack{}));
 }
 
-void GpuServerCtx::stage_horner(size_t count, uint64_t* d_out, hipStream_t s, size_t slot0, bool status_read) {
-    horner_range(count, d_out, 0, G, s, slot0, 0, status_read);
-}
-
 void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0,
                            int lane, bool status_read) {
     if (lane < 0 || lane >= kLanes) throw std::invalid_argument("enqueue: scratch lane out of range");
     TraceRange tr("answer: %zu queries, slots %zu.., lane %d", count, slot0, lane);
-    stage_prep(d_in, count, s, slot0);
     const size_t C = pp.db_cols;
     const size_t nchunks = G / gchunk;
     const hipStream_t hs = hstream[lane];
@@ -981,6 +1037,7 @@ void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, 
         const uint32_t* keys = d_keys + q0 * keys_stride;
         uint32_t* packed = d_packed_b + q0 * packed_stride;
         uint64_t* out = d_out + (q0 - slot0) * resp_u64s;
+        const uint64_t* in = d_in + (q0 - slot0) * qlen;
         DbPlan sp;
         // shape 8 (the collapse inside the streamed pass's launch) takes the
         // direct pass kernel: up to 8 queries, else shape 6
@@ -1015,22 +1072,29 @@ void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, 
             uint32_t* packed_done = pass_done + G;
             const uint32_t pq = pack_width(nq);
             const size_t nblk = (nq + pq - 1) / pq;
-            HIPX(launch_fill_u32(pass_done, (1 + nblk) * G, 0, s));  // this set's last readers are done
+            PrepZero z;  // the flags' last readers are done
+            z.flags = pass_done;
+            z.flag_words = (uint32_t)((1 + nblk) * G);
+            z.skip_lwe = fused;
+            prep_query(in, q0, nq, sp, s, lane, z);
+            // The pack and the chains are released here. Each of their
+            // workgroups needs a whole CU, which they get while the collapse
+            // (6) drains or the LWE digits are made (8); released together
+            // with the pass they would wait for a CU the pass's workgroups
+            // leave wholly free, often its end.
             if (cs != s) {
                 HIPX(hipEventRecord(prep_ev[lane], s));
                 HIPX(hipStreamWaitEvent(cs, prep_ev[lane], 0));
+            } else {
+                HIPX(hipEventRecord(coll_ev[lane][0], s));
             }
-            HIPX(launch_collapse_keys(keys, keys_stride, nq, d_kdig[lane], d_KS[lane], cs));
-            if (!fused)
+            if (fused) {
+                prep_lwe(in, qlen, q0, nq, sp, s, lane);
+            } else {
                 HIPX(launch_collapse(d_precomp, G, d_kdig[lane], d_KS[lane], nq, p2, part2_stride, cs,
                                      collapse_variant));
-            // The pack and the chains are released here (fused: the flags and
-            // key digits in place), before the query digits: each of their
-            // workgroups needs a whole CU, which they get while those small
-            // kernels run; released together with the pass they would wait
-            // for a CU the pass's workgroups leave wholly free, often its end.
-            HIPX(hipEventRecord(coll_ev[lane][0], cs));
-            dbpass_prep(q0, nq, sp, s, lane);
+                if (cs != s) HIPX(hipEventRecord(coll_ev[lane][0], cs));
+            }
             uint32_t* interm = d_interm + q0 * 2 * C;
             const bool direct = sp.slices == 1;
             uint32_t* part = direct ? interm : d_part + q0 * part_stride;
@@ -1043,9 +1107,8 @@ void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, 
             pst.group_done = pass_done;
             mark_pass(s, true);
             if (fused) {
-                HIPX(launch_pass_collapse_stream(db_planes(), d_dig[lane], d_S[lane], nq, part, part_qstride,
-                                                 pp.db_rows, C, sp, d_precomp, d_kdig[lane], d_KS[lane], p2,
-                                                 part2_stride, pass_done, s));
+                HIPX(launch_pass_collapse(db_planes(), d_dig[lane], d_S[lane], nq, part, part_qstride, pp.db_rows, C,
+                                          sp, d_precomp, d_kdig[lane], d_KS[lane], p2, part2_stride, pass_done, s));
             } else if (g_split > 0 && g_split < G) {
                 HIPX(launch_dbpass_mfma(db_planes(), d_dig[lane], d_S[lane], nq, part + g_split * N, part_qstride, C,
                                         pp.db_rows, C, g_split * N, (G - g_split) * N, sp, s, &pst));
@@ -1087,15 +1150,31 @@ void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, 
             continue;
         }
         if (shape == 0) {
-            const DbPlan p = plan_for(nq, C);
-            dbpass_prep(q0, nq, p, s, lane);
+            const DbPlan p = serial_plan(nq);
+            if (q0 == slot0) last_part_slices = p.slices > 1 ? p.slices : 0;
+            // up to 8 queries over a small table: the pass and the collapse in
+            // one launch (kMergeBytes)
+            const bool both = pass_collapse_ok(p, nq) && pp.db_rows * C * 2 + G * PC_GROUP * 4 <= kMergeBytes;
+            PrepZero z;
+            z.part2 = (both ? pass_collapse_ksplit(nq, G) : collapse_row_slices(nq, G, collapse_variant)) > 1;
+            prep_query(in, q0, nq, p, s, lane, z);
             mark_pass(s, true);
-            dbpass_range(q0, nq, 0, G, p, s, lane);
-            mark_pass(s, false);
-            HIPX(launch_collapse_keys(keys, keys_stride, nq, d_kdig[lane], d_KS[lane], s));
-            HIPX(launch_collapse(d_precomp, G, d_kdig[lane], d_KS[lane], nq, p2, part2_stride, s, collapse_variant));
-            HIPX(launch_pack_finalize(d_interm + q0 * 2 * C, C, p2, part2_stride, d_precomp, 0, G, keys, keys_stride,
-                                      packed, packed_stride, nq, nc, s));
+            if (both) {
+                size_t qstride;
+                uint32_t* part = pass_out(q0, p, qstride);
+                HIPX(launch_pass_collapse(db_planes(), d_dig[lane], d_S[lane], nq, part, qstride, pp.db_rows, C, p,
+                                          d_precomp, d_kdig[lane], d_KS[lane], p2, part2_stride, nullptr, s));
+                mark_pass(s, false);
+            } else {
+                dbpass_whole(q0, nq, p, s, lane);
+                mark_pass(s, false);
+                collapse_whole(q0, nq, s, lane, z.part2);
+            }
+            if (G == 1) {  // chains of one ciphertext: the pack writes the responses
+                pack_whole(q0, nq, p, s, out);
+                continue;
+            }
+            pack_whole(q0, nq, p, s);
             if (!defer_n) defer_lo = q0;
             defer_n += nq;
             continue;
@@ -1113,16 +1192,15 @@ void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, 
         const bool first = shape == 4, ahead = shape == 5;
         joined = true;
         const DbPlan p = chunk_plan(nq, gchunk * N);  // every chunk's plan has this one's kernel and digits
+        prep_query(in, q0, nq, p, s, lane);
         if (cs != s) {
             HIPX(hipEventRecord(prep_ev[lane], s));  // the keys are in place
             HIPX(hipStreamWaitEvent(cs, prep_ev[lane], 0));
         }
-        HIPX(launch_collapse_keys(keys, keys_stride, nq, d_kdig[lane], d_KS[lane], cs));
         if (first) {
             TraceRange trc("collapse of all %zu groups", G);
             HIPX(launch_collapse(d_precomp, G, d_kdig[lane], d_KS[lane], nq, p2, part2_stride, s, collapse_variant));
         }
-        dbpass_prep(q0, nq, p, s, lane);
         auto collapse_chunk = [&](size_t k) {
             const size_t g_lo = chunks[k].first, ng = chunks[k].second - g_lo;
             HIPX(launch_collapse(d_precomp + g_lo * PC_GROUP, ng, d_kdig[lane], d_KS[lane], nq, p2 + g_lo * 2 * N,
@@ -1162,8 +1240,8 @@ void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, 
                 HIPX(launch_pack_finalize_wg(d_interm + q0 * 2 * C, C, p2, part2_stride, d_precomp, g_lo, ng, keys,
                                              keys_stride, packed, packed_stride, nq, nc, hs));
             else
-                HIPX(launch_pack_finalize(d_interm + q0 * 2 * C, C, p2, part2_stride, d_precomp, g_lo, ng, keys,
-                                          keys_stride, packed, packed_stride, nq, nc, hs));
+                HIPX(launch_pack_finalize(d_interm + q0 * 2 * C, 2 * C, 1, C, p2, part2_stride, d_precomp, g_lo, ng,
+                                          keys, keys_stride, packed, packed_stride, nq, nc, hs));
             horner_range(nq, out, g_lo, g_hi, hs, q0, lane, status_read, fuse ? &fp : nullptr);
         }
         if (cs != s) {  // the next batch's key digits overwrite the lane's scratch

@@ -51,6 +51,10 @@ struct GpuServerCtx {
     // row slices of the batched chunk plan, timed at setup for plans with
     // chunk_param digit tiles (0: the narrowing rule)
     uint32_t chunk_slices = 0, chunk_param = 0;
+    // row slices of serial answers' full-width pass where timed below the
+    // plan's (0: the plan's); of many-query answers for plans with
+    // serial_param digit tiles
+    uint32_t serial_slices = 0, serial_param = 0, serial_slices1 = 0;
     uint32_t chunk_slices1 = 0;     // the same for one-query answers (plan1's kind)
     // chunks from index late_from on (the collapse beside them has finished)
     // take late_slices row slices instead (0: as the chunks before them);
@@ -122,7 +126,9 @@ struct GpuServerCtx {
     // scratch of the batched database pass, one set per concurrent lane
     static constexpr int kLanes = 4;
     int8_t* d_dig[kLanes] = {};     // query digits [R/16][<=256][16]
-    uint32_t* d_S[kLanes] = {};     // digit-offset corrections [64]
+    uint32_t* d_S[kLanes] = {};     // digit-offset corrections [32][2][kOffsetSumParts]
+    static constexpr size_t kSumWords = ipx::kMfmaMaxQueries * 2 * ipx::kOffsetSumParts;
+    static constexpr size_t kKeySumWords = ipx::kCollapseMaxQueries * 2 * ipx::kKeySumParts;
     // scratch of the collapse pass: key digits [2][2N/16][<=128][16], key sums
     static constexpr size_t kKdigBytes = 2 * (2 * ipx::N / 16) * 128 * 16;
     int8_t* d_kdig[kLanes] = {};
@@ -210,18 +216,39 @@ struct GpuServerCtx {
     void alloc_slots();
     // Pick the fastest database-pass variant on this device and geometry.
     void autotune_dbpass();
-    // Pipeline stages over slots [slot0, slot0+count) on stream s.
-    void stage_prep(const uint64_t* d_in, size_t count, hipStream_t s, size_t slot0);
+    // Pipeline stages over slots [q0, q0+nq) (one sub-batch, at most 32) on
+    // stream s, their int8 operands in scratch set `lane`.
+    // What an answer's first launch zeroes beside its own work.
+    struct PrepZero {
+        uint32_t* flags = nullptr;  // flag_words words
+        uint32_t flag_words = 0;
+        bool part2 = false;         // the collapse sums (a split collapse adds into them)
+        bool skip_lwe = false;      // leave the LWE part to prep_lwe
+    };
+    ipx::PrepArgs prep_args(const uint64_t* d_in, size_t stride, size_t q0, int lane) const;
+    // Keys, RGSW rows and plan p's pass operands of the flat queries at d_in.
+    void prep_query(const uint64_t* d_in, size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s, int lane,
+                    const PrepZero& z);
+    void prep_query(const uint64_t* d_in, size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s, int lane) {
+        prep_query(d_in, q0, nq, p, s, lane, PrepZero{});
+    }
+    // Plan p's pass operands alone, of LWE parts stride words apart.
+    void prep_lwe(const uint64_t* d_in, size_t stride, size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s,
+                  int lane);
+    // Where a full-width pass of plan p writes: its row slices' partials, or interm.
+    uint32_t* pass_out(size_t q0, const ipx::DbPlan& p, size_t& qstride);
+    void dbpass_whole(size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s, int lane);
+    void collapse_whole(size_t q0, size_t nq, hipStream_t s, int lane, bool zeroed = false);
+    // d_out: also the responses (tables of one group)
+    void pack_whole(size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s, uint64_t* d_out = nullptr);
+    // The serial answer's plan: plan_for's at the timed row slices.
+    ipx::DbPlan serial_plan(size_t nq) const;
     // The tuned database-pass plan for nq queries over ncols columns.
     ipx::DbPlan plan_for(size_t nq, size_t ncols) const;
     // The tuned full-width plan narrowed to ncols columns at its workgroup count.
     ipx::DbPlan chunk_plan(size_t nq, size_t ncols) const;
-    // Digits of queries [q0, q0+nq) for an MFMA plan (no-op for fp64).
-    void dbpass_prep(size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s, int lane);
     // Database pass of queries [q0, q0+nq) over the columns of groups [g_lo, g_hi) into interm.
     void dbpass_range(size_t q0, size_t nq, size_t g_lo, size_t g_hi, const ipx::DbPlan& p, hipStream_t s, int lane);
-    // force: -1 the tuned plans, 0 the fp64 pass per query, 1 the MFMA pass
-    void stage_dbpass(size_t count, hipStream_t s, size_t slot0, int lane = 0, int force = -1);
     // The pair kernel only where the caller reads the lane's status after
     // the call (status_read): its bounded wait reports through it.
     bool use_pair(bool status_read) const;
@@ -229,9 +256,6 @@ struct GpuServerCtx {
     // fp: the chains compute their groups' packed b-parts themselves first
     void horner_range(size_t count, uint64_t* d_out, size_t g_lo, size_t g_hi, hipStream_t s, size_t slot0,
                       int lane, bool status_read, const ipx::FusedPack* fp = nullptr);
-    void stage_collapse(size_t count, hipStream_t s, size_t slot0, int lane = 0);
-    void stage_finalize(size_t count, hipStream_t s, size_t slot0);
-    void stage_horner(size_t count, uint64_t* d_out, hipStream_t s, size_t slot0, bool status_read);
     // Throw (and clear) if a pair chain of a call on `lane` reported a fault
     // through its status word; s is the stream the call ran on.
     void check_status(hipStream_t s, int lane);
