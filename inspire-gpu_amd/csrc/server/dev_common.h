@@ -165,6 +165,16 @@ __device__ __forceinline__ void fence_acquire_agent_done() {
     __builtin_amdgcn_s_waitcnt(0);
 }
 
+// A workgroup barrier for data exchanged through LDS only. __syncthreads also
+// waits for every global access in flight (its fence covers global memory),
+// which puts the latency of a prefetch on each step of a serial chain: here
+// loads and stores to global memory stay in flight across the barrier.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // ---------------------------------------------------------------- LDS NTT
 // LDS slot of coefficient e: one pad word per 32 spreads the strided
 // accesses of the register-blocked phases over the banks.

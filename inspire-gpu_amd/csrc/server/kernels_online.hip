@@ -398,7 +398,7 @@ __global__ __launch_bounds__(512, 2) void k_horner(HornerChain h, NttConst nc, N
                     keep[p][k] = c ? cf[p][k + 4] : cf[p][k];
                     xs[4 * p + k][t] = c ? cf[p][k] : cf[p][k + 4];
                 }
-            __syncthreads();
+            lds_barrier();
             uint32_t x[4][8];  // digit polynomials a1, a2, b1, b2: residues + q mod this limb's prime
 #pragma unroll
             for (int p = 0; p < 2; p++)
@@ -409,7 +409,7 @@ __global__ __launch_bounds__(512, 2) void k_horner(HornerChain h, NttConst nc, N
                     dx[c][4 * p + k][0][t] = d.x;
                     dx[c][4 * p + k][1][t] = d.y;
                 }
-            __syncthreads();
+            lds_barrier();
             uint32_t pav[8], pbv[8];  // the step's packed parts, in flight during the transforms
             load8(pav, h.pa_base + (size_t)gs * h.pa_stride);
             if constexpr (!STREAMED) load8(pbv, pb + (size_t)gs * 2 * N);
@@ -423,7 +423,12 @@ __global__ __launch_bounds__(512, 2) void k_horner(HornerChain h, NttConst nc, N
                         x[2 * p + 1][4 * s + k] = dx[s][4 * p + k][1][t] + m.q;
                     }
             nr_forward<4>(x, buf[c], tw, t, m, [&]() {
-                if constexpr (STREAMED) wait_packed((uint32_t)gs);
+                if constexpr (STREAMED) {
+                    wait_packed((uint32_t)gs);
+                    __syncthreads();  // no wave's load of the b-part before the acquire
+                } else {
+                    lds_barrier();
+                }
             });
             if constexpr (STREAMED) {
                 if (sw_abort) {

@@ -18,10 +18,13 @@
 //    independent D x D/2 negacyclic blocks, each done in LDS in one pass
 //    over the DB instead of log2(D)+2 global passes.
 #include "kernels.h"
+#include "ntt_regs.h"
 
 namespace ipx {
 
 namespace {
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint32_t modp(uint32_t x) {  // x mod 65535, any u32
     uint32_t r = (x & 0xffffu) + (x >> 16);
@@ -172,95 +175,138 @@ __global__ __launch_bounds__(256) void k_ntt_rows(uint32_t* __restrict__ rows, N
     for (int k = 0; k < 8; k++) p[t + 256 * k] = buf[ls(t + 256 * k)];
 }
 
+// ------------------------------------------------------------ a_post gather
+// a_post of every step of both directions, F[c][p(s, i)][i], into the words
+// where the chain's digit 0 of that step goes (dtmp [dir][c][s][0][i]): the
+// chain then reads whole lines instead of one line per value. Block (group,
+// limb, 16 slots i): the slots' 16 columns of F in LDS (128 KiB), read and
+// written in 64-byte rows.
+__global__ __launch_bounds__(1024) void k_apost_gather(const uint32_t* __restrict__ F, uint32_t* __restrict__ dtmp) {
+    __shared__ __align__(16) uint32_t T[N][16];
+    __shared__ uint16_t pw[NSTEPS];  // 5^(N/2-2-s) mod 2N
+    const uint32_t it = blockIdx.x % (N / 16), c = (blockIdx.x / (N / 16)) & 1, gl = blockIdx.x / (2 * (N / 16));
+    const uint32_t i0 = it * 16, tid = threadIdx.x;
+    const uint32_t* Fg = F + ((size_t)gl * 2 + c) * N * N + i0;
+    for (uint32_t x = tid; x < N * 4; x += 1024)
+        *reinterpret_cast<u32x4*>(&T[x >> 2][4 * (x & 3)]) =
+            *reinterpret_cast<const u32x4*>(Fg + (size_t)(x >> 2) * N + 4 * (x & 3));
+    if (tid < NSTEPS) {
+        uint32_t ts = 1;
+        for (uint32_t ex = HALF - 2 - tid, b = 5; ex; ex >>= 1, b = (b * b) & (2 * N - 1))
+            if (ex & 1) ts = (ts * b) & (2 * N - 1);
+        pw[tid] = (uint16_t)ts;
+    }
+    __syncthreads();
+    const uint32_t il = tid & 15, v = 2 * brev11(i0 + il) + 1;
+    for (uint32_t r = tid >> 4; r < 2 * NSTEPS; r += 64) {
+        const uint32_t dir = r >= NSTEPS, s = r - dir * NSTEPS;
+        const uint32_t pf = perm_slot(pw[s], v), p = dir ? N - 1 - pf : pf;
+        dtmp[((size_t)gl * 2 + dir) * RD_SZ + ((size_t)c * NSTEPS + s) * D_EFF * N + i0 + il] = T[p][il];
+    }
+}
+
 // ------------------------------------------------------------ collapse
 // One block per (group, direction): 1023 dependent steps. Step s folds
 // k = N/2-1-s: state -> INTT -> gadget digits 1,2 -> NTT -> D[s]; state =
 // a_post[k-1] - sum_j D[s][j] * K[j][perm]. Both the expanded key of step s
 // (tau_{+-5^(k-1)} of ksk5a, reference kskstep = n_steps-1-s) and a_post[k-1]
-// are gathered through the same slot permutation p.
-__global__ __launch_bounds__(1024) void k_collapse_chain(const uint32_t* __restrict__ F,
-                                                         const uint32_t* __restrict__ ksk5a,
-                                                         uint32_t* __restrict__ dtmp,
-                                                         uint32_t* __restrict__ states, NttConst nc, CrtConst cc) {
-    __shared__ uint32_t buf[4][POLY_LDS];
-    __shared__ uint32_t K[4][N];  // [digit*2 + limb][N]
-    __shared__ uint32_t twl[8 * N];
-    const uint32_t gl = blockIdx.x, dir = blockIdx.y, tid = threadIdx.x, team = tid >> 8, t = tid & 255;
-    for (uint32_t x = tid; x < 4 * N; x += 1024) K[x / N][x % N] = ksk5a[x];
-    stage_twiddles(twl, nc, tid, 1024);
-    const int tlimb = (int)(team & 1);
-    const Tw tw = tw_lds(twl, tlimb);
-    const uint32_t inv_n = nc.inv_n[tlimb], inv_n_p = nc.inv_n_p[tlimb];
-    const uint32_t* Fg = F + (size_t)gl * 2 * N * N;
-    uint32_t* Dout = dtmp + ((size_t)gl * 2 + dir) * RD_SZ;
-    uint32_t v[2], st[2][2];  // [e], [limb][e]
-#pragma unroll
-    for (int e = 0; e < 2; e++) v[e] = 2 * brev11(tid + 1024 * e) + 1;
+// are gathered through the same slot permutation p; k_apost_gather has put
+// the latter where the step's first digit will go.
+// A serial chain on one CU, built like the Horner chain: a 256-lane team per
+// limb keeps 8 slots of its polynomials in registers between transforms
+// (ntt_regs.h), the teams swap halves of the CRT lift and the digits through
+// LDS, and the key is kept times 2^32 for Montgomery products. Every
+// transform through LDS by its own 256 lanes of 1024 took 13.3 us per step;
+// with the a_post values gathered in the step (4 bytes of each of 4096 cache
+// lines, the most a CU's misses allow) this form took 11.4.
+__global__ __launch_bounds__(512, 2) void k_collapse_chain(const uint32_t* __restrict__ F,
+                                                           const uint32_t* __restrict__ ksk5a,
+                                                           uint32_t* dtmp,
+                                                           uint32_t* __restrict__ states, NttConst nc, NrGadget gc) {
+    __shared__ __align__(16) uint32_t buf[2][2][POLY4_LDS];
+    __shared__ __align__(16) nr_u32x2 tw2[2][N];
+    __shared__ uint32_t K[2][2][N];         // [limb][digit][slot], times 2^32 mod q
+    __shared__ uint32_t xs[2][4][256];      // lift shares by the team that sent them
+    __shared__ uint32_t dx[2][4][2][256];   // digits by the team that made them
+    const uint32_t gl = blockIdx.x, dir = blockIdx.y, tid = threadIdx.x, t = tid & 255;
+    const int c = __builtin_amdgcn_readfirstlane((int)(tid >> 8));
+    const NrLimb m = nr_limb(c);
+    const uint32_t r32 = c ? (uint32_t)(4294967296ull % Q1) : (uint32_t)(4294967296ull % Q0);
+    const uint32_t qneg = c ? nr_neg_inverse(Q1) : nr_neg_inverse(Q0);
+    nr_stage_twiddles(tw2, nc, tid, 512);
+    for (uint32_t x = t; x < 2 * N; x += 256)  // ksk5a [digit][limb][N]
+        K[c][x / N][x % N] = mul_mod(ksk5a[((size_t)(x / N) * 2 + c) * N + x % N], r32, c);
+    const uint32_t* Fg = F + ((size_t)gl * 2 + c) * N * N;
+    uint32_t* Dout = dtmp + ((size_t)gl * 2 + dir) * RD_SZ + (size_t)c * NSTEPS * D_EFF * N;
+    const nr_u32x2* tw = tw2[c];
     // t = 5^(N/2-1) mod 2N, then 5^(N/2-2-s) for step s
-    uint32_t tk = 1;
+    uint32_t ts = 1;
     for (uint32_t ex = HALF - 1, b = 5; ex; ex >>= 1, b = (b * b) & (2 * N - 1))
-        if (ex & 1) tk = (tk * b) & (2 * N - 1);
+        if (ex & 1) ts = (ts * b) & (2 * N - 1);
+    uint32_t v[8];  // 2 BR(slot) + 1 of this lane's slots 8t + k
 #pragma unroll
-    for (int e = 0; e < 2; e++) {
-        const uint32_t pf = perm_slot(tk, v[e]);
-        const uint32_t p = dir ? N - 1 - pf : pf;
-        const uint32_t i = tid + 1024 * e;
-        st[0][e] = Fg[(size_t)p * N + i];
-        st[1][e] = Fg[((size_t)N + p) * N + i];
-    }
-    uint32_t ts = (tk * 3277u) & (2 * N - 1);
+    for (int k = 0; k < 8; k++) v[k] = 2 * brev11(8 * t + k) + 1;
+    auto slot = [&](int k) {
+        const uint32_t pf = perm_slot(ts, v[k]);
+        return dir ? N - 1 - pf : pf;
+    };
+    uint32_t st[1][8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) st[0][k] = Fg[(size_t)slot(k) * N + 8 * t + k];
+    __syncthreads();
     for (uint32_t s = 0; s < NSTEPS; s++) {
-        uint32_t pidx[2], nxt[2][2];
+        ts = (ts * 3277u) & (2 * N - 1);  // times 5^-1
+        uint32_t p[8];
 #pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const uint32_t pf = perm_slot(ts, v[e]);
-            pidx[e] = dir ? N - 1 - pf : pf;
-            const uint32_t i = tid + 1024 * e;
-            nxt[0][e] = Fg[(size_t)pidx[e] * N + i];
-            nxt[1][e] = Fg[((size_t)N + pidx[e]) * N + i];
+        for (int k = 0; k < 8; k++) p[k] = slot(k);
+        u32x4* D0 = reinterpret_cast<u32x4*>(Dout + (size_t)s * D_EFF * N + 8 * t);
+        const u32x4 nl = D0[0], nh = D0[1];  // this step's a_post, the lane's own words
+        const uint32_t nxt[8] = {nl[0], nl[1], nl[2], nl[3], nh[0], nh[1], nh[2], nh[3]};
+        nr_inverse<1>(st, buf[c], tw, t, m);
+        // team c lifts the coefficients k in [4c, 4c + 4) and sends the others
+        uint32_t keep[4];
+#pragma unroll
+        for (int k = 0; k < 8; k++) st[0][k] = nr_crt_part(st[0][k], gc, c, m);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            keep[k] = c ? st[0][k + 4] : st[0][k];
+            xs[c][k][t] = c ? st[0][k] : st[0][k + 4];
+        }
+        lds_barrier();
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint32_t other = xs[1 - c][k][t];
+            const nr_u32x2 d = nr_digits(c ? other : keep[k], c ? keep[k] : other);
+            dx[c][k][0][t] = d.x;
+            dx[c][k][1][t] = d.y;
+        }
+        lds_barrier();
+        uint32_t x[2][8];  // digit polynomials: residues + q mod this limb's prime
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                x[0][4 * h + k] = dx[h][k][0][t] + (m.q - (1u << 17));
+                x[1][4 * h + k] = dx[h][k][1][t] + m.q;
+            }
+        nr_forward<2>(x, buf[c], tw, t, m, [] { lds_barrier(); });
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) x[j][k] = fold(nr_reduce(x[j][k], m), m.q);  // canonical, from at most 24q
+            u32x4* d = D0 + j * (N / 4);
+            d[0] = u32x4{x[j][0], x[j][1], x[j][2], x[j][3]};
+            d[1] = u32x4{x[j][4], x[j][5], x[j][6], x[j][7]};
         }
 #pragma unroll
-        for (int e = 0; e < 2; e++) {
-            buf[0][ls(tid + 1024 * e)] = st[0][e];
-            buf[1][ls(tid + 1024 * e)] = st[1][e];
+        for (int k = 0; k < 8; k++) {
+            const uint64_t acc = (uint64_t)x[0][k] * K[c][0][p[k]] + (uint64_t)x[1][k] * K[c][1][p[k]];
+            st[0][k] = nxt[k] + (2 * m.q - nr_montgomery(acc, qneg, m.q));  // the product below 1.1q: st below 3q
         }
-        __syncthreads();
-        ntt_inv_lds(buf[team], t, tw, tlimb, inv_n, inv_n_p, team < 2);
-        uint32_t d0[2][2], d1[2][2];
-#pragma unroll
-        for (int e = 0; e < 2; e++) gadget2(buf[0][ls(tid + 1024 * e)], buf[1][ls(tid + 1024 * e)], cc, d0[e], d1[e]);
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < 2; e++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                buf[j * 2 + 0][ls(tid + 1024 * e)] = d0[e][j];
-                buf[j * 2 + 1][ls(tid + 1024 * e)] = d1[e][j];
-            }
-        __syncthreads();
-        ntt_fwd_lds(buf[team], t, tw, tlimb);
-#pragma unroll
-        for (int c = 0; c < 2; c++)
-#pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const uint32_t i = tid + 1024 * e;
-                uint64_t acc = 0;
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const uint32_t dv = buf[j * 2 + c][ls(i)];
-                    Dout[(((size_t)c * NSTEPS + s) * D_EFF + j) * N + i] = dv;
-                    acc += (uint64_t)dv * K[j * 2 + c][pidx[e]];
-                }
-                st[c][e] = sub_mod(nxt[c][e], red64(acc, c), qof(c));
-            }
-        ts = (ts * 3277u) & (2 * N - 1);
-        __syncthreads();
     }
 #pragma unroll
-    for (int c = 0; c < 2; c++)
-#pragma unroll
-        for (int e = 0; e < 2; e++)
-            states[(((size_t)gl * 2 + dir) * 2 + c) * N + tid + 1024 * e] = st[c][e];
+    for (int k = 0; k < 8; k++)
+        states[(((size_t)gl * 2 + dir) * 2 + c) * N + 8 * t + k] = fold(fold(st[0][k], 2 * m.q), m.q);
 }
 
 // Final CollapseOne: digits of the conjugate chain's last state -> D_final;
@@ -347,7 +393,9 @@ hipError_t launch_ring_embed(uint32_t* a32T, size_t ng, const NttConst& nc, hipS
 
 hipError_t launch_collapse_chain(const uint32_t* F, size_t ng, const uint32_t* ksk5a, uint32_t* dtmp,
                                  uint32_t* states, const NttConst& nc, const CrtConst& cc, hipStream_t s) {
-    hipLaunchKernelGGL(k_collapse_chain, dim3((unsigned)ng, 2), dim3(1024), 0, s, F, ksk5a, dtmp, states, nc, cc);
+    hipLaunchKernelGGL(k_apost_gather, dim3((unsigned)(ng * 2 * (N / 16))), dim3(1024), 0, s, F, dtmp);
+    hipLaunchKernelGGL(k_collapse_chain, dim3((unsigned)ng, 2), dim3(512), 0, s, F, ksk5a, dtmp, states, nc,
+                       nr_gadget_const(nc, cc));
     return hipGetLastError();
 }
 

@@ -200,8 +200,7 @@ __device__ __forceinline__ void nr_load(uint32_t (*buf)[POLY4_LDS], uint32_t (&x
 // Forward transform of P polynomials: in, coefficients t + 256k (up to
 // B q, B <= 23); out, NTT slots 8t + k up to (B + 22) q. buf: the team's P
 // LDS polynomials, whose words t + 256k (all lanes' own) must be free; the
-// workgroup runs it together (three barriers; last_barrier() runs just
-// before the third one).
+// workgroup runs it together (three barriers, the third one last_barrier()).
 template <int P, typename F>
 __device__ __forceinline__ void nr_forward(uint32_t (&x)[P][8], uint32_t (*buf)[POLY4_LDS], const nr_u32x2* tw,
                                            uint32_t t, const NrLimb& m, F&& last_barrier) {
@@ -210,18 +209,17 @@ __device__ __forceinline__ void nr_forward(uint32_t (&x)[P][8], uint32_t (*buf)[
     nr_fwd_phase<P, true>(x, w, m);
     nr_store<0, P>(buf, x, t);
     nr_tw_load(w, tw, nr_node(1, t), true);
-    __syncthreads();
+    lds_barrier();
     nr_load<1, P>(buf, x, t);
     nr_fwd_phase<P, true>(x, w, m);
     nr_store<1, P>(buf, x, t);
     nr_tw_load(w, tw, nr_node(2, t), true);
-    __syncthreads();
+    lds_barrier();
     nr_load<2, P>(buf, x, t);
     nr_fwd_phase<P, true>(x, w, m);
     nr_store<2, P>(buf, x, t);
     nr_tw_load(w, tw, nr_node(3, t), false);
     last_barrier();
-    __syncthreads();
     nr_load<3, P>(buf, x, t);
     nr_fwd_phase<P, false>(x, w, m);
 }
@@ -254,19 +252,19 @@ __device__ __forceinline__ void nr_forward1(uint32_t (&x)[1][8], uint32_t (*buf)
         nr_fwd_phase<1, true>(x, w[0], m);
         nr_store<0, 1>(buf, x, t);
     }
-    __syncthreads();
+    lds_barrier();
     if (active) {
         nr_load<1, 1>(buf, x, t);
         nr_fwd_phase<1, true>(x, w[1], m);
         nr_store<1, 1>(buf, x, t);
     }
-    __syncthreads();
+    lds_barrier();
     if (active) {
         nr_load<2, 1>(buf, x, t);
         nr_fwd_phase<1, true>(x, w[2], m);
         nr_store<2, 1>(buf, x, t);
     }
-    __syncthreads();
+    lds_barrier();
     if (active) {
         nr_load<3, 1>(buf, x, t);
         nr_fwd_phase<1, false>(x, w[3], m);
@@ -289,7 +287,7 @@ __device__ __forceinline__ void nr_inverse(uint32_t (&x)[P][8], uint32_t (*buf)[
     }
     nr_store<3, P>(buf, x, t);
     nr_tw_load(w, tw, nr_inv_node(2, t), true);
-    __syncthreads();
+    lds_barrier();
     nr_load<2, P>(buf, x, t);
     nr_inv_phase<P, true, 4>(x, w, m);  // 32q at k = 0, 8q at k = 1, else up to 4q
 #pragma unroll
@@ -299,7 +297,7 @@ __device__ __forceinline__ void nr_inverse(uint32_t (&x)[P][8], uint32_t (*buf)[
     }
     nr_store<2, P>(buf, x, t);
     nr_tw_load(w, tw, nr_inv_node(1, t), true);
-    __syncthreads();
+    lds_barrier();
     nr_load<1, P>(buf, x, t);
     nr_inv_phase<P, true, 4>(x, w, m);
 #pragma unroll
@@ -309,7 +307,7 @@ __device__ __forceinline__ void nr_inverse(uint32_t (&x)[P][8], uint32_t (*buf)[
     }
     nr_store<1, P>(buf, x, t);
     nr_tw_load(w, tw, nr_inv_node(0, t), true);
-    __syncthreads();
+    lds_barrier();
     nr_load<0, P>(buf, x, t);
     nr_inv_phase<P, true, 4>(x, w, m);
 }
