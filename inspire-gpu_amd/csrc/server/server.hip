@@ -511,15 +511,26 @@ void GpuServerCtx::autotune_dbpass() {
     hipEvent_t e0, e1;
     HIPX(hipEventCreate(&e0));
     HIPX(hipEventCreate(&e1));
-    // Candidates are timed round-robin: every round runs each candidate once
-    // (after its own preparation, untimed) and the first round only warms
-    // up. Under sustained int8-MFMA work the power limit lowers the clock
-    // within tens of milliseconds, so timing the candidates one after
-    // another would favour whichever ran first.
+    // Candidates are timed round-robin: every round runs each remaining
+    // candidate once (after its own preparation, untimed). Under sustained
+    // int8-MFMA work the power limit lowers the clock within tens of
+    // milliseconds, so timing the candidates one after another would favour
+    // whichever ran first. After each round the candidates clearly behind the
+    // best one leave: the first round, which also warms up, only drops those
+    // 1.4 times (and 20 us) slower, later ones those above the spread of
+    // repeated runs (a few percent). All candidates through all rounds took
+    // 158 of a 1 GB server's 232 ms.
     auto fastest = [&](size_t n, auto&& prep, auto&& run, int rounds = 4) {
         std::vector<std::vector<float>> got(n);
-        for (int round = 0; round < rounds; round++)
-            for (size_t i = 0; i < n; i++) {
+        std::vector<size_t> left(n);
+        for (size_t i = 0; i < n; i++) left[i] = i;
+        auto median = [&](size_t i) {  // the lower one: a disturbed round does not decide
+            std::vector<float> v = got[i];
+            std::sort(v.begin(), v.end());
+            return v[(v.size() - 1) / 2];
+        };
+        for (int round = 0; round < rounds && left.size() > 1; round++) {
+            for (const size_t i : left) {
                 prep(i);
                 HIPX(hipEventRecord(e0, stream));
                 run(i);
@@ -527,15 +538,14 @@ void GpuServerCtx::autotune_dbpass() {
                 HIPX(hipEventSynchronize(e1));
                 float ms = 0;
                 HIPX(hipEventElapsedTime(&ms, e0, e1));
-                if (round) got[i].push_back(ms);
+                if (round == 1) got[i].clear();  // the warm-up's
+                got[i].push_back(ms);
             }
-        // the lower median: one disturbed round does not decide
-        size_t b = 0;
-        for (size_t i = 0; i < n; i++) {
-            std::sort(got[i].begin(), got[i].end());
-            if (got[i][(got[i].size() - 1) / 2] < got[b][(got[b].size() - 1) / 2]) b = i;
+            std::sort(left.begin(), left.end(), [&](size_t a, size_t b) { return median(a) < median(b); });
+            const float best = median(left[0]), most = round == 0 ? 1.4f * best + 0.02f : round == 1 ? 1.1f * best : 1.06f * best;
+            while (left.size() > 1 && median(left.back()) > most) left.pop_back();
         }
-        return b;
+        return left[0];
     };
     // one full-width database pass of plan x over nq staged queries (zeroed)
     const size_t nq = cfg.max_batch < kMfmaMaxQueries ? cfg.max_batch : kMfmaMaxQueries;
@@ -589,26 +599,42 @@ void GpuServerCtx::autotune_dbpass() {
                     return true;
             return false;
         };
+        // first every form and target at one ring depth, then the ring depths
+        // of the best one and of the other of the two forms that win in
+        // practice (2, shared digits in 8-wave blocks, and 5, power rows)
+        auto add = [&](size_t t, int form, uint32_t d) {
+            const DbPlan x = dbplan_form(R, C, nqc, t, d, form);
+            if (x.depth != d && param >= 8) return;  // a depth this kernel is not built with
+            if (fits(x) && !seen(x)) cands.push_back({x, t, d, form});
+        };
+        auto time_cands = [&] {
+            return fastest(
+                cands.size(), [&](size_t i) { prep_plan(cands[i].x, nqc); },
+                [&](size_t i) { run_plan(cands[i].x, nqc); });
+        };
+        const uint32_t depth0 = depth_forced || param < 8 ? depth_out : 4;
         for (size_t t : kMfmaTargets)
             for (int form = 0; form < kMfmaForms; form++) {
                 if (depth_forced ? form != forced_form
                                  : (form == 1 && param != 16) || (form > 0 && param < 8) || form == 3 || form == 4)
                     continue;
-                for (uint32_t d : kMfmaDepths) {
-                    if ((depth_forced || param < 8) && d != depth_out) continue;
-                    const DbPlan x = dbplan_form(R, C, nqc, t, d, form);
-                    if (x.depth != d && param >= 8) continue;  // a depth this kernel is not built with
-                    if (fits(x) && !seen(x)) cands.push_back({x, t, d, form});
-                }
+                add(t, form, depth0);
             }
-        if (!cands.empty()) {  // empty: a forced depth the forced form is not built with keeps the defaults
-            const size_t b = fastest(
-                cands.size(), [&](size_t i) { prep_plan(cands[i].x, nqc); },
-                [&](size_t i) { run_plan(cands[i].x, nqc); });
-            target_out = cands[b].target;
-            depth_out = cands[b].depth;
-            form_out = cands[b].form;
+        if (cands.empty()) return;  // a forced depth the forced form is not built with keeps the defaults
+        Cand best = cands[time_cands()];
+        if (!depth_forced && param >= 8) {
+            std::vector<Cand> first;
+            for (int form : {best.form, best.form == 5 ? 2 : 5})
+                for (const Cand& y : cands)
+                    if (y.form == form && (form != best.form || y.target == best.target)) first.push_back(y);
+            cands.clear();
+            for (const Cand& y : first)
+                for (uint32_t d : kMfmaDepths) add(y.target, y.form, d);
+            best = cands[time_cands()];
         }
+        target_out = best.target;
+        depth_out = best.depth;
+        form_out = best.form;
     };
     if (nq > 1) {
         tune_batched(nq, mfma_target, mfma_depth, mfma_form);
