@@ -115,9 +115,8 @@ ipir_client_query* ipir_query_build_seeded(const ipir_params* params, uint64_t i
  * report nothing afterwards). The work waits for the server's previous
  * call if that one was on another stream; inside a caller's stream capture
  * the caller orders the captured work itself. For callers that keep
- * queries resident in HBM. Answers of the device's streaming server may
- * run their Horner chains beside a database pass they wait for inside the
- * kernel; such a wait is bounded (about a second or more), and a chain
+ * queries resident in HBM. Answers may run their Horner chains beside a
+ * database pass they wait for inside the kernel; such a wait is bounded (about a second or more), and a chain
  * that gives up writes all-ones words as its response (no residue has
  * that value; it can happen only if the pass gets no CU for that long)
  * and is reported by ipir_device_status. */

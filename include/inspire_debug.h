@@ -167,9 +167,10 @@ int ipir_dbg_get_collapse_variant(const ipir_server* srv);
  * pass's launch, each group's collapse and pass work items together (up to
  * 8 queries; 6 for more). The setup autotuner picks 2, 3, 6 or 8 (4, 5
  * and 7 are tested alternatives that never won at 16 GB).
- * Answers under stream capture, and every answer of a server that is not
- * the device's first live one, take the chunked shape the autotuner picked
- * instead of a streamed one. 1 for other values. */
+ * Answers under stream capture, and answers that find the device's four
+ * slots for streamed answers in flight taken (by other servers' or lanes'
+ * unfinished ones), take the chunked shape the autotuner picked instead of a
+ * streamed one. 1 for other values. */
 int ipir_dbg_set_pipeline(ipir_server* srv, int single, int batched);
 /* Row slices (a power of two <= 16) of the streamed pass of one-query
  * (nq_class 1) or many-query (other values) answers; raised to what the
@@ -181,13 +182,10 @@ int ipir_dbg_set_stream_slices(ipir_server* srv, size_t nq_class, uint32_t slice
  * 0: one launch), the Horner chains starting only after that launch (they
  * hold their CUs from then on). */
 int ipir_dbg_set_stream_split(ipir_server* srv, size_t nq_class, uint32_t eighths);
-/* 1 if this server may take the streamed shapes (the device's first live
- * server), else 0. */
+/* 1 if this server may take the streamed shapes, else 0 (INSPIRE_STREAM=0 at
+ * setup). */
 int ipir_dbg_stream_ok(const ipir_server* srv);
-/* Make srv the device's streaming server; the one that was (if any) then
- * answers with its chunked shapes. Its own mutex is taken: do not call
- * this while that server is inside another call on another thread that
- * itself waits for srv. */
+/* Let srv take the streamed shapes whatever INSPIRE_STREAM said at setup. */
 int ipir_dbg_take_streaming(ipir_server* srv);
 /* Timings (ms, mean of 5 after a warm-up) of the streamed pieces for nq
  * zero queries at `slices` row slices: out[0] the streamed database pass

@@ -45,7 +45,7 @@ struct Req {
 struct Partition {
     size_t slot0 = 0, nslots = 0;
     int lane = 0;  // scratch lane (and status word) of the context this partition uses
-    hipStream_t stream = nullptr;
+    hipStream_t stream = nullptr;  // the lane's own (mstream)
     // device timestamps of the batch in flight (its first and last command),
     // and [start, end) in ms after the loop's reference event of the last
     // completed batch
@@ -216,10 +216,9 @@ ipir_loop* ipir_loop_start(ipir_server* srv, size_t max_inflight) {
         p->slot0 = i * per;
         p->lane = (int)i;
         p->nslots = per;
-        if (hipStreamCreate(&p->stream) != hipSuccess || hipEventCreate(&p->ev0) != hipSuccess ||
-            hipEventCreate(&p->ev1) != hipSuccess) {
+        p->stream = ctx->mstream[i];
+        if (hipEventCreate(&p->ev0) != hipSuccess || hipEventCreate(&p->ev1) != hipSuccess) {
             if (p->ev0) (void)hipEventDestroy(p->ev0);
-            if (p->stream) (void)hipStreamDestroy(p->stream);
             delete p;
             break;
         }
@@ -230,7 +229,6 @@ ipir_loop* ipir_loop_start(ipir_server* srv, size_t max_inflight) {
         for (auto* p : L->parts) {
             (void)hipEventDestroy(p->ev0);
             (void)hipEventDestroy(p->ev1);
-            (void)hipStreamDestroy(p->stream);
             delete p;
         }
         L->parts.clear();
@@ -341,14 +339,13 @@ void ipir_loop_stop(ipir_loop* L) {
         (void)hipStreamSynchronize(p->stream);  // every completer synchronised already
         (void)hipEventDestroy(p->ev0);
         (void)hipEventDestroy(p->ev1);
-        (void)hipStreamDestroy(p->stream);
         delete p;
     }
     (void)hipEventDestroy(L->ev_ref);
     for (auto& kv : L->reqs) delete kv.second;
     {
         std::lock_guard<std::mutex> lk(ctx->mu);
-        ctx->order_stream_set = false;  // the loop's work has finished and its streams are gone
+        ctx->order_stream_set = false;  // the loop's work has finished
         ctx->loop_active = false;
     }
     delete L;

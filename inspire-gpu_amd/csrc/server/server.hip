@@ -255,10 +255,16 @@ GpuServerCtx* gpu_setup_server(const PublicParams& pp, const PreprocessData& pre
 }
 
 namespace {
-// The server of each device that may take the streamed shapes (at most one).
+// Streamed answers in flight, per device: at most kLanes of them, whatever
+// servers and lanes they belong to (StreamSlot). A slot's owner keeps it until
+// another lane finds its last streamed answer finished.
+struct StreamSlot {
+    GpuServerCtx* owner = nullptr;
+    int lane = 0;
+    bool enqueuing = false;  // the owner is between taking it and recording its event
+};
 std::mutex g_stream_mu;
-constexpr size_t kMaxDevices = 64;
-GpuServerCtx* g_streaming[kMaxDevices] = {};
+StreamSlot g_stream_slots[GpuServerCtx::kMaxDevices][GpuServerCtx::kLanes];
 
 // Row slices of a streamed pass over C columns: up to 16, with partials of
 // at most 32 MiB per query.
@@ -404,10 +410,16 @@ void GpuServerCtx::alloc_slots() {
         d_KS[l] = dalloc<uint32_t>(kKeySumWords);
     }
     d_hstate = dalloc<uint32_t>(B * T * 4 * N);
-    trace_name_stream(stream, "server");
+    mstream[0] = stream;
     for (int l = 0; l < kLanes; l++) {
+        // a lane's three streams in a row: three hardware queues
+        if (l > 0) HIPX(hipStreamCreate(&mstream[l]));
         HIPX(hipStreamCreate(&hstream[l]));
         HIPX(hipStreamCreate(&cstream[l]));
+        HIPX(hipEventCreateWithFlags(&hop_in_ev[l], hipEventDisableTiming));
+        HIPX(hipEventCreateWithFlags(&hop_out_ev[l], hipEventDisableTiming));
+        static const char* mn[kLanes] = {"server", "passes lane 1", "passes lane 2", "passes lane 3"};
+        trace_name_stream(mstream[l], mn[l]);
         static const char* hn[kLanes] = {"horner lane 0", "horner lane 1", "horner lane 2", "horner lane 3"};
         static const char* cn[kLanes] = {"collapse lane 0", "collapse lane 1", "collapse lane 2", "collapse lane 3"};
         trace_name_stream(hstream[l], hn[l]);
@@ -424,14 +436,9 @@ void GpuServerCtx::alloc_slots() {
         d_sflags[l] = dalloc<uint32_t>(words);
         HIPX(hipMemset(d_sflags[l], 0, words * 4));
     }
-    // INSPIRE_STREAM=0: no streamed shapes; otherwise the device's first
-    // live server takes them (see stream_ok)
+    // INSPIRE_STREAM=0: no streamed shapes
     const char* se = std::getenv("INSPIRE_STREAM");
-    if (!(se && se[0] == '0')) {
-        std::lock_guard<std::mutex> lk(g_stream_mu);
-        stream_ok = (size_t)device < kMaxDevices && !g_streaming[device];
-        if (stream_ok) g_streaming[device] = this;
-    }
+    stream_ok = !(se && se[0] == '0') && (size_t)device < kMaxDevices;
     d_hxbuf = dalloc<uint32_t>(horner_pair_xbuf_words(B * T));
     d_hflags = dalloc<uint32_t>(2 * B * T);
     d_status = dalloc<uint32_t>(kLanes);
@@ -520,7 +527,8 @@ void GpuServerCtx::autotune_dbpass() {
     // 1.4 times (and 20 us) slower, later ones those above the spread of
     // repeated runs (a few percent). All candidates through all rounds took
     // 158 of a 1 GB server's 232 ms.
-    auto fastest = [&](size_t n, auto&& prep, auto&& run, int rounds = 4) {
+    auto fastest = [&](size_t n, auto&& prep, auto&& run, int rounds = 4, hipStream_t ts = nullptr) {
+        if (!ts) ts = stream;
         std::vector<std::vector<float>> got(n);
         std::vector<size_t> left(n);
         for (size_t i = 0; i < n; i++) left[i] = i;
@@ -532,9 +540,9 @@ void GpuServerCtx::autotune_dbpass() {
         for (int round = 0; round < rounds && left.size() > 1; round++) {
             for (const size_t i : left) {
                 prep(i);
-                HIPX(hipEventRecord(e0, stream));
+                HIPX(hipEventRecord(e0, ts));
                 run(i);
-                HIPX(hipEventRecord(e1, stream));
+                HIPX(hipEventRecord(e1, ts));
                 HIPX(hipEventSynchronize(e1));
                 float ms = 0;
                 HIPX(hipEventElapsedTime(&ms, e0, e1));
@@ -670,6 +678,9 @@ void GpuServerCtx::autotune_dbpass() {
     const bool chunked_ok = G / gchunk > 1;
     if (chunked_ok || can_stream(stream)) {
         const size_t ccols = gchunk * N;
+        // as a caller's stream sees them, the hop of pipelined answers included
+        const hipStream_t caller = mstream[1];
+        HIPX(hipStreamSynchronize(stream));
         for (const size_t count : {(size_t)1, nq}) {
             const DbPlan full = plan_for(count, C);
             const size_t blocks = ccols / dbplan_cols(full);
@@ -756,7 +767,8 @@ void GpuServerCtx::autotune_dbpass() {
             for (const Pick& c : cands) (c.shape >= 6 ? streamed : chunked).push_back(c);
             auto time_picks = [&](std::vector<Pick>& v) {
                 const size_t b = fastest(
-                    v.size(), [&](size_t i) { use(v[i]); }, [&](size_t) { enqueue(d_q, count, d_resp, stream); }, 6);
+                    v.size(), [&](size_t i) { use(v[i]); }, [&](size_t) { enqueue(d_q, count, d_resp, caller); }, 6,
+                    caller);
                 use(v[b]);
                 return v[b];
             };
@@ -892,17 +904,40 @@ DbPlan GpuServerCtx::stream_plan(size_t nq, uint32_t slices, bool fused) const {
     return p;
 }
 
-void GpuServerCtx::take_streaming() {
+bool GpuServerCtx::take_stream_slot(int lane) {
+    std::lock_guard<std::mutex> lk(g_stream_mu);
+    StreamSlot* free_slot = nullptr;
+    // the queries are legal beside another thread's stream capture
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    for (StreamSlot& x : g_stream_slots[device]) {
+        if (x.owner == this && x.lane == lane) {
+            x.enqueuing = true;
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+            return true;
+        }
+        if (!free_slot && !x.enqueuing &&
+            (!x.owner || hipEventQuery(x.owner->horner_done[x.lane]) == hipSuccess))
+            free_slot = &x;
+    }
+    (void)hipGetLastError();  // a query that found work pending is no error
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!free_slot) return false;
+    *free_slot = StreamSlot{this, lane, true};
+    return true;
+}
+
+void GpuServerCtx::settle_stream_slot(int lane) {
+    std::lock_guard<std::mutex> lk(g_stream_mu);
+    for (StreamSlot& x : g_stream_slots[device])
+        if (x.owner == this && x.lane == lane) x.enqueuing = false;
+}
+
+void GpuServerCtx::drop_stream_slots() {
     std::lock_guard<std::mutex> lk(g_stream_mu);
     if ((size_t)device >= kMaxDevices) return;
-    GpuServerCtx* prev = g_streaming[device];
-    if (prev == this) return;
-    if (prev) {
-        std::lock_guard<std::mutex> pl(prev->mu);  // its calls see the change between answers
-        prev->stream_ok = false;
-    }
-    g_streaming[device] = this;
-    stream_ok = true;
+    for (StreamSlot& x : g_stream_slots[device])
+        if (x.owner == this) x = StreamSlot{};
 }
 
 void GpuServerCtx::mark_pass(hipStream_t s, bool first) {
@@ -1027,10 +1062,39 @@ void GpuServerCtx::horner_range(size_t count, uint64_t* d_out, size_t g_lo, size
                            count, nc, cc, s, fp ? *fp : FusedPack{}));
 }
 
+int GpuServerCtx::shape_for(size_t nq) const {
+    int shape = nq == 1 ? pipe_single : pipe_batched;
+    // one chunk: nothing to pipeline but the collapse beside the pass (3)
+    if (shape < 6 && shape != 3 && G == gchunk) shape = 0;
+    // shape 8 (the collapse inside the streamed pass's launch) takes the
+    // direct pass kernel: up to 8 queries, else shape 6
+    if (shape == 8 && (nq > 8 || stream_plan(nq, nq == 1 ? stream_slices1 : stream_slices).param > 4)) shape = 6;
+    return shape;
+}
+
 void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0,
                            int lane, bool status_read) {
     if (lane < 0 || lane >= kLanes) throw std::invalid_argument("enqueue: scratch lane out of range");
     TraceRange tr("answer: %zu queries, slots %zu.., lane %d", count, slot0, lane);
+    // pipelined answers run on the lane's own three streams (mstream);
+    // under capture on s itself, whose replay has no queues to share
+    const size_t last = count % kMfmaMaxQueries;
+    const bool pipelined = (count >= kMfmaMaxQueries && shape_for(kMfmaMaxQueries)) || (last && shape_for(last));
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (pipelined && s != mstream[lane]) HIPX(hipStreamIsCapturing(s, &cap));
+    if (!pipelined || s == mstream[lane] || cap != hipStreamCaptureStatusNone) {
+        enqueue_on(d_in, count, d_out, s, slot0, lane, status_read);
+        return;
+    }
+    HIPX(hipEventRecord(hop_in_ev[lane], s));
+    HIPX(hipStreamWaitEvent(mstream[lane], hop_in_ev[lane], 0));
+    enqueue_on(d_in, count, d_out, mstream[lane], slot0, lane, status_read);
+    HIPX(hipEventRecord(hop_out_ev[lane], mstream[lane]));
+    HIPX(hipStreamWaitEvent(s, hop_out_ev[lane], 0));
+}
+
+void GpuServerCtx::enqueue_on(const uint64_t* d_in, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0,
+                              int lane, bool status_read) {
     const size_t C = pp.db_cols;
     const size_t nchunks = G / gchunk;
     const hipStream_t hs = hstream[lane];
@@ -1042,6 +1106,17 @@ void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, 
     // and through their waits for every collapse.
     bool joined = false;
     const bool streamable = can_stream(s);
+    // the device's slot for this lane's streamed sub-batches, taken with the
+    // first of them and given up for taking over once this answer's event is
+    // recorded
+    struct SlotHold {
+        GpuServerCtx* c;
+        int lane;
+        bool held = false;
+        ~SlotHold() {
+            if (held) c->settle_stream_slot(lane);
+        }
+    } slot_hold{this, lane};
     last_part_slices = 0;  // the first sub-batch's result lands in interm unless it streams with slices
     // Serial sub-batches (shape 0) leave their Horner chains to one launch
     // after the last of them: a sub-batch's nq x T chains each hold a CU for
@@ -1056,25 +1131,22 @@ void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, 
     };
     for (size_t q0 = slot0; q0 < slot0 + count; q0 += kMfmaMaxQueries) {
         const size_t nq = slot0 + count - q0 < kMfmaMaxQueries ? slot0 + count - q0 : kMfmaMaxQueries;
-        int shape = nq == 1 ? pipe_single : pipe_batched;
-        // one chunk: nothing to pipeline but the collapse beside the pass (3)
-        if (shape < 6 && shape != 3 && nchunks == 1) shape = 0;
+        int shape = shape_for(nq);
         uint32_t* p2 = d_part2 + q0 * part2_stride;
         const uint32_t* keys = d_keys + q0 * keys_stride;
         uint32_t* packed = d_packed_b + q0 * packed_stride;
         uint64_t* out = d_out + (q0 - slot0) * resp_u64s;
         const uint64_t* in = d_in + (q0 - slot0) * qlen;
         DbPlan sp;
-        // shape 8 (the collapse inside the streamed pass's launch) takes the
-        // direct pass kernel: up to 8 queries, else shape 6
-        if (shape == 8 && (nq > 8 || stream_plan(nq, nq == 1 ? stream_slices1 : stream_slices).param > 4)) shape = 6;
         if (shape >= 6) {
             sp = stream_plan(nq, nq == 1 ? stream_slices1 : stream_slices, shape == 8);
             // a forced pair Horner cannot wait for a streamed pass, and a
             // sub-batch whose waiting workgroups exceed kStreamMaxWaiters
             // CUs would leave too few to the passes of 4 lanes: the chunked
             // shape then
-            if (!streamable || sp.kind != DbPlan::MFMA || horner_mode == 1 || !stream_fits(nq))
+            if (streamable && sp.kind == DbPlan::MFMA && horner_mode != 1 && stream_fits(nq) && !slot_hold.held)
+                slot_hold.held = take_stream_slot(lane);
+            if (!slot_hold.held || sp.kind != DbPlan::MFMA || !stream_fits(nq))
                 shape = nchunks == 1 ? 0 : nq == 1 ? pipe_single_chunked : pipe_batched_chunked;
         }
         if (shape != 0) flush_deferred();
@@ -1485,21 +1557,24 @@ void gpu_free_server(GpuServerCtx* ctx) {
     dfree(ctx->d_part); dfree(ctx->d_interm); dfree(ctx->d_part2); dfree(ctx->d_packed_b);
     dfree(ctx->d_hxbuf); dfree(ctx->d_hflags); dfree(ctx->d_status); dfree(ctx->d_hstate);
     for (auto& f : ctx->d_sflags) dfree(f);
-    {
-        std::lock_guard<std::mutex> lk(g_stream_mu);
-        if ((size_t)ctx->device < kMaxDevices && g_streaming[ctx->device] == ctx) g_streaming[ctx->device] = nullptr;
-    }
     dfree(ctx->d_qpack); dfree(ctx->d_cmp); dfree(ctx->d_rcmp);
     for (int l = 0; l < GpuServerCtx::kLanes; l++) {
         if (ctx->hstream[l]) (void)hipStreamSynchronize(ctx->hstream[l]);
+        if (l == 0) ctx->drop_stream_slots();  // before their events go
         if (ctx->cstream[l]) (void)hipStreamSynchronize(ctx->cstream[l]);
         for (auto& e : ctx->chunk_ev[l])
             if (e) (void)hipEventDestroy(e);
         for (auto& e : ctx->coll_ev[l])
             if (e) (void)hipEventDestroy(e);
         if (ctx->prep_ev[l]) (void)hipEventDestroy(ctx->prep_ev[l]);
+        if (ctx->hop_in_ev[l]) (void)hipEventDestroy(ctx->hop_in_ev[l]);
+        if (ctx->hop_out_ev[l]) (void)hipEventDestroy(ctx->hop_out_ev[l]);
         if (ctx->pass_ev[l]) (void)hipEventDestroy(ctx->pass_ev[l]);
         if (ctx->horner_done[l]) (void)hipEventDestroy(ctx->horner_done[l]);
+        if (l > 0 && ctx->mstream[l]) {
+            (void)hipStreamSynchronize(ctx->mstream[l]);
+            (void)hipStreamDestroy(ctx->mstream[l]);
+        }
         if (ctx->hstream[l]) (void)hipStreamDestroy(ctx->hstream[l]);
         if (ctx->cstream[l]) (void)hipStreamDestroy(ctx->cstream[l]);
     }

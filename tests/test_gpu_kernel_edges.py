@@ -1,5 +1,7 @@
 """Kernels at the edges of their ranges against the oracle: the largest
 residues through the unfolded transforms of the Horner chain."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -72,3 +74,45 @@ def test_batches_of_every_pass_form_match_oracle(odd_table, nq):
         if want[i] is None:
             want[i] = pc.answer(qs[i]).reshape(-1)
         assert np.array_equal(got[i], want[i]), f"query {i} of {nq}"
+
+
+def test_servers_on_one_device_stream_side_by_side():
+    """Six servers share the device's four slots for streamed answers: each
+    answer streams or takes its chunked shape, enqueued back to back on two
+    streams without waiting, and equals the serial answer; with few in flight
+    a second server streams too."""
+    n, w, rows, nq = 524288, 120, 2048, 3
+    rc, geo = ol.setup(n, w, rows)
+    db = np.random.default_rng(8).integers(0, ol.P, size=(geo["R"], geo["C"]), dtype=np.uint16)
+    lib = ia.load("server")
+    srvs = [ia.Server(db, n, w, rows, max_batch=nq, crs_seed=bytes(SEED)) for _ in range(6)]
+    streams = [lib.ipir_dev_stream_create() for _ in range(2)]
+    qs = np.stack([ol.make_query(geo, SEED, 1000 * k + 5, 70 + k)[0] for k in range(nq)])
+    dq = ia.DeviceBuffer(qs.nbytes, lib)
+    dq.upload(qs)
+    outs = [ia.DeviceBuffer(nq * geo["T"] * 4 * N * 8, lib) for _ in srvs]
+    try:
+        for s in srvs:
+            assert lib.ipir_dbg_stream_ok(s.h) == 1
+            assert lib.ipir_dbg_set_pipeline(s.h, 0, 0) == 0
+        want = srvs[0].answer_batch(list(qs))
+        for s in srvs:
+            assert lib.ipir_dbg_set_stream_slices(s.h, nq, 4) == 0
+            assert lib.ipir_dbg_set_pipeline(s.h, 6, 6) == 0
+        before = [lib.ipir_dbg_streamed_count(s.h) for s in srvs]
+        for s in srvs[:2]:
+            assert np.array_equal(s.answer_batch(list(qs)), want)
+        assert [lib.ipir_dbg_streamed_count(s.h) - b for s, b in zip(srvs[:2], before)] == [1, 1]
+        for rnd in range(4):
+            for k, s in enumerate(srvs):
+                assert lib.ipir_answer_batch_device(s.h, C.c_void_p(dq.p), nq, C.c_void_p(outs[k].p),
+                                                    streams[k % 2]) == 0
+        assert lib.ipir_dev_sync() == 0
+        for k, s in enumerate(srvs):
+            assert lib.ipir_device_status(s.h) == 0
+            assert np.array_equal(outs[k].download(np.zeros_like(want)), want), f"server {k}"
+    finally:
+        for s in srvs:
+            s.close()
+        for st in streams:
+            lib.ipir_dev_stream_destroy(st)
