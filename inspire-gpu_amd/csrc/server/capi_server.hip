@@ -7,6 +7,7 @@
 #include <memory>
 #include <vector>
 
+#include "../host/narrow.h"
 #include "capi.h"
 #include "inspire_debug.h"
 #include "server_ctx.h"
@@ -16,20 +17,21 @@ using namespace inspire;
 
 namespace {
 size_t blk() { return (size_t)D_EFF * 2 * N; }
-
-// copy `count` query views into the context's pinned flat staging
-void stage_views(GpuServerCtx* ctx, const ipir_query_view* qs, size_t count) {
-    const size_t R = ctx->pp.db_rows, b = blk();
-    for (size_t i = 0; i < count; i++) {
-        uint64_t* w = ctx->h_q + i * ctx->qlen;
-        std::memcpy(w, qs[i].lwe_b_limb0, R * 8);
-        std::memcpy(w + R, qs[i].lwe_b_limb1, R * 8);
-        std::memcpy(w + 2 * R, qs[i].ksk5_b, b * 8);
-        std::memcpy(w + 2 * R + b, qs[i].kskneg1_b, b * 8);
-        std::memcpy(w + 2 * R + 2 * b, qs[i].rgsw, 4 * b * 8);
-    }
-}
 }  // namespace
+
+void flatten_view(const ipir_query_view& v, size_t R, uint32_t* w) {
+    const size_t b = (size_t)D_EFF * 2 * N;
+    narrow_residues(v.lwe_b_limb0, w, R, Q0);
+    narrow_residues(v.lwe_b_limb1, w + R, R, Q1);
+    w += 2 * R;
+    // parts of [digit][limb][N]
+    auto parts = [&](const uint64_t* p, size_t n) {
+        for (size_t o = 0; o < n; o += N, w += N) narrow_residues(p + o, w, N, (o / N) & 1 ? Q1 : Q0);
+    };
+    parts(v.ksk5_b, b);
+    parts(v.kskneg1_b, b);
+    parts(v.rgsw, 4 * b);
+}
 
 extern "C" {
 
@@ -87,8 +89,8 @@ int ipir_answer_batch(ipir_server* srv, const ipir_query_view* queries, size_t c
     try {
         std::lock_guard<std::mutex> lk(srv->ctx->mu);
         if (srv->ctx->loop_active) return 5;
-        stage_views(srv->ctx, queries, count);
-        srv->ctx->answer_host(count, out_resp);
+        const size_t R = srv->ctx->pp.db_rows;
+        srv->ctx->answer_host(count, [&](size_t i, uint32_t* w) { flatten_view(queries[i], R, w); }, out_resp);
         return 0;
     } catch (...) {
         return 4;
@@ -124,7 +126,8 @@ int ipir_device_status(ipir_server* srv) {
         if (c->loop_active) return 5;
         hipStream_t s = c->stream;
         c->order_before(s);  // the last call's work, whatever stream it ran on
-        c->check_status(s, 0);
+        hip_check(hipStreamSynchronize(s), "device status");
+        c->check_status(0);
         return 0;
     } catch (...) {
         return 4;
@@ -397,9 +400,15 @@ int ipir_dbg_answer_taps(ipir_server* srv, const uint64_t* query, uint32_t* inte
     try {
         std::lock_guard<std::mutex> lk(c->mu);
         if (c->loop_active) return 5;
-        std::memcpy(c->h_q, query, c->qlen * 8);
+        ipir_query_view v;
+        const size_t R = c->pp.db_rows;
+        v.lwe_b_limb0 = query;
+        v.lwe_b_limb1 = query + R;
+        v.ksk5_b = query + 2 * R;
+        v.kskneg1_b = v.ksk5_b + blk();
+        v.rgsw = v.kskneg1_b + blk();
         std::vector<uint64_t> r(c->resp_u64s);
-        c->answer_host(1, r.data());
+        c->answer_host(1, [&](size_t, uint32_t* w) { flatten_view(v, R, w); }, r.data());
         if (resp) std::memcpy(resp, r.data(), r.size() * 8);
         if (interm && c->last_part_slices > 1) {
             // a streamed pass left row-slice partials (the pack sums them):
@@ -691,7 +700,7 @@ int ipir_dbg_stream_parts(ipir_server* srv, size_t nq, uint32_t slices, double* 
         pk.pass_target = target;
         pk.packed_done = packed_done;
         pk.spin_limit = c->stream_spin_limit;
-        pk.status = c->d_status;
+        pk.status = c->h_status;
         pk.queries = pq;
         out_ms[2] = timed([&] {
             hip_check(ipx::launch_fill_u32(pass_done, G, target, s), "fill");
@@ -706,7 +715,7 @@ int ipir_dbg_stream_parts(ipir_server* srv, size_t nq, uint32_t slices, double* 
         sw.queries = pq;
         sw.stride = (uint32_t)G;
         sw.spin_limit = c->stream_spin_limit;
-        sw.status = c->d_status;
+        sw.status = c->h_status;
         hip_check(ipx::launch_fill_u32(packed_done, nblk * G, 1, s), "fill");
         out_ms[3] = timed([&] {
             hip_check(ipx::launch_horner(c->d_precomp + ipx::PC_A, ipx::PC_GROUP, G, c->Da, c->T, c->d_packed_b,
@@ -723,7 +732,7 @@ int ipir_dbg_stream_parts(ipir_server* srv, size_t nq, uint32_t slices, double* 
         });
         c->order_after(s);
         hip_check(hipStreamSynchronize(s), "sync");
-        c->check_status(s, 0);
+        c->check_status(0);
     } catch (...) {
         rc = 4;
     }
@@ -885,7 +894,6 @@ int ipir_dbg_profile_batch(ipir_server* srv, const uint64_t* d_queries, size_t c
     try {
         for (auto& e : ev) hip_check(hipEventCreate(&e), "event");
         c->order_before(s);
-        c->clear_status(s, 0);
         // kept as staged queries for ipir_dbg_time_dbpass
         hip_check(hipMemcpyAsync(c->d_q, d_queries, count * c->qlen * 8, hipMemcpyDeviceToDevice, s), "stage queries");
         size_t k = 0;
@@ -894,7 +902,9 @@ int ipir_dbg_profile_batch(ipir_server* srv, const uint64_t* d_queries, size_t c
             const size_t nq = count - q0 < step ? count - q0 : step;
             const ipx::DbPlan p = c->serial_plan(nq);
             mark();
-            c->prep_query(c->d_q + q0 * c->qlen, q0, nq, p, s, 0);
+            GpuServerCtx::PrepZero z;
+            if (q0 == 0) z.status = c->h_status;
+            c->prep_query(c->d_q + q0 * c->qlen, q0, nq, p, s, 0, z);
             mark();
             c->dbpass_whole(q0, nq, p, s, 0);
             mark();
@@ -908,7 +918,7 @@ int ipir_dbg_profile_batch(ipir_server* srv, const uint64_t* d_queries, size_t c
         mark();
         c->order_after(s);
         hip_check(hipEventSynchronize(ev[k - 1]), "sync");
-        c->check_status(s, 0);
+        c->check_status(0);
         for (int i = 0; i < 5; i++) stage_ms[i] = 0;
         float ms = 0;
         for (size_t b = 0; b < nsub; b++)

@@ -33,8 +33,8 @@ hipError_t launch_copy16(const void* src, void* dst, size_t bytes, hipStream_t s
 // Bytes of one query in the 53-bit CRT-packed form.
 size_t query_packed_bytes(size_t R);
 // count packed queries (query_packed_bytes(R) bytes each, back to back) ->
-// flat u64 queries (qlen u64s apart).
-hipError_t launch_query_unpack(const uint8_t* packed, size_t count, size_t R, uint64_t* flat, size_t qlen,
+// flat queries of u32 residues (qlen words apart).
+hipError_t launch_query_unpack(const uint8_t* packed, size_t count, size_t R, uint32_t* flat, size_t qlen,
                                hipStream_t s);
 // nct response cts (flat u64, NTT form, [ct][a|b][limb][N]) -> 12288
 // compressed bytes each; scratch holds nct*4*N words.
@@ -91,7 +91,8 @@ constexpr uint32_t kOffsetSumParts = 8;  // row ranges of S: [query][limb][part]
 constexpr uint32_t kKeySumParts = 2;     // KS: [query][limb][digit]
 enum PrepForm : uint32_t { kPrepDoubles, kPrepDigits4, kPrepDigits7, kPrepPower };
 struct PrepArgs {
-    const uint64_t* q = nullptr;  // query 0's words (LWE part first), queries q_stride apart
+    const void* q = nullptr;      // query 0's words (LWE part first), queries q_stride words apart
+    bool narrow = false;          // u32 words instead of u64
     size_t q_stride = 0, R = 0;
     double* bq = nullptr;         // [query][limb][R]
     int8_t* dig = nullptr;
@@ -109,9 +110,11 @@ struct PrepArgs {
     size_t part2_stride = 0, part2_words = 0;
     bool skip_lwe = false;        // keys and RGSW rows only
     // set by launch_prep
-    uint32_t form = 0, parts = 0, Mp = 0, kMp = 0, key_blocks = 0, lwe_blocks = 0, rgsw_blocks = 0;
+    uint32_t first = 0, form = 0, parts = 0, Mp = 0, kMp = 0, key_blocks = 0, lwe_blocks = 0, rgsw_blocks = 0;
 };
-hipError_t launch_prep(PrepArgs a, size_t nq, const DbPlan& p, const NttConst& nc, hipStream_t s);
+// first, count: queries [first, first + count) of the nq only (count 0: all).
+hipError_t launch_prep(PrepArgs a, size_t nq, const DbPlan& p, const NttConst& nc, hipStream_t s, size_t first = 0,
+                       size_t count = 0);
 // Name of the kernel a plan launches (as profilers report it, without arguments).
 std::string dbplan_kernel(const DbPlan& p);
 // Output of the database passes: out points at the first column's residue

@@ -60,14 +60,16 @@ __device__ __forceinline__ void put_digits4(uint32_t (&o)[4], uint32_t val, int 
     }
 }
 
+// W: the words of the query, u64 as on the wire or narrowed to u32.
+template <typename W>
 __global__ __launch_bounds__(256) void k_prep(PrepArgs a, NttConst nc) {
     __shared__ __align__(16) uint32_t lds[2 * kRowLds];  // two limbs of a chunk's rows, or one polynomial
     __shared__ uint64_t red[2][4];
-    const uint32_t t = threadIdx.x, qi = blockIdx.y;
-    const uint64_t* w = a.q + (size_t)qi * a.q_stride;
+    const uint32_t t = threadIdx.x, qi = blockIdx.y + a.first;
+    const W* w = static_cast<const W*>(a.q) + (size_t)qi * a.q_stride;
     const size_t R = a.R;
     uint32_t b = blockIdx.x;
-    if (b == 0 && qi == 0) {
+    if (b == 0 && qi == 0) {  // with the first query
         for (uint32_t x = t; x < a.zero_words; x += 256) a.zero[x] = 0;
         if (a.status && t == 0) *a.status = 0;
     }
@@ -76,7 +78,7 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a, NttConst nc) {
         const int c = (int)(b & 1);
         const uint32_t j = (b >> 1) & 1, key = b >> 2;
         const NrLimb m = nr_limb(c);
-        uint64_t in[8];
+        W in[8];
 #pragma unroll
         for (int k = 0; k < 8; k++) in[k] = w[2 * R + (size_t)b * N + t + 256 * k];
         NrTw tw[4];
@@ -131,8 +133,8 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a, NttConst nc) {
             for (uint32_t l = 0; l < 2; l++) {
                 if (l >= nl) break;
                 const int c = (int)(c0 + l);
-                const uint64_t* src = w + (size_t)c * R + (size_t)kc * 16;
-                uint64_t v[16];
+                const W* src = w + (size_t)c * R + (size_t)kc * 16;
+                W v[16];
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const uint32_t r = t + 256 * i;
@@ -223,9 +225,9 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a, NttConst nc) {
     }
     b -= a.lwe_blocks;
     if (b < a.rgsw_blocks) {
-        const uint64_t* src = w + 2 * R + 2 * BLK + (size_t)b * 4096;
+        const W* src = w + 2 * R + 2 * BLK + (size_t)b * 4096;
         uint32_t* dst = a.rgsw + (size_t)qi * a.rgsw_stride + (size_t)b * 4096;
-        uint64_t v[16];
+        W v[16];
 #pragma unroll
         for (int i = 0; i < 16; i++) v[i] = src[t + 256 * i];
 #pragma unroll
@@ -241,7 +243,11 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a, NttConst nc) {
 
 }  // namespace
 
-hipError_t launch_prep(PrepArgs a, size_t nq, const DbPlan& p, const NttConst& nc, hipStream_t s) {
+hipError_t launch_prep(PrepArgs a, size_t nq, const DbPlan& p, const NttConst& nc, hipStream_t s, size_t first,
+                       size_t count) {
+    if (count == 0) count = nq;
+    if (first + count > nq) return hipErrorInvalidValue;
+    a.first = (uint32_t)first;
     if (nq == 0 || nq > kMfmaMaxQueries || nq > kCollapseMaxQueries || !a.q || a.R == 0 || a.R % N)
         return hipErrorInvalidValue;
     a.Mp = (uint32_t)dbplan_mp(p);
@@ -266,7 +272,11 @@ hipError_t launch_prep(PrepArgs a, size_t nq, const DbPlan& p, const NttConst& n
     }
     if (a.part2_words % 4096 || (a.part2_words && !a.part2) || (a.zero_words && !a.zero)) return hipErrorInvalidValue;
     const size_t blocks = a.key_blocks + a.lwe_blocks + a.rgsw_blocks + a.part2_words / 4096;
-    hipLaunchKernelGGL(k_prep, dim3((unsigned)blocks, (unsigned)nq), dim3(256), 0, s, a, nc);
+    const dim3 grid((unsigned)blocks, (unsigned)count);
+    if (a.narrow)
+        hipLaunchKernelGGL(k_prep<uint32_t>, grid, dim3(256), 0, s, a, nc);
+    else
+        hipLaunchKernelGGL(k_prep<uint64_t>, grid, dim3(256), 0, s, a, nc);
     return hipGetLastError();
 }
 

@@ -34,7 +34,7 @@ using Clock = std::chrono::steady_clock;
 
 struct Req {
     uint64_t ticket = 0;
-    std::vector<uint64_t> q;  // flat query
+    std::vector<uint32_t> q;  // flat query, narrowed
     uint64_t* out = nullptr;
     Clock::time_point t0;
     double lat_us = 0;
@@ -103,16 +103,18 @@ struct ipir_loop {
             if (n > st.max_batch_size) st.max_batch_size = n;
             st.batches++;
             for (size_t i = 0; i < n; i++)
-                std::memcpy(ctx->h_q + (free_p->slot0 + i) * ctx->qlen, free_p->batch[i]->q.data(), ctx->qlen * 8);
+                std::memcpy(ctx->h_q + (free_p->slot0 + i) * ctx->qlen, free_p->batch[i]->q.data(), ctx->qlen * 4);
             lk.unlock();
             bool ok = true;
             try {
                 const size_t s0 = free_p->slot0;
                 hip_check(hipEventRecord(free_p->ev0, free_p->stream), "loop event");
-                hip_check(hipMemcpyAsync(ctx->d_q + s0 * ctx->qlen, ctx->h_q + s0 * ctx->qlen, n * ctx->qlen * 8,
-                                         hipMemcpyHostToDevice, free_p->stream), "loop h2d");
-                ctx->enqueue(ctx->d_q + s0 * ctx->qlen, n, ctx->d_resp + s0 * ctx->resp_u64s, free_p->stream, s0,
-                             free_p->lane, true);
+                // copied, not read in place: the copy engine leaves the CUs to the other partitions
+                uint32_t* dq = ctx->flat32() + s0 * ctx->qlen;
+                hip_check(hipMemcpyAsync(dq, ctx->h_q + s0 * ctx->qlen, n * ctx->qlen * 4, hipMemcpyHostToDevice,
+                                         free_p->stream), "loop h2d");
+                ctx->enqueue(QueryInput(dq), n, ctx->d_resp + s0 * ctx->resp_u64s, free_p->stream, s0, free_p->lane,
+                             true);
                 hip_check(hipMemcpyAsync(ctx->h_resp + s0 * ctx->resp_u64s, ctx->d_resp + s0 * ctx->resp_u64s,
                                          n * ctx->resp_u64s * 8, hipMemcpyDeviceToHost, free_p->stream), "loop d2h");
                 hip_check(hipEventRecord(free_p->ev1, free_p->stream), "loop event");
@@ -136,7 +138,7 @@ struct ipir_loop {
             bool ok = hipStreamSynchronize(p->stream) == hipSuccess;
             if (ok) {
                 try {
-                    ctx->check_status(p->stream, p->lane);
+                    ctx->check_status(p->lane);
                 } catch (...) {
                     ok = false;
                 }
@@ -202,12 +204,12 @@ ipir_loop* ipir_loop_start(ipir_server* srv, size_t max_inflight) {
         ctx->loop_active = true;
     }
     // status words left by earlier asynchronous calls are not this loop's
-    if (hipDeviceSynchronize() != hipSuccess ||
-        hipMemset(ctx->d_status, 0, GpuServerCtx::kLanes * sizeof(uint32_t)) != hipSuccess) {
+    if (hipDeviceSynchronize() != hipSuccess) {
         std::lock_guard<std::mutex> lk(ctx->mu);
         ctx->loop_active = false;
         return nullptr;
     }
+    for (int l = 0; l < GpuServerCtx::kLanes; l++) ctx->h_status[l] = 0;
     auto* L = new ipir_loop;
     L->srv = srv;
     L->ctx = ctx;
@@ -261,13 +263,8 @@ uint64_t ipir_loop_submit(ipir_loop* L, const ipir_query_view* v, uint64_t* out_
     if (!L || !v || !out_resp || !v->lwe_b_limb0 || !v->lwe_b_limb1 || !v->ksk5_b || !v->kskneg1_b || !v->rgsw)
         return 0;
     auto* r = new Req;
-    const size_t R = L->ctx->pp.db_rows, b = (size_t)D_EFF * 2 * N;
     r->q.resize(L->ctx->qlen);
-    std::memcpy(r->q.data(), v->lwe_b_limb0, R * 8);
-    std::memcpy(r->q.data() + R, v->lwe_b_limb1, R * 8);
-    std::memcpy(r->q.data() + 2 * R, v->ksk5_b, b * 8);
-    std::memcpy(r->q.data() + 2 * R + b, v->kskneg1_b, b * 8);
-    std::memcpy(r->q.data() + 2 * R + 2 * b, v->rgsw, 4 * b * 8);
+    flatten_view(*v, L->ctx->pp.db_rows, r->q.data());
     r->out = out_resp;
     std::lock_guard<std::mutex> lk(L->m);
     if (L->stop) {

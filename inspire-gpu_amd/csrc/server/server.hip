@@ -15,8 +15,10 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <vector>
 
+#include "../host/narrow.h"
 #include "gpu_protocol.h"
 #include "kernels.h"
 #include "server_ctx.h"
@@ -346,10 +348,10 @@ ServerFootprint server_footprint(const PublicParams& pp, size_t gchunk) {
     f.per_slot = qlen * 8 + resp * 8 + 2 * R * 8 +
                  (lay.keys_words() + lay.rgsw_words() + part_words + 2 * C + 2 * G * 2 * N) * 4 +
                  (horner_pair_xbuf_words(T) + 2 * T + T * 4 * N) * 4 +
-                 query_packed_bytes(R) + T * 4 * N * 4 + T * GpuServerCtx::kCompressedCtBytes;
+                 T * 4 * N * 4;
     f.fixed = R * C * 2 + G * PC_GROUP * 4 + 8 * N * 4 +
               GpuServerCtx::kLanes *
-                  (R * 256 + GpuServerCtx::kKdigBytes + (GpuServerCtx::kSumWords + GpuServerCtx::kKeySumWords) * 4 + 4);
+                  (R * 256 + GpuServerCtx::kKdigBytes + (GpuServerCtx::kSumWords + GpuServerCtx::kKeySumWords) * 4);
     // streamed answers' flags: one set per lane and 32 slots (rounded up)
     const size_t set_bytes = GpuServerCtx::kStreamSetWords * G * 4;
     f.fixed += GpuServerCtx::kLanes * set_bytes;
@@ -441,8 +443,8 @@ void GpuServerCtx::alloc_slots() {
     stream_ok = !(se && se[0] == '0') && (size_t)device < kMaxDevices;
     d_hxbuf = dalloc<uint32_t>(horner_pair_xbuf_words(B * T));
     d_hflags = dalloc<uint32_t>(2 * B * T);
-    d_status = dalloc<uint32_t>(kLanes);
-    HIPX(hipMemset(d_status, 0, kLanes * 4));
+    HIPX(hipHostMalloc((void**)&h_status, kLanes * 4, hipHostMallocDefault));
+    for (int l = 0; l < kLanes; l++) h_status[l] = 0;
     horner_spin_limit = kHornerSpinLimit;
     stream_spin_limit = kStreamSpinLimit;
     HIPX(hipEventCreateWithFlags(&order_ev, hipEventDisableTiming));
@@ -468,12 +470,13 @@ void GpuServerCtx::alloc_slots() {
             pipe_forced = true;
         }
     }
-    // packed-wire path: packed queries, coefficient-form scratch, compressed responses
+    // packed-wire path: coefficient-form scratch
     qpack_bytes = query_packed_bytes(R);
-    d_qpack = dalloc<uint8_t>(B * qpack_bytes);
     d_cmp = dalloc<uint32_t>(B * T * 4 * N);
-    d_rcmp = dalloc<uint8_t>(B * T * kCompressedCtBytes);
-    HIPX(hipHostMalloc((void**)&h_q, B * qlen * 8, hipHostMallocDefault));
+    HIPX(hipHostMalloc((void**)&h_q, B * (qlen * 4 > qpack_bytes ? qlen * 4 : qpack_bytes), hipHostMallocDefault));
+    // helpers only where a batch has work for them
+    const size_t cpus = std::thread::hardware_concurrency();
+    host_stage.reset(new HostStage(B < 2 || cpus < 2 ? 0 : cpus - 1 < kStageHelpers ? cpus - 1 : kStageHelpers, B));
     HIPX(hipHostMalloc((void**)&h_resp, B * resp_u64s * 8, hipHostMallocDefault));
     resident_bytes = fp.fixed + B * fp.per_slot;
     autotune_dbpass();
@@ -787,9 +790,10 @@ void GpuServerCtx::autotune_dbpass() {
     (void)hipEventDestroy(e1);
 }
 
-PrepArgs GpuServerCtx::prep_args(const uint64_t* d_in, size_t stride, size_t q0, int lane) const {
+PrepArgs GpuServerCtx::prep_args(const QueryInput& in, size_t stride, size_t q0, int lane) const {
     PrepArgs a;
-    a.q = d_in;
+    a.q = in.q;
+    a.narrow = in.narrow;
     a.q_stride = stride;
     a.R = pp.db_rows;
     a.bq = d_bq + q0 * 2 * pp.db_rows;
@@ -798,14 +802,14 @@ PrepArgs GpuServerCtx::prep_args(const uint64_t* d_in, size_t stride, size_t q0,
     return a;
 }
 
-void GpuServerCtx::prep_lwe(const uint64_t* d_in, size_t stride, size_t q0, size_t nq, const DbPlan& p, hipStream_t s,
+void GpuServerCtx::prep_lwe(const QueryInput& in, size_t stride, size_t q0, size_t nq, const DbPlan& p, hipStream_t s,
                             int lane) {
-    HIPX(launch_prep(prep_args(d_in, stride, q0, lane), nq, p, nc, s));
+    HIPX(launch_prep(prep_args(in, stride, q0, lane), nq, p, nc, s));
 }
 
-void GpuServerCtx::prep_query(const uint64_t* d_in, size_t q0, size_t nq, const DbPlan& p, hipStream_t s, int lane,
+void GpuServerCtx::prep_query(const QueryInput& in, size_t q0, size_t nq, const DbPlan& p, hipStream_t s, int lane,
                               const PrepZero& z) {
-    PrepArgs a = prep_args(d_in, qlen, q0, lane);
+    PrepArgs a = prep_args(in, qlen, q0, lane);
     a.keys = d_keys + q0 * keys_stride;
     a.keys_stride = keys_stride;
     a.rgsw = d_rgsw + q0 * rgsw_stride;
@@ -818,7 +822,17 @@ void GpuServerCtx::prep_query(const uint64_t* d_in, size_t q0, size_t nq, const 
     a.part2 = d_part2 + q0 * part2_stride;
     a.part2_stride = part2_stride;
     a.part2_words = z.part2 ? G * 2 * N : 0;
-    HIPX(launch_prep(a, nq, p, nc, s));
+    a.status = z.status;
+    if (!in.stage) {
+        HIPX(launch_prep(a, nq, p, nc, s));
+        return;
+    }
+    // a few queries at a time, while the host stages the next ones
+    for (size_t f = 0; f < nq; f += kStagePiece) {
+        const size_t n = nq - f < kStagePiece ? nq - f : kStagePiece;
+        in.stage->wait(in.first + f + n);
+        HIPX(launch_prep(a, nq, p, nc, s, f, n));
+    }
 }
 
 DbPlan GpuServerCtx::plan_for(size_t nq, size_t ncols) const {
@@ -1055,7 +1069,7 @@ void GpuServerCtx::horner_range(size_t count, uint64_t* d_out, size_t g_lo, size
                                 packed_stride, d_rgsw + slot0 * rgsw_stride, rgsw_stride, d_out,
                                 d_hstate + slot0 * T * 4 * N, g_lo, g_hi, count,
                                 d_hxbuf + horner_pair_xbuf_words(slot0 * T), d_hflags + 2 * slot0 * T,
-                                d_status + lane, horner_spin_limit, nc, cc, s));
+                                h_status + lane, horner_spin_limit, nc, cc, s));
     else
         HIPX(launch_horner(d_precomp + PC_A, PC_GROUP, G, Da, T, d_packed_b + slot0 * packed_stride, packed_stride,
                            d_rgsw + slot0 * rgsw_stride, rgsw_stride, d_out, d_hstate + slot0 * T * 4 * N, g_lo, g_hi,
@@ -1072,7 +1086,7 @@ int GpuServerCtx::shape_for(size_t nq) const {
     return shape;
 }
 
-void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0,
+void GpuServerCtx::enqueue(const QueryInput& in, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0,
                            int lane, bool status_read) {
     if (lane < 0 || lane >= kLanes) throw std::invalid_argument("enqueue: scratch lane out of range");
     TraceRange tr("answer: %zu queries, slots %zu.., lane %d", count, slot0, lane);
@@ -1083,17 +1097,17 @@ void GpuServerCtx::enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, 
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (pipelined && s != mstream[lane]) HIPX(hipStreamIsCapturing(s, &cap));
     if (!pipelined || s == mstream[lane] || cap != hipStreamCaptureStatusNone) {
-        enqueue_on(d_in, count, d_out, s, slot0, lane, status_read);
+        enqueue_on(in, count, d_out, s, slot0, lane, status_read);
         return;
     }
     HIPX(hipEventRecord(hop_in_ev[lane], s));
     HIPX(hipStreamWaitEvent(mstream[lane], hop_in_ev[lane], 0));
-    enqueue_on(d_in, count, d_out, mstream[lane], slot0, lane, status_read);
+    enqueue_on(in, count, d_out, mstream[lane], slot0, lane, status_read);
     HIPX(hipEventRecord(hop_out_ev[lane], mstream[lane]));
     HIPX(hipStreamWaitEvent(s, hop_out_ev[lane], 0));
 }
 
-void GpuServerCtx::enqueue_on(const uint64_t* d_in, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0,
+void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0,
                               int lane, bool status_read) {
     const size_t C = pp.db_cols;
     const size_t nchunks = G / gchunk;
@@ -1136,7 +1150,9 @@ void GpuServerCtx::enqueue_on(const uint64_t* d_in, size_t count, uint64_t* d_ou
         const uint32_t* keys = d_keys + q0 * keys_stride;
         uint32_t* packed = d_packed_b + q0 * packed_stride;
         uint64_t* out = d_out + (q0 - slot0) * resp_u64s;
-        const uint64_t* in = d_in + (q0 - slot0) * qlen;
+        const QueryInput in = input.at(q0 - slot0, qlen);
+        PrepZero z;
+        if (status_read && q0 == slot0) z.status = h_status + lane;  // an earlier call's report is not this one's
         DbPlan sp;
         if (shape >= 6) {
             sp = stream_plan(nq, nq == 1 ? stream_slices1 : stream_slices, shape == 8);
@@ -1170,8 +1186,7 @@ void GpuServerCtx::enqueue_on(const uint64_t* d_in, size_t count, uint64_t* d_ou
             uint32_t* packed_done = pass_done + G;
             const uint32_t pq = pack_width(nq);
             const size_t nblk = (nq + pq - 1) / pq;
-            PrepZero z;  // the flags' last readers are done
-            z.flags = pass_done;
+            z.flags = pass_done;  // their last readers are done
             z.flag_words = (uint32_t)((1 + nblk) * G);
             z.skip_lwe = fused;
             prep_query(in, q0, nq, sp, s, lane, z);
@@ -1228,7 +1243,7 @@ void GpuServerCtx::enqueue_on(const uint64_t* d_in, size_t count, uint64_t* d_ou
             pk.pass_target = fused ? pass_collapse_target(sp, nq, G) : (uint32_t)(N / dbplan_cols(sp) * sp.slices);
             pk.packed_done = packed_done;
             pk.spin_limit = stream_spin_limit;
-            pk.status = d_status + lane;
+            pk.status = h_status + lane;
             pk.queries = pq;
             HIPX(launch_pack_stream(pk, p2, part2_stride, d_precomp, keys, keys_stride, packed, packed_stride, G, nq,
                                     nc, ps_s));
@@ -1239,7 +1254,7 @@ void GpuServerCtx::enqueue_on(const uint64_t* d_in, size_t count, uint64_t* d_ou
             sw.queries = pq;
             sw.stride = (uint32_t)G;
             sw.spin_limit = stream_spin_limit;
-            sw.status = d_status + lane;
+            sw.status = h_status + lane;
             HIPX(launch_horner(d_precomp + PC_A, PC_GROUP, G, Da, T, packed, packed_stride, d_rgsw + q0 * rgsw_stride,
                                rgsw_stride, out, d_hstate + q0 * T * 4 * N, 0, G, nq, nc, cc, hs, FusedPack{}, sw));
             // the next sub-batch's key digits and flags wait for the collapse and the pack
@@ -1253,7 +1268,6 @@ void GpuServerCtx::enqueue_on(const uint64_t* d_in, size_t count, uint64_t* d_ou
             // up to 8 queries over a small table: the pass and the collapse in
             // one launch (kMergeBytes)
             const bool both = pass_collapse_ok(p, nq) && pp.db_rows * C * 2 + G * PC_GROUP * 4 <= kMergeBytes;
-            PrepZero z;
             z.part2 = (both ? pass_collapse_ksplit(nq, G) : collapse_row_slices(nq, G, collapse_variant)) > 1;
             prep_query(in, q0, nq, p, s, lane, z);
             mark_pass(s, true);
@@ -1290,7 +1304,7 @@ void GpuServerCtx::enqueue_on(const uint64_t* d_in, size_t count, uint64_t* d_ou
         const bool first = shape == 4, ahead = shape == 5;
         joined = true;
         const DbPlan p = chunk_plan(nq, gchunk * N);  // every chunk's plan has this one's kernel and digits
-        prep_query(in, q0, nq, p, s, lane);
+        prep_query(in, q0, nq, p, s, lane, z);
         if (cs != s) {
             HIPX(hipEventRecord(prep_ev[lane], s));  // the keys are in place
             HIPX(hipStreamWaitEvent(cs, prep_ev[lane], 0));
@@ -1406,46 +1420,67 @@ void GpuServerCtx::drop_graphs() {
 }
 
 void GpuServerCtx::enqueue_packed(const uint8_t* d_in, size_t count, uint8_t* d_out, hipStream_t s, size_t slot0,
-                                  int lane, bool status_read) {
-    uint64_t* dq = d_q + slot0 * qlen;
+                                  int lane, bool status_read, HostStage* stage) {
+    uint32_t* dq = flat32() + slot0 * qlen;
     uint64_t* dr = d_resp + slot0 * resp_u64s;
-    HIPX(launch_query_unpack(d_in, count, pp.db_rows, dq, qlen, s));
-    enqueue(dq, count, dr, s, slot0, lane, status_read);
+    for (size_t f = 0; f < count; f += stage ? kStagePiece : count) {
+        const size_t n = stage && count - f > kStagePiece ? kStagePiece : count - f;
+        if (stage) stage->wait(f + n);
+        HIPX(launch_query_unpack(d_in + f * qpack_bytes, n, pp.db_rows, dq + f * qlen, qlen, s));
+    }
+    enqueue(QueryInput(dq), count, dr, s, slot0, lane, status_read);
     HIPX(launch_compress(dr, count * T, d_cmp + slot0 * T * 4 * N, d_out, nc, cc, s));
+}
+
+namespace {
+// A host job that ends with the call, also when the call throws.
+struct StagedJob {
+    HostStage& st;
+    StagedJob(HostStage& x, size_t n, std::function<void(size_t)> fn) : st(x) {
+        // waking the helpers costs tens of microseconds: from two queries on
+        st.begin(n, std::move(fn), n > 1);
+    }
+    ~StagedJob() { st.finish(); }
+};
+}  // namespace
+
+void GpuServerCtx::copy_out(size_t count, size_t bytes, void* out) {
+    // query i's response from the pinned staging, in pieces of several
+    const char* src = reinterpret_cast<const char*>(h_resp);
+    if (count * bytes < (size_t)1 << 19) {
+        std::memcpy(out, src, count * bytes);
+        return;
+    }
+    StagedJob job(*host_stage, count, [&](size_t i) {
+        std::memcpy(static_cast<char*>(out) + i * bytes, src + i * bytes, bytes);
+    });
 }
 
 void GpuServerCtx::answer_packed_host(const uint8_t* in, size_t count, uint8_t* out) {
     hipStream_t s = stream;
-    uint8_t* hq = reinterpret_cast<uint8_t*>(h_q);     // packed queries fit the flat staging
-    uint8_t* hr = reinterpret_cast<uint8_t*>(h_resp);  // so do compressed responses
-    std::memcpy(hq, in, count * qpack_bytes);
-    order_before(s);
-    clear_status(s, 0);
-    HIPX(hipMemcpyAsync(d_qpack, hq, count * qpack_bytes, hipMemcpyHostToDevice, s));
-    run_step(d_qpack, d_rcmp, count, 0, 0, 1, s, [&] { enqueue_packed(d_qpack, count, d_rcmp, s, 0, 0, true); });
-    HIPX(hipMemcpyAsync(hr, d_rcmp, count * T * kCompressedCtBytes, hipMemcpyDeviceToHost, s));
-    order_after(s);
-    HIPX(hipStreamSynchronize(s));
-    check_status(s, 0);
-    std::memcpy(out, hr, count * T * kCompressedCtBytes);
-}
-
-void GpuServerCtx::check_status(hipStream_t s, int lane) {
-    uint32_t st = 0;
-    HIPX(hipMemcpyAsync(&st, d_status + lane, 4, hipMemcpyDeviceToHost, s));
-    HIPX(hipStreamSynchronize(s));
-    if (st) {
-        HIPX(hipMemsetAsync(d_status + lane, 0, 4, s));
-        HIPX(hipStreamSynchronize(s));
-        throw std::runtime_error(
-            "a Horner chain exceeded its wait bound (pair exchange or streamed database pass); responses of this "
-            "call are invalid");
+    uint8_t* hq = reinterpret_cast<uint8_t*>(h_q);
+    uint8_t* hr = reinterpret_cast<uint8_t*>(h_resp);
+    TraceRange tr("host-staged packed answer: %zu queries", count);
+    {
+        StagedJob job(*host_stage, count,
+                      [&](size_t i) { std::memcpy(hq + i * qpack_bytes, in + i * qpack_bytes, qpack_bytes); });
+        order_before(s);
+        if (graph_mode) host_stage->wait(count);  // a replayed graph waits for nothing
+        run_step(hq, hr, count, 0, 0, 1, s,
+                 [&] { enqueue_packed(hq, count, hr, s, 0, 0, true, graph_mode ? nullptr : host_stage.get()); });
+        order_after(s);
     }
+    HIPX(hipStreamSynchronize(s));
+    check_status(0);
+    copy_out(count, T * kCompressedCtBytes, out);
 }
 
-void GpuServerCtx::clear_status(hipStream_t s, int lane) {
-    // a kernel, not a memset: the call may be captured
-    HIPX(launch_fill_u32(d_status + lane, 1, 0, s));
+void GpuServerCtx::check_status(int lane) {
+    if (!__atomic_load_n(h_status + lane, __ATOMIC_RELAXED)) return;
+    h_status[lane] = 0;
+    throw std::runtime_error(
+        "a Horner chain exceeded its wait bound (pair exchange or streamed database pass); responses of this call "
+        "are invalid");
 }
 
 void GpuServerCtx::order_before(hipStream_t s) {
@@ -1464,22 +1499,25 @@ void GpuServerCtx::order_after(hipStream_t s) {
     order_stream_set = true;
 }
 
-void GpuServerCtx::answer_host(size_t count, uint64_t* out, hipStream_t s, size_t slot0) {
-    if (!s) s = stream;
-    uint64_t* hq = h_q + slot0 * qlen;
-    uint64_t* hr = h_resp + slot0 * resp_u64s;
-    uint64_t* dq = d_q + slot0 * qlen;
-    uint64_t* dr = d_resp + slot0 * resp_u64s;
+void GpuServerCtx::answer_host(size_t count, const std::function<void(size_t, uint32_t*)>& fill, uint64_t* out) {
+    hipStream_t s = stream;
     TraceRange tr("host-staged answer: %zu queries", count);
-    order_before(s);
-    clear_status(s, 0);
-    HIPX(hipMemcpyAsync(dq, hq, count * qlen * 8, hipMemcpyHostToDevice, s));
-    run_step(dq, dr, count, slot0, 0, 0, s, [&] { enqueue(dq, count, dr, s, slot0, 0, true); });
-    HIPX(hipMemcpyAsync(hr, dr, count * resp_u64s * 8, hipMemcpyDeviceToHost, s));
-    order_after(s);
+    {
+        // The queries are narrowed into pinned memory that the preparation
+        // kernel reads, piece by piece as they come, and the chains write the
+        // responses to pinned memory: no copies of their own, half the bytes.
+        // At 1 GB, 32 queries, one thread's copies to and from the staging
+        // took 1.1 ms and the device copy 0.53 ms of a 2.1-2.5 ms call.
+        StagedJob job(*host_stage, count, [&](size_t i) { fill(i, h_q + i * qlen); });
+        order_before(s);
+        if (graph_mode) host_stage->wait(count);  // a replayed graph waits for nothing
+        const QueryInput in(h_q, graph_mode ? nullptr : host_stage.get());
+        run_step(h_q, h_resp, count, 0, 0, 0, s, [&] { enqueue(in, count, h_resp, s, 0, 0, true); });
+        order_after(s);
+    }
     HIPX(hipStreamSynchronize(s));
-    check_status(s, 0);
-    if (out) std::memcpy(out, hr, count * resp_u64s * 8);
+    check_status(0);
+    copy_out(count, resp_u64s * 8, out);
 }
 
 GpuServerCaps gpu_server_caps(const GpuServerCtx* ctx) {
@@ -1493,19 +1531,24 @@ GpuServerCaps gpu_server_caps(const GpuServerCtx* ctx) {
 }
 
 namespace {
-void flatten_query(const QueryMessage& m, size_t R, uint64_t* w) {
+void check_query(const QueryMessage& m, size_t R) {
     if (m.lwe.b_limb0.size() != R || m.lwe.b_limb1.size() != R)
         throw std::invalid_argument("gpu_answer_batch: query length differs from db_rows");
-    std::memcpy(w, m.lwe.b_limb0.data(), R * 8);
-    std::memcpy(w + R, m.lwe.b_limb1.data(), R * 8);
+    for (const std::vector<RnsPoly>* v : {&m.ksk_5.b_parts, &m.ksk_neg1.b_parts, &m.rgsw.top.a_parts,
+                                          &m.rgsw.top.b_parts, &m.rgsw.bottom.a_parts, &m.rgsw.bottom.b_parts})
+        if (v->size() != (size_t)D_EFF) throw std::invalid_argument("gpu_answer_batch: wrong digit count");
+}
+
+void flatten_query(const QueryMessage& m, size_t R, uint32_t* w) {
+    narrow_residues(m.lwe.b_limb0.data(), w, R, Q0);
+    narrow_residues(m.lwe.b_limb1.data(), w + R, R, Q1);
     w += 2 * R;
     auto parts = [&](const std::vector<RnsPoly>& v, bool want_ntt) {
-        if (v.size() != (size_t)D_EFF) throw std::invalid_argument("gpu_answer_batch: wrong digit count");
         for (const RnsPoly& p0 : v) {
             RnsPoly p = p0;
             if (want_ntt) p.to_ntt(); else p.to_coeff();
-            std::memcpy(w, p.limbs[0].data(), N * 8);
-            std::memcpy(w + N, p.limbs[1].data(), N * 8);
+            narrow_residues(p.limbs[0].data(), w, N, Q0);
+            narrow_residues(p.limbs[1].data(), w + N, N, Q1);
             w += 2 * N;
         }
     };
@@ -1524,9 +1567,9 @@ std::vector<std::vector<RlweCt>> gpu_answer_batch(GpuServerCtx* ctx, const Query
     if (count > ctx->cfg.max_batch) throw std::invalid_argument("gpu_answer_batch: count exceeds max_batch");
     std::lock_guard<std::mutex> lk(ctx->mu);
     if (ctx->loop_active) throw std::runtime_error("gpu_answer_batch: a serving loop owns this server");
-    for (size_t i = 0; i < count; i++) flatten_query(queries[i], ctx->pp.db_rows, ctx->h_q + i * ctx->qlen);
+    for (size_t i = 0; i < count; i++) check_query(queries[i], ctx->pp.db_rows);
     std::vector<uint64_t> flat(count * ctx->resp_u64s);
-    ctx->answer_host(count, flat.data());
+    ctx->answer_host(count, [&](size_t i, uint32_t* w) { flatten_query(queries[i], ctx->pp.db_rows, w); }, flat.data());
     std::vector<std::vector<RlweCt>> out(count, std::vector<RlweCt>(ctx->T));
     const uint64_t* r = flat.data();
     for (auto& resp : out)
@@ -1555,9 +1598,9 @@ void gpu_free_server(GpuServerCtx* ctx) {
     dfree(ctx->d_tw); dfree(ctx->d_db); dfree(ctx->d_precomp);
     dfree(ctx->d_q); dfree(ctx->d_resp); dfree(ctx->d_bq); dfree(ctx->d_keys); dfree(ctx->d_rgsw);
     dfree(ctx->d_part); dfree(ctx->d_interm); dfree(ctx->d_part2); dfree(ctx->d_packed_b);
-    dfree(ctx->d_hxbuf); dfree(ctx->d_hflags); dfree(ctx->d_status); dfree(ctx->d_hstate);
+    dfree(ctx->d_hxbuf); dfree(ctx->d_hflags); dfree(ctx->d_hstate);
     for (auto& f : ctx->d_sflags) dfree(f);
-    dfree(ctx->d_qpack); dfree(ctx->d_cmp); dfree(ctx->d_rcmp);
+    dfree(ctx->d_cmp);
     for (int l = 0; l < GpuServerCtx::kLanes; l++) {
         if (ctx->hstream[l]) (void)hipStreamSynchronize(ctx->hstream[l]);
         if (l == 0) ctx->drop_stream_slots();  // before their events go
@@ -1582,6 +1625,8 @@ void gpu_free_server(GpuServerCtx* ctx) {
     for (int l = 0; l < GpuServerCtx::kLanes; l++) {
         dfree(ctx->d_dig[l]); dfree(ctx->d_S[l]); dfree(ctx->d_kdig[l]); dfree(ctx->d_KS[l]);
     }
+    ctx->host_stage.reset();
+    if (ctx->h_status) (void)hipHostFree(ctx->h_status);
     if (ctx->h_q) (void)hipHostFree(ctx->h_q);
     if (ctx->h_resp) (void)hipHostFree(ctx->h_resp);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);

@@ -8,7 +8,9 @@
 #include <utility>
 #include <vector>
 
+#include "capi.h"
 #include "gpu_protocol.h"
+#include "host_stage.h"
 #include "kernels.h"
 
 namespace inspire {
@@ -17,6 +19,24 @@ void hip_check(hipError_t e, const char* what);
 inline void dfree(void* p) {
     if (p) (void)hipFree(p);
 }
+
+// Flat queries an answer starts from: u64 wire words, or words narrowed to
+// u32 (back to back, qlen words each), in device or pinned host memory; with
+// `stage`, queries that a host job is still writing (query 0 is its item 0).
+struct QueryInput {
+    const void* q = nullptr;
+    bool narrow = false;
+    HostStage* stage = nullptr;
+    size_t first = 0;  // item of query 0
+    QueryInput(const uint64_t* d) : q(d) {}
+    QueryInput(const uint32_t* d, HostStage* st = nullptr) : q(d), narrow(true), stage(st) {}
+    QueryInput at(size_t k, size_t qlen) const {
+        QueryInput x = *this;
+        x.q = static_cast<const char*>(q) + k * qlen * (narrow ? 4 : 8);
+        x.first += k;
+        return x;
+    }
+};
 
 struct GpuServerCtx {
     PublicParams pp{};
@@ -177,19 +197,26 @@ struct GpuServerCtx {
     uint32_t* d_hflags = nullptr;   // pair step flags [B*T][2]
     // per scratch lane: nonzero once a pair chain of that lane's calls gave
     // up its bounded wait (read and cleared by check_status)
-    uint32_t* d_status = nullptr;   // [kLanes]
+    // (pinned host memory the kernels write: reading it after the call costs
+    // no copy; a call whose status is read zeroes it in its first kernel)
+    uint32_t* h_status = nullptr;   // [kLanes]
     uint32_t horner_spin_limit = 0; // the pair kernel's wait bound in sleeps (0: report at once)
     uint32_t stream_spin_limit = 0; // the same for chains waiting for a streamed pass's groups
     uint32_t* d_hstate = nullptr;   // Horner chain state between chunk launches [B*T][4][N]
-    uint64_t* h_q = nullptr;        // pinned host staging
+    // Pinned host staging, which kernels read and write directly: queries
+    // narrowed to u32 words (qlen per slot), or packed ones; flat or
+    // compressed responses.
+    uint32_t* h_q = nullptr;
     uint64_t* h_resp = nullptr;
+    std::unique_ptr<HostStage> host_stage;  // fills h_q and empties h_resp
+    static constexpr size_t kStageHelpers = 3;
+    static constexpr size_t kStagePiece = 4;  // queries per preparation launch while the rest is staged
+    uint32_t* flat32() const { return reinterpret_cast<uint32_t*>(d_q); }  // unpacked queries
 
     // packed-wire path (53-bit CRT-packed queries in, compressed responses out)
     static constexpr size_t kCompressedCtBytes = ipx::N * (28 + 20) / 8;  // 12288
     size_t qpack_bytes = 0;
-    uint8_t* d_qpack = nullptr;     // packed query staging [B][qpack_bytes]
     uint32_t* d_cmp = nullptr;      // coefficient-form responses [B*T][4][N]
-    uint8_t* d_rcmp = nullptr;      // compressed response staging [B*T][12288]
 
     size_t resident_bytes = 0;
     // mu serialises every entry point that touches the slots, scratch lanes
@@ -238,16 +265,17 @@ struct GpuServerCtx {
         uint32_t flag_words = 0;
         bool part2 = false;         // the collapse sums (a split collapse adds into them)
         bool skip_lwe = false;      // leave the LWE part to prep_lwe
+        uint32_t* status = nullptr; // a word
     };
-    ipx::PrepArgs prep_args(const uint64_t* d_in, size_t stride, size_t q0, int lane) const;
+    ipx::PrepArgs prep_args(const QueryInput& in, size_t stride, size_t q0, int lane) const;
     // Keys, RGSW rows and plan p's pass operands of the flat queries at d_in.
-    void prep_query(const uint64_t* d_in, size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s, int lane,
+    void prep_query(const QueryInput& in, size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s, int lane,
                     const PrepZero& z);
-    void prep_query(const uint64_t* d_in, size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s, int lane) {
-        prep_query(d_in, q0, nq, p, s, lane, PrepZero{});
+    void prep_query(const QueryInput& in, size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s, int lane) {
+        prep_query(in, q0, nq, p, s, lane, PrepZero{});
     }
     // Plan p's pass operands alone, of LWE parts stride words apart.
-    void prep_lwe(const uint64_t* d_in, size_t stride, size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s,
+    void prep_lwe(const QueryInput& in, size_t stride, size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s,
                   int lane);
     // Where a full-width pass of plan p writes: its row slices' partials, or interm.
     uint32_t* pass_out(size_t q0, const ipx::DbPlan& p, size_t& qstride);
@@ -271,11 +299,8 @@ struct GpuServerCtx {
     void horner_range(size_t count, uint64_t* d_out, size_t g_lo, size_t g_hi, hipStream_t s, size_t slot0,
                       int lane, bool status_read, const ipx::FusedPack* fp = nullptr);
     // Throw (and clear) if a pair chain of a call on `lane` reported a fault
-    // through its status word; s is the stream the call ran on.
-    void check_status(hipStream_t s, int lane);
-    // Zero the lane's status word on s (before a call whose status is read,
-    // so an earlier asynchronous call's report is not taken for its own).
-    void clear_status(hipStream_t s, int lane);
+    // through its status word; the call's stream has been waited for.
+    void check_status(int lane);
     std::atomic<size_t> n_streamed{0};  // streamed sub-batches enqueued (a test counter)
     // row slices whose partials the last answer's first sub-batch left in
     // d_part instead of a sum in d_interm (a streamed pass; 0: summed)
@@ -301,21 +326,24 @@ struct GpuServerCtx {
     // set `lane` (work that may overlap on the device uses distinct lanes).
     // status_read: the caller reads the lane's status word after the call
     // (check_status), so the pair Horner kernel may be used.
-    void enqueue(const uint64_t* d_in, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0 = 0,
+    void enqueue(const QueryInput& in, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0 = 0,
                  int lane = 0, bool status_read = false);
     // The same wholly on s and the lane's two side streams.
-    void enqueue_on(const uint64_t* d_in, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0, int lane,
+    void enqueue_on(const QueryInput& in, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0, int lane,
                     bool status_read);
     // The pipeline shape of a sub-batch of nq queries where nothing stands
     // against it (capture, stream slots).
     int shape_for(size_t nq) const;
-    // Host-staged round trip through the pinned staging of slots
-    // [slot0, slot0+count): h_q -> device -> h_resp, then copy to out.
-    void answer_host(size_t count, uint64_t* out, hipStream_t s = nullptr, size_t slot0 = 0);
+    // Host-staged answer: fill(i, words) writes query i's qlen u32 words
+    // (called from several threads); the flat responses go to out.
+    void answer_host(size_t count, const std::function<void(size_t, uint32_t*)>& fill, uint64_t* out);
     // enqueue() behind the device wire codecs: count packed queries at d_in
     // (device, qpack_bytes each) -> count*T compressed cts at d_out (device).
+    // (stage: a host job still writing them)
     void enqueue_packed(const uint8_t* d_in, size_t count, uint8_t* d_out, hipStream_t s, size_t slot0 = 0,
-                        int lane = 0, bool status_read = false);
+                        int lane = 0, bool status_read = false, HostStage* stage = nullptr);
+    // count responses of `bytes` bytes from the pinned staging to out.
+    void copy_out(size_t count, size_t bytes, void* out);
     // Host round trip of the packed forms through the pinned staging.
     void answer_packed_host(const uint8_t* in, size_t count, uint8_t* out);
 };
@@ -340,3 +368,5 @@ struct ipir_server {
     inspire::GpuServerCtx* ctx;
 };
 
+// One query's words (a C ABI view), narrowed to u32 as the server stages them.
+void flatten_view(const ipir_query_view& v, size_t R, uint32_t* w);

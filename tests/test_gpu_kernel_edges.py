@@ -116,3 +116,36 @@ def test_servers_on_one_device_stream_side_by_side():
             s.close()
         for st in streams:
             lib.ipir_dev_stream_destroy(st)
+
+
+def test_wire_words_beyond_32_bits_and_unaligned_packed_buffers(odd_table):
+    """Residues plus large multiples of their prime, over 2^32, through the
+    narrowing host entry and the 64-bit device entry; packed queries and
+    compressed responses at odd device addresses."""
+    geo, pc, srv, qs, want = odd_table
+    lib, R, nq = srv.lib, geo["R"], 5
+    base = srv.answer_batch(qs[:nq])
+    wide = np.stack([q.copy() for q in qs[:nq]])
+    rng = np.random.default_rng(12)
+    limb = np.concatenate([np.zeros(R, int), np.ones(R, int), np.tile(np.repeat([0, 1], N), 12)])
+    k = rng.integers(0, 1 << 36, wide.shape, dtype=np.uint64)
+    k[:, ::3] = 0  # some words stay canonical
+    wide += k * Q[limb][None, :]
+    assert wide.max() > 1 << 60
+    assert np.array_equal(srv.answer_batch(list(wide)), base)
+    dq, dout = ia.DeviceBuffer(wide.nbytes, lib), ia.DeviceBuffer(base.nbytes, lib)
+    dq.upload(wide)
+    assert lib.ipir_answer_batch_device(srv.h, C.c_void_p(dq.p), nq, C.c_void_p(dout.p), None) == 0
+    assert lib.ipir_dev_sync() == 0
+    assert np.array_equal(dout.download(np.zeros_like(base)), base)
+    cl = ia.Client(srv.params, lib)
+    packed = np.stack([cl.pack_query(q) for q in qs[:nq]])
+    comp = srv.answer_packed(packed)
+    assert np.array_equal(comp, np.stack([cl.compress(r) for r in base]))
+    for off in (1, 8, 16):
+        src = np.concatenate([np.zeros(off, np.uint8), packed.reshape(-1)])
+        dp, dc = ia.DeviceBuffer(src.nbytes, lib), ia.DeviceBuffer(comp.nbytes + off, lib)
+        dp.upload(src)
+        assert lib.ipir_answer_batch_packed_device(srv.h, C.c_void_p(dp.p + off), nq, C.c_void_p(dc.p + off), None) == 0
+        assert lib.ipir_dev_sync() == 0
+        assert np.array_equal(dc.download(np.zeros(comp.nbytes + off, np.uint8))[off:], comp.reshape(-1)), off
