@@ -167,10 +167,8 @@ int ipir_dbg_get_collapse_variant(const ipir_server* srv);
  * pass's launch, each group's collapse and pass work items together (up to
  * 8 queries; 6 for more). The setup autotuner picks 2, 3, 6 or 8 (4, 5
  * and 7 are tested alternatives that never won at 16 GB).
- * Answers under stream capture, and answers that find the device's four
- * slots for streamed answers in flight taken (by other servers' or lanes'
- * unfinished ones), take the chunked shape the autotuner picked instead of a
- * streamed one. 1 for other values. */
+ * Answers under stream capture take the chunked shape the autotuner picked
+ * instead of a streamed one. 1 for other values. */
 int ipir_dbg_set_pipeline(ipir_server* srv, int single, int batched);
 /* Row slices (a power of two <= 16) of the streamed pass of one-query
  * (nq_class 1) or many-query (other values) answers; raised to what the

@@ -776,7 +776,6 @@ int ipir_dbg_take_streaming(ipir_server* srv) {
     if (!srv) return 1;
     std::lock_guard<std::mutex> lk(srv->ctx->mu);
     if (srv->ctx->loop_active) return 5;
-    if (srv->ctx->device < 0 || (size_t)srv->ctx->device >= GpuServerCtx::kMaxDevices) return 1;
     srv->ctx->stream_ok = true;
     srv->ctx->drop_graphs();
     return 0;

@@ -45,7 +45,7 @@ struct Req {
 struct Partition {
     size_t slot0 = 0, nslots = 0;
     int lane = 0;  // scratch lane (and status word) of the context this partition uses
-    hipStream_t stream = nullptr;  // the lane's own (mstream)
+    hipStream_t stream = nullptr;  // the lane's passes
     // device timestamps of the batch in flight (its first and last command),
     // and [start, end) in ms after the loop's reference event of the last
     // completed batch
@@ -218,7 +218,7 @@ ipir_loop* ipir_loop_start(ipir_server* srv, size_t max_inflight) {
         p->slot0 = i * per;
         p->lane = (int)i;
         p->nslots = per;
-        p->stream = ctx->mstream[i];
+        p->stream = ctx->lanes[i].pass;
         if (hipEventCreate(&p->ev0) != hipSuccess || hipEventCreate(&p->ev1) != hipSuccess) {
             if (p->ev0) (void)hipEventDestroy(p->ev0);
             delete p;

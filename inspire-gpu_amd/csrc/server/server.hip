@@ -257,17 +257,6 @@ GpuServerCtx* gpu_setup_server(const PublicParams& pp, const PreprocessData& pre
 }
 
 namespace {
-// Streamed answers in flight, per device: at most kLanes of them, whatever
-// servers and lanes they belong to (StreamSlot). A slot's owner keeps it until
-// another lane finds its last streamed answer finished.
-struct StreamSlot {
-    GpuServerCtx* owner = nullptr;
-    int lane = 0;
-    bool enqueuing = false;  // the owner is between taking it and recording its event
-};
-std::mutex g_stream_mu;
-StreamSlot g_stream_slots[GpuServerCtx::kMaxDevices][GpuServerCtx::kLanes];
-
 // Row slices of a streamed pass over C columns: up to 16, with partials of
 // at most 32 MiB per query.
 constexpr uint32_t kStreamSlicesMax = 16;
@@ -412,20 +401,12 @@ void GpuServerCtx::alloc_slots() {
         d_KS[l] = dalloc<uint32_t>(kKeySumWords);
     }
     d_hstate = dalloc<uint32_t>(B * T * 4 * N);
-    mstream[0] = stream;
+    trace_name_stream(stream, "server");
+    static_assert(kLanes == kLaneSets, "a lane set per scratch lane");
+    lane_first = acquire_lanes(device, lanes);
     for (int l = 0; l < kLanes; l++) {
-        // a lane's three streams in a row: three hardware queues
-        if (l > 0) HIPX(hipStreamCreate(&mstream[l]));
-        HIPX(hipStreamCreate(&hstream[l]));
-        HIPX(hipStreamCreate(&cstream[l]));
         HIPX(hipEventCreateWithFlags(&hop_in_ev[l], hipEventDisableTiming));
         HIPX(hipEventCreateWithFlags(&hop_out_ev[l], hipEventDisableTiming));
-        static const char* mn[kLanes] = {"server", "passes lane 1", "passes lane 2", "passes lane 3"};
-        trace_name_stream(mstream[l], mn[l]);
-        static const char* hn[kLanes] = {"horner lane 0", "horner lane 1", "horner lane 2", "horner lane 3"};
-        static const char* cn[kLanes] = {"collapse lane 0", "collapse lane 1", "collapse lane 2", "collapse lane 3"};
-        trace_name_stream(hstream[l], hn[l]);
-        trace_name_stream(cstream[l], cn[l]);
         for (auto& e : chunk_ev[l]) HIPX(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         for (auto& e : coll_ev[l]) HIPX(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         HIPX(hipEventCreateWithFlags(&prep_ev[l], hipEventDisableTiming));
@@ -440,7 +421,7 @@ void GpuServerCtx::alloc_slots() {
     }
     // INSPIRE_STREAM=0: no streamed shapes
     const char* se = std::getenv("INSPIRE_STREAM");
-    stream_ok = !(se && se[0] == '0') && (size_t)device < kMaxDevices;
+    stream_ok = !(se && se[0] == '0');
     d_hxbuf = dalloc<uint32_t>(horner_pair_xbuf_words(B * T));
     d_hflags = dalloc<uint32_t>(2 * B * T);
     HIPX(hipHostMalloc((void**)&h_status, kLanes * 4, hipHostMallocDefault));
@@ -682,8 +663,7 @@ void GpuServerCtx::autotune_dbpass() {
     if (chunked_ok || can_stream(stream)) {
         const size_t ccols = gchunk * N;
         // as a caller's stream sees them, the hop of pipelined answers included
-        const hipStream_t caller = mstream[1];
-        HIPX(hipStreamSynchronize(stream));
+        const hipStream_t caller = stream;
         for (const size_t count : {(size_t)1, nq}) {
             const DbPlan full = plan_for(count, C);
             const size_t blocks = ccols / dbplan_cols(full);
@@ -918,42 +898,6 @@ DbPlan GpuServerCtx::stream_plan(size_t nq, uint32_t slices, bool fused) const {
     return p;
 }
 
-bool GpuServerCtx::take_stream_slot(int lane) {
-    std::lock_guard<std::mutex> lk(g_stream_mu);
-    StreamSlot* free_slot = nullptr;
-    // the queries are legal beside another thread's stream capture
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
-    for (StreamSlot& x : g_stream_slots[device]) {
-        if (x.owner == this && x.lane == lane) {
-            x.enqueuing = true;
-            (void)hipThreadExchangeStreamCaptureMode(&mode);
-            return true;
-        }
-        if (!free_slot && !x.enqueuing &&
-            (!x.owner || hipEventQuery(x.owner->horner_done[x.lane]) == hipSuccess))
-            free_slot = &x;
-    }
-    (void)hipGetLastError();  // a query that found work pending is no error
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
-    if (!free_slot) return false;
-    *free_slot = StreamSlot{this, lane, true};
-    return true;
-}
-
-void GpuServerCtx::settle_stream_slot(int lane) {
-    std::lock_guard<std::mutex> lk(g_stream_mu);
-    for (StreamSlot& x : g_stream_slots[device])
-        if (x.owner == this && x.lane == lane) x.enqueuing = false;
-}
-
-void GpuServerCtx::drop_stream_slots() {
-    std::lock_guard<std::mutex> lk(g_stream_mu);
-    if ((size_t)device >= kMaxDevices) return;
-    for (StreamSlot& x : g_stream_slots[device])
-        if (x.owner == this) x = StreamSlot{};
-}
-
 void GpuServerCtx::mark_pass(hipStream_t s, bool first) {
     if (!time_pass) return;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -1090,28 +1034,44 @@ void GpuServerCtx::enqueue(const QueryInput& in, size_t count, uint64_t* d_out, 
                            int lane, bool status_read) {
     if (lane < 0 || lane >= kLanes) throw std::invalid_argument("enqueue: scratch lane out of range");
     TraceRange tr("answer: %zu queries, slots %zu.., lane %d", count, slot0, lane);
-    // pipelined answers run on the lane's own three streams (mstream);
-    // under capture on s itself, whose replay has no queues to share
-    const size_t last = count % kMfmaMaxQueries;
-    const bool pipelined = (count >= kMfmaMaxQueries && shape_for(kMfmaMaxQueries)) || (last && shape_for(last));
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (pipelined && s != mstream[lane]) HIPX(hipStreamIsCapturing(s, &cap));
-    if (!pipelined || s == mstream[lane] || cap != hipStreamCaptureStatusNone) {
+    // pipelined answers run on the lane's set of streams; under capture on s
+    // itself, whose replay has no queues to share
+    const hipStream_t ms = lanes[lane].pass;
+    if (!pipelined(count) || s == ms || is_capturing(s)) {
         enqueue_on(in, count, d_out, s, slot0, lane, status_read);
         return;
     }
     HIPX(hipEventRecord(hop_in_ev[lane], s));
-    HIPX(hipStreamWaitEvent(mstream[lane], hop_in_ev[lane], 0));
-    enqueue_on(in, count, d_out, mstream[lane], slot0, lane, status_read);
-    HIPX(hipEventRecord(hop_out_ev[lane], mstream[lane]));
+    HIPX(hipStreamWaitEvent(ms, hop_in_ev[lane], 0));
+    enqueue_on(in, count, d_out, ms, slot0, lane, status_read);
+    HIPX(hipEventRecord(hop_out_ev[lane], ms));
     HIPX(hipStreamWaitEvent(s, hop_out_ev[lane], 0));
+}
+
+bool GpuServerCtx::is_capturing(hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (s) HIPX(hipStreamIsCapturing(s, &cap));
+    return cap != hipStreamCaptureStatusNone;
+}
+
+bool GpuServerCtx::pipelined(size_t count) const {
+    const size_t last = count % kMfmaMaxQueries;
+    return (count >= kMfmaMaxQueries && shape_for(kMfmaMaxQueries)) || (last && shape_for(last));
 }
 
 void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0,
                               int lane, bool status_read) {
     const size_t C = pp.db_cols;
     const size_t nchunks = G / gchunk;
-    const hipStream_t hs = hstream[lane];
+    // Side streams: the lane's, or under capture the server's own pair (a
+    // shared stream must not join one server's capture while others use it).
+    hipStream_t hs = lanes[lane].horner, ps_side = lanes[lane].side;
+    if (is_capturing(s)) {
+        if (!capture_horner) HIPX(hipStreamCreate(&capture_horner));
+        if (!capture_side) HIPX(hipStreamCreate(&capture_side));
+        hs = capture_horner;
+        ps_side = capture_side;
+    }
     // Pipelined over group chunks, highest first (the order every Horner
     // chain consumes groups). The database pass (on s) and the collapse (on
     // s, or on the lane's collapse stream) need nothing from each other; the
@@ -1120,17 +1080,6 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
     // and through their waits for every collapse.
     bool joined = false;
     const bool streamable = can_stream(s);
-    // the device's slot for this lane's streamed sub-batches, taken with the
-    // first of them and given up for taking over once this answer's event is
-    // recorded
-    struct SlotHold {
-        GpuServerCtx* c;
-        int lane;
-        bool held = false;
-        ~SlotHold() {
-            if (held) c->settle_stream_slot(lane);
-        }
-    } slot_hold{this, lane};
     last_part_slices = 0;  // the first sub-batch's result lands in interm unless it streams with slices
     // Serial sub-batches (shape 0) leave their Horner chains to one launch
     // after the last of them: a sub-batch's nq x T chains each hold a CU for
@@ -1160,9 +1109,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             // sub-batch whose waiting workgroups exceed kStreamMaxWaiters
             // CUs would leave too few to the passes of 4 lanes: the chunked
             // shape then
-            if (streamable && sp.kind == DbPlan::MFMA && horner_mode != 1 && stream_fits(nq) && !slot_hold.held)
-                slot_hold.held = take_stream_slot(lane);
-            if (!slot_hold.held || sp.kind != DbPlan::MFMA || !stream_fits(nq))
+            if (!streamable || sp.kind != DbPlan::MFMA || horner_mode == 1 || !stream_fits(nq))
                 shape = nchunks == 1 ? 0 : nq == 1 ? pipe_single_chunked : pipe_batched_chunked;
         }
         if (shape != 0) flush_deferred();
@@ -1180,7 +1127,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             n_streamed.fetch_add(1, std::memory_order_relaxed);
             if (q0 == slot0) last_part_slices = sp.slices;
             const bool fused = shape == 8;
-            const hipStream_t ps_s = cstream[lane], cs = shape == 7 ? ps_s : s;
+            const hipStream_t ps_s = ps_side, cs = shape == 7 ? ps_s : s;
             joined = true;
             uint32_t* pass_done = d_sflags[lane] + ((q0 - slot0) / kMfmaMaxQueries) * kStreamSetWords * G;
             uint32_t* packed_done = pass_done + G;
@@ -1300,7 +1247,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
         // the first collapse chunk: the collapse stream then stays a chunk
         // ahead, so each chunk's pack and Horner steps wait for its database
         // pass only, and the last ones follow the last pass at once
-        const hipStream_t cs = shape == 3 || shape == 5 ? cstream[lane] : s;
+        const hipStream_t cs = shape == 3 || shape == 5 ? ps_side : s;
         const bool first = shape == 4, ahead = shape == 5;
         joined = true;
         const DbPlan p = chunk_plan(nq, gchunk * N);  // every chunk's plan has this one's kernel and digits
@@ -1457,7 +1404,7 @@ void GpuServerCtx::copy_out(size_t count, size_t bytes, void* out) {
 }
 
 void GpuServerCtx::answer_packed_host(const uint8_t* in, size_t count, uint8_t* out) {
-    hipStream_t s = stream;
+    hipStream_t s = pipelined(count) && !graph_mode ? lanes[0].pass : stream;
     uint8_t* hq = reinterpret_cast<uint8_t*>(h_q);
     uint8_t* hr = reinterpret_cast<uint8_t*>(h_resp);
     TraceRange tr("host-staged packed answer: %zu queries", count);
@@ -1500,7 +1447,7 @@ void GpuServerCtx::order_after(hipStream_t s) {
 }
 
 void GpuServerCtx::answer_host(size_t count, const std::function<void(size_t, uint32_t*)>& fill, uint64_t* out) {
-    hipStream_t s = stream;
+    hipStream_t s = pipelined(count) && !graph_mode ? lanes[0].pass : stream;
     TraceRange tr("host-staged answer: %zu queries", count);
     {
         // The queries are narrowed into pinned memory that the preparation
@@ -1602,9 +1549,8 @@ void gpu_free_server(GpuServerCtx* ctx) {
     for (auto& f : ctx->d_sflags) dfree(f);
     dfree(ctx->d_cmp);
     for (int l = 0; l < GpuServerCtx::kLanes; l++) {
-        if (ctx->hstream[l]) (void)hipStreamSynchronize(ctx->hstream[l]);
-        if (l == 0) ctx->drop_stream_slots();  // before their events go
-        if (ctx->cstream[l]) (void)hipStreamSynchronize(ctx->cstream[l]);
+        for (hipStream_t x : {ctx->lanes[l].pass, ctx->lanes[l].horner, ctx->lanes[l].side})
+            if (x) (void)hipStreamSynchronize(x);
         for (auto& e : ctx->chunk_ev[l])
             if (e) (void)hipEventDestroy(e);
         for (auto& e : ctx->coll_ev[l])
@@ -1614,13 +1560,13 @@ void gpu_free_server(GpuServerCtx* ctx) {
         if (ctx->hop_out_ev[l]) (void)hipEventDestroy(ctx->hop_out_ev[l]);
         if (ctx->pass_ev[l]) (void)hipEventDestroy(ctx->pass_ev[l]);
         if (ctx->horner_done[l]) (void)hipEventDestroy(ctx->horner_done[l]);
-        if (l > 0 && ctx->mstream[l]) {
-            (void)hipStreamSynchronize(ctx->mstream[l]);
-            (void)hipStreamDestroy(ctx->mstream[l]);
-        }
-        if (ctx->hstream[l]) (void)hipStreamDestroy(ctx->hstream[l]);
-        if (ctx->cstream[l]) (void)hipStreamDestroy(ctx->cstream[l]);
     }
+    if (ctx->lane_first >= 0) release_lanes(ctx->device, ctx->lane_first);
+    for (hipStream_t x : {ctx->capture_horner, ctx->capture_side})
+        if (x) {
+            (void)hipStreamSynchronize(x);
+            (void)hipStreamDestroy(x);
+        }
     for (hipEvent_t e : ctx->pass_marks) (void)hipEventDestroy(e);
     for (int l = 0; l < GpuServerCtx::kLanes; l++) {
         dfree(ctx->d_dig[l]); dfree(ctx->d_S[l]); dfree(ctx->d_kdig[l]); dfree(ctx->d_KS[l]);

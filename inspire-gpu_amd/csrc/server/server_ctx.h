@@ -12,6 +12,7 @@
 #include "gpu_protocol.h"
 #include "host_stage.h"
 #include "kernels.h"
+#include "lanes.h"
 
 namespace inspire {
 
@@ -104,17 +105,15 @@ struct GpuServerCtx {
     int pipe_single_chunked = 3, pipe_batched_chunked = 3;  // where a streamed shape cannot run
     bool pipe_forced = false;       // INSPIRE_PIPELINE set the shapes (not autotuned)
     // row slices of the streamed pass (one query, many), and whether this
-    // server may stream at all. The workgroups of a streamed answer hold
-    // their CUs while they wait, so a device has kLanes slots for streamed
-    // answers in flight, shared by its servers' lanes: a lane takes a free
-    // one, or one whose owner's last streamed answer has finished; with none
-    // the answer takes its chunked shape.
+    // server may stream at all (INSPIRE_STREAM). The workgroups of a streamed
+    // answer hold their CUs while they wait; the device's lane sets are
+    // shared by its servers and run one answer's chains at a time each, so
+    // at most kLanes answers wait, whatever servers they belong to.
     uint32_t stream_slices1 = 4, stream_slices = 4;
     // eighths of the groups (from the top) in a streamed pass's first
     // launch, the chains starting after it (0: one launch, chains at once)
     uint32_t stream_split1 = 0, stream_split = 0;
     bool stream_ok = false;
-    static constexpr size_t kMaxDevices = 64;  // devices with slots
     // The streamed pass's plan for nq queries (the tuned kernel, the streamed
     // slice count, at least the slices exactness needs); kind F64 if none fits.
     // One- and two-query passes stream with 128-column tiles per wave (fewer,
@@ -133,11 +132,6 @@ struct GpuServerCtx {
     // of small batches), kPackQueries above (two rounds, fewer CUs held
     // beside the slower 17..32-query pass).
     static uint32_t pack_width(size_t nq) { return nq <= 16 ? 2u : ipx::kPackQueries; }
-    // The device's slot for this server's lane, taken before a streamed
-    // answer is enqueued (false: none is free now).
-    bool take_stream_slot(int lane);
-    void settle_stream_slot(int lane);  // the answer's horner_done event is recorded
-    void drop_stream_slots();
     size_t qlen = 0, resp_u64s = 0;
     size_t part_stride = 0, part2_stride = 0, keys_stride = 0, rgsw_stride = 0, packed_stride = 0;
     uint64_t* d_q = nullptr;        // flat queries (device staging)
@@ -166,19 +160,15 @@ struct GpuServerCtx {
     static_assert(16 / 2 <= ipx::kMfmaMaxQueries / ipx::kPackQueries, "pack workgroups of a 16-query sub-batch");
     uint32_t* d_sflags[kLanes] = {};
     size_t stream_sets = 0;
-    // per lane: the streams the collapse and the Horner chains run on beside
-    // the database pass, and the events that hand each group chunk over
+    // Per lane, the streams of pipelined answers: the database passes, and
+    // beside them the Horner chains and the collapse or pack (lanes.h), with
+    // the events that hand each group chunk over. A caller's stream may share
+    // a hardware queue with either side stream, so pipelined answers hop from
+    // it to the passes' stream and back.
     static constexpr int kChunkEvents = 16;
-    hipStream_t hstream[kLanes] = {};
-    hipStream_t cstream[kLanes] = {};
-    // The stream a lane's database passes run on beside them (lane 0: the
-    // server's own). The three must sit on three of the process's 4 hardware
-    // queues or the chains wait for the pass to end; streams created one
-    // after another do. A caller's stream may share a queue with either, so
-    // pipelined answers hop from it to this one and back (two events): at
-    // 16 GB, 32 queries, answers on 8 streams of a caller took 5.45-5.55 ms on
-    // half of them and 7.0-8.1 ms on the others.
-    hipStream_t mstream[kLanes] = {};
+    LaneStreams lanes[kLanes];
+    int lane_first = -1;  // acquire_lanes' answer
+    hipStream_t capture_horner = nullptr, capture_side = nullptr;  // the side streams of captured answers
     hipEvent_t hop_in_ev[kLanes] = {}, hop_out_ev[kLanes] = {};
     hipEvent_t chunk_ev[kLanes][kChunkEvents] = {};  // database pass of a chunk done
     hipEvent_t coll_ev[kLanes][kChunkEvents] = {};   // collapse of a chunk done
@@ -332,8 +322,10 @@ struct GpuServerCtx {
     void enqueue_on(const QueryInput& in, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0, int lane,
                     bool status_read);
     // The pipeline shape of a sub-batch of nq queries where nothing stands
-    // against it (capture, stream slots).
+    // against it (capture), and whether an answer has a pipelined sub-batch.
     int shape_for(size_t nq) const;
+    bool pipelined(size_t count) const;
+    static bool is_capturing(hipStream_t s);
     // Host-staged answer: fill(i, words) writes query i's qlen u32 words
     // (called from several threads); the flat responses go to out.
     void answer_host(size_t count, const std::function<void(size_t, uint32_t*)>& fill, uint64_t* out);
