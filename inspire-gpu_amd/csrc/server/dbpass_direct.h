@@ -19,10 +19,19 @@ __device__ __forceinline__ uint32_t offset_sum(const uint32_t* __restrict__ S, u
     return (uint32_t)(a[0] + a[1] + a[2] + a[3] + b[0] + b[1] + b[2] + b[3]);
 }
 
+// A pass's output word: agent scope where a streamed pass hands it over.
+__device__ __forceinline__ void pass_store(uint32_t* p, uint32_t v, bool streamed) {
+    if (streamed)
+        agent_store(p, v);
+    else
+        *p = v;
+}
+
 // Recombine one lane's accumulators of pair pr and store the canonical residue.
 __device__ __forceinline__ void store_pair(const i32x4& al, const i32x4& ah, uint32_t pr, uint32_t nq, bool corr,
                                            const uint32_t* __restrict__ S, uint32_t* __restrict__ out,
-                                           size_t out_qstride, uint32_t slice, uint32_t OC, uint32_t col) {
+                                           size_t out_qstride, uint32_t slice, uint32_t OC, uint32_t col,
+                                           bool streamed) {
     const uint32_t q = pr >> 1;
     const int c = (int)(pr & 1);
     if (q >= nq) return;
@@ -33,8 +42,8 @@ __device__ __forceinline__ void store_pair(const i32x4& al, const i32x4& ah, uin
     // of q_c above that to make it non-negative
     const uint64_t qc = c ? Q1 : Q0;
     const uint64_t off = qc * ((1ull << 59) / qc);
-    out[(size_t)q * out_qstride + (size_t)slice * 2 * OC + (size_t)c * OC + col] =
-        red64((uint64_t)(s + (int64_t)off), c);
+    pass_store(out + (size_t)q * out_qstride + (size_t)slice * 2 * OC + (size_t)c * OC + col,
+               red64((uint64_t)(s + (int64_t)off), c), streamed);
 }
 
 // Up to 2*MT queries (Mp = 16*MT digit rows) over column tile xt (4 waves x
@@ -47,7 +56,7 @@ template <int MT, int NT>
 __device__ __forceinline__ void dbpass_direct_body(const uint8_t* __restrict__ db, const int8_t* __restrict__ dig,
                                                    const uint32_t* __restrict__ S, uint32_t* __restrict__ out,
                                                    size_t out_qstride, uint32_t C, uint32_t OC, uint32_t nq,
-                                                   uint32_t kbps, uint32_t xt, uint32_t slice) {
+                                                   uint32_t kbps, uint32_t xt, uint32_t slice, bool streamed) {
     constexpr uint32_t Mp = 16 * MT;
     const uint32_t w = threadIdx.x >> 6, l = threadIdx.x & 63;
     const uint32_t col0 = (xt * 4 + w) * NT * 16;
@@ -98,7 +107,7 @@ __device__ __forceinline__ void dbpass_direct_body(const uint8_t* __restrict__ d
 #pragma unroll
         for (int n = 0; n < NT; n++)
             store_pair(acc[a][n][0], acc[a][n][1], (uint32_t)a * 4 + (l >> 4), nq, slice == 0, S, out, out_qstride,
-                       slice, OC, col0 + n * 16 + (l & 15));
+                       slice, OC, col0 + n * 16 + (l & 15), streamed);
 }
 
 }  // namespace

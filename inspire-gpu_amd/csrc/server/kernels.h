@@ -131,7 +131,7 @@ hipError_t launch_dbpass_f64(const uint8_t* db, const double* bq, uint32_t* out,
 // forms only) hands its groups over while it runs: its 1-D grid takes the
 // column tiles from the highest down (the order the Horner chains consume
 // groups), each tile's row slices in a row; every workgroup, once its
-// stores are complete at agent scope (one release per workgroup), adds 1 to
+// stores (agent scope) are complete, adds 1 to
 // ps.group_done[column / N]. A group's columns are in place (out: one
 // slice's final values, or [q][slice][limb][OC] partials) when its word
 // reaches (N / dbplan_cols(p)) * p.slices. group_done must be zero before
@@ -248,8 +248,8 @@ struct StreamWait {
 // for each it waits until pass_done[g] reaches pass_target, then packs the
 // group's b-parts of its queries (the pass's row-slice partials summed, NTT,
 // minus the collapse sums and Df x Kn: launch_pack_finalize's output) into
-// packed_b and publishes them: packed_done[block * G + g] = 1 after an
-// agent-scope release. packed_done must be zero before the launch. A wait
+// packed_b (agent scope) and publishes them: packed_done[block * G + g] = 1 once
+// they are complete. packed_done must be zero before the launch. A wait
 // longer than spin_limit sleeps sets *status to 1 and ends the workgroup
 // (its chains then give up their own waits).
 constexpr uint32_t kPackQueries = 4;

@@ -150,7 +150,8 @@ __device__ __forceinline__ KSlice kslice(uint32_t sl, uint32_t ksplit) {
 __device__ __forceinline__ KSlice slice_of(uint32_t ksplit) { return kslice(blockIdx.z % ksplit, ksplit); }
 __device__ __forceinline__ void collapse_store(const i32x4 (&acc)[4], uint32_t q, int c, uint32_t g, uint32_t i,
                                                const uint32_t* __restrict__ KS, uint32_t* __restrict__ part2,
-                                               size_t p2_stride, const KSlice& ks = KSlice{}) {
+                                               size_t p2_stride, const KSlice& ks = KSlice{},
+                                               bool streamed = false) {
     const uint64_t qc = c ? Q1 : Q0;
     int64_t lv[7] = {0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
@@ -172,7 +173,7 @@ __device__ __forceinline__ void collapse_store(const i32x4 (&acc)[4], uint32_t q
     if (ks.add)
         atomicAdd(dst, r);
     else
-        *dst = r;
+        pass_store(dst, r, streamed);
 }
 
 // Block (4*NT*16-slot tile of i, limb, group): 4 waves of NT 16-slot tiles,
@@ -188,7 +189,8 @@ __device__ __forceinline__ void collapse_mfma_body(const uint32_t* __restrict__ 
                                                    const int8_t* __restrict__ kdig,
                                                    const uint32_t* __restrict__ KS,
                                                    uint32_t* __restrict__ part2, size_t p2_stride, uint32_t nq,
-                                                   uint32_t it, int c, uint32_t g, const KSlice& ksl = KSlice{}) {
+                                                   uint32_t it, int c, uint32_t g, const KSlice& ksl = KSlice{},
+                                                   bool streamed = false) {
     constexpr uint32_t Mp = 16 * MT;
     constexpr uint32_t NKB = DD_K / 16;
     constexpr uint32_t AU = SHARED ? Mp * 4 / 256 : 1;  // 16-byte units of a step's digit tile per thread
@@ -280,7 +282,8 @@ __device__ __forceinline__ void collapse_mfma_body(const uint32_t* __restrict__ 
         if (q >= nq) continue;
 #pragma unroll
         for (int n = 0; n < NT; n++)
-            collapse_store(acc[a][n], q, c, g, col0 + n * 16 + (l & 15), KS, part2, p2_stride, ksl);
+            collapse_store(acc[a][n], q, c, g, col0 + n * 16 + (l & 15), KS, part2, p2_stride, ksl,
+                           streamed);
     }
 }
 
@@ -300,7 +303,7 @@ __global__ __launch_bounds__(256, 2) void k_collapse_mfma(const uint32_t* __rest
 // PNT-wide column tiles), all 256-lane workgroups of the same footprint, so
 // the two HBM streams of a group run together and groups complete in the
 // order the Horner chains consume them. Every work item, once its stores
-// are complete (one agent-scope release per workgroup), adds 1 to its
+// (agent scope) are complete, adds 1 to its
 // group's counter; a group is in place at 2 N/(64 CNT) + (N/(64 PNT)) x
 // slices.
 // Without counters (group_done null) it is the serial answer's pass and
@@ -321,19 +324,16 @@ __global__ __launch_bounds__(256, 2) void k_pass_collapse_stream(
     if (r < CB) {
         const uint32_t sl = r / (2 * CIT), it = r % (2 * CIT);
         collapse_mfma_body<CMT, CNT, false>(precomp, kdig, KS, part2, p2_stride, nq, it % CIT, (int)(it / CIT), g,
-                                            kslice(sl, ksplit));
+                                            kslice(sl, ksplit), group_done != nullptr);
     } else {
         const uint32_t pr = r - CB;
         dbpass_direct_body<PMT, PNT>(db, dig, S, out, out_qstride, C, C, nq, kbps, g * TPG + (pr >> slice_shift),
-                                     pr & ((1u << slice_shift) - 1));
+                                     pr & ((1u << slice_shift) - 1), group_done != nullptr);
     }
     if (!group_done) return;
     __builtin_amdgcn_s_waitcnt(0);  // this wave's stores are complete
     __syncthreads();
-    if (threadIdx.x == 0) {
-        fence_release_agent_done();
-        __hip_atomic_fetch_add(group_done + g, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (threadIdx.x == 0) __hip_atomic_fetch_add(group_done + g, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // 17..32 queries (8 key-digit tiles) in the load pattern of the batched

@@ -188,18 +188,14 @@ __device__ __forceinline__ void pass_coords(const PassStream& ps, uint32_t& xt, 
     }
 }
 
-// Streamed pass, after the workgroup's stores of column tile xt: count the
-// workgroup into its group. One agent-scope release per workgroup (it
-// writes back the L2): every wave first waits for its own stores, the
-// barrier orders them before lane 0's release.
+// Streamed pass, after the workgroup's stores of column tile xt (agent
+// scope): count the workgroup into its group once every wave's are complete.
 __device__ __forceinline__ void pass_handover(const PassStream& ps, uint32_t xt) {
     __builtin_amdgcn_s_waitcnt(0);  // this wave's stores are complete
     __syncthreads();
-    if (threadIdx.x == 0) {
-        fence_release_agent_done();
+    if (threadIdx.x == 0)
         __hip_atomic_fetch_add(ps.group_done + ps.group_base + xt / ps.tiles_per_group, 1u, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
-    }
 }
 
 // Up to 2*MT queries: dbpass_direct_body over the grid's (tile, slice).
@@ -212,7 +208,7 @@ __global__ __launch_bounds__(256, 2) void k_dbpass_mfma(const uint8_t* __restric
                                                         PassStream ps) {
     uint32_t xt, slice;
     pass_coords(ps, xt, slice);
-    dbpass_direct_body<MT, NT>(db, dig, S, out, out_qstride, C, OC, nq, kbps, xt, slice);
+    dbpass_direct_body<MT, NT>(db, dig, S, out, out_qstride, C, OC, nq, kbps, xt, slice, ps.group_done != nullptr);
     if (ps.group_done) pass_handover(ps, xt);
 }
 
@@ -410,8 +406,8 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void k_dbpass_mfma_sa(const uint8_
                     if (q < nq) {
                         const uint32_t r0 = pow_residue(pk, slice == 0 ? offset_sum(S, 2 * q) : 0, 0);
                         const uint32_t r1 = pow_residue(pk, slice == 0 ? offset_sum(S, 2 * q + 1) : 0, 1);
-                        o[0] = r0;
-                        o[OC] = r1;
+                        pass_store(o, r0, ps.group_done != nullptr);
+                        pass_store(o + OC, r1, ps.group_done != nullptr);
                     }
                 }
             }
@@ -439,7 +435,9 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void k_dbpass_mfma_sa(const uint8_
                 if (q < nq) {
                     uint32_t* o = out + (size_t)q * out_qstride + (size_t)slice * 2 * OC + col0 + cl;
 #pragma unroll
-                    for (int c = 0; c < 2; c++) o[(size_t)c * OC] = crt7_residue(t, slice == 0 ? offset_sum(S, 2 * q + c) : 0, c);
+                    for (int c = 0; c < 2; c++)
+                        pass_store(o + (size_t)c * OC, crt7_residue(t, slice == 0 ? offset_sum(S, 2 * q + c) : 0, c),
+                                   ps.group_done != nullptr);
                 }
             }
             __syncthreads();  // the second half reuses the region
@@ -450,7 +448,7 @@ __global__ __launch_bounds__(64 * WAVES, OCC) void k_dbpass_mfma_sa(const uint8_
 #pragma unroll
             for (int n = 0; n < NT; n++)
                 store_pair(acc[a][n][0], acc[a][n][1], (uint32_t)a * 4 + (l >> 4), nq, slice == 0, S, out,
-                           out_qstride, slice, OC, col0 + n * 16 + (l & 15));
+                           out_qstride, slice, OC, col0 + n * 16 + (l & 15), ps.group_done != nullptr);
     }
     if (ps.group_done) pass_handover(ps, xt);
 }
@@ -552,7 +550,7 @@ __global__ __launch_bounds__(256, 2) void k_dbpass_mfma_bs(const uint8_t* __rest
 #pragma unroll
         for (int n = 0; n < NT; n++)
             store_pair(acc[a][n][0], acc[a][n][1], (uint32_t)(MW * w + a) * 4 + (l >> 4), nq, slice == 0, S, out,
-                       out_qstride, slice, OC, bcol0 + n * 16 + (l & 15));
+                       out_qstride, slice, OC, bcol0 + n * 16 + (l & 15), false);
 }
 
 // Largest power-of-two slice count s with blocks*s <= target that keeps

@@ -278,9 +278,9 @@ __global__ __launch_bounds__(512, 2) void k_horner(HornerChain h, NttConst nc, N
     if (lo >= hi) return;
     const NrLimb m = nr_limb(c);
     // Beside a streamed pack: lane 0 waits until this chain's packed b-part
-    // of group g is published and acquires (the hand-over rules in
-    // dev_common.h); the caller's next barrier publishes sw_abort, set where
-    // the wait exceeded its bound.
+    // of group g is published (the hand-over rules in dev_common.h); the
+    // caller's next barrier publishes sw_abort, set where the wait exceeded
+    // its bound.
     const uint32_t* sw_done = sw.done + (size_t)(qi / sw.queries) * sw.stride;
     auto wait_packed = [&](uint32_t g) {
         if (tid == 0) {
@@ -294,7 +294,6 @@ __global__ __launch_bounds__(512, 2) void k_horner(HornerChain h, NttConst nc, N
                 }
                 __builtin_amdgcn_s_sleep(kSpinSleep);
             }
-            fence_acquire_agent_done();
             sw_abort = ab;
         }
     };
@@ -340,6 +339,19 @@ __global__ __launch_bounds__(512, 2) void k_horner(HornerChain h, NttConst nc, N
             x[k + 4] = u[k];
         }
     };
+    // the same of a b-part: handed over by a streamed pack, or ordinary
+    auto load8b = [&](uint32_t (&x)[8], const uint32_t* p) {
+        if constexpr (STREAMED) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const uint64_t v = agent_load2(p + (size_t)c * N + 8 * t + 2 * k);
+                x[2 * k] = (uint32_t)v;
+                x[2 * k + 1] = (uint32_t)(v >> 32);
+            }
+        } else {
+            load8(x, p);
+        }
+    };
     uint32_t acc[2][8];  // a and b part, slots 8t + k
     int first;
     if (top < h.g_hi) {  // the chain starts here: acc = packed[top]
@@ -352,7 +364,7 @@ __global__ __launch_bounds__(512, 2) void k_horner(HornerChain h, NttConst nc, N
             }
         }
         load8(acc[0], h.pa_base + (size_t)top * h.pa_stride);
-        load8(acc[1], pb + (size_t)top * 2 * N);
+        load8b(acc[1], pb + (size_t)top * 2 * N);
         first = (int)top - 1;
     } else {
         load8(acc[0], hs);
@@ -425,7 +437,7 @@ __global__ __launch_bounds__(512, 2) void k_horner(HornerChain h, NttConst nc, N
             nr_forward<4>(x, buf[c], tw, t, m, [&]() {
                 if constexpr (STREAMED) {
                     wait_packed((uint32_t)gs);
-                    __syncthreads();  // no wave's load of the b-part before the acquire
+                    __syncthreads();  // no wave's load of the b-part before the flag was seen
                 } else {
                     lds_barrier();
                 }
@@ -435,7 +447,7 @@ __global__ __launch_bounds__(512, 2) void k_horner(HornerChain h, NttConst nc, N
                     poison();
                     return;
                 }
-                load8(pbv, pb + (size_t)gs * 2 * N);
+                load8b(pbv, pb + (size_t)gs * 2 * N);
             }
 #pragma unroll
             for (int k = 0; k < 8; k++) {
@@ -481,41 +493,44 @@ __global__ __launch_bounds__(512, 2) void k_horner(HornerChain h, NttConst nc, N
 // Beside a streamed database pass (launch_pack_stream): workgroup b packs
 // queries [b*ps.queries, ...) group by group from the top; team k of
 // round r takes polynomial 4r + k = (query, limb), the limb of its own
-// twiddles. The subtrahend of round 0 (collapse sums + Df x Kn, in place
-// before the launch) is loaded while lane 0 waits for the group.
+// twiddles, and transforms it in registers (ntt_regs.h). Df x Kn of round 0
+// (in place before the launch) is computed while lane 0 waits for the group;
+// the partials and the collapse sums are read at agent scope, all of a
+// lane's in flight together.
 __global__ __launch_bounds__(1024) void k_pack_stream(PackStream ps, const uint32_t* __restrict__ part2,
                                                       size_t p2_stride, const uint32_t* __restrict__ precomp,
                                                       const uint32_t* __restrict__ keys, size_t kstride,
                                                       uint32_t* __restrict__ packed_b, size_t pstride, uint32_t G,
                                                       uint32_t nq, NttConst nc) {
-    __shared__ uint32_t buf[4][POLY_LDS];
-    __shared__ uint32_t twl[8 * N];
+    __shared__ __align__(16) uint32_t buf[4][1][POLY4_LDS];
+    __shared__ __align__(16) nr_u32x2 tw2[2][N];
     __shared__ uint32_t abort_flag;
-    const uint32_t tid = threadIdx.x, team = tid >> 8, t = tid & 255, blk = blockIdx.x;
+    const uint32_t tid = threadIdx.x, t = tid & 255, blk = blockIdx.x;
+    const uint32_t team = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 8));
     const uint32_t q0 = blk * ps.queries;
     const uint32_t nqb = nq - q0 < ps.queries ? nq - q0 : ps.queries;
     const uint32_t npoly = 2 * nqb, rounds = (npoly + 3) / 4;
     const int c = (int)(team & 1);
-    const uint32_t q = qof(c);
-    const Tw tw = tw_lds(twl, c);
+    const NrLimb m = nr_limb(c);
     const size_t sstride = 2 * (size_t)ps.C;  // one row slice of the pass's partials
-    stage_twiddles(twl, nc, tid, 1024);        // published by the first barrier below
+    nr_stage_twiddles(tw2, nc, tid, 1024);    // published by the first barrier below
     for (int g = (int)G - 1; g >= 0; g--) {
         for (uint32_t r = 0; r < rounds; r++) {  // every lane runs every round (barriers inside)
             const uint32_t k = 4 * r + team;
             const bool active = k < npoly;
             const uint32_t qi = q0 + (active ? k >> 1 : 0);
-            // Df x Kn (precomp and keys, in place before the launch) now;
-            // the collapse sums after the wait, since a pass may produce them
-            // with the group (the collapse in the pass's launch)
             uint32_t sub[8];
             if (active) {
-                const uint32_t* Df = precomp + (size_t)g * PC_GROUP + PC_DF + (size_t)c * D_EFF * N;
-                const uint32_t* Kn = keys + qi * kstride + BLK + (size_t)c * N;
+                const u32x4* Df = reinterpret_cast<const u32x4*>(precomp + (size_t)g * PC_GROUP + PC_DF +
+                                                                 (size_t)c * D_EFF * N + 8 * t);
+                const u32x4* Kn =
+                    reinterpret_cast<const u32x4*>(keys + (size_t)qi * kstride + BLK + (size_t)c * N + 8 * t);
 #pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const uint32_t x = t + 256 * e;
-                    sub[e] = red64((uint64_t)Df[x] * Kn[x] + (uint64_t)Df[N + x] * Kn[2 * N + x], c);
+                for (int h = 0; h < 2; h++) {
+                    const u32x4 d0 = Df[h], d1 = Df[N / 4 + h], k0 = Kn[h], k1 = Kn[2 * N / 4 + h];
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        sub[4 * h + e] = red64((uint64_t)d0[e] * k0[e] + (uint64_t)d1[e] * k1[e], c);
                 }
             }
             if (r == 0) {
@@ -530,44 +545,54 @@ __global__ __launch_bounds__(1024) void k_pack_stream(PackStream ps, const uint3
                         }
                         __builtin_amdgcn_s_sleep(kSpinSleep);
                     }
-                    fence_acquire_agent_done();  // the pass's partials
                     abort_flag = ab;
                 }
-                __syncthreads();
+                __syncthreads();  // no wave's load of the partials before the count was seen
                 if (abort_flag) return;
             }
+            uint32_t x[1][8];
             if (active) {
-                // partials are residues (< 2^27) and at most 16 are summed:
-                // 32-bit sums, the 8 loads of a slice in flight together
-                const uint32_t* src = ps.part + qi * ps.part_qstride + (size_t)c * ps.C + (size_t)g * N + t;
-                const uint32_t* p2 = part2 + qi * p2_stride + (size_t)g * 2 * N + (size_t)c * N + t;
+                // columns 2t + 512k (a pair each) of every slice: residues below
+                // 2^27, at most 16 of them, so 32-bit sums below 16q
+                const uint32_t* src = ps.part + qi * ps.part_qstride + (size_t)c * ps.C + (size_t)g * N + 2 * t;
+                const uint32_t* p2 = part2 + qi * p2_stride + (size_t)g * 2 * N + (size_t)c * N + 8 * t;
                 uint32_t a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-                for (uint32_t sl = 0; sl < ps.slices; sl++) {
+                uint64_t s2[4];
 #pragma unroll
-                    for (int e = 0; e < 8; e++) a[e] += src[sl * sstride + 256 * e];
-                }
+                for (int e = 0; e < 4; e++) s2[e] = agent_load2(p2 + 2 * e);
+#pragma unroll 4
+                for (uint32_t sl = 0; sl < ps.slices; sl++)
 #pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    buf[team][ls(t + 256 * e)] = red64(a[e], c);
-                    sub[e] = red64((uint64_t)sub[e] + p2[256 * e], c);
+                    for (int e = 0; e < 4; e++) {
+                        const uint64_t v = agent_load2(src + sl * sstride + 512 * e);
+                        a[2 * e] += (uint32_t)v;
+                        a[2 * e + 1] += (uint32_t)(v >> 32);
+                    }
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const uint32_t col = 2 * t + 512 * e;
+                    *reinterpret_cast<u32x2*>(&buf[team][0][col + 4 * (col >> 5)]) = u32x2{a[2 * e], a[2 * e + 1]};
+                    sub[2 * e] = red64((uint64_t)sub[2 * e] + (uint32_t)s2[e], c);
+                    sub[2 * e + 1] = red64((uint64_t)sub[2 * e + 1] + (uint32_t)(s2[e] >> 32), c);
                 }
             }
-            __syncthreads();
-            ntt_fwd_lds(buf[team], t, tw, c, active);
+            lds_barrier();
+            if (active) nr_load<0, 1>(buf[team], x, t);
+            nr_forward<1>(x, buf[team], tw2[c], t, m, [] { lds_barrier(); });  // from 16q: below 38q
             if (active) {
-                uint32_t* dst = packed_b + qi * pstride + (size_t)g * 2 * N + (size_t)c * N;
+                uint32_t* dst = packed_b + qi * pstride + (size_t)g * 2 * N + (size_t)c * N + 8 * t;
 #pragma unroll
-                for (int e = 0; e < 8; e++) dst[t + 256 * e] = sub_mod(buf[team][ls(t + 256 * e)], sub[e], q);
+                for (int e = 0; e < 8; e++) x[0][e] = sub_mod(fold(nr_reduce(x[0][e], m), m.q), sub[e], m.q);
+#pragma unroll
+                for (int e = 0; e < 4; e++) agent_store2(dst + 2 * e, x[0][2 * e], x[0][2 * e + 1]);
             }
-            __syncthreads();  // the buffers are free for the next round
+            lds_barrier();  // the buffers are free for the next round
         }
-        // publish the group: every wave's stores complete, then one release
+        // publish the group once every wave's stores are complete
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        if (tid == 0) {
-            fence_release_agent_done();
+        if (tid == 0)
             __hip_atomic_store(ps.packed_done + (size_t)blk * G + g, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
     }
 }
 

@@ -57,7 +57,7 @@ __device__ __forceinline__ NrLimb nr_limb(int c) { return NrLimb{qof(c), 0u - qo
 __device__ __forceinline__ uint32_t nr_mul(uint32_t x, uint32_t w, uint32_t wp, const NrLimb& m) {
     return nr_mad_s(mulhi32(x, wp), m.nq, nr_low(x * w)).x;
 }
-// x mod q up to a little more than q (below 1.4q) for x <= 32q:
+// x mod q up to a little more than q (below 1.5q) for any x < 2^32:
 // floor(2^32/q) = 45 for both primes.
 __device__ __forceinline__ uint32_t nr_reduce(uint32_t x, const NrLimb& m) {
     return nr_mad_s(mulhi32(x, 45u), m.nq, nr_low(x)).x;
