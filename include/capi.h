@@ -116,10 +116,11 @@ ipir_client_query* ipir_query_build_seeded(const ipir_params* params, uint64_t i
  * call if that one was on another stream; inside a caller's stream capture
  * the caller orders the captured work itself. For callers that keep
  * queries resident in HBM. Answers may run their Horner chains beside a
- * database pass they wait for inside the kernel; such a wait is bounded (about a second or more), and a chain
- * that gives up writes all-ones words as its response (no residue has
- * that value; it can happen only if the pass gets no CU for that long)
- * and is reported by ipir_device_status. */
+ * database pass they wait for inside the kernel, or as two workgroups that
+ * wait for each other; such a wait is bounded (about a second or more), and
+ * a chain that gives up writes all-ones words as its response (no residue
+ * has that value; it can happen only if the pass or the other workgroup gets
+ * no CU for that long) and is reported by ipir_device_status. */
 int ipir_answer_batch_device(ipir_server* srv, const uint64_t* d_queries, size_t count,
                              uint64_t* d_out_resp, void* hip_stream);
 

@@ -92,13 +92,13 @@ int ipir_dbg_set_group_chunk(ipir_server* srv, size_t groups);
  * overrides it). 1 for values outside 0..3. */
 int ipir_dbg_set_tail_split(ipir_server* srv, int on);
 /* Select the Horner kernel a server's answers use: mode as variant above,
- * or -1 (the default): one workgroup per chain, the faster one. Whatever
- * the mode, the asynchronous device entry points
- * (ipir_answer_batch_device, ipir_answer_batch_packed_device) never use the
- * pair: its bounded wait reports through a status word that only the
- * blocking entry points and the serving loop read. */
+ * or -1 (the default): pairs for up to 128 chains at once. With mode 1 the
+ * asynchronous device entry points (ipir_answer_batch_device,
+ * ipir_answer_batch_packed_device) use one workgroup per chain; pairs
+ * chosen by the default report there as streamed chains do
+ * (ipir_device_status). */
 int ipir_dbg_set_horner(ipir_server* srv, int mode);
-/* Bound of the pair kernel's partner wait, in sleeps (default 2^26, ~2 s).
+/* Bound of the pair kernel's partner wait, in loads (default 2^21, ~2 s).
  * 0 makes every pair chain report the bound exceeded at its first
  * exchange and stop (all kernels still end normally): the call that ran it
  * then returns 4, and later calls are unaffected. 5 while a loop runs. */

@@ -850,13 +850,13 @@ int ipir_dbg_horner_variant(const uint64_t* cts, size_t L, const uint64_t* rgsw,
             pb[g * 2 * N + x] = (uint32_t)(cts[g * 4 * N + 2 * N + x] % q);
         }
     for (size_t x = 0; x < 4 * b; x++) rg[x] = (uint32_t)(rgsw[x] % ((x / N) % 2 ? Q1 : Q0));
-    uint32_t *d_pa = nullptr, *d_pb = nullptr, *d_rg = nullptr, *d_x = nullptr, *d_f = nullptr, *d_st = nullptr;
+    uint32_t *d_pa = nullptr, *d_pb = nullptr, *d_rg = nullptr, *d_x = nullptr, *d_st = nullptr;
     uint32_t* d_hs = nullptr;
     uint64_t* d_o = nullptr;
     int rc = 0;
     if (hipMalloc(&d_pa, pa.size() * 4) || hipMalloc(&d_pb, pb.size() * 4) || hipMalloc(&d_rg, rg.size() * 4) ||
-        hipMalloc(&d_o, 4 * N * 8) || hipMalloc(&d_x, ipx::horner_pair_xbuf_words(1) * 4) || hipMalloc(&d_f, 8) ||
-        hipMalloc(&d_st, 4) || hipMemset(d_st, 0, 4) || hipMalloc(&d_hs, 4 * N * 4))
+        hipMalloc(&d_o, 4 * N * 8) || hipMalloc(&d_x, ipx::horner_pair_xbuf_words(1) * 4) ||
+        hipMemset(d_x, 0, ipx::horner_pair_xbuf_words(1) * 4) || hipMalloc(&d_st, 4) || hipMemset(d_st, 0, 4) || hipMalloc(&d_hs, 4 * N * 4))
         rc = 4;
     if (!rc && (hipMemcpy(d_pa, pa.data(), pa.size() * 4, hipMemcpyHostToDevice) ||
                 hipMemcpy(d_pb, pb.data(), pb.size() * 4, hipMemcpyHostToDevice) ||
@@ -865,7 +865,7 @@ int ipir_dbg_horner_variant(const uint64_t* cts, size_t L, const uint64_t* rgsw,
     if (!rc) {
         const hipError_t e =
             variant == 1 ? ipx::launch_horner_pair(d_pa, 2 * N, L, L, 1, d_pb, L * 2 * N, d_rg, 4 * b, d_o, d_hs, 0, L,
-                                                   1, d_x, d_f, d_st, GpuServerCtx::kHornerSpinLimit, st->nc, st->cc,
+                                                   1, d_x, d_st, GpuServerCtx::kHornerSpinLimit, st->nc, st->cc,
                                                    nullptr)
                          : ipx::launch_horner(d_pa, 2 * N, L, L, 1, d_pb, L * 2 * N, d_rg, 4 * b, d_o, d_hs, 0, L, 1,
                                               st->nc, st->cc, nullptr);
@@ -874,7 +874,7 @@ int ipir_dbg_horner_variant(const uint64_t* cts, size_t L, const uint64_t* rgsw,
             hipMemcpy(&status, d_st, 4, hipMemcpyDeviceToHost) || status)
             rc = 4;
     }
-    dfree(d_pa); dfree(d_pb); dfree(d_rg); dfree(d_o); dfree(d_x); dfree(d_f); dfree(d_st); dfree(d_hs);
+    dfree(d_pa); dfree(d_pb); dfree(d_rg); dfree(d_o); dfree(d_x); dfree(d_st); dfree(d_hs);
     return rc;
 }
 
@@ -903,6 +903,7 @@ int ipir_dbg_profile_batch(ipir_server* srv, const uint64_t* d_queries, size_t c
             mark();
             GpuServerCtx::PrepZero z;
             if (q0 == 0) z.status = c->h_status;
+            z.pair = c->use_pair(count, true);
             c->prep_query(c->d_q + q0 * c->qlen, q0, nq, p, s, 0, z);
             mark();
             c->dbpass_whole(q0, nq, p, s, 0);
@@ -913,7 +914,7 @@ int ipir_dbg_profile_batch(ipir_server* srv, const uint64_t* d_queries, size_t c
             mark();
         }
         mark();
-        c->horner_range(count, d_out, 0, c->G, s, 0, 0, true);
+        c->horner_range(count, d_out, 0, c->G, s, 0, 0, c->use_pair(count, true));
         mark();
         c->order_after(s);
         hip_check(hipEventSynchronize(ev[k - 1]), "sync");

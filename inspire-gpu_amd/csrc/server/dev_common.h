@@ -166,21 +166,6 @@ __device__ __forceinline__ void agent_store2(uint32_t* p, uint32_t lo, uint32_t 
 __device__ __forceinline__ uint64_t agent_load2(const uint32_t* p) {
     return __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// The workgroup pair of the two-workgroup Horner chain exchanges ordinary
-// accesses through the fences: the producer lane writes the L2 back after the
-// block's barrier and waits for that before the flag; the lane that saw the
-// flag invalidates and waits before the block's barrier. The waits are
-// written out: after an explicit s_waitcnt the compiler drops the fence's
-// own, which would let the flag overtake the write-back and other waves'
-// loads overtake the invalidation.
-__device__ __forceinline__ void fence_release_agent_done() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __builtin_amdgcn_s_waitcnt(0);
-}
-__device__ __forceinline__ void fence_acquire_agent_done() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    __builtin_amdgcn_s_waitcnt(0);
-}
 
 // A workgroup barrier for data exchanged through LDS only. __syncthreads also
 // waits for every global access in flight (its fence covers global memory),

@@ -108,6 +108,8 @@ struct PrepArgs {
     uint32_t* status = nullptr;   // a word set to zero
     uint32_t* part2 = nullptr;    // part2_words (a multiple of 4096) words per query set to zero
     size_t part2_stride = 0, part2_words = 0;
+    uint32_t* xbuf = nullptr;     // the same of xbuf_words words per query, queries back to back
+    size_t xbuf_words = 0;
     bool skip_lwe = false;        // keys and RGSW rows only
     // set by launch_prep
     uint32_t first = 0, form = 0, parts = 0, Mp = 0, kMp = 0, key_blocks = 0, lwe_blocks = 0, rgsw_blocks = 0;
@@ -275,17 +277,17 @@ hipError_t launch_horner(const uint32_t* pa_base, size_t pa_stride, size_t G, si
                          const StreamWait& wait = StreamWait{});
 
 // The same chains with two workgroups per chain (one per limb) exchanging
-// coefficient-form values once per step. xbuf holds
-// horner_pair_xbuf_words(nq*T) words and flags 2*nq*T words (reset by the
-// launch); a partner wait longer than spin_limit sleeps sets *status to 1
-// and the chain's output is then undefined. spin_limit 0 sets it at the
-// first exchange.
+// shares of the CRT lift once per step through xbuf,
+// horner_pair_xbuf_words(nq*T) words that are zero before a chain's first
+// launch. A partner wait of more than spin_limit loads sets *status to 1 and
+// makes the chain's output all-ones words. spin_limit 0 does so at the first
+// exchange.
 size_t horner_pair_xbuf_words(size_t nchains);
 hipError_t launch_horner_pair(const uint32_t* pa_base, size_t pa_stride, size_t G, size_t Da, size_t T,
                               const uint32_t* packed_b, size_t packed_stride, const uint32_t* rgsw,
                               size_t rgsw_stride, uint64_t* out, uint32_t* hstate, size_t g_lo, size_t g_hi,
-                              size_t nq, uint32_t* xbuf, uint32_t* flags, uint32_t* status, uint32_t spin_limit,
-                              const NttConst& nc, const CrtConst& cc, hipStream_t s);
+                              size_t nq, uint32_t* xbuf, uint32_t* status, uint32_t spin_limit, const NttConst& nc,
+                              const CrtConst& cc, hipStream_t s);
 
 // ---------------------------------------------------------------- preprocess
 hipError_t launch_encode(uint16_t* db, size_t R, size_t C, size_t Da, hipStream_t s);

@@ -4,193 +4,217 @@
 // src/gpu_online.cu:474-540, src/crypto.cpp:219-279) costs 4 INTTs, two
 // gadget decompositions and 8 NTTs. Only the decomposition couples the
 // limbs (its CRT lift needs both residues of a coefficient), so each limb's
-// workgroup inverts its own two polynomials, swaps the coefficient-form
-// values with its partner through global memory, decomposes every
-// coefficient itself and transforms the four digit polynomials mod its own
+// workgroup inverts its own two polynomials, swaps its shares of the lift
+// with its partner through global memory, cuts every coefficient into
+// digits itself and transforms the four digit polynomials mod its own
 // prime: 6 transforms per workgroup and one exchange per step instead of 12
-// transforms in one workgroup.
+// transforms in one workgroup. Inside a workgroup, team p of 256 lanes has
+// part p (a or b) of the accumulator: its inverse transform, its digits and
+// their products with the query's rows; the teams add each other's half of
+// the products through LDS. Transforms and layouts as in ntt_regs.h.
+//
+// Bound: like the one-workgroup chain, VALU issue of a serial chain, here on
+// two CUs (about 4.3 us of a step), plus the exchange's latency (about 1.6).
+// A step takes 5.9 us against the one workgroup's 8.6 (63 steps, one chain:
+// 376 and 541 us); with transforms through LDS, and flags behind L2
+// write-backs for the exchange, it took 12.
 //
 // Pairing: block b serves chain (b/16)*8 + b%8, limb (b/8)%2, so partners
 // are b and b^8 (consecutive workgroups are spread over the XCDs
-// round-robin, which puts partners on the same XCD and L2). The exchange
-// is a release store of the step number and a bounded wait for the
-// partner's (acquire at agent scope, so correctness does not depend on the
-// placement); a wait that exceeds the bound sets *status and ends both
-// workgroups, so every wave always reaches the end (a bound of zero takes
-// that path at the first exchange).
+// round-robin, which puts partners on the same XCD). The exchange has no
+// flag: a share takes 27 bits of a word, and the 5 upper bits of two words
+// stored together (agent_store2, an 8-byte access, so they arrive together)
+// hold the step's number; the partner loads them until the number is
+// there. Against a counter behind the data that saves the wait for the
+// stores and one trip through memory per step, and correctness depends on
+// neither placement nor caches. Steps alternate between two buffers: a
+// workgroup stores step n + 2 only after all of its lanes have seen the
+// partner's step n + 1, which the partner's lanes store after they have read
+// step n. The words must hold no number of this chain's steps beforehand
+// (they are zeroed in the answer's preparation launch).
+// The wait is bounded: a workgroup whose wait exceeds the bound sets
+// *status, fills its limb of the response with all-ones words (no residue;
+// where the chain continues in a later launch, of the state, which passes
+// them on) and ends; its partner's wait then ends the same way (a bound of
+// zero takes that path at the first exchange).
 #include "kernels.h"
+#include "ntt_regs.h"
 
 namespace ipx {
 
 namespace {
 
 constexpr size_t BLK = (size_t)D_EFF * 2 * N;
+constexpr uint32_t kShareMask = (1u << 27) - 1, kShareCentre = 1u << 26;
+static_assert(Q1 <= kShareMask && Q0 / 2 < kShareCentre, "a share fits 27 bits");
 
 __global__ __launch_bounds__(256) void k_fill_u32(uint32_t* __restrict__ p, size_t n, uint32_t v) {
     for (size_t x = (size_t)blockIdx.x * 256 + threadIdx.x; x < n; x += (size_t)gridDim.x * 256) p[x] = v;
 }
 
-__global__ __launch_bounds__(1024) void k_horner_pair(const uint32_t* __restrict__ pa_base, size_t pa_stride,
-                                                      uint32_t G, uint32_t Da, uint32_t T,
-                                                      const uint32_t* __restrict__ packed_b, size_t pstride,
-                                                      const uint32_t* __restrict__ rgsw, size_t rstride,
-                                                      uint64_t* __restrict__ out, uint32_t* __restrict__ hstate,
-                                                      uint32_t g_lo, uint32_t g_hi, uint32_t* __restrict__ xbuf,
-                                                      uint32_t* __restrict__ flags, uint32_t* __restrict__ status,
-                                                      uint32_t nchains, uint32_t spin_limit, NttConst nc,
-                                                      CrtConst cc) {
-    __shared__ uint32_t buf[4][POLY_LDS];
-    __shared__ uint32_t twl[4 * N];
-    __shared__ uint32_t rgl[4][2][N];  // this limb's RGSW rows [part][digit][coeff]
+__global__ __launch_bounds__(512, 2) void k_horner_pair(const uint32_t* __restrict__ pa_base, size_t pa_stride,
+                                                        uint32_t G, uint32_t Da, uint32_t T,
+                                                        const uint32_t* __restrict__ packed_b, size_t pstride,
+                                                        const uint32_t* __restrict__ rgsw, size_t rstride,
+                                                        uint64_t* __restrict__ out, uint32_t* __restrict__ hstate,
+                                                        uint32_t g_lo, uint32_t g_hi, uint32_t* xbuf,
+                                                        uint32_t* status, uint32_t nchains, uint32_t spin_limit,
+                                                        NttConst nc, NrGadget gc) {
+    __shared__ __align__(16) uint32_t buf[2][2][POLY4_LDS];  // [team][digit polynomial]
+    __shared__ __align__(16) nr_u32x2 tw[N];
+    __shared__ uint32_t sx[2][8][256];  // products by the team that made them, for the other's part
     __shared__ uint32_t abort_flag;
     const uint32_t b = blockIdx.x, chain = (b >> 4) * 8 + (b & 7);
     const int c = (int)((b >> 3) & 1);
     if (chain >= nchains) return;  // both partners of a padding chain leave
-    const uint32_t ct = chain % T, qi = chain / T;
+    const uint32_t ct = chain % T, qi = chain / T, tid = threadIdx.x, t = tid & 255;
+    const uint32_t p = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 8));  // this team's part
     const uint32_t start = ct * Da;
     const uint32_t L = (G - start) < Da ? (G - start) : Da;
     const uint32_t top = start + L - 1;
     // this launch covers the chain's groups in [lo, hi), highest first
     const uint32_t lo = start > g_lo ? start : g_lo, hi = start + L < g_hi ? start + L : g_hi;
     if (lo >= hi) return;  // both partners leave
-    const uint32_t tid = threadIdx.x, team = tid >> 8, t = tid & 255;
-    const uint32_t q = qof(c);
-    for (uint32_t x = tid; x < 4 * N; x += 1024) twl[x] = nc.tw[(size_t)c * 4 * N + x];
-    if (tid == 0) abort_flag = 0;
-    const Tw tw{twl, twl + N, twl + 2 * N, twl + 3 * N};
-    const uint32_t* pb = packed_b + qi * pstride;
-    const uint32_t* rg = rgsw + qi * rstride;
-    for (uint32_t x = tid; x < 8 * N; x += 1024) {
-        const uint32_t part = x / (2 * N), j = (x / N) & 1, i = x % N;
-        rgl[part][j][i] = rg[(size_t)part * BLK + ((size_t)j * 2 + c) * N + i];
-    }
+    const NrLimb m = nr_limb(c);
+    // this team's part of a group: 8 consecutive slots of the limb
+    auto load8 = [&](uint32_t (&x)[8], const uint32_t* src) {
+        const nr_u32x4* s = reinterpret_cast<const nr_u32x4*>(src + (size_t)c * N + 8 * t);
+        const nr_u32x4 l = s[0], u = s[1];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            x[k] = l[k];
+            x[k + 4] = u[k];
+        }
+    };
+    const uint32_t* pk = p ? packed_b + qi * pstride : pa_base;
+    const size_t pk_stride = p ? 2 * (size_t)N : pa_stride;
     uint32_t* hs = hstate + ((size_t)qi * T + ct) * 4 * N;  // chain state between launches, [a|b][limb][N]
-    uint32_t acc_a[2], acc_b[2];
-    int first;
-    if (top < g_hi) {  // the chain starts here: acc = packed[top]
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const uint32_t i = tid + 1024 * e;
-            acc_a[e] = pa_base[(size_t)top * pa_stride + (size_t)c * N + i];
-            acc_b[e] = pb[(size_t)top * 2 * N + (size_t)c * N + i];
-        }
-        first = (int)top - 1;
-    } else {
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const uint32_t i = tid + 1024 * e;
-            acc_a[e] = hs[(size_t)c * N + i];
-            acc_b[e] = hs[2 * (size_t)N + (size_t)c * N + i];
-        }
-        first = (int)hi - 1;
-    }
-    uint32_t* xb = xbuf + (size_t)chain * 2 * 2 * 2 * N;  // [parity][limb][a|b][N]
-    uint32_t* my_flag = flags + (size_t)chain * 2 + c;
-    uint32_t* other_flag = flags + (size_t)chain * 2 + (1 - c);
-    __syncthreads();
-    uint32_t k = 0;
-    for (int gs = first; gs >= (int)lo; gs--) {
-        k++;
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-            buf[0][ls(tid + 1024 * e)] = acc_a[e];
-            buf[1][ls(tid + 1024 * e)] = acc_b[e];
-        }
-        __syncthreads();
-        ntt_inv_lds(buf[team & 1], t, tw, c, nc.inv_n[c], nc.inv_n_p[c], team < 2);
-        uint32_t own_a[2], own_b[2];
-        uint32_t* xw = xb + (size_t)(k & 1) * 4 * N + (size_t)c * 2 * N;
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const uint32_t i = tid + 1024 * e;
-            own_a[e] = buf[0][ls(i)];
-            own_b[e] = buf[1][ls(i)];
-            xw[i] = own_a[e];
-            xw[N + i] = own_b[e];
-        }
-        // the hand-over rules in dev_common.h: every wave's stores complete,
-        // one release, the flag; the partner's flag, one acquire, the barrier
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        if (tid == 0) {
-            fence_release_agent_done();
-            __hip_atomic_store(my_flag, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            // a zero bound reports at the first exchange whatever the partner
-            // did (a deterministic way into this failure path)
-            uint32_t spins = 0;
-            while (spin_limit == 0 || __hip_atomic_load(other_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < k) {
-                if (++spins > spin_limit) {
-                    __hip_atomic_store(status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    abort_flag = 1;
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
-            }
-            fence_acquire_agent_done();  // the partner's values, for every wave after the barrier
-        }
-        __syncthreads();
-        if (abort_flag) {
-            // let the partner stop waiting for this step too
-            if (tid == 0) __hip_atomic_store(my_flag, 0xffffffffu, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    uint64_t* o = out + ((size_t)qi * T + ct) * 4 * N;
+    auto give_up = [&]() {
+        if (lo > start) {
+            nr_u32x4* d = reinterpret_cast<nr_u32x4*>(hs + ((size_t)2 * p + c) * N + 8 * t);
+            d[0] = d[1] = nr_u32x4{~0u, ~0u, ~0u, ~0u};
             return;
         }
-        const uint32_t* xr = xb + (size_t)(k & 1) * 4 * N + (size_t)(1 - c) * 2 * N;
-        uint32_t dA[2][2], dB[2][2];  // [e][digit], residues mod this limb's prime
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const uint32_t i = tid + 1024 * e;
-            const uint32_t oa = xr[i], ob = xr[N + i];
-            uint32_t d0[2], d1[2];
-            gadget2(c ? oa : own_a[e], c ? own_a[e] : oa, cc, d0, d1);
-            dA[e][0] = c ? d1[0] : d0[0];
-            dA[e][1] = c ? d1[1] : d0[1];
-            gadget2(c ? ob : own_b[e], c ? own_b[e] : ob, cc, d0, d1);
-            dB[e][0] = c ? d1[0] : d0[0];
-            dB[e][1] = c ? d1[1] : d0[1];
+        for (int k = 0; k < 8; k++) o[((size_t)2 * p + c) * N + t + 256 * k] = ~0ull;
+    };
+    uint32_t acc[1][8];  // slots 8t + k
+    int first;
+    if (top < g_hi) {  // the chain starts here: acc = packed[top]
+        load8(acc[0], pk + (size_t)top * pk_stride);
+        first = (int)top - 1;
+    } else {
+        load8(acc[0], hs + (size_t)p * 2 * N);
+        first = (int)hi - 1;
+        if (acc[0][0] == ~0u) {  // every lane: the chain gave up in an earlier launch
+            give_up();
+            return;
         }
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const uint32_t i = tid + 1024 * e;
-            buf[0][ls(i)] = dA[e][0];
-            buf[1][ls(i)] = dA[e][1];
-            buf[2][ls(i)] = dB[e][0];
-            buf[3][ls(i)] = dB[e][1];
+    }
+    if (first >= (int)lo) {
+        for (uint32_t x = tid; x < N; x += 512) {  // published by the barrier below
+            const uint32_t* f = nc.tw + (size_t)c * 4 * N;
+            tw[x] = nr_u32x2{f[x], f[N + x]};
         }
-        __syncthreads();
-        ntt_fwd_lds(buf[team], t, tw, c);
-        // RGSW parts: 0 top_a, 1 top_b, 2 bot_a, 3 bot_b (a-digits use top, b-digits bottom)
-        const uint32_t gi = (uint32_t)gs;
+        if (tid == 0) abort_flag = 0;
+        // the query's rows for this part's digits [to a | to b][digit][slot], times 2^32 mod q
+        const uint32_t r32 = c ? (uint32_t)(4294967296ull % Q1) : (uint32_t)(4294967296ull % Q0);
+        const uint32_t qneg = c ? nr_neg_inverse(Q1) : nr_neg_inverse(Q0);
+        const uint32_t* rg = rgsw + qi * rstride + (size_t)2 * p * BLK;
+        uint32_t rows[2][2][8];
 #pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const uint32_t i = tid + 1024 * e;
-            uint64_t sa = 0, sb = 0;
+        for (int r = 0; r < 2; r++)
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                const uint64_t xa = buf[j][ls(i)], xbv = buf[2 + j][ls(i)];
-                sa += xa * rgl[0][j][i] + xbv * rgl[2][j][i];
-                sb += xa * rgl[1][j][i] + xbv * rgl[3][j][i];
+                load8(rows[r][j], rg + (size_t)r * BLK + (size_t)j * 2 * N);
+#pragma unroll
+                for (int k = 0; k < 8; k++) rows[r][j][k] = mul_mod(rows[r][j][k], r32, c);
             }
-            acc_a[e] = add_mod(red64(sa, c), pa_base[(size_t)gi * pa_stride + (size_t)c * N + i], q);
-            acc_b[e] = add_mod(red64(sb, c), pb[(size_t)gi * 2 * N + (size_t)c * N + i], q);
-        }
+        // [parity][limb][part][k/2][lane][2]
+        uint32_t* xw = xbuf + (size_t)chain * 8 * N + ((size_t)c * 2 + p) * N + 2 * t;
+        const uint32_t* xr = xbuf + (size_t)chain * 8 * N + ((size_t)(1 - c) * 2 + p) * N + 2 * t;
         __syncthreads();
+        for (int gs = first; gs >= (int)lo; gs--) {
+            const uint32_t step = top - (uint32_t)gs;  // 1, 2, ...
+            const uint32_t par = (step & 1) * 4 * N;
+            // 1..1023: 5 bits in each of the two words of an access
+            const uint32_t num = (step - 1) % 1023 + 1, tag0 = num << 27, tag1 = (num >> 5) << 27;
+            uint32_t cf[1][8];  // coefficients t + 256k
+#pragma unroll
+            for (int k = 0; k < 8; k++) cf[0][k] = acc[0][k];
+            nr_inverse<1, 6>(cf, buf[p], tw, t, m);
+#pragma unroll
+            for (int k = 0; k < 8; k++) cf[0][k] = nr_crt_part(cf[0][k], gc, c, m);
+            const uint32_t off = c ? 0 : kShareCentre;
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                agent_store2(xw + par + 512 * k, (cf[0][2 * k] + off) | tag0, (cf[0][2 * k + 1] + off) | tag1);
+            uint32_t pv[8];  // the step's packed part, in flight during the exchange
+            load8(pv, pk + (size_t)gs * pk_stride);
+            uint32_t other[8];
+            uint32_t spins = 0;
+            bool late = spin_limit == 0;
+            while (!late) {
+                uint32_t diff = 0;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const uint64_t v = agent_load2(xr + par + 512 * k);
+                    other[2 * k] = (uint32_t)v;
+                    other[2 * k + 1] = (uint32_t)(v >> 32);
+                    diff |= (other[2 * k] ^ tag0) | (other[2 * k + 1] ^ tag1);
+                }
+                if (diff <= kShareMask) break;
+                late = ++spins > spin_limit;
+            }
+            if (late) {
+                __hip_atomic_store(status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                abort_flag = 1;
+            }
+            lds_barrier();
+            if (abort_flag) {
+                give_up();
+                return;
+            }
+            uint32_t x[2][8];  // digit polynomials: residues + q mod this limb's prime
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const uint32_t got = (other[k] & kShareMask) - (c ? kShareCentre : 0);
+                const nr_u32x2 d = nr_digits(c ? got : cf[0][k], c ? cf[0][k] : got);
+                x[0][k] = d.x + (m.q - (1u << 17));
+                x[1][k] = d.y + m.q;
+            }
+            nr_forward<2>(x, buf[p], tw, t, m, [] { lds_barrier(); });
+            uint32_t mine[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                // digits below 23.1q, rows below q: the sums stay below 47 q^2, a product below 2.1q
+                uint64_t s[2];
+#pragma unroll
+                for (int r = 0; r < 2; r++)
+                    s[r] = (uint64_t)x[0][k] * rows[r][0][k] + (uint64_t)x[1][k] * rows[r][1][k];
+                mine[k] = nr_montgomery(p ? s[1] : s[0], qneg, m.q);
+                sx[p][k][t] = nr_montgomery(p ? s[0] : s[1], qneg, m.q);
+            }
+            lds_barrier();
+#pragma unroll
+            for (int k = 0; k < 8; k++) acc[0][k] = mine[k] + sx[1 - p][k][t] + pv[k];  // below 5.2q
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++) acc[0][k] = fold(fold(fold(acc[0][k], 4 * m.q), 2 * m.q), m.q);
     }
     if (lo > start) {  // the chain continues in a later launch
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const uint32_t i = tid + 1024 * e;
-            hs[(size_t)c * N + i] = acc_a[e];
-            hs[2 * (size_t)N + (size_t)c * N + i] = acc_b[e];
-        }
+        nr_u32x4* d = reinterpret_cast<nr_u32x4*>(hs + ((size_t)2 * p + c) * N + 8 * t);
+        d[0] = nr_u32x4{acc[0][0], acc[0][1], acc[0][2], acc[0][3]};
+        d[1] = nr_u32x4{acc[0][4], acc[0][5], acc[0][6], acc[0][7]};
         return;
     }
-    uint64_t* o = out + ((size_t)qi * T + ct) * 4 * N;
+    // the response, through LDS for whole lines of 8-byte words (a lane's own
+    // words of the last exchange)
+    nr_store<3, 1>(buf[p], acc, t);
+    __syncthreads();
 #pragma unroll
-    for (int e = 0; e < 2; e++) {
-        const uint32_t i = tid + 1024 * e;
-        o[(size_t)c * N + i] = acc_a[e];
-        o[2 * (size_t)N + (size_t)c * N + i] = acc_b[e];
-    }
+    for (int k = 0; k < 8; k++)
+        o[((size_t)2 * p + c) * N + t + 256 * k] = buf[p][0][nr_base(0, t) + nr_stride<0>() * k];
 }
 
 }  // namespace
@@ -200,15 +224,15 @@ size_t horner_pair_xbuf_words(size_t nchains) { return nchains * 2 * 2 * 2 * N; 
 hipError_t launch_horner_pair(const uint32_t* pa_base, size_t pa_stride, size_t G, size_t Da, size_t T,
                               const uint32_t* packed_b, size_t packed_stride, const uint32_t* rgsw,
                               size_t rgsw_stride, uint64_t* out, uint32_t* hstate, size_t g_lo, size_t g_hi,
-                              size_t nq, uint32_t* xbuf, uint32_t* flags, uint32_t* status, uint32_t spin_limit,
-                              const NttConst& nc, const CrtConst& cc, hipStream_t s) {
+                              size_t nq, uint32_t* xbuf, uint32_t* status, uint32_t spin_limit, const NttConst& nc,
+                              const CrtConst& cc, hipStream_t s) {
     const size_t nchains = nq * T;
     if (nchains == 0 || g_lo >= g_hi) return hipSuccess;
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, s, flags, 2 * nchains, 0u);
     const size_t blocks = 16 * ((nchains + 7) / 8);
-    hipLaunchKernelGGL(k_horner_pair, dim3((unsigned)blocks), dim3(1024), 0, s, pa_base, pa_stride, (uint32_t)G,
+    hipLaunchKernelGGL(k_horner_pair, dim3((unsigned)blocks), dim3(512), 0, s, pa_base, pa_stride, (uint32_t)G,
                        (uint32_t)Da, (uint32_t)T, packed_b, packed_stride, rgsw, rgsw_stride, out, hstate,
-                       (uint32_t)g_lo, (uint32_t)g_hi, xbuf, flags, status, (uint32_t)nchains, spin_limit, nc, cc);
+                       (uint32_t)g_lo, (uint32_t)g_hi, xbuf, status, (uint32_t)nchains, spin_limit, nc,
+                       nr_gadget_const(nc, cc));
     return hipGetLastError();
 }
 

@@ -234,9 +234,11 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a, NttConst nc) {
         for (int i = 0; i < 16; i++) dst[t + 256 * i] = red64(v[i], i >> 3);  // [..][limb][N]: 4096 words = both limbs
         return;
     }
-    // collapse sums a split collapse adds into
+    // collapse sums a split collapse adds into; the pair chains' exchange words
     b -= a.rgsw_blocks;
-    uint32_t* p2 = a.part2 + (size_t)qi * a.part2_stride + (size_t)b * 4096;
+    const uint32_t nb2 = (uint32_t)(a.part2_words / 4096);
+    uint32_t* p2 = b < nb2 ? a.part2 + (size_t)qi * a.part2_stride + (size_t)b * 4096
+                           : a.xbuf + (size_t)qi * a.xbuf_words + (size_t)(b - nb2) * 4096;
 #pragma unroll
     for (int i = 0; i < 4; i++) *reinterpret_cast<u32x4*>(p2 + 4 * (t + 256 * i)) = u32x4{0, 0, 0, 0};
 }
@@ -270,8 +272,10 @@ hipError_t launch_prep(PrepArgs a, size_t nq, const DbPlan& p, const NttConst& n
         a.key_blocks = kKeyBlocks;
         a.rgsw_blocks = kRgswBlocks;
     }
-    if (a.part2_words % 4096 || (a.part2_words && !a.part2) || (a.zero_words && !a.zero)) return hipErrorInvalidValue;
-    const size_t blocks = a.key_blocks + a.lwe_blocks + a.rgsw_blocks + a.part2_words / 4096;
+    if (a.part2_words % 4096 || (a.part2_words && !a.part2) || (a.zero_words && !a.zero) || a.xbuf_words % 4096 ||
+        (a.xbuf_words && !a.xbuf))
+        return hipErrorInvalidValue;
+    const size_t blocks = a.key_blocks + a.lwe_blocks + a.rgsw_blocks + (a.part2_words + a.xbuf_words) / 4096;
     const dim3 grid((unsigned)blocks, (unsigned)count);
     if (a.narrow)
         hipLaunchKernelGGL(k_prep<uint32_t>, grid, dim3(256), 0, s, a, nc);

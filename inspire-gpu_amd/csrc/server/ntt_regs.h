@@ -272,14 +272,14 @@ __device__ __forceinline__ void nr_forward1(uint32_t (&x)[1][8], uint32_t (*buf)
 }
 
 // Inverse transform without its N^-1 scale: in, NTT slots 8t + k up to
-// 5q; out, coefficients t + 256k up to 32q. buf as above, with the words
+// B q (B <= 8); out, coefficients t + 256k up to 32q. buf as above, with the words
 // 8t + k (own) free.
-template <int P>
+template <int P, uint32_t B = 5>
 __device__ __forceinline__ void nr_inverse(uint32_t (&x)[P][8], uint32_t (*buf)[POLY4_LDS], const nr_u32x2* tw,
                                            uint32_t t, const NrLimb& m) {
     NrTw w;
     nr_tw_load(w, tw, nr_inv_node(3, t), false);
-    nr_inv_phase<P, false, 5>(x, w, m);  // sums of four: 20q at k = 0 and 4, else up to 4q
+    nr_inv_phase<P, false, B>(x, w, m);  // sums of four: 4B q at k = 0 and 4, else up to 4q
 #pragma unroll
     for (int p = 0; p < P; p++) {
         x[p][0] = nr_reduce(x[p][0], m);

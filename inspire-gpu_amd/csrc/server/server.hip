@@ -336,7 +336,7 @@ ServerFootprint server_footprint(const PublicParams& pp, size_t gchunk) {
     const size_t qlen = lay.query_u64s(), resp = T * 4 * N;
     f.per_slot = qlen * 8 + resp * 8 + 2 * R * 8 +
                  (lay.keys_words() + lay.rgsw_words() + part_words + 2 * C + 2 * G * 2 * N) * 4 +
-                 (horner_pair_xbuf_words(T) + 2 * T + T * 4 * N) * 4 +
+                 (horner_pair_xbuf_words(T) + T * 4 * N) * 4 +
                  T * 4 * N * 4;
     f.fixed = R * C * 2 + G * PC_GROUP * 4 + 8 * N * 4 +
               GpuServerCtx::kLanes *
@@ -423,7 +423,6 @@ void GpuServerCtx::alloc_slots() {
     const char* se = std::getenv("INSPIRE_STREAM");
     stream_ok = !(se && se[0] == '0');
     d_hxbuf = dalloc<uint32_t>(horner_pair_xbuf_words(B * T));
-    d_hflags = dalloc<uint32_t>(2 * B * T);
     HIPX(hipHostMalloc((void**)&h_status, kLanes * 4, hipHostMallocDefault));
     for (int l = 0; l < kLanes; l++) h_status[l] = 0;
     horner_spin_limit = kHornerSpinLimit;
@@ -802,6 +801,8 @@ void GpuServerCtx::prep_query(const QueryInput& in, size_t q0, size_t nq, const 
     a.part2 = d_part2 + q0 * part2_stride;
     a.part2_stride = part2_stride;
     a.part2_words = z.part2 ? G * 2 * N : 0;
+    a.xbuf = d_hxbuf + horner_pair_xbuf_words(q0 * T);
+    a.xbuf_words = z.pair ? horner_pair_xbuf_words(T) : 0;
     a.status = z.status;
     if (!in.stage) {
         HIPX(launch_prep(a, nq, p, nc, s));
@@ -998,22 +999,23 @@ void GpuServerCtx::pack_whole(size_t q0, size_t nq, const DbPlan& p, hipStream_t
                               packed_stride, nq, nc, s, d_out));
 }
 
-bool GpuServerCtx::use_pair(bool status_read) const {
-    // only where set by hand, and never where nobody reads the status its
-    // bounded wait reports through: the Horner stage of a serial one-query
-    // answer at 1 GB (7 steps) takes 87 us with the pair, 72 us with one
-    // workgroup
-    return status_read && horner_mode == 1;
+bool GpuServerCtx::use_pair(size_t count, bool status_read) const {
+    // set by hand: never where nobody reads the status its bounded wait
+    // reports through
+    if (horner_mode >= 0) return horner_mode == 1 && status_read;
+    // else wherever the answer's chains all find two CUs; a chain fused with
+    // its pack has one workgroup
+    return pack_wg != 2 && G > 1 && count * T <= kPairMaxChains;
 }
 
 void GpuServerCtx::horner_range(size_t count, uint64_t* d_out, size_t g_lo, size_t g_hi, hipStream_t s,
-                                size_t slot0, int lane, bool status_read, const FusedPack* fp) {
-    if (use_pair(status_read))
+                                size_t slot0, int lane, bool pair, const FusedPack* fp) {
+    if (pair)
         HIPX(launch_horner_pair(d_precomp + PC_A, PC_GROUP, G, Da, T, d_packed_b + slot0 * packed_stride,
                                 packed_stride, d_rgsw + slot0 * rgsw_stride, rgsw_stride, d_out,
                                 d_hstate + slot0 * T * 4 * N, g_lo, g_hi, count,
-                                d_hxbuf + horner_pair_xbuf_words(slot0 * T), d_hflags + 2 * slot0 * T,
-                                h_status + lane, horner_spin_limit, nc, cc, s));
+                                d_hxbuf + horner_pair_xbuf_words(slot0 * T), h_status + lane, horner_spin_limit, nc,
+                                cc, s));
     else
         HIPX(launch_horner(d_precomp + PC_A, PC_GROUP, G, Da, T, d_packed_b + slot0 * packed_stride, packed_stride,
                            d_rgsw + slot0 * rgsw_stride, rgsw_stride, d_out, d_hstate + slot0 * T * 4 * N, g_lo, g_hi,
@@ -1079,7 +1081,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
     // wait for both halves of that chunk. s finally waits for the chains,
     // and through their waits for every collapse.
     bool joined = false;
-    const bool streamable = can_stream(s);
+    const bool streamable = can_stream(s), pair = use_pair(count, status_read);
     last_part_slices = 0;  // the first sub-batch's result lands in interm unless it streams with slices
     // Serial sub-batches (shape 0) leave their Horner chains to one launch
     // after the last of them: a sub-batch's nq x T chains each hold a CU for
@@ -1089,7 +1091,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
     size_t defer_lo = 0, defer_n = 0;
     auto flush_deferred = [&]() {
         if (defer_n)
-            horner_range(defer_n, d_out + (defer_lo - slot0) * resp_u64s, 0, G, s, defer_lo, lane, status_read);
+            horner_range(defer_n, d_out + (defer_lo - slot0) * resp_u64s, 0, G, s, defer_lo, lane, pair);
         defer_n = 0;
     };
     for (size_t q0 = slot0; q0 < slot0 + count; q0 += kMfmaMaxQueries) {
@@ -1216,6 +1218,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             // one launch (kMergeBytes)
             const bool both = pass_collapse_ok(p, nq) && pp.db_rows * C * 2 + G * PC_GROUP * 4 <= kMergeBytes;
             z.part2 = (both ? pass_collapse_ksplit(nq, G) : collapse_row_slices(nq, G, collapse_variant)) > 1;
+            z.pair = pair;
             prep_query(in, q0, nq, p, s, lane, z);
             mark_pass(s, true);
             if (both) {
@@ -1251,6 +1254,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
         const bool first = shape == 4, ahead = shape == 5;
         joined = true;
         const DbPlan p = chunk_plan(nq, gchunk * N);  // every chunk's plan has this one's kernel and digits
+        z.pair = pair;
         prep_query(in, q0, nq, p, s, lane, z);
         if (cs != s) {
             HIPX(hipEventRecord(prep_ev[lane], s));  // the keys are in place
@@ -1291,7 +1295,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             if (cs != s) HIPX(hipStreamWaitEvent(hs, dbe, 0));
             HIPX(hipStreamWaitEvent(hs, ce, 0));
             // the pack: fused into the one-workgroup Horner chains, or a kernel of its own
-            const bool fuse = pack_wg == 2 && !use_pair(status_read);
+            const bool fuse = pack_wg == 2 && !pair;
             const FusedPack fp{d_interm + q0 * 2 * C, C, p2, part2_stride, d_precomp, keys, keys_stride};
             if (fuse)
                 ;
@@ -1301,7 +1305,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             else
                 HIPX(launch_pack_finalize(d_interm + q0 * 2 * C, 2 * C, 1, C, p2, part2_stride, d_precomp, g_lo, ng,
                                           keys, keys_stride, packed, packed_stride, nq, nc, hs));
-            horner_range(nq, out, g_lo, g_hi, hs, q0, lane, status_read, fuse ? &fp : nullptr);
+            horner_range(nq, out, g_lo, g_hi, hs, q0, lane, pair, fuse ? &fp : nullptr);
         }
         if (cs != s) {  // the next batch's key digits overwrite the lane's scratch
             HIPX(hipEventRecord(prep_ev[lane], cs));
@@ -1545,7 +1549,7 @@ void gpu_free_server(GpuServerCtx* ctx) {
     dfree(ctx->d_tw); dfree(ctx->d_db); dfree(ctx->d_precomp);
     dfree(ctx->d_q); dfree(ctx->d_resp); dfree(ctx->d_bq); dfree(ctx->d_keys); dfree(ctx->d_rgsw);
     dfree(ctx->d_part); dfree(ctx->d_interm); dfree(ctx->d_part2); dfree(ctx->d_packed_b);
-    dfree(ctx->d_hxbuf); dfree(ctx->d_hflags); dfree(ctx->d_hstate);
+    dfree(ctx->d_hxbuf); dfree(ctx->d_hstate);
     for (auto& f : ctx->d_sflags) dfree(f);
     dfree(ctx->d_cmp);
     for (int l = 0; l < GpuServerCtx::kLanes; l++) {

@@ -184,13 +184,12 @@ struct GpuServerCtx {
     // the Horner chains' own workgroups (where the one-workgroup Horner runs)
     int pack_wg = 0;
     uint32_t* d_hxbuf = nullptr;    // pair exchange buffers [B*T chains]
-    uint32_t* d_hflags = nullptr;   // pair step flags [B*T][2]
     // per scratch lane: nonzero once a pair chain of that lane's calls gave
     // up its bounded wait (read and cleared by check_status)
     // (pinned host memory the kernels write: reading it after the call costs
     // no copy; a call whose status is read zeroes it in its first kernel)
     uint32_t* h_status = nullptr;   // [kLanes]
-    uint32_t horner_spin_limit = 0; // the pair kernel's wait bound in sleeps (0: report at once)
+    uint32_t horner_spin_limit = 0; // the pair kernel's wait bound in loads (0: report at once)
     uint32_t stream_spin_limit = 0; // the same for chains waiting for a streamed pass's groups
     uint32_t* d_hstate = nullptr;   // Horner chain state between chunk launches [B*T][4][N]
     // Pinned host staging, which kernels read and write directly: queries
@@ -254,6 +253,7 @@ struct GpuServerCtx {
         uint32_t* flags = nullptr;  // flag_words words
         uint32_t flag_words = 0;
         bool part2 = false;         // the collapse sums (a split collapse adds into them)
+        bool pair = false;          // the pair chains' exchange words
         bool skip_lwe = false;      // leave the LWE part to prep_lwe
         uint32_t* status = nullptr; // a word
     };
@@ -281,13 +281,14 @@ struct GpuServerCtx {
     ipx::DbPlan chunk_plan(size_t nq, size_t ncols) const;
     // Database pass of queries [q0, q0+nq) over the columns of groups [g_lo, g_hi) into interm.
     void dbpass_range(size_t q0, size_t nq, size_t g_lo, size_t g_hi, const ipx::DbPlan& p, hipStream_t s, int lane);
-    // The pair kernel only where the caller reads the lane's status after
-    // the call (status_read): its bounded wait reports through it.
-    bool use_pair(bool status_read) const;
+    // Whether an answer's chains (of count queries) run as workgroup pairs.
+    // Where set by hand, only where the caller reads the lane's status after
+    // the call (status_read).
+    bool use_pair(size_t count, bool status_read) const;
     // Horner chains of `count` queries over groups [g_lo, g_hi).
     // fp: the chains compute their groups' packed b-parts themselves first
     void horner_range(size_t count, uint64_t* d_out, size_t g_lo, size_t g_hi, hipStream_t s, size_t slot0,
-                      int lane, bool status_read, const ipx::FusedPack* fp = nullptr);
+                      int lane, bool pair, const ipx::FusedPack* fp = nullptr);
     // Throw (and clear) if a pair chain of a call on `lane` reported a fault
     // through its status word; the call's stream has been waited for.
     void check_status(int lane);
@@ -304,10 +305,14 @@ struct GpuServerCtx {
     std::vector<hipEvent_t> pass_marks;
     size_t pass_marks_used = 0, passes_timed = 0;
     void mark_pass(hipStream_t s, bool first);
-    // Seconds of sleeps: far above any partner skew or any streamed pass's
-    // time to reach a group, bounded so a chain whose partner or pass never
-    // runs still ends.
-    static constexpr uint32_t kHornerSpinLimit = 1u << 26;
+    // Loads of about 1 us: far above any partner skew, bounded so a chain
+    // whose partner never runs still ends.
+    static constexpr uint32_t kHornerSpinLimit = 1u << 21;
+    // Most chains of an answer that run as pairs: a CU for each of their
+    // workgroups. 63 steps, all chains in one launch, one workgroup and pair:
+    // 541 / 376 us for 1 chain, 555 / 394 for 32, 612 / 464 for 128, 632 / 875
+    // for 192 (two workgroups to a CU).
+    static constexpr size_t kPairMaxChains = 128;
     // The streamed chains' bound: ~1 s or more of sleeps, far above a
     // database pass's time even queued behind other batches on the device.
     static constexpr uint32_t kStreamSpinLimit = 1u << 23;

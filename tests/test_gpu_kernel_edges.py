@@ -148,3 +148,71 @@ def test_wire_words_beyond_32_bits_and_unaligned_packed_buffers(odd_table):
         assert lib.ipir_answer_batch_packed_device(srv.h, C.c_void_p(dp.p + off), nq, C.c_void_p(dc.p + off), None) == 0
         assert lib.ipir_dev_sync() == 0
         assert np.array_equal(dc.download(np.zeros(comp.nbytes + off, np.uint8))[off:], comp.reshape(-1)), off
+
+
+@pytest.mark.parametrize("rgsw", ["largest", "alternating", "random"])
+@pytest.mark.parametrize("cts", ["largest", "alternating", "sparse", "random"])
+def test_pair_chain_of_extreme_residues(cts, rgsw):
+    """The same chain by a workgroup pair, whose teams add two products."""
+    L = 4
+    c = _polys(cts, (L, 2), 1).reshape(-1)
+    r = _polys(rgsw, (4, 2), 2).reshape(-1)
+    out, want = np.zeros(4 * N, np.uint64), np.zeros(4 * N, np.uint64)
+    assert ia.load("server").ipir_dbg_horner_variant(ia.ptr(c), L, ia.ptr(r), ia.ptr(out), 1) == 0
+    ol.oracle().orc_horner(c, L, r, want)
+    assert np.array_equal(out, want)
+
+
+def test_pair_chain_longer_than_its_step_numbers():
+    """1030 steps: the exchange's numbers 1..1023 start again."""
+    L = 1031
+    c = _polys("random", (L, 2), 5).reshape(-1)
+    r = _polys("random", (4, 2), 6).reshape(-1)
+    out, want = np.zeros(4 * N, np.uint64), np.zeros(4 * N, np.uint64)
+    assert ia.load("server").ipir_dbg_horner_variant(ia.ptr(c), L, ia.ptr(r), ia.ptr(out), 1) == 0
+    ol.oracle().orc_horner(c, L, r, want)
+    assert np.array_equal(out, want)
+
+
+@pytest.mark.parametrize("shape", [0, 2])
+def test_pair_chains_of_plain_answers(shape):
+    """Answers whose chains run as pairs by themselves, in one launch and in
+    one per chunk: equal to the one-workgroup kernel's, on blocking and
+    device calls; a wait over its bound (0: every kernel still ends) is
+    reported and leaves no residue in the response, and the next answer is
+    right again."""
+    n, w, rows, nq = 524288, 120, 2048, 3
+    rc, geo = ol.setup(n, w, rows)
+    db = np.random.default_rng(8).integers(0, ol.P, size=(geo["R"], geo["C"]), dtype=np.uint16)
+    lib = ia.load("server")
+    srv = ia.Server(db, n, w, rows, max_batch=nq, crs_seed=bytes(SEED))
+    qs = np.stack([ol.make_query(geo, SEED, 1000 * k + 5, 70 + k)[0] for k in range(nq)])
+    dq = ia.DeviceBuffer(qs.nbytes, lib)
+    dq.upload(qs)
+    out = ia.DeviceBuffer(nq * geo["T"] * 4 * N * 8, lib)
+
+    def device():
+        assert lib.ipir_answer_batch_device(srv.h, C.c_void_p(dq.p), nq, C.c_void_p(out.p), None) == 0
+        assert lib.ipir_dev_sync() == 0
+        return out.download(np.zeros_like(want))
+
+    try:
+        assert lib.ipir_dbg_set_group_chunk(srv.h, 2) == 0
+        assert lib.ipir_dbg_set_pipeline(srv.h, shape, shape) == 0
+        assert lib.ipir_dbg_set_horner(srv.h, 0) == 0
+        want = srv.answer_batch(list(qs))
+        assert lib.ipir_dbg_set_horner(srv.h, -1) == 0
+        for _ in range(3):
+            assert np.array_equal(srv.answer_batch(list(qs)), want)
+            assert np.array_equal(device(), want)
+        assert lib.ipir_dbg_set_horner_spin_limit(srv.h, 0) == 0
+        assert (device() == ~np.uint64(0)).all()
+        assert lib.ipir_device_status(srv.h) == 4
+        assert lib.ipir_answer_batch(srv.h, srv.views(list(qs)), nq, ia.ptr(np.zeros_like(want))) == 4
+        assert lib.ipir_dbg_set_horner_spin_limit(srv.h, 1 << 21) == 0
+        assert np.array_equal(device(), want)
+        assert lib.ipir_device_status(srv.h) == 0
+    finally:
+        out.free()
+        dq.free()
+        srv.close()
