@@ -108,8 +108,8 @@ int ipir_answer_batch_device(ipir_server* srv, const uint64_t* d_queries, size_t
         if (c->loop_active) return 5;
         hipStream_t s = hip_stream ? static_cast<hipStream_t>(hip_stream) : c->stream;
         c->order_before(s);
-        // nobody reads a status word after an asynchronous call, so its
-        // answers never take the pair Horner kernel (enqueue's default)
+        // nobody reads a status word after an asynchronous call: a pair Horner
+        // set by hand is for the others (enqueue's default)
         c->run_step(d_queries, d_out_resp, count, 0, 0, 0, s, [&] { c->enqueue(d_queries, count, d_out_resp, s); });
         c->order_after(s);
         return 0;

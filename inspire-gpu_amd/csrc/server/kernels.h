@@ -108,7 +108,7 @@ struct PrepArgs {
     uint32_t* status = nullptr;   // a word set to zero
     uint32_t* part2 = nullptr;    // part2_words (a multiple of 4096) words per query set to zero
     size_t part2_stride = 0, part2_words = 0;
-    uint32_t* xbuf = nullptr;     // the same of xbuf_words words per query, queries back to back
+    uint32_t* xbuf = nullptr;     // xbuf_words words per query, queries back to back, set to zero (with keys)
     size_t xbuf_words = 0;
     bool skip_lwe = false;        // keys and RGSW rows only
     // set by launch_prep
