@@ -19,11 +19,13 @@ namespace {
 size_t blk() { return (size_t)D_EFF * 2 * N; }
 }  // namespace
 
-void flatten_view(const ipir_query_view& v, size_t R, uint32_t* w) {
+void flatten_view(const ipir_query_view& v, size_t R, uint32_t* lwe, uint32_t* w) {
     const size_t b = (size_t)D_EFF * 2 * N;
-    narrow_residues(v.lwe_b_limb0, w, R, Q0);
-    narrow_residues(v.lwe_b_limb1, w + R, R, Q1);
-    w += 2 * R;
+    if (lwe) {
+        narrow_residues(v.lwe_b_limb0, lwe, R, Q0);
+        narrow_residues(v.lwe_b_limb1, lwe + R, R, Q1);
+    }
+    if (!w) return;
     // parts of [digit][limb][N]
     auto parts = [&](const uint64_t* p, size_t n) {
         for (size_t o = 0; o < n; o += N, w += N) narrow_residues(p + o, w, N, (o / N) & 1 ? Q1 : Q0);
@@ -90,7 +92,8 @@ int ipir_answer_batch(ipir_server* srv, const ipir_query_view* queries, size_t c
         std::lock_guard<std::mutex> lk(srv->ctx->mu);
         if (srv->ctx->loop_active) return 5;
         const size_t R = srv->ctx->pp.db_rows;
-        srv->ctx->answer_host(count, [&](size_t i, uint32_t* w) { flatten_view(queries[i], R, w); }, out_resp);
+        srv->ctx->answer_host(
+            count, [&](size_t i, uint32_t* lwe, uint32_t* rest) { flatten_view(queries[i], R, lwe, rest); }, out_resp);
         return 0;
     } catch (...) {
         return 4;
@@ -408,7 +411,7 @@ int ipir_dbg_answer_taps(ipir_server* srv, const uint64_t* query, uint32_t* inte
         v.kskneg1_b = v.ksk5_b + blk();
         v.rgsw = v.kskneg1_b + blk();
         std::vector<uint64_t> r(c->resp_u64s);
-        c->answer_host(1, [&](size_t, uint32_t* w) { flatten_view(v, R, w); }, r.data());
+        c->answer_host(1, [&](size_t, uint32_t* lwe, uint32_t* rest) { flatten_view(v, R, lwe, rest); }, r.data());
         if (resp) std::memcpy(resp, r.data(), r.size() * 8);
         if (interm && c->last_part_slices > 1) {
             // a streamed pass left row-slice partials (the pack sums them):

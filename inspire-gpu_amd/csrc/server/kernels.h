@@ -36,6 +36,9 @@ size_t query_packed_bytes(size_t R);
 // flat queries of u32 residues (qlen words apart).
 hipError_t launch_query_unpack(const uint8_t* packed, size_t count, size_t R, uint32_t* flat, size_t qlen,
                                hipStream_t s);
+// Values [v0, v0 + nv) alone (multiples of 256), whose bytes are pstride apart.
+hipError_t launch_query_unpack_part(const uint8_t* packed, size_t pstride, size_t v0, size_t nv, size_t count,
+                                    size_t R, uint32_t* flat, size_t qlen, hipStream_t s);
 // nct response cts (flat u64, NTT form, [ct][a|b][limb][N]) -> 12288
 // compressed bytes each; scratch holds nct*4*N words.
 hipError_t launch_compress(const uint64_t* resp, size_t nct, uint32_t* scratch, uint8_t* out, const NttConst& nc,
@@ -94,6 +97,7 @@ struct PrepArgs {
     const void* q = nullptr;      // query 0's words (LWE part first), queries q_stride words apart
     bool narrow = false;          // u32 words instead of u64
     size_t q_stride = 0, R = 0;
+    size_t keys_at = 0;           // word of the key part (2R in a flat query), the RGSW part behind it
     double* bq = nullptr;         // [query][limb][R]
     int8_t* dig = nullptr;
     uint32_t* S = nullptr;

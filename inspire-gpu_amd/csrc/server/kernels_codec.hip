@@ -21,10 +21,10 @@ constexpr int BETA = 53;  // bits of one CRT-packed value (Q0*Q1 < 2^53)
 // aligned).
 constexpr uint32_t kFieldBytes = 256 * BETA / 8;
 template <bool WIDE>
-__global__ __launch_bounds__(256) void k_query_unpack(const uint8_t* __restrict__ packed, size_t pbytes, uint32_t R,
-                                                      uint32_t* __restrict__ flat, size_t qlen) {
+__global__ __launch_bounds__(256) void k_query_unpack(const uint8_t* __restrict__ packed, size_t pbytes, uint32_t v0,
+                                                      uint32_t R, uint32_t* __restrict__ flat, size_t qlen) {
     __shared__ __align__(16) uint8_t sb[kFieldBytes];
-    const uint32_t t = threadIdx.x, v = blockIdx.x * 256 + t;
+    const uint32_t t = threadIdx.x, v = v0 + blockIdx.x * 256 + t;
     const uint8_t* src = packed + (size_t)blockIdx.y * pbytes + (size_t)blockIdx.x * kFieldBytes;
     if (WIDE) {
         if (t < kFieldBytes / 16)
@@ -129,21 +129,27 @@ __global__ __launch_bounds__(256) void k_compress(const uint32_t* __restrict__ c
 
 size_t query_packed_bytes(size_t R) { return ((R + 6 * (size_t)D_EFF * N) * BETA + 7) / 8; }
 
-hipError_t launch_query_unpack(const uint8_t* packed, size_t count, size_t R, uint32_t* flat, size_t qlen,
-                               hipStream_t s) {
-    if (count == 0) return hipSuccess;
-    if (qlen < 2 * R + 12 * (size_t)D_EFF * N) return hipErrorInvalidValue;
+hipError_t launch_query_unpack_part(const uint8_t* packed, size_t pstride, size_t v0, size_t nv, size_t count,
+                                    size_t R, uint32_t* flat, size_t qlen, hipStream_t s) {
+    if (count == 0 || nv == 0) return hipSuccess;
     const size_t V = R + 6 * (size_t)D_EFF * N;
-    // V is a multiple of 2048: whole blocks, and queries start 16-byte aligned if the buffer does
-    if (V % 256 || query_packed_bytes(R) % 16) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)(V / 256), (unsigned)count);
-    if (reinterpret_cast<uintptr_t>(packed) % 16 == 0)
-        hipLaunchKernelGGL(k_query_unpack<true>, grid, dim3(256), 0, s, packed, query_packed_bytes(R), (uint32_t)R,
+    // whole blocks of 256 fields; every query starts 16-byte aligned if the buffer does
+    if (qlen < 2 * R + 12 * (size_t)D_EFF * N || v0 % 256 || nv % 256 || v0 + nv > V || pstride < nv / 256 * kFieldBytes)
+        return hipErrorInvalidValue;
+    const dim3 grid((unsigned)(nv / 256), (unsigned)count);
+    if (reinterpret_cast<uintptr_t>(packed) % 16 == 0 && pstride % 16 == 0)
+        hipLaunchKernelGGL(k_query_unpack<true>, grid, dim3(256), 0, s, packed, pstride, (uint32_t)v0, (uint32_t)R,
                            flat, qlen);
     else
-        hipLaunchKernelGGL(k_query_unpack<false>, grid, dim3(256), 0, s, packed, query_packed_bytes(R), (uint32_t)R,
+        hipLaunchKernelGGL(k_query_unpack<false>, grid, dim3(256), 0, s, packed, pstride, (uint32_t)v0, (uint32_t)R,
                            flat, qlen);
     return hipGetLastError();
+}
+
+hipError_t launch_query_unpack(const uint8_t* packed, size_t count, size_t R, uint32_t* flat, size_t qlen,
+                               hipStream_t s) {
+    return launch_query_unpack_part(packed, query_packed_bytes(R), 0, R + 6 * (size_t)D_EFF * N, count, R, flat, qlen,
+                                    s);
 }
 
 hipError_t launch_compress(const uint64_t* resp, size_t nct, uint32_t* scratch, uint8_t* out, const NttConst& nc,

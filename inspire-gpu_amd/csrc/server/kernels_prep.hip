@@ -82,7 +82,7 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a, NttConst nc) {
         const NrLimb m = nr_limb(c);
         W in[8];
 #pragma unroll
-        for (int k = 0; k < 8; k++) in[k] = w[2 * R + (size_t)b * N + t + 256 * k];
+        for (int k = 0; k < 8; k++) in[k] = w[a.keys_at + (size_t)b * N + t + 256 * k];
         // the pair chains' exchange words, an eighth per block while the keys load
         u32x4* xz = reinterpret_cast<u32x4*>(a.xbuf + (size_t)qi * a.xbuf_words + b * (a.xbuf_words / kKeyBlocks));
         for (uint32_t x = t; x < a.xbuf_words / kKeyBlocks / 4; x += 256) xz[x] = u32x4{0, 0, 0, 0};
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a, NttConst nc) {
     }
     b -= a.lwe_blocks;
     if (b < a.rgsw_blocks) {
-        const W* src = w + 2 * R + 2 * BLK + (size_t)b * 4096;
+        const W* src = w + a.keys_at + 2 * BLK + (size_t)b * 4096;
         uint32_t* dst = a.rgsw + (size_t)qi * a.rgsw_stride + (size_t)b * 4096;
         W v[16];
 #pragma unroll

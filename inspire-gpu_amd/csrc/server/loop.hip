@@ -264,7 +264,7 @@ uint64_t ipir_loop_submit(ipir_loop* L, const ipir_query_view* v, uint64_t* out_
         return 0;
     auto* r = new Req;
     r->q.resize(L->ctx->qlen);
-    flatten_view(*v, L->ctx->pp.db_rows, r->q.data());
+    flatten_view(*v, L->ctx->pp.db_rows, r->q.data(), r->q.data() + 2 * L->ctx->pp.db_rows);
     r->out = out_resp;
     std::lock_guard<std::mutex> lk(L->m);
     if (L->stop) {

@@ -456,7 +456,7 @@ void GpuServerCtx::alloc_slots() {
     HIPX(hipHostMalloc((void**)&h_q, B * (qlen * 4 > qpack_bytes ? qlen * 4 : qpack_bytes), hipHostMallocDefault));
     // helpers only where a batch has work for them
     const size_t cpus = std::thread::hardware_concurrency();
-    host_stage.reset(new HostStage(B < 2 || cpus < 2 ? 0 : cpus - 1 < kStageHelpers ? cpus - 1 : kStageHelpers, B));
+    host_stage.reset(new HostStage(B < 2 || cpus < 2 ? 0 : cpus - 1 < kStageHelpers ? cpus - 1 : kStageHelpers, 2 * B));
     HIPX(hipHostMalloc((void**)&h_resp, B * resp_u64s * 8, hipHostMallocDefault));
     resident_bytes = fp.fixed + B * fp.per_slot;
     autotune_dbpass();
@@ -775,6 +775,7 @@ PrepArgs GpuServerCtx::prep_args(const QueryInput& in, size_t stride, size_t q0,
     a.narrow = in.narrow;
     a.q_stride = stride;
     a.R = pp.db_rows;
+    a.keys_at = 2 * pp.db_rows;
     a.bq = d_bq + q0 * 2 * pp.db_rows;
     a.dig = d_dig[lane];
     a.S = d_S[lane];
@@ -783,27 +784,10 @@ PrepArgs GpuServerCtx::prep_args(const QueryInput& in, size_t stride, size_t q0,
 
 void GpuServerCtx::prep_lwe(const QueryInput& in, size_t stride, size_t q0, size_t nq, const DbPlan& p, hipStream_t s,
                             int lane) {
-    HIPX(launch_prep(prep_args(in, stride, q0, lane), nq, p, nc, s));
+    launch_pieces(prep_args(in, stride, q0, lane), in, nq, p, s);
 }
 
-void GpuServerCtx::prep_query(const QueryInput& in, size_t q0, size_t nq, const DbPlan& p, hipStream_t s, int lane,
-                              const PrepZero& z) {
-    PrepArgs a = prep_args(in, qlen, q0, lane);
-    a.keys = d_keys + q0 * keys_stride;
-    a.keys_stride = keys_stride;
-    a.rgsw = d_rgsw + q0 * rgsw_stride;
-    a.rgsw_stride = rgsw_stride;
-    a.kdig = d_kdig[lane];
-    a.KS = d_KS[lane];
-    a.skip_lwe = z.skip_lwe;
-    a.zero = z.flags;
-    a.zero_words = z.flag_words;
-    a.part2 = d_part2 + q0 * part2_stride;
-    a.part2_stride = part2_stride;
-    a.part2_words = z.part2 ? G * 2 * N : 0;
-    a.xbuf = d_hxbuf + horner_pair_xbuf_words(q0 * T);
-    a.xbuf_words = z.pair ? horner_pair_xbuf_words(T) : 0;
-    a.status = z.status;
+void GpuServerCtx::launch_pieces(const PrepArgs& a, const QueryInput& in, size_t nq, const DbPlan& p, hipStream_t s) {
     if (!in.stage) {
         HIPX(launch_prep(a, nq, p, nc, s));
         return;
@@ -814,6 +798,35 @@ void GpuServerCtx::prep_query(const QueryInput& in, size_t q0, size_t nq, const 
         in.stage->wait(in.first + f + n);
         HIPX(launch_prep(a, nq, p, nc, s, f, n));
     }
+}
+
+void GpuServerCtx::prep_query(const QueryInput& in, size_t q0, size_t nq, const DbPlan& p, hipStream_t s, int lane,
+                              const PrepZero& z) {
+    PrepArgs a = prep_args(in, qlen, q0, lane);
+    if (in.late) {  // the late part, in place on the device
+        a.q = in.late->words;
+        a.q_stride = in.late->stride;
+        a.keys_at = 0;
+    }
+    a.keys = d_keys + q0 * keys_stride;
+    a.keys_stride = keys_stride;
+    a.rgsw = d_rgsw + q0 * rgsw_stride;
+    a.rgsw_stride = rgsw_stride;
+    a.kdig = d_kdig[lane];
+    a.KS = d_KS[lane];
+    a.skip_lwe = z.skip_lwe || in.late;
+    a.zero = z.flags;
+    a.zero_words = z.flag_words;
+    a.part2 = d_part2 + q0 * part2_stride;
+    a.part2_stride = part2_stride;
+    a.part2_words = z.part2 ? G * 2 * N : 0;
+    a.xbuf = d_hxbuf + horner_pair_xbuf_words(q0 * T);
+    a.xbuf_words = z.pair ? horner_pair_xbuf_words(T) : 0;
+    a.status = z.status;
+    if (in.late)
+        HIPX(launch_prep(a, nq, p, nc, s));
+    else
+        launch_pieces(a, in, nq, p, s);
 }
 
 DbPlan GpuServerCtx::plan_for(size_t nq, size_t ncols) const {
@@ -1151,7 +1164,9 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
                 HIPX(hipEventRecord(coll_ev[lane][0], s));
             }
             if (fused) {
-                prep_lwe(in, qlen, q0, nq, sp, s, lane);
+                QueryInput staged = in;
+                staged.stage = nullptr;  // prep_query has waited for all of it
+                prep_lwe(staged, qlen, q0, nq, sp, s, lane);
             } else {
                 HIPX(launch_collapse(d_precomp, G, d_kdig[lane], d_KS[lane], nq, p2, part2_stride, cs,
                                      collapse_variant));
@@ -1219,7 +1234,26 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             const bool both = pass_collapse_ok(p, nq) && pp.db_rows * C * 2 + G * PC_GROUP * 4 <= kMergeBytes;
             z.part2 = (both ? pass_collapse_ksplit(nq, G) : collapse_row_slices(nq, G, collapse_variant)) > 1;
             z.pair = pair;
+            if (in.late) {
+                HIPX(hipEventRecord(prep_ev[lane], s));  // earlier readers of the copy's target are done
+                HIPX(hipStreamWaitEvent(ps_side, prep_ev[lane], 0));
+                prep_lwe(in, in.lwe_stride, q0, nq, p, s, lane);
+                mark_pass(s, true);
+                dbpass_whole(q0, nq, p, s, lane);
+                mark_pass(s, false);
+                in.late->copy(ps_side);
+                HIPX(hipEventRecord(coll_ev[lane][0], ps_side));
+                HIPX(hipStreamWaitEvent(s, coll_ev[lane][0], 0));
+                if (in.late->after) in.late->after(s);
+            }
             prep_query(in, q0, nq, p, s, lane, z);
+            if (in.late) {
+                collapse_whole(q0, nq, s, lane, z.part2);
+                pack_whole(q0, nq, p, s);
+                defer_lo = q0;  // one sub-batch
+                defer_n = nq;
+                continue;
+            }
             mark_pass(s, true);
             if (both) {
                 size_t qstride;
@@ -1371,15 +1405,23 @@ void GpuServerCtx::drop_graphs() {
 }
 
 void GpuServerCtx::enqueue_packed(const uint8_t* d_in, size_t count, uint8_t* d_out, hipStream_t s, size_t slot0,
-                                  int lane, bool status_read, HostStage* stage) {
+                                  int lane, bool status_read, HostStage* stage, const LateKeys* late) {
     uint32_t* dq = flat32() + slot0 * qlen;
     uint64_t* dr = d_resp + slot0 * resp_u64s;
+    QueryInput in(dq);
+    in.late = late;
+    in.lwe_stride = qlen;
+    const size_t R = pp.db_rows;
     for (size_t f = 0; f < count; f += stage ? kStagePiece : count) {
         const size_t n = stage && count - f > kStagePiece ? kStagePiece : count - f;
         if (stage) stage->wait(f + n);
-        HIPX(launch_query_unpack(d_in + f * qpack_bytes, n, pp.db_rows, dq + f * qlen, qlen, s));
+        if (late)
+            HIPX(launch_query_unpack_part(d_in + f * lwe_packed_bytes(), lwe_packed_bytes(), 0, R, n, R,
+                                          dq + f * qlen, qlen, s));
+        else
+            HIPX(launch_query_unpack(d_in + f * qpack_bytes, n, R, dq + f * qlen, qlen, s));
     }
-    enqueue(QueryInput(dq), count, dr, s, slot0, lane, status_read);
+    enqueue(in, count, dr, s, slot0, lane, status_read);
     HIPX(launch_compress(dr, count * T, d_cmp + slot0 * T * 4 * N, d_out, nc, cc, s));
 }
 
@@ -1413,12 +1455,42 @@ void GpuServerCtx::answer_packed_host(const uint8_t* in, size_t count, uint8_t* 
     uint8_t* hr = reinterpret_cast<uint8_t*>(h_resp);
     TraceRange tr("host-staged packed answer: %zu queries", count);
     {
-        StagedJob job(*host_stage, count,
-                      [&](size_t i) { std::memcpy(hq + i * qpack_bytes, in + i * qpack_bytes, qpack_bytes); });
+        // split: the LWE parts' bytes, then the others' (both 16-byte multiples)
+        const bool split = late_keys(count);
+        const size_t lwe = lwe_packed_bytes(), rest = qpack_bytes - lwe;
+        uint8_t* const hq_rest = hq + count * lwe;
+        StagedJob job(*host_stage, split ? 2 * count : count, [&](size_t i) {
+            if (!split)
+                std::memcpy(hq + i * qpack_bytes, in + i * qpack_bytes, qpack_bytes);
+            else if (i < count)
+                std::memcpy(hq + i * lwe, in + i * qpack_bytes, lwe);
+            else
+                std::memcpy(hq_rest + (i - count) * rest, in + (i - count) * qpack_bytes + lwe, rest);
+        });
         order_before(s);
         if (graph_mode) host_stage->wait(count);  // a replayed graph waits for nothing
-        run_step(hq, hr, count, 0, 0, 1, s,
-                 [&] { enqueue_packed(hq, count, hr, s, 0, 0, true, graph_mode ? nullptr : host_stage.get()); });
+        LateKeys late;
+        if (split) {
+            // the bytes go behind the unpacked queries (half of d_q is free)
+            uint8_t* const d_rest = reinterpret_cast<uint8_t*>(flat32() + cfg.max_batch * qlen);
+            late.copy = [=](hipStream_t side) {
+                for (size_t f = 0; f < count; f += kLatePiece) {
+                    const size_t n = count - f < kLatePiece ? count - f : kLatePiece;
+                    host_stage->wait(count + f + n);
+                    HIPX(hipMemcpyAsync(d_rest + f * rest, hq_rest + f * rest, n * rest, hipMemcpyHostToDevice, side));
+                }
+            };
+            late.after = [=](hipStream_t st) {
+                HIPX(launch_query_unpack_part(d_rest, rest, pp.db_rows, 6 * (size_t)D_EFF * N, count, pp.db_rows,
+                                              flat32(), qlen, st));
+            };
+            late.words = flat32() + 2 * pp.db_rows;
+            late.stride = qlen;
+        }
+        run_step(hq, hr, count, 0, 0, 1, s, [&] {
+            enqueue_packed(hq, count, hr, s, 0, 0, true, graph_mode ? nullptr : host_stage.get(),
+                           split ? &late : nullptr);
+        });
         order_after(s);
     }
     HIPX(hipStreamSynchronize(s));
@@ -1450,7 +1522,12 @@ void GpuServerCtx::order_after(hipStream_t s) {
     order_stream_set = true;
 }
 
-void GpuServerCtx::answer_host(size_t count, const std::function<void(size_t, uint32_t*)>& fill, uint64_t* out) {
+bool GpuServerCtx::late_keys(size_t count) const {
+    return !graph_mode && count >= kLateQueries && count <= kMfmaMaxQueries && G > 1 && shape_for(count) == 0 &&
+           plan_for(count, pp.db_cols).kind == DbPlan::MFMA && pp.db_rows * pp.db_cols * 2 >= kLateTableBytes;
+}
+
+void GpuServerCtx::answer_host(size_t count, const FillQuery& fill, uint64_t* out) {
     hipStream_t s = pipelined(count) && !graph_mode ? lanes[0].pass : stream;
     TraceRange tr("host-staged answer: %zu queries", count);
     {
@@ -1459,10 +1536,35 @@ void GpuServerCtx::answer_host(size_t count, const std::function<void(size_t, ui
         // responses to pinned memory: no copies of their own, half the bytes.
         // At 1 GB, 32 queries, one thread's copies to and from the staging
         // took 1.1 ms and the device copy 0.53 ms of a 2.1-2.5 ms call.
-        StagedJob job(*host_stage, count, [&](size_t i) { fill(i, h_q + i * qlen); });
+        const size_t R2 = 2 * pp.db_rows, rest = qlen - R2;
+        const bool split = late_keys(count);
+        uint32_t* const h_rest = h_q + count * R2;  // split: the LWE parts, then the others
+        StagedJob job(*host_stage, split ? 2 * count : count, [&](size_t i) {
+            if (!split)
+                fill(i, h_q + i * qlen, h_q + i * qlen + R2);
+            else if (i < count)
+                fill(i, h_q + i * R2, nullptr);
+            else
+                fill(i - count, nullptr, h_rest + (i - count) * rest);
+        });
         order_before(s);
         if (graph_mode) host_stage->wait(count);  // a replayed graph waits for nothing
-        const QueryInput in(h_q, graph_mode ? nullptr : host_stage.get());
+        QueryInput in(h_q, graph_mode ? nullptr : host_stage.get());
+        LateKeys late;
+        if (split) {
+            late.copy = [&](hipStream_t side) {
+                for (size_t f = 0; f < count; f += kLatePiece) {
+                    const size_t n = count - f < kLatePiece ? count - f : kLatePiece;
+                    host_stage->wait(count + f + n);
+                    HIPX(hipMemcpyAsync(flat32() + f * rest, h_rest + f * rest, n * rest * 4, hipMemcpyHostToDevice,
+                                        side));
+                }
+            };
+            late.words = flat32();
+            late.stride = rest;
+            in.late = &late;
+            in.lwe_stride = R2;
+        }
         run_step(h_q, h_resp, count, 0, 0, 0, s, [&] { enqueue(in, count, h_resp, s, 0, 0, true); });
         order_after(s);
     }
@@ -1490,10 +1592,12 @@ void check_query(const QueryMessage& m, size_t R) {
         if (v->size() != (size_t)D_EFF) throw std::invalid_argument("gpu_answer_batch: wrong digit count");
 }
 
-void flatten_query(const QueryMessage& m, size_t R, uint32_t* w) {
-    narrow_residues(m.lwe.b_limb0.data(), w, R, Q0);
-    narrow_residues(m.lwe.b_limb1.data(), w + R, R, Q1);
-    w += 2 * R;
+void flatten_query(const QueryMessage& m, size_t R, uint32_t* lwe, uint32_t* w) {
+    if (lwe) {
+        narrow_residues(m.lwe.b_limb0.data(), lwe, R, Q0);
+        narrow_residues(m.lwe.b_limb1.data(), lwe + R, R, Q1);
+    }
+    if (!w) return;
     auto parts = [&](const std::vector<RnsPoly>& v, bool want_ntt) {
         for (const RnsPoly& p0 : v) {
             RnsPoly p = p0;
@@ -1520,7 +1624,10 @@ std::vector<std::vector<RlweCt>> gpu_answer_batch(GpuServerCtx* ctx, const Query
     if (ctx->loop_active) throw std::runtime_error("gpu_answer_batch: a serving loop owns this server");
     for (size_t i = 0; i < count; i++) check_query(queries[i], ctx->pp.db_rows);
     std::vector<uint64_t> flat(count * ctx->resp_u64s);
-    ctx->answer_host(count, [&](size_t i, uint32_t* w) { flatten_query(queries[i], ctx->pp.db_rows, w); }, flat.data());
+    ctx->answer_host(
+        count,
+        [&](size_t i, uint32_t* lwe, uint32_t* rest) { flatten_query(queries[i], ctx->pp.db_rows, lwe, rest); },
+        flat.data());
     std::vector<std::vector<RlweCt>> out(count, std::vector<RlweCt>(ctx->T));
     const uint64_t* r = flat.data();
     for (auto& resp : out)

@@ -21,14 +21,26 @@ inline void dfree(void* p) {
     if (p) (void)hipFree(p);
 }
 
+// The key and RGSW parts of staged queries that reach the device beside the
+// database pass, which needs the LWE parts alone.
+struct LateKeys {
+    std::function<void(hipStream_t)> copy;  // to the device, on the side stream (waits for the host job)
+    std::function<void(hipStream_t)> after; // what is left to do behind the copy, on the answer's stream
+    const uint32_t* words = nullptr;        // then: stride words per query, the key part first
+    size_t stride = 0;
+};
+
 // Flat queries an answer starts from: u64 wire words, or words narrowed to
 // u32 (back to back, qlen words each), in device or pinned host memory; with
 // `stage`, queries that a host job is still writing (query 0 is its item 0).
+// With `late` (one sub-batch) the LWE parts alone, lwe_stride words apart.
 struct QueryInput {
     const void* q = nullptr;
     bool narrow = false;
     HostStage* stage = nullptr;
     size_t first = 0;  // item of query 0
+    const LateKeys* late = nullptr;
+    size_t lwe_stride = 0;
     QueryInput(const uint64_t* d) : q(d) {}
     QueryInput(const uint32_t* d, HostStage* st = nullptr) : q(d), narrow(true), stage(st) {}
     QueryInput at(size_t k, size_t qlen) const {
@@ -200,6 +212,13 @@ struct GpuServerCtx {
     std::unique_ptr<HostStage> host_stage;  // fills h_q and empties h_resp
     static constexpr size_t kStageHelpers = 3;
     static constexpr size_t kStagePiece = 4;  // queries per preparation launch while the rest is staged
+    // late_keys: from this many queries over a table of this size (bytes; a
+    // pass of 20 us). Host calls of 3, 6, 9, 32 queries with everything before
+    // the pass and with the late part: 240 MB 166 / 180, 215 / 229, 295 / 246,
+    // 603 / 523 us; 1 GB 377 / 384, 417 / 408, 520 / 483, 887 / 794.
+    static constexpr size_t kLateQueries = 9, kLateTableBytes = (size_t)1 << 27;
+    static constexpr size_t kLatePiece = 8;   // queries per copy
+    size_t lwe_packed_bytes() const { return pp.db_rows / 8 * 53; }  // of a packed query
     uint32_t* flat32() const { return reinterpret_cast<uint32_t*>(d_q); }  // unpacked queries
 
     // packed-wire path (53-bit CRT-packed queries in, compressed responses out)
@@ -264,9 +283,11 @@ struct GpuServerCtx {
     void prep_query(const QueryInput& in, size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s, int lane) {
         prep_query(in, q0, nq, p, s, lane, PrepZero{});
     }
-    // Plan p's pass operands alone, of LWE parts stride words apart.
+    // Plan p's pass operands alone, of LWE parts stride words apart (staged
+    // ones piece by piece).
     void prep_lwe(const QueryInput& in, size_t stride, size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s,
                   int lane);
+    void launch_pieces(const ipx::PrepArgs& a, const QueryInput& in, size_t nq, const ipx::DbPlan& p, hipStream_t s);
     // Where a full-width pass of plan p writes: its row slices' partials, or interm.
     uint32_t* pass_out(size_t q0, const ipx::DbPlan& p, size_t& qstride);
     void dbpass_whole(size_t q0, size_t nq, const ipx::DbPlan& p, hipStream_t s, int lane);
@@ -331,14 +352,22 @@ struct GpuServerCtx {
     int shape_for(size_t nq) const;
     bool pipelined(size_t count) const;
     static bool is_capturing(hipStream_t s);
-    // Host-staged answer: fill(i, words) writes query i's qlen u32 words
-    // (called from several threads); the flat responses go to out.
-    void answer_host(size_t count, const std::function<void(size_t, uint32_t*)>& fill, uint64_t* out);
+    // Host-staged answer: fill(i, lwe, rest) writes the u32 words of query i's
+    // LWE part and of its keys and RGSW rows, each where not null (called from
+    // several threads); the flat responses go to out.
+    using FillQuery = std::function<void(size_t, uint32_t*, uint32_t*)>;
+    void answer_host(size_t count, const FillQuery& fill, uint64_t* out);
+    // Whether a staged answer's keys and RGSW rows (43% of a query of 32768
+    // rows) go to the device beside the database pass: a serial answer of one
+    // sub-batch, with a pass long enough to hide the copy engine's transfer.
+    bool late_keys(size_t count) const;
     // enqueue() behind the device wire codecs: count packed queries at d_in
     // (device, qpack_bytes each) -> count*T compressed cts at d_out (device).
-    // (stage: a host job still writing them)
+    // (stage: a host job still writing them; late: d_in has their LWE parts'
+    // bytes alone)
     void enqueue_packed(const uint8_t* d_in, size_t count, uint8_t* d_out, hipStream_t s, size_t slot0 = 0,
-                        int lane = 0, bool status_read = false, HostStage* stage = nullptr);
+                        int lane = 0, bool status_read = false, HostStage* stage = nullptr,
+                        const LateKeys* late = nullptr);
     // count responses of `bytes` bytes from the pinned staging to out.
     void copy_out(size_t count, size_t bytes, void* out);
     // Host round trip of the packed forms through the pinned staging.
@@ -366,4 +395,5 @@ struct ipir_server {
 };
 
 // One query's words (a C ABI view), narrowed to u32 as the server stages them.
-void flatten_view(const ipir_query_view& v, size_t R, uint32_t* w);
+// The view's words, each part where not null.
+void flatten_view(const ipir_query_view& v, size_t R, uint32_t* lwe, uint32_t* rest);

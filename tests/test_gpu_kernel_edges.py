@@ -216,3 +216,37 @@ def test_pair_chains_of_plain_answers(shape):
         out.free()
         dq.free()
         srv.close()
+
+
+@pytest.mark.parametrize("groups,shape", [(1, 0), (2, 0), (2, 3)])
+def test_staged_batches_whose_keys_follow_the_pass(groups, shape):
+    """Host and packed calls of 8 to 33 queries over 128 and 240 MB (from 9
+    to 32 and two groups on, serial, the keys and RGSW rows reach the device
+    beside the pass), a different set of queries each call: equal to the
+    device entry's answers."""
+    n, w, rows = groups << 20, 120 if groups > 1 else 60, 32768
+    rc, geo = ol.setup(n, w, rows)
+    assert rc == 0 and geo["G"] == groups
+    db = np.random.default_rng(4).integers(0, ol.P, size=(geo["R"], geo["C"]), dtype=np.uint16)
+    lib = ia.load("server")
+    srv = ia.Server(db, n, w, rows, max_batch=33, crs_seed=bytes(SEED))
+    try:
+        assert lib.ipir_dbg_set_pipeline(srv.h, shape, shape) == 0
+        qs = np.stack([ol.make_query(geo, SEED, 7919 * k, 40 + k)[0] for k in range(33)])
+        dq = ia.DeviceBuffer(qs.nbytes, lib)
+        dq.upload(qs)
+        out = ia.DeviceBuffer(33 * geo["T"] * 4 * N * 8, lib)
+        assert lib.ipir_answer_batch_device(srv.h, C.c_void_p(dq.p), 33, C.c_void_p(out.p), None) == 0
+        assert lib.ipir_dev_sync() == 0
+        want = out.download(np.zeros((33, geo["T"] * 4 * N), np.uint64))
+        cl = ia.Client(srv.params, lib)
+        packed = np.stack([cl.pack_query(q) for q in qs])
+        comp = np.stack([cl.compress(r) for r in want])
+        for first, nq in ((0, 8), (3, 9), (20, 13), (1, 32), (0, 33), (11, 10)):
+            part = slice(first, first + nq)
+            assert np.array_equal(srv.answer_batch(list(qs[part])), want[part]), (first, nq)
+            assert np.array_equal(srv.answer_packed(packed[part]), comp[part]), (first, nq)
+        dq.free()
+        out.free()
+    finally:
+        srv.close()
