@@ -839,22 +839,38 @@ DbPlan GpuServerCtx::plan_for(size_t nq, size_t ncols) const {
 }
 
 void GpuServerCtx::set_chunks() {
+    // The chunks of every response ciphertext's chain, highest first, taken
+    // in turns where chunks end with the ciphertexts: the chains of several
+    // then advance side by side, and only a chunk's steps of each are left
+    // after the last pass.
     chunks.clear();
-    const size_t n = G / gchunk, h = gchunk / 2, q = gchunk / 4;
-    const bool quarters = n > 1 && gchunk % 4 == 0;
-    for (size_t k = n; k-- > 0;) {
-        const size_t lo = k * gchunk, hi = lo + gchunk;
-        if (quarters && head_split && k == n - 1) {
-            chunks.push_back({hi - q, hi});
-            chunks.push_back({hi - h, hi - q});
-            chunks.push_back({lo, hi - h});
-        } else if (quarters && tail_split && k == 0) {
-            chunks.push_back({lo + h, hi});
-            chunks.push_back({lo + q, lo + h});
-            chunks.push_back({lo, lo + q});
-        } else {
-            chunks.push_back({lo, hi});
+    const bool turns = T > 1 && G % T == 0 && G / T == Da && Da % gchunk == 0;
+    const size_t nct = turns ? T : 1, per = G / nct, n = per / gchunk, h = gchunk / 2, q = gchunk / 4;
+    const bool quarters = G > gchunk && gchunk % 4 == 0;
+    std::vector<std::vector<std::pair<size_t, size_t>>> lists(nct);
+    for (size_t ct = 0; ct < nct; ct++)
+        for (size_t k = n; k-- > 0;) {
+            const size_t lo = ct * per + k * gchunk, hi = lo + gchunk;
+            auto& l = lists[ct];
+            if (quarters && head_split && hi == G) {
+                l.push_back({hi - q, hi});
+                l.push_back({hi - h, hi - q});
+                l.push_back({lo, hi - h});
+            } else if (quarters && tail_split && lo == 0) {
+                l.push_back({lo + h, hi});
+                l.push_back({lo + q, lo + h});
+                l.push_back({lo, lo + q});
+            } else {
+                l.push_back({lo, hi});
+            }
         }
+    for (size_t r = 0, left = nct; left; r++) {
+        left = 0;
+        for (size_t ct = nct; ct-- > 0;)
+            if (r < lists[ct].size()) {
+                chunks.push_back(lists[ct][r]);
+                left++;
+            }
     }
 }
 
@@ -1093,7 +1109,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
     // pack and the Horner chains of a chunk (on the lane's Horner stream)
     // wait for both halves of that chunk. s finally waits for the chains,
     // and through their waits for every collapse.
-    bool joined = false;
+    bool joined = false, side_chains = false;
     const bool streamable = can_stream(s), pair = use_pair(count, status_read);
     last_part_slices = 0;  // the first sub-batch's result lands in interm unless it streams with slices
     // Serial sub-batches (shape 0) leave their Horner chains to one launch
@@ -1326,8 +1342,12 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
                                          p2 + g_lo * 2 * N, part2_stride, cs, collapse_variant));
                 HIPX(hipEventRecord(ce, cs));
             }
-            if (cs != s) HIPX(hipStreamWaitEvent(hs, dbe, 0));
-            HIPX(hipStreamWaitEvent(hs, ce, 0));
+            // with the side stream free, every other ciphertext's chains run on it
+            const bool aside = cs == s && (T - 1 - g_lo / Da) % 2 == 1;
+            const hipStream_t ks = aside ? ps_side : hs;
+            side_chains = side_chains || aside;
+            if (cs != s) HIPX(hipStreamWaitEvent(ks, dbe, 0));
+            HIPX(hipStreamWaitEvent(ks, ce, 0));
             // the pack: fused into the one-workgroup Horner chains, or a kernel of its own
             const bool fuse = pack_wg == 2 && !pair;
             const FusedPack fp{d_interm + q0 * 2 * C, C, p2, part2_stride, d_precomp, keys, keys_stride};
@@ -1335,11 +1355,11 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
                 ;
             else if (nq == 1 ? pack_wg != 0 : pack_wg == 1)
                 HIPX(launch_pack_finalize_wg(d_interm + q0 * 2 * C, C, p2, part2_stride, d_precomp, g_lo, ng, keys,
-                                             keys_stride, packed, packed_stride, nq, nc, hs));
+                                             keys_stride, packed, packed_stride, nq, nc, ks));
             else
                 HIPX(launch_pack_finalize(d_interm + q0 * 2 * C, 2 * C, 1, C, p2, part2_stride, d_precomp, g_lo, ng,
-                                          keys, keys_stride, packed, packed_stride, nq, nc, hs));
-            horner_range(nq, out, g_lo, g_hi, hs, q0, lane, pair, fuse ? &fp : nullptr);
+                                          keys, keys_stride, packed, packed_stride, nq, nc, ks));
+            horner_range(nq, out, g_lo, g_hi, ks, q0, lane, pair, fuse ? &fp : nullptr);
         }
         if (cs != s) {  // the next batch's key digits overwrite the lane's scratch
             HIPX(hipEventRecord(prep_ev[lane], cs));
@@ -1350,6 +1370,10 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
     if (joined) {
         HIPX(hipEventRecord(horner_done[lane], hs));
         HIPX(hipStreamWaitEvent(s, horner_done[lane], 0));
+    }
+    if (side_chains) {
+        HIPX(hipEventRecord(prep_ev[lane], ps_side));
+        HIPX(hipStreamWaitEvent(s, prep_ev[lane], 0));
     }
 }
 
