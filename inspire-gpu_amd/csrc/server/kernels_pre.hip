@@ -37,32 +37,38 @@ __device__ __forceinline__ uint32_t modp(uint32_t x) {  // x mod 65535, any u32
 // index mod S = 2N/Da: y[d][k1] = x[d][k0 + S*k1], k1 < Da/2, on which
 // X^S acts as a negacyclic shift. out[m] = Da^-1 sum_d y[d] * X^(-2N d m/Da)
 // computed as a radix-2 DIT FFT (bit-reversed load, natural-order output).
-__global__ __launch_bounds__(1024) void k_encode(uint16_t* __restrict__ db, uint32_t C, uint32_t Da, uint32_t logDa,
-                                                 uint32_t KC, uint32_t nchunk, uint32_t Dinv) {
-    __shared__ uint16_t y[32768];
-    const uint32_t row = blockIdx.x, ct = blockIdx.y / nchunk, chunk = blockIdx.y % nchunk;
-    const uint32_t S = 2 * N / Da, L1 = Da / 2, E = KC * Da * L1;
-    uint16_t* base = db + (size_t)row * C + (size_t)ct * Da * N + (size_t)chunk * KC;
+// Bound: index arithmetic and LDS; every extent is a power of two, given by
+// its logarithm, and consecutive lanes take consecutive k0 (then k1), hence
+// consecutive LDS words. With divisions by the extents and k0 outermost
+// (64-byte strides between lanes) 1 GB took 3.3 ms, now 2.1. The chunks of one
+// row share cache lines: workgroup numbers 8 apart, one XCD, hold them.
+__global__ __launch_bounds__(1024) void k_encode(uint16_t* __restrict__ db, uint32_t C, uint32_t T, uint32_t lda,
+                                                 uint32_t lkc, uint32_t lch, uint32_t Dinv) {
+    __shared__ uint16_t y[32768];  // [d][k1][k0]
+    const uint32_t idx = blockIdx.x >> 3, unit = ((idx >> lch) << 3) + (blockIdx.x & 7);
+    const uint32_t row = unit / T, ct = unit % T, chunk = idx & ((1u << lch) - 1);
+    const uint32_t l1 = lda - 1, S = 2 * N >> lda, L1 = 1u << l1, lrow = l1 + lkc, E = 1u << (lda + lrow);
+    const uint32_t mk = (1u << lkc) - 1, m1 = L1 - 1;
+    uint16_t* base = db + (size_t)row * C + (((size_t)ct * N) << lda) + ((size_t)chunk << lkc);
     for (uint32_t x = threadIdx.x; x < E; x += 1024) {
-        const uint32_t k0 = x % KC, rest = x / KC, k1 = rest % L1, d = rest / L1;
-        const uint32_t dr = __builtin_bitreverse32(d) >> (32 - logDa);
-        y[(k0 * Da + dr) * L1 + k1] = base[(size_t)d * N + (size_t)S * k1 + k0];
+        const uint32_t k0 = x & mk, k1 = (x >> lkc) & m1, d = x >> lrow;
+        const uint32_t dr = __builtin_bitreverse32(d) >> (32 - lda);
+        y[(dr << lrow) + (x & ((1u << lrow) - 1))] = base[(size_t)d * N + S * k1 + k0];
     }
     __syncthreads();
     const uint32_t npairs = E / 2;
-    for (uint32_t lv = 0; lv < logDa; lv++) {
-        const uint32_t half = 1u << lv, size = half << 1;
+    for (uint32_t lv = 0; lv < lda; lv++) {
+        const uint32_t half = 1u << lv;
         uint16_t sum[16], dif[16];
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const uint32_t z = threadIdx.x + 1024 * r;
             if (z < npairs) {
-                const uint32_t k1 = z % L1, rest = z / L1, k0 = rest % KC, pidx = rest / KC;
-                const uint32_t de = (pidx / half) * size + pidx % half, dodd = de + half;
-                const uint32_t sh = (Da / size) * (pidx % half);
-                const uint32_t e = y[(k0 * Da + de) * L1 + k1];
-                const uint32_t src = k1 + sh;
-                uint32_t o = src < L1 ? y[(k0 * Da + dodd) * L1 + src] : y[(k0 * Da + dodd) * L1 + src - L1];
+                const uint32_t k0 = z & mk, k1 = (z >> lkc) & m1, pidx = z >> lrow, ph = pidx & (half - 1);
+                const uint32_t de = ((pidx >> lv) << (lv + 1)) + ph, dodd = de + half;
+                const uint32_t src = k1 + (ph << (lda - lv - 1));
+                const uint32_t e = y[(de << lrow) + (k1 << lkc) + k0];
+                uint32_t o = y[(dodd << lrow) + ((src & m1) << lkc) + k0];
                 if (src >= L1 && o) o = PMOD - o;
                 uint32_t a = e + o;
                 if (a >= PMOD) a -= PMOD;
@@ -77,86 +83,92 @@ __global__ __launch_bounds__(1024) void k_encode(uint16_t* __restrict__ db, uint
         for (int r = 0; r < 16; r++) {
             const uint32_t z = threadIdx.x + 1024 * r;
             if (z < npairs) {
-                const uint32_t k1 = z % L1, rest = z / L1, k0 = rest % KC, pidx = rest / KC;
-                const uint32_t de = (pidx / half) * size + pidx % half, dodd = de + half;
-                y[(k0 * Da + de) * L1 + k1] = sum[r];
-                y[(k0 * Da + dodd) * L1 + k1] = dif[r];
+                const uint32_t pidx = z >> lrow, in = z & ((1u << lrow) - 1);
+                const uint32_t de = ((pidx >> lv) << (lv + 1)) + (pidx & (half - 1)), dodd = de + half;
+                y[(de << lrow) + in] = sum[r];
+                y[(dodd << lrow) + in] = dif[r];
             }
         }
         __syncthreads();
     }
     for (uint32_t x = threadIdx.x; x < E; x += 1024) {
-        const uint32_t k0 = x % KC, rest = x / KC, k1 = rest % L1, d = rest / L1;
-        base[(size_t)d * N + (size_t)S * k1 + k0] = (uint16_t)modp((uint32_t)y[(k0 * Da + d) * L1 + k1] * Dinv);
+        const uint32_t k0 = x & mk, k1 = (x >> lkc) & m1, d = x >> lrow;
+        base[(size_t)d * N + S * k1 + k0] = (uint16_t)modp((uint32_t)y[x] * Dinv);
     }
 }
 
 // ------------------------------------------------------------ a-side
 // Block (group, 4 columns) over the resident DB (byte planes in 16-row
 // blocks): acc[col][c] = sum_r NTT(db[rN..rN+N-1][col]) * crs[r][c]; a32T[g][c][k][col] = N^-1 * acc[col][c][N-1-k].
-// Polynomial p = col*2 + c; team tm transforms p = tm and p = tm + 4.
-__global__ __launch_bounds__(1024) void k_aside(const uint8_t* __restrict__ db, uint32_t C, uint32_t nr, uint32_t g0,
-                                                const uint32_t* __restrict__ crs, uint32_t* __restrict__ a32T,
-                                                NttConst nc) {
-    __shared__ uint32_t buf[8][POLY_LDS];
-    __shared__ uint32_t twl[8 * N];
+// Team c of 256 lanes transforms the 4 columns mod its limb's prime in
+// registers (ntt_regs.h) and keeps 8 slots of each sum. The columns' units
+// (one per lane and plane, the next polynomial's in flight during the
+// transforms) become 16-bit values in LDS, which both teams read. Products
+// (below 23q * q < 2^58) add up in 64 bits, reduced every 32 polynomials.
+// Bound: VALU issue. With every transform through LDS and byte loads (1024
+// lanes, two polynomials per team) 1 GB took 3.7 ms, now 1.6.
+__global__ __launch_bounds__(512, 2) void k_aside(const uint8_t* __restrict__ db, uint32_t C, uint32_t nr, uint32_t g0,
+                                                  const uint32_t* __restrict__ crs, uint32_t* __restrict__ a32T,
+                                                  NttConst nc) {
+    __shared__ __align__(16) uint32_t buf[2][4][POLY4_LDS];
+    __shared__ __align__(16) nr_u32x2 tw2[2][N];
+    __shared__ __align__(16) uint16_t xin[4][N + 16];
     const uint32_t gl = blockIdx.x / (N / 4), j0 = (blockIdx.x % (N / 4)) * 4;
-    const uint32_t tid = threadIdx.x, team = tid >> 8, t = tid & 255;
-    stage_twiddles(twl, nc, tid, 1024);
-    const int c = (int)(team & 1);  // p = team + 4*rr has limb team&1
-    const Tw tw = tw_lds(twl, c);
-    const size_t col0 = (size_t)(g0 + gl) * N + j0;
-    uint32_t acc[2][8];
+    const uint32_t tid = threadIdx.x, t = tid & 255;
+    const int c = __builtin_amdgcn_readfirstlane((int)(tid >> 8));
+    const NrLimb m = nr_limb(c);
+    nr_stage_twiddles(tw2, nc, tid, 512);  // published by the first barrier below
+    const uint32_t kb = tid >> 2, col = tid & 3;  // this lane's unit
+    const u32x4* src = reinterpret_cast<const u32x4*>(db) + (size_t)kb * 2 * C + (size_t)(g0 + gl) * N + j0 + col;
+    const size_t rstep = (size_t)(N / 16) * 2 * C;
+    u32x4 lo = src[0], hi = src[C];
+    uint64_t acc[4][8];
 #pragma unroll
-    for (int rr = 0; rr < 2; rr++)
+    for (int p = 0; p < 4; p++)
 #pragma unroll
-        for (int k = 0; k < 8; k++) acc[rr][k] = 0;
+        for (int k = 0; k < 8; k++) acc[p][k] = 0;
     for (uint32_t r = 0; r < nr; r++) {
+        // the transforms' barriers below keep this behind the last reads
+        u32x4* d = reinterpret_cast<u32x4*>(&xin[col][16 * kb]);
+        u32x4 v[2];
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const uint32_t i = tid + 1024 * h;
-            const size_t row = (size_t)r * N + i;  // plane p of (row, col) at ((row/16)*2 + p)*C*16 + col*16 + row%16
-            const uint8_t* src = db + ((row >> 4) * 2 * C + col0) * 16 + (row & 15);
-#pragma unroll
-            for (int col = 0; col < 4; col++) {
-                const uint32_t x = (uint32_t)src[col * 16] | ((uint32_t)src[(size_t)C * 16 + col * 16] << 8);
-                buf[col * 2][ls(i)] = x;
-                buf[col * 2 + 1][ls(i)] = x;
-            }
+        for (int w = 0; w < 4; w++) {
+            v[w >> 1][2 * (w & 1)] = __builtin_amdgcn_perm(hi[w], lo[w], 0x05010400u);
+            v[w >> 1][2 * (w & 1) + 1] = __builtin_amdgcn_perm(hi[w], lo[w], 0x07030602u);
         }
-        __syncthreads();
-        ntt_fwd_lds(buf[team], t, tw, c);
-        ntt_fwd_lds(buf[team + 4], t, tw, c);
-#pragma unroll
-        for (int rr = 0; rr < 2; rr++) {
-            const uint32_t p = team + 4 * rr;
-            const uint32_t* A = crs + ((size_t)r * 2 + c) * N;
-#pragma unroll
-            for (int k = 0; k < 8; k++) {
-                const uint32_t e = t + 256 * k;
-                acc[rr][k] = add_mod(acc[rr][k], mul_mod(buf[p][ls(e)], A[e], c), qof(c));
-            }
+        d[0] = v[0];
+        d[1] = v[1];
+        lds_barrier();
+        if (r + 1 < nr) {
+            lo = src[(r + 1) * rstep];
+            hi = src[(r + 1) * rstep + C];
         }
-        __syncthreads();
-    }
+        const u32x4* A = reinterpret_cast<const u32x4*>(crs + ((size_t)r * 2 + c) * N + 8 * t);
+        const u32x4 a0 = A[0], a1 = A[1];
+        uint32_t x[4][8];
 #pragma unroll
-    for (int rr = 0; rr < 2; rr++) {
-        const uint32_t p = team + 4 * rr;
+        for (int p = 0; p < 4; p++)
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const uint32_t e = t + 256 * k;
-            buf[p][ls(e)] = mul_shoup(acc[rr][k], nc.inv_n[c], nc.inv_n_p[c], qof(c));
+            for (int k = 0; k < 8; k++) x[p][k] = xin[p][t + 256 * k];
+        nr_forward<4>(x, buf[c], tw2[c], t, m, [] { lds_barrier(); });
+#pragma unroll
+        for (int p = 0; p < 4; p++)
+#pragma unroll
+            for (int k = 0; k < 8; k++) acc[p][k] += (uint64_t)x[p][k] * (k < 4 ? a0[k & 3] : a1[k & 3]);
+        if ((r & 31) == 31) {
+#pragma unroll
+            for (int p = 0; p < 4; p++)
+#pragma unroll
+                for (int k = 0; k < 8; k++) acc[p][k] = red64(acc[p][k], c);
         }
     }
-    __syncthreads();
-    for (uint32_t x = tid; x < 2 * N; x += 1024) {
-        const uint32_t cc = x / N, k = x % N, e = N - 1 - k;
-        uint4 o;
-        o.x = buf[0 * 2 + cc][ls(e)];
-        o.y = buf[1 * 2 + cc][ls(e)];
-        o.z = buf[2 * 2 + cc][ls(e)];
-        o.w = buf[3 * 2 + cc][ls(e)];
-        *reinterpret_cast<uint4*>(a32T + (((size_t)gl * 2 + cc) * N + k) * N + j0) = o;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        uint32_t o[4];
+#pragma unroll
+        for (int p = 0; p < 4; p++) o[p] = mul_shoup(red64(acc[p][k], c), nc.inv_n[c], nc.inv_n_p[c], m.q);
+        *reinterpret_cast<u32x4*>(a32T + (((size_t)gl * 2 + c) * N + (N - 1 - (8 * t + k))) * N + j0) =
+            u32x4{o[0], o[1], o[2], o[3]};
     }
 }
 
@@ -364,24 +376,24 @@ __global__ __launch_bounds__(1024) void k_collapse_final(const uint32_t* __restr
 
 hipError_t launch_encode(uint16_t* db, size_t R, size_t C, size_t Da, hipStream_t s) {
     if (Da <= 1) return hipSuccess;
-    uint32_t logDa = 0;
-    while ((1u << logDa) < Da) logDa++;
-    const uint32_t S = (uint32_t)(2 * N / Da), L1 = (uint32_t)(Da / 2);
-    uint32_t KC = 32768u / ((uint32_t)Da * L1);
-    if (KC > S) KC = S;
-    const uint32_t nchunk = S / KC;
+    uint32_t lda = 0, lkc = 0, lch = 0;
+    while ((1u << lda) < Da) lda++;
+    const size_t S = 2 * N / Da, T = C / (Da * N);
+    // a chunk's Da x Da/2 x KC values fill the LDS, or KC is all of S
+    while ((Da * Da / 2 << (lkc + 1)) <= 32768 && ((size_t)2 << lkc) <= S) lkc++;
+    while (((size_t)1 << (lkc + lch)) < S) lch++;
+    if ((Da & (Da - 1)) || Da > 256 || R * T % 8 || (R * T << lch) > 0x7fffffffu) return hipErrorInvalidValue;
     uint32_t Dinv = 0;  // Da^-1 mod 65535 (Da a power of two, odd modulus)
     for (uint32_t x = 1; x < PMOD; x++)
         if ((uint64_t)x * Da % PMOD == 1) { Dinv = x; break; }
-    const size_t T = C / (Da * N);
-    hipLaunchKernelGGL(k_encode, dim3((unsigned)R, (unsigned)(T * nchunk)), dim3(1024), 0, s, db, (uint32_t)C,
-                       (uint32_t)Da, logDa, KC, nchunk, Dinv);
+    hipLaunchKernelGGL(k_encode, dim3((unsigned)(R * T << lch)), dim3(1024), 0, s, db, (uint32_t)C, (uint32_t)T, lda,
+                       lkc, lch, Dinv);
     return hipGetLastError();
 }
 
 hipError_t launch_aside(const uint8_t* db, size_t R, size_t C, size_t g0, size_t ng, const uint32_t* crs,
                         uint32_t* a32T, const NttConst& nc, hipStream_t s) {
-    hipLaunchKernelGGL(k_aside, dim3((unsigned)(ng * (N / 4))), dim3(1024), 0, s, db, (uint32_t)C,
+    hipLaunchKernelGGL(k_aside, dim3((unsigned)(ng * (N / 4))), dim3(512), 0, s, db, (uint32_t)C,
                        (uint32_t)(R / N), (uint32_t)g0, crs, a32T, nc);
     return hipGetLastError();
 }

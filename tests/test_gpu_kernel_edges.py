@@ -250,3 +250,22 @@ def test_staged_batches_whose_keys_follow_the_pass(groups, shape):
         out.free()
     finally:
         srv.close()
+
+
+@pytest.mark.parametrize("groups,rows", [(2, 2048), (4, 2048), (16, 2048), (32, 2048), (64, 2048), (1, 34 * 2048)])
+def test_preprocessing_of_every_group_count_extracts(groups, rows):
+    """The encode's power-of-two extents (2..64 groups of interpolation
+    points) and a-side sums of 1 and of 34 polynomials (past the 32 between
+    reductions): first, middle and last entry extract."""
+    n, w = groups * rows * N // 64, 120
+    rc, geo = ol.setup(n, w, rows)
+    assert rc == 0 and geo["G"] == groups
+    db = np.random.default_rng(groups).integers(0, ol.P, size=(geo["R"], geo["C"]), dtype=np.uint16)
+    srv = ia.Server(db, n, w, rows, max_batch=1, crs_seed=bytes(SEED))
+    try:
+        for k, idx in enumerate((0, n // 2 + 1, n - 1)):
+            q, st = ol.make_query(geo, SEED, idx, 50 + k)
+            got = ol.extract(geo, st, srv.answer_batch([q])[0].reshape(geo["T"], -1))
+            assert np.array_equal(got, ol.expected_slots(geo, db, idx)), f"entry {idx}"
+    finally:
+        srv.close()
