@@ -298,8 +298,14 @@ DbPlan narrow_plan(const DbPlan& full, size_t target, size_t R, size_t C, size_t
 }  // namespace
 
 // Tables (with their tensors) up to this size run the pass and the collapse
-// of up to 8 queries in one launch.
-constexpr size_t kMergeBytes = (size_t)1 << 30;
+// in one launch: up to 4 queries, and 5..8, whose pass tiles take all the
+// registers of two workgroups per CU, so that the collapse's share of the
+// launch runs at their occupancy. Two launches and one, whole answers of 1, 3
+// and 8 queries: 0.07 GB 32.9 / 30.0, 39.0 / 35.0, 41.9 / 34.7 us; 0.19 GB
+// 52.6 / 49.6, 71.5 / 65.8, 67.6 / 63.4; 0.39 GB 93.4 / 89.4, 99.4 / 91.0,
+// 105 / 110; 0.77 GB 166 / 152, 167 / 161, 169 / 200; 1.5 GB 296 / 301,
+// 301 / 300, 308 / 385.
+constexpr size_t merge_bytes(size_t nq) { return (size_t)1 << (nq <= 4 ? 30 : 28); }
 
 size_t default_group_chunk(size_t G) {
     // group chunks of the pipelined answer: about 8, of at least 8 groups
@@ -1246,8 +1252,8 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             const DbPlan p = serial_plan(nq);
             if (q0 == slot0) last_part_slices = p.slices > 1 ? p.slices : 0;
             // up to 8 queries over a small table: the pass and the collapse in
-            // one launch (kMergeBytes)
-            const bool both = pass_collapse_ok(p, nq) && pp.db_rows * C * 2 + G * PC_GROUP * 4 <= kMergeBytes;
+            // one launch (merge_bytes)
+            const bool both = pass_collapse_ok(p, nq) && pp.db_rows * C * 2 + G * PC_GROUP * 4 <= merge_bytes(nq);
             z.part2 = (both ? pass_collapse_ksplit(nq, G) : collapse_row_slices(nq, G, collapse_variant)) > 1;
             z.pair = pair;
             if (in.late) {
