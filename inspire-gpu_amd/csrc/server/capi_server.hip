@@ -372,7 +372,7 @@ int ipir_dbg_tuning(const ipir_server* srv, char* out, size_t cap) {
     if (c->G / c->gchunk > 1)
         s += "; chunks of " + std::to_string(c->gchunk) + " groups: batch1 " + plan(c->chunk_plan(1, c->gchunk * ipx::N)) +
              ", batch" + std::to_string(nq) + " " + plan(c->chunk_plan(nq, c->gchunk * ipx::N));
-    if (c->chunks.size() > c->G / c->gchunk) {
+    if (c->layout.chunks.size() > c->G / c->gchunk) {
         s += c->tail_split ? " (lowest split in 1/2, 1/4, 1/4" : " (";
         s += c->head_split ? std::string(c->tail_split ? "; " : "") + "highest split in 1/4, 1/4, 1/2)" : ")";
     }

@@ -845,39 +845,7 @@ DbPlan GpuServerCtx::plan_for(size_t nq, size_t ncols) const {
 }
 
 void GpuServerCtx::set_chunks() {
-    // The chunks of every response ciphertext's chain, highest first, taken
-    // in turns where chunks end with the ciphertexts: the chains of several
-    // then advance side by side, and only a chunk's steps of each are left
-    // after the last pass.
-    chunks.clear();
-    const bool turns = T > 1 && G % T == 0 && G / T == Da && Da % gchunk == 0;
-    const size_t nct = turns ? T : 1, per = G / nct, n = per / gchunk, h = gchunk / 2, q = gchunk / 4;
-    const bool quarters = G > gchunk && gchunk % 4 == 0;
-    std::vector<std::vector<std::pair<size_t, size_t>>> lists(nct);
-    for (size_t ct = 0; ct < nct; ct++)
-        for (size_t k = n; k-- > 0;) {
-            const size_t lo = ct * per + k * gchunk, hi = lo + gchunk;
-            auto& l = lists[ct];
-            if (quarters && head_split && hi == G) {
-                l.push_back({hi - q, hi});
-                l.push_back({hi - h, hi - q});
-                l.push_back({lo, hi - h});
-            } else if (quarters && tail_split && lo == 0) {
-                l.push_back({lo + h, hi});
-                l.push_back({lo + q, lo + h});
-                l.push_back({lo, lo + q});
-            } else {
-                l.push_back({lo, hi});
-            }
-        }
-    for (size_t r = 0, left = nct; left; r++) {
-        left = 0;
-        for (size_t ct = nct; ct-- > 0;)
-            if (r < lists[ct].size()) {
-                chunks.push_back(lists[ct][r]);
-                left++;
-            }
-    }
+    layout = layout_chunks(G, T, Da, gchunk, head_split, tail_split);
 }
 
 // The chunk plan over ncols (<= gchunk N) columns: a timed slice count sets
@@ -1321,7 +1289,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             HIPX(launch_collapse(d_precomp, G, d_kdig[lane], d_KS[lane], nq, p2, part2_stride, s, collapse_variant));
         }
         auto collapse_chunk = [&](size_t k) {
-            const size_t g_lo = chunks[k].first, ng = chunks[k].second - g_lo;
+            const size_t g_lo = layout.chunks[k].first, ng = layout.chunks[k].second - g_lo;
             HIPX(launch_collapse(d_precomp + g_lo * PC_GROUP, ng, d_kdig[lane], d_KS[lane], nq, p2 + g_lo * 2 * N,
                                  part2_stride, cs, collapse_variant));
             HIPX(hipEventRecord(coll_ev[lane][k % kChunkEvents], cs));
@@ -1330,8 +1298,8 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             collapse_chunk(0);
             HIPX(hipStreamWaitEvent(s, coll_ev[lane][0], 0));
         }
-        for (size_t k = 0; k < chunks.size(); k++) {
-            const size_t g_lo = chunks[k].first, g_hi = chunks[k].second, ng = g_hi - g_lo;
+        for (size_t k = 0; k < layout.chunks.size(); k++) {
+            const size_t g_lo = layout.chunks[k].first, g_hi = layout.chunks[k].second, ng = g_hi - g_lo;
             TraceRange trk("chunk %zu: groups %zu..%zu (DB pass, collapse, pack, Horner)", k, g_lo, g_hi - 1);
             hipEvent_t dbe = chunk_ev[lane][k % kChunkEvents], ce = coll_ev[lane][k % kChunkEvents];
             mark_pass(s, k == 0);
@@ -1341,7 +1309,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             // event record costs the stream a few microseconds of idle)
             if (cs != s) HIPX(hipEventRecord(dbe, s));
             if (ahead) {
-                if (k + 1 < chunks.size()) collapse_chunk(k + 1);  // ce of chunk k was recorded a chunk earlier
+                if (k + 1 < layout.chunks.size()) collapse_chunk(k + 1);  // ce of chunk k was recorded a chunk earlier
             } else {
                 if (!first)
                     HIPX(launch_collapse(d_precomp + g_lo * PC_GROUP, ng, d_kdig[lane], d_KS[lane], nq,
@@ -1349,7 +1317,8 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
                 HIPX(hipEventRecord(ce, cs));
             }
             // with the side stream free, every other ciphertext's chains run on it
-            const bool aside = cs == s && (T - 1 - g_lo / Da) % 2 == 1;
+            // (chunks of one ciphertext each: ChunkLayout)
+            const bool aside = cs == s && layout.aside(k);
             const hipStream_t ks = aside ? ps_side : hs;
             side_chains = side_chains || aside;
             if (cs != s) HIPX(hipStreamWaitEvent(ks, dbe, 0));

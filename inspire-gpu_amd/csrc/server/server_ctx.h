@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "capi.h"
+#include "chunks.h"
 #include "gpu_protocol.h"
 #include "host_stage.h"
 #include "kernels.h"
@@ -97,13 +98,13 @@ struct GpuServerCtx {
     ipx::DbPlan chunk_plan_at(size_t nq, size_t k, size_t ng, const ipx::DbPlan& whole) const;
     int collapse_variant = 0;       // 17..32-query collapse pass form (launch_collapse)
     size_t gchunk = 0;              // groups per chunk of the pipelined answer
-    // the pipelined answer's chunks [lo, hi), highest groups first (of several
-    // response ciphertexts in turns): chunks of gchunk groups, the lowest one split into gchunk/2, /4, /4 when
+    // the pipelined answer's chunks: of gchunk groups, the lowest one split
+    // into gchunk/2, /4, /4 when
     // tail_split (its Horner steps are the ones left after every pass), the
     // highest one into gchunk/4, /4, /2 when head_split (the chains start
     // after a quarter chunk's passes)
     bool tail_split = true, head_split = false;
-    std::vector<std::pair<size_t, size_t>> chunks;
+    ChunkLayout layout;
     void set_chunks();
     // pipeline shape of one-query and many-query calls: 0 serial on the
     // caller's stream, 2 Horner chains beside the passes, 3 collapse beside
