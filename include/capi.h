@@ -111,16 +111,15 @@ ipir_client_query* ipir_query_build_seeded(const ipir_params* params, uint64_t i
  * memory (count * ipir_query_u64s u64s), writing the flat responses to
  * DEVICE memory, on the given HIP stream (NULL = the server's own stream).
  * Asynchronous: returns after enqueueing. Return codes as
- * ipir_answer_batch (4 only for launch failures: the answer's kernels
- * report nothing afterwards). The work waits for the server's previous
- * call if that one was on another stream; inside a caller's stream capture
- * the caller orders the captured work itself. For callers that keep
- * queries resident in HBM. Answers may run their Horner chains beside a
+ * ipir_answer_batch (4 only for launch failures). The work waits for the
+ * server's previous call if that one was on another stream; inside a caller's
+ * stream capture the caller orders the captured work itself. For callers that
+ * keep queries resident in HBM. Answers may run their Horner chains beside a
  * database pass they wait for inside the kernel, or as two workgroups that
  * wait for each other; such a wait is bounded (about a second or more), and
- * a chain that gives up writes all-ones words as its response (no residue
- * has that value; it can happen only if the pass or the other workgroup gets
- * no CU for that long) and is reported by ipir_device_status. */
+ * an answer in which one ends at its bound (the pass or the other workgroup
+ * got no CU for that long) has its chains made again, without waits, before
+ * the stream goes on. */
 int ipir_answer_batch_device(ipir_server* srv, const uint64_t* d_queries, size_t count,
                              uint64_t* d_out_resp, void* hip_stream);
 
@@ -134,16 +133,16 @@ int ipir_answer_batch_device(ipir_server* srv, const uint64_t* d_queries, size_t
 int ipir_answer_batch_packed(ipir_server* srv, const uint8_t* packed_queries, size_t count,
                              uint8_t* out_compressed);
 /* The same over DEVICE buffers, asynchronous on the given HIP stream (NULL
- * = the server's own stream), like ipir_answer_batch_device (a chain that
- * gives up its bounded wait leaves its compressed response undefined). */
+ * = the server's own stream), like ipir_answer_batch_device. */
 int ipir_answer_batch_packed_device(ipir_server* srv, const uint8_t* d_packed_queries, size_t count,
                                     uint8_t* d_out_compressed, void* hip_stream);
 
 /* For callers of the asynchronous entry points (no counterpart in the
- * reference): waits for the server's last call and returns 4 if a Horner
- * chain of an asynchronous call gave up a bounded wait since the last
- * blocking call or status query (those responses are invalid), else 0;
- * then clears the report. 5 while a serving loop owns the server. */
+ * reference): waits for the server's last call and returns 4 if responses of
+ * an asynchronous call since the last blocking call or status query are
+ * invalid (a Horner chain gave up its wait where the wait bound was set to
+ * zero, inspire_debug.h), else 0; then clears the report. 5 while a serving
+ * loop owns the server. */
 int ipir_device_status(ipir_server* srv);
 
 /* Device memory of a server of this geometry (setup()'s rules; 1 if it

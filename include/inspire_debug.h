@@ -94,19 +94,24 @@ int ipir_dbg_set_tail_split(ipir_server* srv, int on);
 /* Select the Horner kernel a server's answers use: mode as variant above,
  * or -1 (the default): pairs for up to 128 chains at once. With mode 1 the
  * asynchronous device entry points (ipir_answer_batch_device,
- * ipir_answer_batch_packed_device) use one workgroup per chain; pairs
- * chosen by the default report there as streamed chains do
- * (ipir_device_status). */
+ * ipir_answer_batch_packed_device) use one workgroup per chain. */
 int ipir_dbg_set_horner(ipir_server* srv, int mode);
-/* Bound of the pair kernel's partner wait, in loads (default 2^21, ~2 s).
+/* Bound of the pair kernel's partner wait, in loads (default 2^21, ~2 s); an
+ * answer in which a wait ends at its bound is made again at its end.
  * 0 makes every pair chain report the bound exceeded at its first
- * exchange and stop (all kernels still end normally): the call that ran it
- * then returns 4, and later calls are unaffected. 5 while a loop runs. */
+ * exchange and stop (all kernels still end normally), and nothing is made
+ * again: the response is all-ones words, the call that ran it returns 4 (the
+ * asynchronous ones report it through ipir_device_status), and later calls
+ * are unaffected. 5 while a loop runs. */
 int ipir_dbg_set_horner_spin_limit(ipir_server* srv, uint32_t limit);
 /* The same bound for Horner chains waiting for a streamed database pass's
  * groups (default 2^23; 0: give up at once and report, as above; the pass
  * itself runs to its end). */
 int ipir_dbg_set_stream_spin_limit(ipir_server* srv, uint32_t limit);
+/* 1 if chains of an answer were made again since the last call because a
+ * wait inside a kernel ended at its bound, else 0 (-1: no server). Read it
+ * once the answers in question are complete. */
+int ipir_dbg_chains_redone(ipir_server* srv);
 /* Keep a serving loop's partitions busy after their device work finished
  * (on = 1) until released (on = 0): requests admitted meanwhile go to the
  * other partitions or wait. For tests of admission while batches are in

@@ -840,6 +840,11 @@ int ipir_dbg_set_stream_spin_limit(ipir_server* srv, uint32_t limit) {
     return 0;
 }
 
+int ipir_dbg_chains_redone(ipir_server* srv) {
+    if (!srv) return -1;
+    return (int)__atomic_exchange_n(srv->ctx->h_status + GpuServerCtx::kLanes, 0u, __ATOMIC_RELAXED);
+}
+
 int ipir_dbg_horner_variant(const uint64_t* cts, size_t L, const uint64_t* rgsw, uint64_t* out, int variant) {
     if (!cts || !rgsw || !out || L == 0 || variant < 0 || variant > 1) return 1;
     Standalone* st = standalone();
@@ -905,7 +910,10 @@ int ipir_dbg_profile_batch(ipir_server* srv, const uint64_t* d_queries, size_t c
             const ipx::DbPlan p = c->serial_plan(nq);
             mark();
             GpuServerCtx::PrepZero z;
-            if (q0 == 0) z.status = c->h_status;
+            if (q0 == 0) {
+                z.status = c->h_status;
+                z.gave_up = c->d_gave_up;
+            }
             z.pair = c->use_pair(count, true);
             c->prep_query(c->d_q + q0 * c->qlen, q0, nq, p, s, 0, z);
             mark();
@@ -919,6 +927,7 @@ int ipir_dbg_profile_batch(ipir_server* srv, const uint64_t* d_queries, size_t c
         mark();
         c->horner_range(count, d_out, 0, c->G, s, 0, 0, c->use_pair(count, true));
         mark();
+        if (c->use_pair(count, true) && c->horner_spin_limit) c->horner_again(count, d_out, s, 0, 0);
         c->order_after(s);
         hip_check(hipEventSynchronize(ev[k - 1]), "sync");
         c->check_status(0);

@@ -109,7 +109,7 @@ struct PrepArgs {
     uint32_t* KS = nullptr;
     uint32_t* zero = nullptr;     // zero_words words set to zero (hand-over flags)
     uint32_t zero_words = 0;
-    uint32_t* status = nullptr;   // a word set to zero
+    uint32_t *status = nullptr, *gave_up = nullptr;  // words set to zero
     uint32_t* part2 = nullptr;    // part2_words (a multiple of 4096) words per query set to zero
     size_t part2_stride = 0, part2_words = 0;
     uint32_t* xbuf = nullptr;     // xbuf_words words per query, queries back to back, set to zero (with keys)
@@ -270,6 +270,13 @@ struct PackStream {
     uint32_t spin_limit = 0;
     uint32_t* status = nullptr;
     uint32_t queries = kPackQueries;  // queries per workgroup
+    const uint32_t* only_if = nullptr;  // set: the launch does nothing while this word is zero
+};
+// A launch that makes chains again: it does nothing while *only_if is zero,
+// else it sets *redone.
+struct HornerAgain {
+    const uint32_t* only_if = nullptr;
+    uint32_t* redone = nullptr;
 };
 hipError_t launch_pack_stream(const PackStream& ps, const uint32_t* part2, size_t part2_stride,
                               const uint32_t* precomp, const uint32_t* keys, size_t keys_stride, uint32_t* packed_b,
@@ -278,7 +285,7 @@ hipError_t launch_horner(const uint32_t* pa_base, size_t pa_stride, size_t G, si
                          uint32_t* packed_b, size_t packed_stride, const uint32_t* rgsw, size_t rgsw_stride,
                          uint64_t* out, uint32_t* hstate, size_t g_lo, size_t g_hi, size_t nq, const NttConst& nc,
                          const CrtConst& cc, hipStream_t s, const FusedPack& pack = FusedPack{},
-                         const StreamWait& wait = StreamWait{});
+                         const StreamWait& wait = StreamWait{}, const HornerAgain& again = HornerAgain{});
 
 // The same chains with two workgroups per chain (one per limb) exchanging
 // shares of the CRT lift once per step through xbuf,

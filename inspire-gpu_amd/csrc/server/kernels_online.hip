@@ -259,6 +259,7 @@ struct HornerChain {
     uint64_t* out;
     uint32_t* hstate;
     uint32_t g_lo, g_hi;
+    HornerAgain again;
 };
 
 template <bool STREAMED>
@@ -269,6 +270,10 @@ __global__ __launch_bounds__(512, 2) void k_horner(HornerChain h, NttConst nc, N
     __shared__ uint32_t dx[2][8][2][256];  // digits by the team that made them: [4a + .., 4b + ..][d1, d2][lane]
     __shared__ uint32_t sw_abort;
     const uint32_t ct = blockIdx.x, qi = blockIdx.y, tid = threadIdx.x, t = tid & 255;
+    if (!STREAMED && h.again.only_if) {
+        if (*h.again.only_if == 0) return;
+        if (tid == 0) *h.again.redone = 1;
+    }
     const int c = __builtin_amdgcn_readfirstlane((int)(tid >> 8));  // this team's limb
     const uint32_t start = ct * h.Da;
     const uint32_t L = (h.G - start) < h.Da ? (h.G - start) : h.Da;
@@ -506,6 +511,7 @@ __global__ __launch_bounds__(1024) void k_pack_stream(PackStream ps, const uint3
     __shared__ __align__(16) nr_u32x2 tw2[2][N];
     __shared__ uint32_t abort_flag;
     const uint32_t tid = threadIdx.x, t = tid & 255, blk = blockIdx.x;
+    if (ps.only_if && *ps.only_if == 0) return;
     const uint32_t team = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 8));
     const uint32_t q0 = blk * ps.queries;
     const uint32_t nqb = nq - q0 < ps.queries ? nq - q0 : ps.queries;
@@ -674,11 +680,13 @@ hipError_t launch_pack_stream(const PackStream& ps, const uint32_t* part2, size_
 hipError_t launch_horner(const uint32_t* pa_base, size_t pa_stride, size_t G, size_t Da, size_t T,
                          uint32_t* packed_b, size_t packed_stride, const uint32_t* rgsw, size_t rgsw_stride,
                          uint64_t* out, uint32_t* hstate, size_t g_lo, size_t g_hi, size_t nq, const NttConst& nc,
-                         const CrtConst& cc, hipStream_t s, const FusedPack& pack, const StreamWait& wait) {
+                         const CrtConst& cc, hipStream_t s, const FusedPack& pack, const StreamWait& wait,
+                         const HornerAgain& again) {
     if (nq == 0 || g_lo >= g_hi) return hipSuccess;
     if (wait.done && (!wait.status || wait.queries == 0)) return hipErrorInvalidValue;
+    if (again.only_if && (!again.redone || wait.done || pack.interm)) return hipErrorInvalidValue;
     const HornerChain h{pa_base, pa_stride, (uint32_t)G, (uint32_t)Da, (uint32_t)T, packed_b, packed_stride,
-                        rgsw, rgsw_stride, out, hstate, (uint32_t)g_lo, (uint32_t)g_hi};
+                        rgsw, rgsw_stride, out, hstate, (uint32_t)g_lo, (uint32_t)g_hi, again};
     const NrGadget gc = nr_gadget_const(nc, cc);
     const dim3 grid((unsigned)T, (unsigned)nq);
     if (wait.done)

@@ -74,6 +74,7 @@ __global__ __launch_bounds__(256) void k_prep(PrepArgs a, NttConst nc) {
     if (b == 0 && qi == 0) {  // with the first query
         for (uint32_t x = t; x < a.zero_words; x += 256) a.zero[x] = 0;
         if (a.status && t == 0) *a.status = 0;
+        if (a.gave_up && t == 0) *a.gave_up = 0;
     }
     if (b < a.key_blocks) {
         // key polynomial b = key*4 + digit*2 + limb

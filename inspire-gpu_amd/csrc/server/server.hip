@@ -346,7 +346,7 @@ ServerFootprint server_footprint(const PublicParams& pp, size_t gchunk) {
                  T * 4 * N * 4;
     f.fixed = R * C * 2 + G * PC_GROUP * 4 + 8 * N * 4 +
               GpuServerCtx::kLanes *
-                  (R * 256 + GpuServerCtx::kKdigBytes + (GpuServerCtx::kSumWords + GpuServerCtx::kKeySumWords) * 4);
+                  (R * 256 + GpuServerCtx::kKdigBytes + (GpuServerCtx::kSumWords + GpuServerCtx::kKeySumWords + 1) * 4);
     // streamed answers' flags: one set per lane and 32 slots (rounded up)
     const size_t set_bytes = GpuServerCtx::kStreamSetWords * G * 4;
     f.fixed += GpuServerCtx::kLanes * set_bytes;
@@ -429,8 +429,10 @@ void GpuServerCtx::alloc_slots() {
     const char* se = std::getenv("INSPIRE_STREAM");
     stream_ok = !(se && se[0] == '0');
     d_hxbuf = dalloc<uint32_t>(horner_pair_xbuf_words(B * T));
-    HIPX(hipHostMalloc((void**)&h_status, kLanes * 4, hipHostMallocDefault));
-    for (int l = 0; l < kLanes; l++) h_status[l] = 0;
+    d_gave_up = dalloc<uint32_t>(kLanes);
+    HIPX(hipMemset(d_gave_up, 0, kLanes * 4));
+    HIPX(hipHostMalloc((void**)&h_status, (kLanes + 1) * 4, hipHostMallocDefault));
+    for (int l = 0; l <= kLanes; l++) h_status[l] = 0;
     horner_spin_limit = kHornerSpinLimit;
     stream_spin_limit = kStreamSpinLimit;
     HIPX(hipEventCreateWithFlags(&order_ev, hipEventDisableTiming));
@@ -829,6 +831,7 @@ void GpuServerCtx::prep_query(const QueryInput& in, size_t q0, size_t nq, const 
     a.xbuf = d_hxbuf + horner_pair_xbuf_words(q0 * T);
     a.xbuf_words = z.pair ? horner_pair_xbuf_words(T) : 0;
     a.status = z.status;
+    a.gave_up = z.gave_up;
     if (in.late)
         HIPX(launch_prep(a, nq, p, nc, s));
     else
@@ -1017,12 +1020,21 @@ void GpuServerCtx::horner_range(size_t count, uint64_t* d_out, size_t g_lo, size
         HIPX(launch_horner_pair(d_precomp + PC_A, PC_GROUP, G, Da, T, d_packed_b + slot0 * packed_stride,
                                 packed_stride, d_rgsw + slot0 * rgsw_stride, rgsw_stride, d_out,
                                 d_hstate + slot0 * T * 4 * N, g_lo, g_hi, count,
-                                d_hxbuf + horner_pair_xbuf_words(slot0 * T), h_status + lane, horner_spin_limit, nc,
-                                cc, s));
+                                d_hxbuf + horner_pair_xbuf_words(slot0 * T), wait_status(lane, horner_spin_limit),
+                                horner_spin_limit, nc, cc, s));
     else
         HIPX(launch_horner(d_precomp + PC_A, PC_GROUP, G, Da, T, d_packed_b + slot0 * packed_stride, packed_stride,
                            d_rgsw + slot0 * rgsw_stride, rgsw_stride, d_out, d_hstate + slot0 * T * 4 * N, g_lo, g_hi,
                            count, nc, cc, s, fp ? *fp : FusedPack{}));
+}
+
+void GpuServerCtx::horner_again(size_t count, uint64_t* d_out, hipStream_t s, size_t slot0, int lane) {
+    HornerAgain again;
+    again.only_if = d_gave_up + lane;
+    again.redone = h_status + kLanes;
+    HIPX(launch_horner(d_precomp + PC_A, PC_GROUP, G, Da, T, d_packed_b + slot0 * packed_stride, packed_stride,
+                       d_rgsw + slot0 * rgsw_stride, rgsw_stride, d_out, d_hstate + slot0 * T * 4 * N, 0, G, count,
+                       nc, cc, s, FusedPack{}, StreamWait{}, again));
 }
 
 int GpuServerCtx::shape_for(size_t nq) const {
@@ -1092,9 +1104,22 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
     // device (at 128 GB, 4 x 128 chains in two rounds over the 256 CUs
     // instead of four rounds over 128). Contiguous slots [defer_lo, +defer_n).
     size_t defer_lo = 0, defer_n = 0;
+    // The answer's last launches: sub-batches whose chains wait inside their
+    // kernels are made again where a wait ended at its bound (d_gave_up), so
+    // that bound is no limit to what the device may run beside an answer. A
+    // launch that finds the word at zero takes 2 to 3 us (1 GB, one query 297.5 to
+    // 299.2, 32 queries 370.8 to 374.2; pairs still pay from one step on: two
+    // groups 91.0 single, 87.7 in pairs).
+    std::vector<std::function<void()>> again;
+    auto chains_again = [&](size_t q0, size_t nq) {
+        if (pair && horner_spin_limit)
+            again.push_back([=] { horner_again(nq, d_out + (q0 - slot0) * resp_u64s, s, q0, lane); });
+    };
     auto flush_deferred = [&]() {
-        if (defer_n)
+        if (defer_n) {
             horner_range(defer_n, d_out + (defer_lo - slot0) * resp_u64s, 0, G, s, defer_lo, lane, pair);
+            chains_again(defer_lo, defer_n);
+        }
         defer_n = 0;
     };
     for (size_t q0 = slot0; q0 < slot0 + count; q0 += kMfmaMaxQueries) {
@@ -1107,6 +1132,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
         const QueryInput in = input.at(q0 - slot0, qlen);
         PrepZero z;
         if (status_read && q0 == slot0) z.status = h_status + lane;  // an earlier call's report is not this one's
+        if (q0 == slot0) z.gave_up = d_gave_up + lane;
         DbPlan sp;
         if (shape >= 6) {
             sp = stream_plan(nq, nq == 1 ? stream_slices1 : stream_slices, shape == 8);
@@ -1197,7 +1223,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             pk.pass_target = fused ? pass_collapse_target(sp, nq, G) : (uint32_t)(N / dbplan_cols(sp) * sp.slices);
             pk.packed_done = packed_done;
             pk.spin_limit = stream_spin_limit;
-            pk.status = h_status + lane;
+            pk.status = wait_status(lane, stream_spin_limit);
             pk.queries = pq;
             HIPX(launch_pack_stream(pk, p2, part2_stride, d_precomp, keys, keys_stride, packed, packed_stride, G, nq,
                                     nc, ps_s));
@@ -1208,12 +1234,20 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             sw.queries = pq;
             sw.stride = (uint32_t)G;
             sw.spin_limit = stream_spin_limit;
-            sw.status = h_status + lane;
+            sw.status = wait_status(lane, stream_spin_limit);
             HIPX(launch_horner(d_precomp + PC_A, PC_GROUP, G, Da, T, packed, packed_stride, d_rgsw + q0 * rgsw_stride,
                                rgsw_stride, out, d_hstate + q0 * T * 4 * N, 0, G, nq, nc, cc, hs, FusedPack{}, sw));
             // the next sub-batch's key digits and flags wait for the collapse and the pack
             HIPX(hipEventRecord(prep_ev[lane], ps_s));
             HIPX(hipStreamWaitEvent(s, prep_ev[lane], 0));
+            if (stream_spin_limit)
+                again.push_back([=] {  // the pass and its counters are complete by then
+                    PackStream pa = pk;
+                    pa.only_if = d_gave_up + lane;
+                    HIPX(launch_pack_stream(pa, p2, part2_stride, d_precomp, keys, keys_stride, packed,
+                                            packed_stride, G, nq, nc, s));
+                    horner_again(nq, out, s, q0, lane);
+                });
             continue;
         }
         if (shape == 0) {
@@ -1336,6 +1370,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
                                           keys, keys_stride, packed, packed_stride, nq, nc, ks));
             horner_range(nq, out, g_lo, g_hi, ks, q0, lane, pair, fuse ? &fp : nullptr);
         }
+        chains_again(q0, nq);
         if (cs != s) {  // the next batch's key digits overwrite the lane's scratch
             HIPX(hipEventRecord(prep_ev[lane], cs));
             HIPX(hipStreamWaitEvent(s, prep_ev[lane], 0));
@@ -1350,6 +1385,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
         HIPX(hipEventRecord(prep_ev[lane], ps_side));
         HIPX(hipStreamWaitEvent(s, prep_ev[lane], 0));
     }
+    for (const auto& f : again) f();
 }
 
 void GpuServerCtx::run_step(const void* in, void* out, size_t count, size_t slot0, int lane, int packed,
@@ -1501,8 +1537,7 @@ void GpuServerCtx::check_status(int lane) {
     if (!__atomic_load_n(h_status + lane, __ATOMIC_RELAXED)) return;
     h_status[lane] = 0;
     throw std::runtime_error(
-        "a Horner chain exceeded its wait bound (pair exchange or streamed database pass); responses of this call "
-        "are invalid");
+        "a Horner chain gave up its wait (bound set to zero); responses of this call are invalid");
 }
 
 void GpuServerCtx::order_before(hipStream_t s) {
@@ -1655,7 +1690,7 @@ void gpu_free_server(GpuServerCtx* ctx) {
     dfree(ctx->d_tw); dfree(ctx->d_db); dfree(ctx->d_precomp);
     dfree(ctx->d_q); dfree(ctx->d_resp); dfree(ctx->d_bq); dfree(ctx->d_keys); dfree(ctx->d_rgsw);
     dfree(ctx->d_part); dfree(ctx->d_interm); dfree(ctx->d_part2); dfree(ctx->d_packed_b);
-    dfree(ctx->d_hxbuf); dfree(ctx->d_hstate);
+    dfree(ctx->d_hxbuf); dfree(ctx->d_hstate); dfree(ctx->d_gave_up);
     for (auto& f : ctx->d_sflags) dfree(f);
     dfree(ctx->d_cmp);
     for (int l = 0; l < GpuServerCtx::kLanes; l++) {

@@ -197,11 +197,17 @@ struct GpuServerCtx {
     // the Horner chains' own workgroups (where the one-workgroup Horner runs)
     int pack_wg = 0;
     uint32_t* d_hxbuf = nullptr;    // pair exchange buffers [B*T chains]
-    // per scratch lane: nonzero once a pair chain of that lane's calls gave
-    // up its bounded wait (read and cleared by check_status)
-    // (pinned host memory the kernels write: reading it after the call costs
-    // no copy; a call whose status is read zeroes it in its first kernel)
-    uint32_t* h_status = nullptr;   // [kLanes]
+    // Waits inside a kernel (a pair chain's for its partner, a streamed pack's
+    // or chain's for its pass) are bounded. Per scratch lane, d_gave_up is
+    // zeroed by an answer's first kernel and set by a wait that ends at its
+    // bound; the answer's last launches make its waiting sub-batches again,
+    // without waits, where it is set, and set h_status[kLanes] (pinned host
+    // memory). With a bound of zero (chains that end at once, for tests)
+    // nothing is made again, the report goes to h_status[lane], and
+    // check_status reads and clears it.
+    uint32_t* d_gave_up = nullptr;  // [kLanes]
+    uint32_t* h_status = nullptr;   // [kLanes + 1]
+    uint32_t* wait_status(int lane, uint32_t limit) const { return limit ? d_gave_up + lane : h_status + lane; }
     uint32_t horner_spin_limit = 0; // the pair kernel's wait bound in loads (0: report at once)
     uint32_t stream_spin_limit = 0; // the same for chains waiting for a streamed pass's groups
     uint32_t* d_hstate = nullptr;   // Horner chain state between chunk launches [B*T][4][N]
@@ -275,7 +281,7 @@ struct GpuServerCtx {
         bool part2 = false;         // the collapse sums (a split collapse adds into them)
         bool pair = false;          // the pair chains' exchange words
         bool skip_lwe = false;      // leave the LWE part to prep_lwe
-        uint32_t* status = nullptr; // a word
+        uint32_t* status = nullptr, *gave_up = nullptr;  // a word each
     };
     ipx::PrepArgs prep_args(const QueryInput& in, size_t stride, size_t q0, int lane) const;
     // Keys, RGSW rows and plan p's pass operands of the flat queries at d_in.
@@ -311,6 +317,9 @@ struct GpuServerCtx {
     // fp: the chains compute their groups' packed b-parts themselves first
     void horner_range(size_t count, uint64_t* d_out, size_t g_lo, size_t g_hi, hipStream_t s, size_t slot0,
                       int lane, bool pair, const ipx::FusedPack* fp = nullptr);
+    // The chains of `count` queries in one launch and without waits, where a
+    // wait of the lane's answer ended at its bound.
+    void horner_again(size_t count, uint64_t* d_out, hipStream_t s, size_t slot0, int lane);
     // Throw (and clear) if a pair chain of a call on `lane` reported a fault
     // through its status word; the call's stream has been waited for.
     void check_status(int lane);
