@@ -145,6 +145,11 @@ int acquire_lanes(int device, LaneStreams (&out)[kLaneSets]) {
     return first;
 }
 
+std::recursive_mutex& QueueTurn::mutex(int device) {
+    static std::recursive_mutex m[kMaxDevices];
+    return m[device >= 0 && device < kMaxDevices ? device : 0];
+}
+
 void release_lanes(int device, int first) {
     std::lock_guard<std::mutex> lk(g_mu);
     DeviceLanes& d = g_lanes[device];

@@ -1059,10 +1059,10 @@ void GpuServerCtx::enqueue(const QueryInput& in, size_t count, uint64_t* d_out, 
         return;
     }
     HIPX(hipEventRecord(hop_in_ev[lane], s));
-    HIPX(hipStreamWaitEvent(ms, hop_in_ev[lane], 0));
+    stream_wait(ms, hop_in_ev[lane]);
     enqueue_on(in, count, d_out, ms, slot0, lane, status_read);
     HIPX(hipEventRecord(hop_out_ev[lane], ms));
-    HIPX(hipStreamWaitEvent(s, hop_out_ev[lane], 0));
+    stream_wait(s, hop_out_ev[lane]);
 }
 
 bool GpuServerCtx::is_capturing(hipStream_t s) {
@@ -1173,9 +1173,16 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             // (6) drains or the LWE digits are made (8); released together
             // with the pass they would wait for a CU the pass's workgroups
             // leave wholly free, often its end.
+            // Once released they wait inside the kernel, so nothing that may
+            // take long must come between what they wait for and its queue
+            // (hardware queues are few, and shared with other streams and
+            // servers): the pass follows the release under one QueueTurn,
+            // and the chains are released only when the pack's queue has
+            // reached the pack.
+            const QueueTurn turn(device);
             if (cs != s) {
                 HIPX(hipEventRecord(prep_ev[lane], s));
-                HIPX(hipStreamWaitEvent(cs, prep_ev[lane], 0));
+                stream_wait(cs, prep_ev[lane]);
             } else {
                 HIPX(hipEventRecord(coll_ev[lane][0], s));
             }
@@ -1213,7 +1220,12 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
                                         C, 0, C, sp, s, &pst));
             }
             mark_pass(s, false);
-            if (ps_s != cs) HIPX(hipStreamWaitEvent(ps_s, coll_ev[lane][0], 0));
+            hipEvent_t pack_next = coll_ev[lane][0];  // recorded on ps_s where the collapse is beside the pass
+            if (ps_s != cs) {
+                stream_wait(ps_s, coll_ev[lane][0]);
+                pack_next = chunk_ev[lane][0];
+                HIPX(hipEventRecord(pack_next, ps_s));
+            }
             PackStream pk;
             pk.part = part;
             pk.part_qstride = part_qstride;
@@ -1227,8 +1239,8 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             pk.queries = pq;
             HIPX(launch_pack_stream(pk, p2, part2_stride, d_precomp, keys, keys_stride, packed, packed_stride, G, nq,
                                     nc, ps_s));
-            HIPX(hipStreamWaitEvent(hs, coll_ev[lane][0], 0));
-            if (g_split > 0 && g_split < G) HIPX(hipStreamWaitEvent(hs, pass_ev[lane], 0));
+            stream_wait(hs, pack_next);
+            if (g_split > 0 && g_split < G) stream_wait(hs, pass_ev[lane]);
             StreamWait sw;
             sw.done = packed_done;
             sw.queries = pq;
@@ -1239,7 +1251,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
                                rgsw_stride, out, d_hstate + q0 * T * 4 * N, 0, G, nq, nc, cc, hs, FusedPack{}, sw));
             // the next sub-batch's key digits and flags wait for the collapse and the pack
             HIPX(hipEventRecord(prep_ev[lane], ps_s));
-            HIPX(hipStreamWaitEvent(s, prep_ev[lane], 0));
+            stream_wait(s, prep_ev[lane]);
             if (stream_spin_limit)
                 again.push_back([=] {  // the pass and its counters are complete by then
                     PackStream pa = pk;
@@ -1260,14 +1272,14 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             z.pair = pair;
             if (in.late) {
                 HIPX(hipEventRecord(prep_ev[lane], s));  // earlier readers of the copy's target are done
-                HIPX(hipStreamWaitEvent(ps_side, prep_ev[lane], 0));
+                stream_wait(ps_side, prep_ev[lane]);
                 prep_lwe(in, in.lwe_stride, q0, nq, p, s, lane);
                 mark_pass(s, true);
                 dbpass_whole(q0, nq, p, s, lane);
                 mark_pass(s, false);
                 in.late->copy(ps_side);
                 HIPX(hipEventRecord(coll_ev[lane][0], ps_side));
-                HIPX(hipStreamWaitEvent(s, coll_ev[lane][0], 0));
+                stream_wait(s, coll_ev[lane][0]);
                 if (in.late->after) in.late->after(s);
             }
             prep_query(in, q0, nq, p, s, lane, z);
@@ -1316,7 +1328,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
         prep_query(in, q0, nq, p, s, lane, z);
         if (cs != s) {
             HIPX(hipEventRecord(prep_ev[lane], s));  // the keys are in place
-            HIPX(hipStreamWaitEvent(cs, prep_ev[lane], 0));
+            stream_wait(cs, prep_ev[lane]);
         }
         if (first) {
             TraceRange trc("collapse of all %zu groups", G);
@@ -1330,7 +1342,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
         };
         if (ahead) {
             collapse_chunk(0);
-            HIPX(hipStreamWaitEvent(s, coll_ev[lane][0], 0));
+            stream_wait(s, coll_ev[lane][0]);
         }
         for (size_t k = 0; k < layout.chunks.size(); k++) {
             const size_t g_lo = layout.chunks[k].first, g_hi = layout.chunks[k].second, ng = g_hi - g_lo;
@@ -1355,8 +1367,8 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             const bool aside = cs == s && layout.aside(k);
             const hipStream_t ks = aside ? ps_side : hs;
             side_chains = side_chains || aside;
-            if (cs != s) HIPX(hipStreamWaitEvent(ks, dbe, 0));
-            HIPX(hipStreamWaitEvent(ks, ce, 0));
+            if (cs != s) stream_wait(ks, dbe);
+            stream_wait(ks, ce);
             // the pack: fused into the one-workgroup Horner chains, or a kernel of its own
             const bool fuse = pack_wg == 2 && !pair;
             const FusedPack fp{d_interm + q0 * 2 * C, C, p2, part2_stride, d_precomp, keys, keys_stride};
@@ -1373,17 +1385,17 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
         chains_again(q0, nq);
         if (cs != s) {  // the next batch's key digits overwrite the lane's scratch
             HIPX(hipEventRecord(prep_ev[lane], cs));
-            HIPX(hipStreamWaitEvent(s, prep_ev[lane], 0));
+            stream_wait(s, prep_ev[lane]);
         }
     }
     flush_deferred();
     if (joined) {
         HIPX(hipEventRecord(horner_done[lane], hs));
-        HIPX(hipStreamWaitEvent(s, horner_done[lane], 0));
+        stream_wait(s, horner_done[lane]);
     }
     if (side_chains) {
         HIPX(hipEventRecord(prep_ev[lane], ps_side));
-        HIPX(hipStreamWaitEvent(s, prep_ev[lane], 0));
+        stream_wait(s, prep_ev[lane]);
     }
     for (const auto& f : again) f();
 }
@@ -1404,6 +1416,7 @@ void GpuServerCtx::run_step(const void* in, void* out, size_t count, size_t slot
     for (const StepGraph& g : graphs)
         if (g.in == in && g.out == out && g.count == count && g.slot0 == slot0 && g.lane == lane &&
             g.packed == packed) {
+            const QueueTurn turn(device);  // branches of a graph wait for each other
             HIPX(hipGraphLaunch(g.exec, s));
             return;
         }
@@ -1428,6 +1441,7 @@ void GpuServerCtx::run_step(const void* in, void* out, size_t count, size_t slot
         graphs.erase(graphs.begin());
     }
     graphs.push_back({in, out, count, slot0, lane, packed, exec});
+    const QueueTurn turn(device);
     HIPX(hipGraphLaunch(exec, s));
 }
 
@@ -1540,11 +1554,16 @@ void GpuServerCtx::check_status(int lane) {
         "a Horner chain gave up its wait (bound set to zero); responses of this call are invalid");
 }
 
+void GpuServerCtx::stream_wait(hipStream_t s, hipEvent_t e) {
+    const QueueTurn turn(device);
+    HIPX(hipStreamWaitEvent(s, e, 0));
+}
+
 void GpuServerCtx::order_before(hipStream_t s) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     HIPX(hipStreamIsCapturing(s, &cap));
     if (cap != hipStreamCaptureStatusNone) return;  // a caller's capture orders its own work
-    if (order_stream_set && order_stream != s) HIPX(hipStreamWaitEvent(s, order_ev, 0));
+    if (order_stream_set && order_stream != s) stream_wait(s, order_ev);
 }
 
 void GpuServerCtx::order_after(hipStream_t s) {

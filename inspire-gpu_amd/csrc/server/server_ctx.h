@@ -247,6 +247,9 @@ struct GpuServerCtx {
     bool order_stream_set = false;
     void order_before(hipStream_t s);
     void order_after(hipStream_t s);
+    // s waits for e, in a queue turn: every wait this library puts on a
+    // stream goes through here (lanes.h, QueueTurn).
+    void stream_wait(hipStream_t s, hipEvent_t e);
 
     // Captured answer steps: with graph_mode on, the first answer of a given
     // (input, output, count, slots, lane, form) is captured from its stream
