@@ -18,7 +18,14 @@ namespace inspire {
 class HostStage {
 public:
     explicit HostStage(size_t helpers, size_t max_items) : done_(new std::atomic<uint8_t>[max_items]) {
-        for (size_t i = 0; i < helpers; i++) threads_.emplace_back([this] { help(); });
+        threads_.reserve(helpers);
+        try {
+            for (size_t i = 0; i < helpers; i++) threads_.emplace_back([this] { help(); });
+        } catch (...) {
+            // no more threads to be had: a job goes with those there are, or
+            // with its caller alone (leaving here would end the process,
+            // whose threads nothing joins)
+        }
     }
     ~HostStage() {
         {
