@@ -9,7 +9,6 @@
 #include <functional>
 #include <memory>
 #include <mutex>
-#include <stdexcept>
 #include <thread>
 #include <vector>
 
@@ -51,25 +50,25 @@ public:
         }
         if (open_) cv_.notify_all();
     }
-    // Return once items [0, upto) are done, taking part; throws if one failed.
+    // Return once items [0, upto) are done or have failed, taking part. A
+    // failure does not end the wait: what the caller has enqueued by then is
+    // followed by the rest, and it learns of the failure from finish().
     void wait(size_t upto) {
-        settle(upto);
-        if (failed_.load()) throw std::runtime_error("staging a query failed");
-    }
-    // Every item done and no helper inside the job any more (never throws).
-    void finish() {
-        settle(n_);
-        std::unique_lock<std::mutex> lk(m_);
-        open_ = false;
-        idle_.wait(lk, [&] { return active_ == 0; });
-    }
-
-private:
-    void settle(size_t upto) {
         for (size_t i = 0; i < upto; i++)
             while (!done_[i].load(std::memory_order_acquire))
                 if (!take()) std::this_thread::yield();
     }
+    // Every item done and no helper inside the job any more; whether none of
+    // them failed.
+    bool finish() {
+        wait(n_);
+        std::unique_lock<std::mutex> lk(m_);
+        open_ = false;
+        idle_.wait(lk, [&] { return active_ == 0; });
+        return !failed_.load();
+    }
+
+private:
     bool take() {
         const size_t i = next_.fetch_add(1);
         if (i >= n_) return false;

@@ -1483,6 +1483,9 @@ struct StagedJob {
         st.begin(n, std::move(fn), n > 1);
     }
     ~StagedJob() { st.finish(); }
+    // The call's work is enqueued whole, ordered before the next call's, and
+    // waited for before it fails for a query that could not be staged.
+    bool finish() { return st.finish(); }
 };
 }  // namespace
 
@@ -1503,6 +1506,7 @@ void GpuServerCtx::answer_packed_host(const uint8_t* in, size_t count, uint8_t* 
     uint8_t* hq = reinterpret_cast<uint8_t*>(h_q);
     uint8_t* hr = reinterpret_cast<uint8_t*>(h_resp);
     TraceRange tr("host-staged packed answer: %zu queries", count);
+    bool staged = false;
     {
         // split: the LWE parts' bytes, then the others' (both 16-byte multiples)
         const bool split = late_keys(count);
@@ -1541,8 +1545,10 @@ void GpuServerCtx::answer_packed_host(const uint8_t* in, size_t count, uint8_t* 
                            split ? &late : nullptr);
         });
         order_after(s);
+        staged = job.finish();
     }
     HIPX(hipStreamSynchronize(s));
+    if (!staged) throw std::runtime_error("staging a query failed");
     check_status(0);
     copy_out(count, T * kCompressedCtBytes, out);
 }
@@ -1583,6 +1589,7 @@ bool GpuServerCtx::late_keys(size_t count) const {
 void GpuServerCtx::answer_host(size_t count, const FillQuery& fill, uint64_t* out) {
     hipStream_t s = pipelined(count) && !graph_mode ? lanes[0].pass : stream;
     TraceRange tr("host-staged answer: %zu queries", count);
+    bool staged = false;
     {
         // The queries are narrowed into pinned memory that the preparation
         // kernel reads, piece by piece as they come, and the chains write the
@@ -1620,8 +1627,10 @@ void GpuServerCtx::answer_host(size_t count, const FillQuery& fill, uint64_t* ou
         }
         run_step(h_q, h_resp, count, 0, 0, 0, s, [&] { enqueue(in, count, h_resp, s, 0, 0, true); });
         order_after(s);
+        staged = job.finish();
     }
     HIPX(hipStreamSynchronize(s));
+    if (!staged) throw std::runtime_error("staging a query failed");
     check_status(0);
     copy_out(count, resp_u64s * 8, out);
 }

@@ -1,7 +1,7 @@
 // HostStage (inspire-gpu_amd/csrc/server/host_stage.h) on the CPU: with as
 // many helper threads as the process can have (fewer than asked for, here by
 // a limit on its address space), every item of a job is done once, and a
-// failed one is reported.
+// failed one is reported once everything has been waited for.
 #include <pthread.h>
 #include <sys/resource.h>
 
@@ -34,9 +34,10 @@ static void run_jobs(size_t helpers) {
             } catch (const std::runtime_error&) {
                 threw = true;
             }
-            st.finish();
+            const bool ok = st.finish();
             for (size_t i = 0; i < kItems; i++) check(times[i] == (i < n ? 1 : 0), "every item once");
-            check(threw == (bad != 0), "failures are reported");
+            check(!threw, "a failed item does not end the waits");
+            check(ok == (bad == 0) && st.finish() == ok, "failures are reported at the end");
         }
     }
 }
