@@ -96,14 +96,17 @@ int ipir_dbg_set_tail_split(ipir_server* srv, int on);
  * asynchronous device entry points (ipir_answer_batch_device,
  * ipir_answer_batch_packed_device) use one workgroup per chain. */
 int ipir_dbg_set_horner(ipir_server* srv, int mode);
-/* Bound of the pair kernel's partner wait, in loads (default 2^21, ~2 s); an
- * answer in which a wait ends at its bound is made again at its end.
+/* Bound of the pair kernel's partner wait, in loads (default 2^21, ~2 s, and
+ * no more: larger values set the default, among them 2^26, which was the
+ * default while the bound counted shorter sleeps); an answer in which a wait
+ * ends at its bound is made again at its end.
  * 0 makes every pair chain report the bound exceeded at its first
  * exchange and stop (all kernels still end normally), and nothing is made
  * again: the response is all-ones words, the call that ran it returns 4 (the
  * asynchronous ones report it through ipir_device_status), and later calls
  * are unaffected. 5 while a loop runs. */
 int ipir_dbg_set_horner_spin_limit(ipir_server* srv, uint32_t limit);
+uint32_t ipir_dbg_horner_spin_limit(const ipir_server* srv);
 /* The same bound for Horner chains waiting for a streamed database pass's
  * groups (default 2^23; 0: give up at once and report, as above; the pass
  * itself runs to its end). */

@@ -826,10 +826,12 @@ int ipir_dbg_set_horner_spin_limit(ipir_server* srv, uint32_t limit) {
     if (!srv) return 1;
     std::lock_guard<std::mutex> lk(srv->ctx->mu);
     if (srv->ctx->loop_active) return 5;
-    srv->ctx->horner_spin_limit = limit;
+    srv->ctx->horner_spin_limit = limit < GpuServerCtx::kHornerSpinLimit ? limit : GpuServerCtx::kHornerSpinLimit;
     srv->ctx->drop_graphs();  // their kernels carry the old bound
     return 0;
 }
+
+uint32_t ipir_dbg_horner_spin_limit(const ipir_server* srv) { return srv ? srv->ctx->horner_spin_limit : 0; }
 
 int ipir_dbg_set_stream_spin_limit(ipir_server* srv, uint32_t limit) {
     if (!srv) return 1;

@@ -94,6 +94,7 @@ SERVER_FUNCS = [
     ("ipir_fit_max_batch", SZ, [SZ, SZ, SZ, SZ, SZ]),
     ("ipir_dbg_db_block", C.c_int, [VP, SZ, SZ, SZ, SZ, VP]),
     ("ipir_dbg_set_horner_spin_limit", C.c_int, [VP, C.c_uint32]),
+    ("ipir_dbg_horner_spin_limit", C.c_uint32, [VP]),
     ("ipir_dbg_set_stream_spin_limit", C.c_int, [VP, C.c_uint32]),
     ("ipir_dbg_chains_redone", C.c_int, [VP]),
     ("ipir_dbg_loop_hold", C.c_int, [VP, C.c_int]),

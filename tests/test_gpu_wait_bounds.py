@@ -83,3 +83,15 @@ def test_answers_past_their_wait_bounds(table, shape, limit):
     assert lib.ipir_answer_batch(srv.h, srv.views(qs[:3]), 3, ia.ptr(out)) == 0
     assert np.array_equal(out, want[:3])
     assert lib.ipir_dbg_chains_redone(srv.h) == 0, "ordinary bounds are not reached"
+
+
+def test_pair_bound_is_at_most_the_default(table):
+    """A bound past the default (2^26 was it, in another unit) is the default:
+    no pair holds its CUs for minutes."""
+    _, srv, _, _ = table
+    lib = srv.lib
+    default = lib.ipir_dbg_horner_spin_limit(srv.h)
+    assert default == 1 << 21
+    for limit, got in ((0, 0), (7, 7), (1 << 26, default), (1 << 21, default), ((1 << 32) - 1, default)):
+        assert lib.ipir_dbg_set_horner_spin_limit(srv.h, limit) == 0
+        assert lib.ipir_dbg_horner_spin_limit(srv.h) == got, limit
