@@ -34,10 +34,17 @@ int ipir_dbg_db_pass(ipir_server* srv, const uint64_t* b, size_t nq, int path, u
 /* Device time of the full-width database pass alone (the pass kernel of
  * the plan answer_batch uses for nq <= 32 queries, and its slice reduction
  * if the plan has row slices, on the server stream) over the first nq
- * query slots as last staged (by a host-staged answer or
- * ipir_dbg_profile_batch), averaged over iters passes; the query digits are
- * prepared once, outside the timed launches. */
+ * queries that the last call staged, averaged over iters passes; the query
+ * digits are prepared once, outside the timed launches. Every call stages
+ * its queries (blocking and packed answers, a serving loop,
+ * ipir_dbg_profile_batch, ipir_dbg_db_pass) except ipir_answer_batch_device,
+ * whose queries stay the caller's; at first they are zero. Leaves the passes'
+ * result as ipir_dbg_interm reads it. */
 int ipir_dbg_time_dbpass(ipir_server* srv, size_t nq, int iters, double* ms_per_pass);
+/* The pass's result as last left for the first nq query slots,
+ * interm [nq][2][db_cols] (an answer whose pass has row slices leaves it as
+ * it was). Waits for the server's last call; 5 while a loop runs. */
+int ipir_dbg_interm(ipir_server* srv, size_t nq, uint32_t* interm);
 /* The database-pass kernel (profiler name) and row-slice count the server
  * uses for a batch of nq queries, NUL-terminated into out[cap]. */
 int ipir_dbg_dbpass_kernel(const ipir_server* srv, size_t nq, char* out, size_t cap);

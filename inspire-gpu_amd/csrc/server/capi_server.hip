@@ -292,6 +292,7 @@ int ipir_dbg_db_pass(ipir_server* srv, const uint64_t* b, size_t nq, int path, u
         c->order_before(c->stream);
         // the LWE parts, 2R words apart, in the flat query staging
         hip_check(hipMemcpy(c->d_q, b, nq * 2 * R * 8, hipMemcpyHostToDevice), "dbg db pass upload");
+        c->set_staged(c->d_q, 2 * R);
         const size_t step = path == 0 ? 1 : ipx::kMfmaMaxQueries;
         for (size_t q0 = 0; q0 < nq; q0 += step) {
             const size_t n = nq - q0 < step ? nq - q0 : step;
@@ -329,7 +330,7 @@ int ipir_dbg_time_dbpass(ipir_server* srv, size_t nq, int iters, double* ms_per_
         // the query digits once; then the pass's own launches (the kernel and,
         // for a plan with row slices, the slice reduction)
         const ipx::DbPlan p = c->plan_for(nq, c->pp.db_cols);
-        c->prep_lwe(c->d_q, c->qlen, 0, nq, p, c->stream, 0);
+        c->prep_lwe(c->staged, c->staged_stride, 0, nq, p, c->stream, 0);
         c->dbpass_range(0, nq, 0, c->G, p, c->stream, 0);  // warm-up
         hip_check(hipEventRecord(e0, c->stream), "record");
         for (int i = 0; i < iters; i++) c->dbpass_range(0, nq, 0, c->G, p, c->stream, 0);
@@ -345,6 +346,21 @@ int ipir_dbg_time_dbpass(ipir_server* srv, size_t nq, int iters, double* ms_per_
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     return rc;
+}
+
+int ipir_dbg_interm(ipir_server* srv, size_t nq, uint32_t* interm) {
+    if (!srv || !interm || nq == 0 || nq > srv->ctx->cfg.max_batch) return 1;
+    GpuServerCtx* c = srv->ctx;
+    std::lock_guard<std::mutex> lk(c->mu);
+    if (c->loop_active) return 5;
+    try {
+        c->order_before(c->stream);
+        hip_check(hipStreamSynchronize(c->stream), "interm");
+        hip_check(hipMemcpy(interm, c->d_interm, nq * 2 * c->pp.db_cols * 4, hipMemcpyDeviceToHost), "interm");
+        return 0;
+    } catch (...) {
+        return 4;
+    }
 }
 
 int ipir_dbg_dbpass_kernel(const ipir_server* srv, size_t nq, char* out, size_t cap) {
@@ -671,6 +687,7 @@ int ipir_dbg_stream_parts(ipir_server* srv, size_t nq, uint32_t slices, double* 
         const size_t part_qstride = direct ? 2 * C : c->part_stride;
         c->order_before(s);
         hip_check(hipMemsetAsync(c->d_q, 0, nq * c->qlen * 8, s), "zero");
+        c->set_staged(c->d_q, c->qlen);
         c->prep_lwe(c->d_q, c->qlen, 0, nq, p, s, 0);
         auto timed = [&](const std::function<void()>& fn) {
             fn();  // warm
@@ -903,8 +920,8 @@ int ipir_dbg_profile_batch(ipir_server* srv, const uint64_t* d_queries, size_t c
     try {
         for (auto& e : ev) hip_check(hipEventCreate(&e), "event");
         c->order_before(s);
-        // kept as staged queries for ipir_dbg_time_dbpass
         hip_check(hipMemcpyAsync(c->d_q, d_queries, count * c->qlen * 8, hipMemcpyDeviceToDevice, s), "stage queries");
+        c->set_staged(c->d_q, c->qlen);
         size_t k = 0;
         auto mark = [&] { hip_check(hipEventRecord(ev[k++], s), "event"); };
         for (size_t q0 = 0; q0 < count; q0 += step) {

@@ -343,6 +343,7 @@ void ipir_loop_stop(ipir_loop* L) {
     {
         std::lock_guard<std::mutex> lk(ctx->mu);
         ctx->order_stream_set = false;  // the loop's work has finished
+        ctx->set_staged(ctx->flat32(), ctx->qlen);  // its batches' copies
         ctx->loop_active = false;
     }
     delete L;

@@ -551,6 +551,7 @@ void GpuServerCtx::autotune_dbpass() {
     // one full-width database pass of plan x over nq staged queries (zeroed)
     const size_t nq = cfg.max_batch < kMfmaMaxQueries ? cfg.max_batch : kMfmaMaxQueries;
     HIPX(hipMemset(d_q, 0, nq * qlen * 8));
+    set_staged(d_q, qlen);
     auto prep_plan = [&](const DbPlan& x, size_t n) { prep_lwe(d_q, qlen, 0, n, x, stream, 0); };
     auto run_plan = [&](const DbPlan& x, size_t nq) {
         if (x.kind == DbPlan::F64)
@@ -1460,6 +1461,7 @@ void GpuServerCtx::enqueue_packed(const uint8_t* d_in, size_t count, uint8_t* d_
     QueryInput in(dq);
     in.late = late;
     in.lwe_stride = qlen;
+    set_staged(in, qlen);
     const size_t R = pp.db_rows;
     for (size_t f = 0; f < count; f += stage ? kStagePiece : count) {
         const size_t n = stage && count - f > kStagePiece ? kStagePiece : count - f;
@@ -1625,6 +1627,7 @@ void GpuServerCtx::answer_host(size_t count, const FillQuery& fill, uint64_t* ou
             in.late = &late;
             in.lwe_stride = R2;
         }
+        set_staged(in, split ? R2 : qlen);
         run_step(h_q, h_resp, count, 0, 0, 0, s, [&] { enqueue(in, count, h_resp, s, 0, 0, true); });
         order_after(s);
         staged = job.finish();

@@ -381,6 +381,17 @@ struct GpuServerCtx {
     void enqueue_packed(const uint8_t* d_in, size_t count, uint8_t* d_out, hipStream_t s, size_t slot0 = 0,
                         int lane = 0, bool status_read = false, HostStage* stage = nullptr,
                         const LateKeys* late = nullptr);
+    // The LWE parts that ipir_dbg_time_dbpass prepares: those the last call
+    // but a flat device one left in the staging (else zeros), wherever it put
+    // them.
+    QueryInput staged{(const uint64_t*)nullptr};
+    size_t staged_stride = 0;
+    void set_staged(const QueryInput& in, size_t stride) {
+        staged = in;
+        staged.stage = nullptr;
+        staged.late = nullptr;
+        staged_stride = stride;
+    }
     // count responses of `bytes` bytes from the pinned staging to out.
     void copy_out(size_t count, size_t bytes, void* out);
     // Host round trip of the packed forms through the pinned staging.
