@@ -198,6 +198,10 @@ int ipir_dbg_set_stream_split(ipir_server* srv, size_t nq_class, uint32_t eighth
 /* 1 if this server may take the streamed shapes, else 0 (INSPIRE_STREAM=0 at
  * setup). */
 int ipir_dbg_stream_ok(const ipir_server* srv);
+/* How many of the device's four sets of streams for pipelined answers have
+ * streams whose kernels run side by side (call it on an idle device); -1 on
+ * errors. */
+int ipir_dbg_lanes_apart(const ipir_server* srv);
 /* Let srv take the streamed shapes whatever INSPIRE_STREAM said at setup. */
 int ipir_dbg_take_streaming(ipir_server* srv);
 /* Timings (ms, mean of 5 after a warm-up) of the streamed pieces for nq

@@ -661,6 +661,15 @@ int ipir_dbg_set_stream_split(ipir_server* srv, size_t nq_class, uint32_t eighth
     return 0;
 }
 
+int ipir_dbg_lanes_apart(const ipir_server* srv) {
+    if (!srv) return -1;
+    try {
+        return lanes_apart(srv->ctx->device);
+    } catch (...) {
+        return -1;
+    }
+}
+
 int ipir_dbg_stream_ok(const ipir_server* srv) { return srv && srv->ctx->stream_ok ? 1 : 0; }
 
 int ipir_dbg_stream_parts(ipir_server* srv, size_t nq, uint32_t slices, double* out_ms) {

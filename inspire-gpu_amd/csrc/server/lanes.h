@@ -16,6 +16,9 @@ struct LaneStreams {
 // Throws std::runtime_error where the streams cannot be created.
 int acquire_lanes(int device, LaneStreams (&out)[kLaneSets]);
 void release_lanes(int device, int first);
+// How many of a device's sets have streams that run side by side now (on an
+// idle device).
+int lanes_apart(int device);
 
 // A thread's turn to put waits into a device's queues. Streams share a few
 // hardware queues, and a stream's wait for an event holds up whatever was

@@ -7,6 +7,7 @@
 // are seen to run side by side.
 #include "lanes.h"
 
+#include <algorithm>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -20,8 +21,13 @@ namespace inspire {
 namespace {
 
 constexpr int kMaxDevices = 64;
-// polls of 128 clocks: about 0.1 ms, far above the launch of a second kernel
-constexpr uint32_t kProbePolls = 2000;
+// Polls of 128 clocks and a load, about 1 ms: far above the launch of a second
+// kernel on an idle device. Beside other work that launch may take longer
+// (four threads with 2 ms of kernels in flight each: sets of one to three
+// streams apart were found), so where a set stays incomplete its remaining
+// candidates are tried again with the longer wait, which only a kernel behind
+// the waiting one on its own queue uses up.
+constexpr uint32_t kProbePolls[] = {2000, 60000};
 constexpr int kProbeStreams = 10;  // candidates tried for one set
 
 // words: [0] the flag, [1] whether the waiting kernel saw it
@@ -42,10 +48,10 @@ void check(hipError_t e, const char* what) {
 }
 
 // Whether a kernel on b runs while one enqueued before it on a still runs.
-bool side_by_side(hipStream_t a, hipStream_t b, uint32_t* d_words) {
+bool side_by_side(hipStream_t a, hipStream_t b, uint32_t* d_words, uint32_t polls = kProbePolls[0]) {
     check(ipx::launch_fill_u32(d_words, 2, 0, a), "stream probe");
     check(hipStreamSynchronize(a), "stream probe");
-    hipLaunchKernelGGL(k_probe_wait, dim3(1), dim3(1), 0, a, d_words, kProbePolls);
+    hipLaunchKernelGGL(k_probe_wait, dim3(1), dim3(1), 0, a, d_words, polls);
     hipLaunchKernelGGL(k_probe_set, dim3(1), dim3(1), 0, b, d_words);
     check(hipGetLastError(), "stream probe");
     check(hipStreamSynchronize(a), "stream probe");
@@ -74,6 +80,7 @@ void destroy(DeviceLanes& d) {
 void create(DeviceLanes& d) {
     uint32_t* words = nullptr;
     std::vector<hipStream_t> spare;
+    bool few = false;  // the longer waits did not complete a set either
     auto cleanup = [&] {
         for (hipStream_t x : spare) (void)hipStreamDestroy(x);
         if (words) (void)hipFree(words);
@@ -85,19 +92,22 @@ void create(DeviceLanes& d) {
             // Streams left over from earlier sets first, then new ones. The
             // rejected ones live until every set is complete: destroyed early,
             // their queue would be the next stream's again.
-            for (int k = 0; k < kProbeStreams && got.size() < 3; k++) {
-                hipStream_t x = nullptr;
-                if ((size_t)k < spare.size()) {
-                    x = spare[k];
-                } else {
-                    check(hipStreamCreate(&x), "hipStreamCreate");
-                    spare.push_back(x);
+            for (const uint32_t polls : kProbePolls) {
+                if (polls != kProbePolls[0] && few) break;
+                for (int k = 0; k < kProbeStreams && got.size() < 3; k++) {
+                    if ((size_t)k >= spare.size()) {
+                        hipStream_t x = nullptr;
+                        check(hipStreamCreate(&x), "hipStreamCreate");
+                        spare.push_back(x);
+                    }
+                    const hipStream_t x = spare[k];
+                    bool apart = std::find(got.begin(), got.end(), x) == got.end();
+                    for (size_t i = 0; i < got.size() && apart; i++) apart = side_by_side(got[i], x, words, polls);
+                    if (apart) got.push_back(x);
                 }
-                bool apart = true;
-                for (hipStream_t y : got) apart = apart && side_by_side(y, x, words);
-                if (apart) got.push_back(x);
             }
-            for (size_t k = 0; got.size() < 3; k++) {  // fewer queues than roles (or a busy device): any will do
+            few = few || got.size() < 3;
+            while (got.size() < 3) {  // fewer queues than roles, or a very busy device: any will do
                 hipStream_t x = nullptr;
                 check(hipStreamCreate(&x), "hipStreamCreate");
                 spare.push_back(x);
@@ -148,6 +158,26 @@ int acquire_lanes(int device, LaneStreams (&out)[kLaneSets]) {
 std::recursive_mutex& QueueTurn::mutex(int device) {
     static std::recursive_mutex m[kMaxDevices];
     return m[device >= 0 && device < kMaxDevices ? device : 0];
+}
+
+int lanes_apart(int device) {
+    if (device < 0 || device >= kMaxDevices) return 0;
+    std::lock_guard<std::mutex> lk(g_mu);
+    DeviceLanes& d = g_lanes[device];
+    if (d.servers == 0) return 0;
+    uint32_t* words = nullptr;
+    check(hipMalloc((void**)&words, 8), "stream probe");
+    int n = 0;
+    try {
+        for (const LaneStreams& s : d.set)
+            n += side_by_side(s.pass, s.horner, words) && side_by_side(s.pass, s.side, words) &&
+                 side_by_side(s.horner, s.side, words);
+    } catch (...) {
+        (void)hipFree(words);
+        throw;
+    }
+    (void)hipFree(words);
+    return n;
 }
 
 void release_lanes(int device, int first) {

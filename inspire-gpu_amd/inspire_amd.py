@@ -129,6 +129,7 @@ SERVER_FUNCS = [
     ("ipir_dbg_get_collapse_variant", C.c_int, [VP]),
     ("ipir_dbg_set_pipeline", C.c_int, [VP, C.c_int, C.c_int]),
     ("ipir_dbg_set_stream_slices", C.c_int, [VP, SZ, C.c_uint32]),
+    ("ipir_dbg_lanes_apart", C.c_int, [VP]),
     ("ipir_dbg_stream_ok", C.c_int, [VP]),
     ("ipir_dbg_set_stream_split", C.c_int, [VP, SZ, C.c_uint32]),
     ("ipir_dbg_take_streaming", C.c_int, [VP]),
