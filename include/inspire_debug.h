@@ -177,7 +177,7 @@ int ipir_dbg_get_collapse_variant(const ipir_server* srv);
  * collapse stream a chunk ahead of the database pass; streamed: one
  * full-width database pass that hands each group over as its columns are
  * final, the Horner chains waiting for the groups inside the kernel (a
- * bounded wait, reported like the pair kernel's), 6 after the collapse of
+ * bounded wait, like the pair kernel's), 6 after the collapse of
  * all groups, 7 with the collapse beside it, 8 with the collapse inside the
  * pass's launch, each group's collapse and pass work items together (up to
  * 8 queries; 6 for more). The setup autotuner picks 2, 3, 6 or 8 (4, 5
@@ -217,11 +217,13 @@ size_t ipir_dbg_streamed_count(const ipir_server* srv);
  * around every sub-batch's database-pass launches (the streamed launch, or
  * each chunk's pass) on the stream they run on; on = 0 stops, waits for
  * them and returns the summed pass time and the number of sub-batch passes
- * (each over all columns). 1 if more than 4096 launches were marked (the
- * rest went untimed). */
+ * (each over all columns). Where the pass and the collapse are one launch
+ * (shape 8, and serial answers of up to 8 queries over small tables) the
+ * time is that launch's. 1 if more than 4096 launches were marked (the rest
+ * went untimed). */
 int ipir_dbg_pass_timing(ipir_server* srv, int on, double* total_ms, size_t* passes);
 /* Per-stage device time (ms) of the last ipir_dbg_profile_batch run:
- * [unmarshal+key NTT, DB pass, collapse pass, pack finalize, Horner]. */
+ * [preparation, DB pass, collapse pass, pack finalize, Horner]. */
 int ipir_dbg_profile_batch(ipir_server* srv, const uint64_t* d_queries, size_t count, uint64_t* d_out,
                            double* stage_ms);
 

@@ -13,9 +13,9 @@
 namespace ipx {
 
 // ---------------------------------------------------------------- online
-// Per-query device layout produced by unmarshal (one "slot"):
-//   bq  : double [2][R]            (b residues as exact doubles, DB pass)
-//   keys: u32 [2 keys][digit][limb][N]  (ksk5, kskneg1; coeff -> NTT in place)
+// Per-query device layout that the preparation launch writes (one "slot"):
+//   bq  : double [2][R]            (b residues as exact doubles, fp64 passes)
+//   keys: u32 [2 keys][digit][limb][N]  (ksk5, kskneg1; NTT form)
 //   rgsw: u32 [4 parts][digit][limb][N]  (NTT form)
 struct SlotLayout {
     size_t R, C, G;

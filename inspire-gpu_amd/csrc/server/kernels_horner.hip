@@ -36,7 +36,8 @@
 // *status, fills its limb of the response with all-ones words (no residue;
 // where the chain continues in a later launch, of the state, which passes
 // them on) and ends; its partner's wait then ends the same way (a bound of
-// zero takes that path at the first exchange).
+// zero takes that path at the first exchange). The answer then makes its
+// chains again (HornerAgain).
 #include "kernels.h"
 #include "ntt_regs.h"
 

@@ -1,7 +1,7 @@
-// Online (per-query) kernels for gfx950: query unmarshal, batched NTT, the
-// row-slice reduction of the database pass, pack finalize, and the
-// persistent Horner/external-product chain (the database and collapse
-// passes live in kernels_db.hip and kernels_collapse.hip).
+// Online (per-query) kernels for gfx950: batched NTT, the row-slice
+// reduction of the database pass, pack finalize, and the persistent
+// Horner/external-product chain (preparation, database and collapse passes
+// live in kernels_prep.hip, kernels_db.hip and kernels_collapse.hip).
 //
 // Semantics follow the reference's online path (src/gpu_protocol.cu:
 // 1121-1339): mat-vec interm_c = DB^T b_c mod q_c (src/gpu_online.cu:23-41);

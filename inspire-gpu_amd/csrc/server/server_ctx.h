@@ -99,10 +99,9 @@ struct GpuServerCtx {
     int collapse_variant = 0;       // 17..32-query collapse pass form (launch_collapse)
     size_t gchunk = 0;              // groups per chunk of the pipelined answer
     // the pipelined answer's chunks: of gchunk groups, the lowest one split
-    // into gchunk/2, /4, /4 when
-    // tail_split (its Horner steps are the ones left after every pass), the
-    // highest one into gchunk/4, /4, /2 when head_split (the chains start
-    // after a quarter chunk's passes)
+    // into gchunk/2, /4, /4 when tail_split (its Horner steps are the ones
+    // left after every pass), the highest one into gchunk/4, /4, /2 when
+    // head_split (the chains start after a quarter chunk's passes)
     bool tail_split = true, head_split = false;
     ChunkLayout layout;
     void set_chunks();
@@ -121,7 +120,8 @@ struct GpuServerCtx {
     // server may stream at all (INSPIRE_STREAM). The workgroups of a streamed
     // answer hold their CUs while they wait; the device's lane sets are
     // shared by its servers and run one answer's chains at a time each, so
-    // at most kLanes answers wait, whatever servers they belong to.
+    // at most kLanes answers wait, whatever servers they belong to. What they
+    // wait for follows their release in its queue (lanes.h, QueueTurn).
     uint32_t stream_slices1 = 4, stream_slices = 4;
     // eighths of the groups (from the top) in a streamed pass's first
     // launch, the chains starting after it (0: one launch, chains at once)
@@ -189,8 +189,10 @@ struct GpuServerCtx {
     hipEvent_t pass_ev[kLanes] = {};                 // a split streamed pass's first launch done
     hipEvent_t horner_done[kLanes] = {};
     uint32_t* d_packed_b = nullptr;
-    // Horner: 1 = a workgroup pair per chain (one per limb) where its status
-    // is read, 0 and -1 = one workgroup per chain (faster everywhere)
+    // Horner kernel of chains that do not wait for a streamed pass: -1 = a
+    // workgroup pair per chain (one per limb) for up to kPairMaxChains of an
+    // answer, else one workgroup; 0 = one workgroup always; 1 = pairs
+    // always, except where nobody reads the call's status
     int horner_mode = -1;
     // pack kernel of pipelined chunks: 1 one workgroup per query, 0 a grid
     // over (group, limb), -1 one workgroup for one-query calls, 2 fused into
@@ -323,8 +325,8 @@ struct GpuServerCtx {
     // The chains of `count` queries in one launch and without waits, where a
     // wait of the lane's answer ended at its bound.
     void horner_again(size_t count, uint64_t* d_out, hipStream_t s, size_t slot0, int lane);
-    // Throw (and clear) if a pair chain of a call on `lane` reported a fault
-    // through its status word; the call's stream has been waited for.
+    // Throw (and clear) if a chain of a call on `lane` gave up its wait with a
+    // bound of zero (h_status); the call's stream has been waited for.
     void check_status(int lane);
     std::atomic<size_t> n_streamed{0};  // streamed sub-batches enqueued (a test counter)
     // row slices whose partials the last answer's first sub-batch left in
@@ -354,7 +356,7 @@ struct GpuServerCtx {
     // (device) on stream s, using slots [slot0, slot0 + count) and scratch
     // set `lane` (work that may overlap on the device uses distinct lanes).
     // status_read: the caller reads the lane's status word after the call
-    // (check_status), so the pair Horner kernel may be used.
+    // (check_status): the first kernel clears it.
     void enqueue(const QueryInput& in, size_t count, uint64_t* d_out, hipStream_t s, size_t slot0 = 0,
                  int lane = 0, bool status_read = false);
     // The same wholly on s and the lane's two side streams.
