@@ -105,8 +105,8 @@ int ipir_dbg_set_tail_split(ipir_server* srv, int on);
 int ipir_dbg_set_horner(ipir_server* srv, int mode);
 /* Bound of the pair kernel's partner wait, in loads (default 2^21, ~2 s, and
  * no more: larger values set the default, among them 2^26, which was the
- * default while the bound counted shorter sleeps); an answer in which a wait
- * ends at its bound is made again at its end.
+ * default while the bound counted shorter sleeps); a workgroup whose wait
+ * ends at its bound makes its chain alone.
  * 0 makes every pair chain report the bound exceeded at its first
  * exchange and stop (all kernels still end normally), and nothing is made
  * again: the response is all-ones words, the call that ran it returns 4 (the
@@ -115,8 +115,9 @@ int ipir_dbg_set_horner(ipir_server* srv, int mode);
 int ipir_dbg_set_horner_spin_limit(ipir_server* srv, uint32_t limit);
 uint32_t ipir_dbg_horner_spin_limit(const ipir_server* srv);
 /* The same bound for Horner chains waiting for a streamed database pass's
- * groups (default 2^23; 0: give up at once and report, as above; the pass
- * itself runs to its end). */
+ * groups (default 2^23, a second or more); an answer in which one ends at its
+ * bound is packed and chained again at its end. 0: give up at once and
+ * report, as above; the pass itself runs to its end. */
 int ipir_dbg_set_stream_spin_limit(ipir_server* srv, uint32_t limit);
 /* 1 if chains of an answer were made again since the last call because a
  * wait inside a kernel ended at its bound, else 0 (-1: no server). Read it

@@ -955,7 +955,6 @@ int ipir_dbg_profile_batch(ipir_server* srv, const uint64_t* d_queries, size_t c
         mark();
         c->horner_range(count, d_out, 0, c->G, s, 0, 0, c->use_pair(count, true));
         mark();
-        if (c->use_pair(count, true) && c->horner_spin_limit) c->horner_again(count, d_out, s, 0, 0);
         c->order_after(s);
         hip_check(hipEventSynchronize(ev[k - 1]), "sync");
         c->check_status(0);

@@ -290,9 +290,10 @@ hipError_t launch_horner(const uint32_t* pa_base, size_t pa_stride, size_t G, si
 // The same chains with two workgroups per chain (one per limb) exchanging
 // shares of the CRT lift once per step through xbuf,
 // horner_pair_xbuf_words(nq*T) words that are zero before a chain's first
-// launch. A partner wait of more than spin_limit loads sets *status to 1 and
-// makes the chain's output all-ones words. spin_limit 0 does so at the first
-// exchange.
+// launch. A workgroup that waits for more than spin_limit loads sets *status
+// to 1 and makes its chain alone, from the highest group (the packed parts of
+// all groups from g_lo up are read). spin_limit 0: it sets *status at the
+// first exchange and makes the chain's output all-ones words.
 size_t horner_pair_xbuf_words(size_t nchains);
 hipError_t launch_horner_pair(const uint32_t* pa_base, size_t pa_stride, size_t G, size_t Da, size_t T,
                               const uint32_t* packed_b, size_t packed_stride, const uint32_t* rgsw,

@@ -32,12 +32,16 @@
 // partner's step n + 1, which the partner's lanes store after they have read
 // step n. The words must hold no number of this chain's steps beforehand
 // (they are zeroed in the answer's preparation launch).
-// The wait is bounded: a workgroup whose wait exceeds the bound sets
-// *status, fills its limb of the response with all-ones words (no residue;
-// where the chain continues in a later launch, of the state, which passes
-// them on) and ends; its partner's wait then ends the same way (a bound of
-// zero takes that path at the first exchange). The answer then makes its
-// chains again (HornerAgain).
+// The wait is bounded: a workgroup whose wait exceeds the bound (its partner
+// has not had a CU for that long) sets *status and makes the whole chain, from
+// its highest group, by itself: both limbs' polynomials in turn through the
+// same buffers, the twiddles staged anew for each. It writes its own limb
+// only, as ever, so its partner, whose wait then ends the same way, may run
+// at any time. (The kernel takes 176 VGPRs with that path and 158 without:
+// one workgroup to a CU either way.)
+// With a bound of zero (to see chains give up) a workgroup fills its limb of
+// the response with all-ones words instead (no residue; where the chain
+// continues in a later launch, of the state, which passes them on).
 #include "kernels.h"
 #include "ntt_regs.h"
 
@@ -101,6 +105,7 @@ __global__ __launch_bounds__(512, 2) void k_horner_pair(const uint32_t* __restri
     };
     uint32_t acc[1][8];  // slots 8t + k
     int first;
+    bool alone = false;
     if (top < g_hi) {  // the chain starts here: acc = packed[top]
         load8(acc[0], pk + (size_t)top * pk_stride);
         first = (int)top - 1;
@@ -173,8 +178,12 @@ __global__ __launch_bounds__(512, 2) void k_horner_pair(const uint32_t* __restri
             }
             lds_barrier();
             if (abort_flag) {
-                give_up();
-                return;
+                if (spin_limit == 0) {
+                    give_up();
+                    return;
+                }
+                alone = true;
+                break;
             }
             uint32_t x[2][8];  // digit polynomials: residues + q mod this limb's prime
 #pragma unroll
@@ -199,6 +208,79 @@ __global__ __launch_bounds__(512, 2) void k_horner_pair(const uint32_t* __restri
             lds_barrier();
 #pragma unroll
             for (int k = 0; k < 8; k++) acc[0][k] = mine[k] + sx[1 - p][k][t] + pv[k];  // below 5.2q
+        }
+        if (alone) {
+            // this team's part of both limbs, canonical between steps
+            uint32_t a0[8], a1[8];
+            auto load_limb = [&](uint32_t (&x)[8], const uint32_t* src, int l) {
+#pragma unroll
+                for (int k = 0; k < 8; k++) x[k] = src[(size_t)l * N + 8 * t + k];
+            };
+            load_limb(a0, pk + (size_t)top * pk_stride, 0);
+            load_limb(a1, pk + (size_t)top * pk_stride, 1);
+#pragma unroll 1
+            for (int gs = (int)top - 1; gs >= (int)lo; gs--) {
+                uint32_t s0[8], s1[8];  // shares of the lift, then the digits
+#pragma unroll 1
+                for (int half = 0; half < 4; half++) {  // inverse of limb 0, 1, then products mod limb 0, 1
+                    const int l = half & 1;
+                    const NrLimb ml = nr_limb(l);
+                    __syncthreads();  // the last transform's twiddles and products are read
+                    for (uint32_t x = tid; x < N; x += 512) {
+                        const uint32_t* f = nc.tw + (size_t)l * 4 * N;
+                        tw[x] = nr_u32x2{f[x], f[N + x]};
+                    }
+                    __syncthreads();
+                    if (half < 2) {
+                        uint32_t cf[1][8];
+#pragma unroll
+                        for (int k = 0; k < 8; k++) cf[0][k] = l ? a1[k] : a0[k];
+                        nr_inverse<1, 6>(cf, buf[p], tw, t, ml);
+#pragma unroll
+                        for (int k = 0; k < 8; k++) {
+                            const uint32_t v = nr_crt_part(cf[0][k], gc, l, ml);
+                            s0[k] = l ? s0[k] : v;
+                            s1[k] = l ? v : s1[k];
+                        }
+                        if (half == 0) continue;
+#pragma unroll
+                        for (int k = 0; k < 8; k++) {
+                            const nr_u32x2 d = nr_digits(s0[k], s1[k]);
+                            s0[k] = d.x;
+                            s1[k] = d.y;
+                        }
+                        continue;
+                    }
+                    uint32_t x[2][8];
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {
+                        x[0][k] = s0[k] + (ml.q - (1u << 17));
+                        x[1][k] = s1[k] + ml.q;
+                    }
+                    nr_forward<2>(x, buf[p], tw, t, ml, [] { lds_barrier(); });
+                    uint32_t pv[8];
+                    load_limb(pv, pk + (size_t)gs * pk_stride, l);
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {
+#pragma unroll
+                        for (int j = 0; j < 2; j++) x[j][k] = fold(nr_reduce(x[j][k], ml), ml.q);
+                        const uint32_t* r = rg + (size_t)l * N + 8 * t + k;
+                        const uint32_t ta = red64((uint64_t)x[0][k] * r[0] + (uint64_t)x[1][k] * r[2 * N], l);
+                        const uint32_t tb = red64((uint64_t)x[0][k] * r[BLK] + (uint64_t)x[1][k] * r[BLK + 2 * N], l);
+                        pv[k] = add_mod(pv[k], p ? tb : ta, ml.q);
+                        sx[p][k][t] = p ? ta : tb;
+                    }
+                    __syncthreads();
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {
+                        const uint32_t v = add_mod(pv[k], sx[1 - p][k][t], ml.q);
+                        a0[k] = l ? a0[k] : v;
+                        a1[k] = l ? v : a1[k];
+                    }
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 8; k++) acc[0][k] = c ? a1[k] : a0[k];
         }
 #pragma unroll
         for (int k = 0; k < 8; k++) acc[0][k] = fold(fold(fold(acc[0][k], 4 * m.q), 2 * m.q), m.q);

@@ -1023,7 +1023,7 @@ void GpuServerCtx::horner_range(size_t count, uint64_t* d_out, size_t g_lo, size
         HIPX(launch_horner_pair(d_precomp + PC_A, PC_GROUP, G, Da, T, d_packed_b + slot0 * packed_stride,
                                 packed_stride, d_rgsw + slot0 * rgsw_stride, rgsw_stride, d_out,
                                 d_hstate + slot0 * T * 4 * N, g_lo, g_hi, count,
-                                d_hxbuf + horner_pair_xbuf_words(slot0 * T), wait_status(lane, horner_spin_limit),
+                                d_hxbuf + horner_pair_xbuf_words(slot0 * T), horner_spin_limit ? h_status + kLanes : h_status + lane,
                                 horner_spin_limit, nc, cc, s));
     else
         HIPX(launch_horner(d_precomp + PC_A, PC_GROUP, G, Da, T, d_packed_b + slot0 * packed_stride, packed_stride,
@@ -1105,22 +1105,14 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
     // device (at 128 GB, 4 x 128 chains in two rounds over the 256 CUs
     // instead of four rounds over 128). Contiguous slots [defer_lo, +defer_n).
     size_t defer_lo = 0, defer_n = 0;
-    // The answer's last launches: sub-batches whose chains wait inside their
-    // kernels are made again where a wait ended at its bound (d_gave_up), so
-    // that bound is no limit to what the device may run beside an answer. A
-    // launch that finds the word at zero takes 2 to 3 us (1 GB, one query 297.5 to
-    // 299.2, 32 queries 370.8 to 374.2; pairs still pay from one step on: two
-    // groups 91.0 single, 87.7 in pairs).
+    // The answer's last launches: streamed sub-batches are packed and chained
+    // again where a wait ended at its bound (d_gave_up), so that bound is no
+    // limit to what the device may run beside an answer. A launch that finds
+    // the word at zero takes 2 to 3 us of an answer of a millisecond or more.
     std::vector<std::function<void()>> again;
-    auto chains_again = [&](size_t q0, size_t nq) {
-        if (pair && horner_spin_limit)
-            again.push_back([=] { horner_again(nq, d_out + (q0 - slot0) * resp_u64s, s, q0, lane); });
-    };
     auto flush_deferred = [&]() {
-        if (defer_n) {
+        if (defer_n)
             horner_range(defer_n, d_out + (defer_lo - slot0) * resp_u64s, 0, G, s, defer_lo, lane, pair);
-            chains_again(defer_lo, defer_n);
-        }
         defer_n = 0;
     };
     for (size_t q0 = slot0; q0 < slot0 + count; q0 += kMfmaMaxQueries) {
@@ -1236,7 +1228,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             pk.pass_target = fused ? pass_collapse_target(sp, nq, G) : (uint32_t)(N / dbplan_cols(sp) * sp.slices);
             pk.packed_done = packed_done;
             pk.spin_limit = stream_spin_limit;
-            pk.status = wait_status(lane, stream_spin_limit);
+            pk.status = stream_spin_limit ? d_gave_up + lane : h_status + lane;
             pk.queries = pq;
             HIPX(launch_pack_stream(pk, p2, part2_stride, d_precomp, keys, keys_stride, packed, packed_stride, G, nq,
                                     nc, ps_s));
@@ -1247,7 +1239,7 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
             sw.queries = pq;
             sw.stride = (uint32_t)G;
             sw.spin_limit = stream_spin_limit;
-            sw.status = wait_status(lane, stream_spin_limit);
+            sw.status = pk.status;
             HIPX(launch_horner(d_precomp + PC_A, PC_GROUP, G, Da, T, packed, packed_stride, d_rgsw + q0 * rgsw_stride,
                                rgsw_stride, out, d_hstate + q0 * T * 4 * N, 0, G, nq, nc, cc, hs, FusedPack{}, sw));
             // the next sub-batch's key digits and flags wait for the collapse and the pack
@@ -1383,7 +1375,6 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
                                           keys, keys_stride, packed, packed_stride, nq, nc, ks));
             horner_range(nq, out, g_lo, g_hi, ks, q0, lane, pair, fuse ? &fp : nullptr);
         }
-        chains_again(q0, nq);
         if (cs != s) {  // the next batch's key digits overwrite the lane's scratch
             HIPX(hipEventRecord(prep_ev[lane], cs));
             stream_wait(s, prep_ev[lane]);

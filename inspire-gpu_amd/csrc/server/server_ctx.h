@@ -200,16 +200,16 @@ struct GpuServerCtx {
     int pack_wg = 0;
     uint32_t* d_hxbuf = nullptr;    // pair exchange buffers [B*T chains]
     // Waits inside a kernel (a pair chain's for its partner, a streamed pack's
-    // or chain's for its pass) are bounded. Per scratch lane, d_gave_up is
-    // zeroed by an answer's first kernel and set by a wait that ends at its
-    // bound; the answer's last launches make its waiting sub-batches again,
-    // without waits, where it is set, and set h_status[kLanes] (pinned host
-    // memory). With a bound of zero (chains that end at once, for tests)
-    // nothing is made again, the report goes to h_status[lane], and
-    // check_status reads and clears it.
+    // or chain's for its pass) are bounded. A pair's workgroup whose wait ends
+    // at its bound makes the chain alone (kernels_horner.hip). Streamed: per
+    // scratch lane, d_gave_up is zeroed by an answer's first kernel and set by
+    // such a wait, and the answer's last launches make its streamed
+    // sub-batches again, without waits, where it is set. Both then set
+    // h_status[kLanes] (pinned host memory). With a bound of zero (chains
+    // that end at once, for tests) nothing is made again, the report goes to
+    // h_status[lane], and check_status reads and clears it.
     uint32_t* d_gave_up = nullptr;  // [kLanes]
     uint32_t* h_status = nullptr;   // [kLanes + 1]
-    uint32_t* wait_status(int lane, uint32_t limit) const { return limit ? d_gave_up + lane : h_status + lane; }
     uint32_t horner_spin_limit = 0; // the pair kernel's wait bound in loads (0: report at once)
     uint32_t stream_spin_limit = 0; // the same for chains waiting for a streamed pass's groups
     uint32_t* d_hstate = nullptr;   // Horner chain state between chunk launches [B*T][4][N]
@@ -323,7 +323,7 @@ struct GpuServerCtx {
     void horner_range(size_t count, uint64_t* d_out, size_t g_lo, size_t g_hi, hipStream_t s, size_t slot0,
                       int lane, bool pair, const ipx::FusedPack* fp = nullptr);
     // The chains of `count` queries in one launch and without waits, where a
-    // wait of the lane's answer ended at its bound.
+    // streamed wait of the lane's answer ended at its bound.
     void horner_again(size_t count, uint64_t* d_out, hipStream_t s, size_t slot0, int lane);
     // Throw (and clear) if a chain of a call on `lane` gave up its wait with a
     // bound of zero (h_status); the call's stream has been waited for.

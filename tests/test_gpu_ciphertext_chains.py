@@ -40,5 +40,11 @@ def test_chunked_answers_of_several_ciphertexts(cts):
                     for order in ([0, 1, 2], [2, 0, 1], [1]):  # other queries in the same slots
                         got = srv.answer_batch([qs[j] for j in order])
                         assert np.array_equal(got, want[order]), (shape, split, mode, order)
+        # pairs that do not wait for their partner: each workgroup makes its chain alone
+        assert lib.ipir_dbg_set_horner_spin_limit(srv.h, 1) == 0
+        for shape in (0, 2, 3):
+            assert lib.ipir_dbg_set_pipeline(srv.h, shape, shape) == 0
+            print(f"[{cts} cts] shape {shape}, bound of one load", flush=True)
+            assert np.array_equal(srv.answer_batch(list(qs)), want), f"alone, shape {shape}"
     finally:
         srv.close()

@@ -1,5 +1,6 @@
-"""Waits inside kernels end at a bound: an answer in which one does is made
-again before its stream goes on."""
+"""Waits inside kernels end at a bound: a pair's workgroup then makes its chain
+alone, and a streamed answer is packed and chained again before its stream
+goes on."""
 import ctypes as C
 
 import numpy as np
