@@ -410,8 +410,6 @@ void GpuServerCtx::alloc_slots() {
     trace_name_stream(stream, "server");
     static_assert(kLanes == kLaneSets, "a lane set per scratch lane");
     lane_first = acquire_lanes(device, lanes);
-    HIPX(hipStreamCreate(&capture_horner));
-    HIPX(hipStreamCreate(&capture_side));
     for (int l = 0; l < kLanes; l++) {
         HIPX(hipEventCreateWithFlags(&hop_in_ev[l], hipEventDisableTiming));
         HIPX(hipEventCreateWithFlags(&hop_out_ev[l], hipEventDisableTiming));
@@ -1086,7 +1084,12 @@ void GpuServerCtx::enqueue_on(const QueryInput& input, size_t count, uint64_t* d
     // Side streams: the lane's, or under capture the server's own pair (a
     // shared stream must not join one server's capture while others use it).
     hipStream_t hs = lanes[lane].horner, ps_side = lanes[lane].side;
+    // Made by the first captured answer: made with the server, they changed
+    // which hardware queues later servers' streams fall on (chunked answers
+    // of two ciphertexts in a process's second server 6130 -> 6350 us).
     if (is_capturing(s)) {
+        if (!capture_horner) HIPX(hipStreamCreate(&capture_horner));
+        if (!capture_side) HIPX(hipStreamCreate(&capture_side));
         hs = capture_horner;
         ps_side = capture_side;
     }
