@@ -220,7 +220,7 @@ __global__ __launch_bounds__(512, 2) void k_horner_pair(const uint32_t* __restri
             load_limb(a1, pk + (size_t)top * pk_stride, 1);
 #pragma unroll 1
             for (int gs = (int)top - 1; gs >= (int)lo; gs--) {
-                uint32_t s0[8], s1[8];  // shares of the lift, then the digits
+                uint32_t s0[8] = {}, s1[8] = {};  // shares of the lift, then the digits
 #pragma unroll 1
                 for (int half = 0; half < 4; half++) {  // inverse of limb 0, 1, then products mod limb 0, 1
                     const int l = half & 1;
